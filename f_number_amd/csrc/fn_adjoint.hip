@@ -329,7 +329,8 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(const float *__rest
         re += P[base + off_re];
         im += P[base + off_im];
     }
-    Z[((size_t)b * n_tx + a) * n_el + k] = make_float2(re, im);
+    // the truncated phases' mean rotation, conjugate to the forward kernels' (PHASE_BACK)
+    Z[((size_t)b * n_tx + a) * n_el + k] = make_float2(fmaf(PHASE_BACK, im, re), fmaf(-PHASE_BACK, re, im));
 }
 
 // (A^H y)[ch][t] = Re sum_b Z[b][ch] e^{+j 2 pi (n_lb + b) t / N}, ch = a n_el + k, as a

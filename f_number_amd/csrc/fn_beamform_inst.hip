@@ -124,8 +124,9 @@ hipError_t FN_LBL_LAUNCHER(INST_KI)(int wcr, dim3 grid, hipStream_t s, const Bea
 #endif
 
 #if INST_MODE == 0 && !FN_WIDE
-// ensemble variant: frames x angles as transmit rows, up to four tiles per group (fp16
-// at 128 elements up to eight)
+// ensemble variant: frames x angles as transmit rows, up to four tiles per group (FP32 and
+// the fp16 split at 128 elements five, fp16 eight).  FP32: the linear class only (FP32
+// plans of every other window run the fp16 split)
 #define FN_ENS_LAUNCHER(k, p) FN_CAT6(launch_beamform_ens, _k, k, _p, p, )
 template <int MT, int WCR, bool STK>
 static hipError_t launch_ens_one(dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
@@ -142,12 +143,17 @@ template <int MT, bool STK>
 static hipError_t launch_ens_mt(int wcr, dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
 {
     switch (wcr) {
-    case WC_RANGE: return launch_ens_one<MT, WC_RANGE, STK>(grid, lds, s, A);
     case WC_LINEAR: return launch_ens_one<MT, WC_LINEAR, STK>(grid, lds, s, A);
+#if INST_PREC == 0
+    default: return hipErrorInvalidValue;
+    }
+#else
+    case WC_RANGE: return launch_ens_one<MT, WC_RANGE, STK>(grid, lds, s, A);
     case WC_COS_ALL: return launch_ens_one<MT, WC_COS_ALL, STK>(grid, lds, s, A);
     case WC_COS_RF: return launch_ens_one<MT, WC_COS_RF, STK>(grid, lds, s, A);
     default: return launch_ens_one<MT, WC_COS, STK>(grid, lds, s, A);
     }
+#endif
 }
 
 // stack != 0: a row stack (rows of several acquisitions, each its own transmit phase)
@@ -172,8 +178,8 @@ hipError_t FN_ENS_LAUNCHER(INST_KI, INST_PREC)(int mt, int wcr, dim3 grid, size_
     case 2: return launch_ens_mt<2, false>(wcr, grid, lds, s, A);
     case 3: return launch_ens_mt<3, false>(wcr, grid, lds, s, A);
     case 4: return launch_ens_mt<4, false>(wcr, grid, lds, s, A);
-#if INST_PREC == 0 && INST_KI == 32
-    // FP32 at 128 elements: 5 tiles (the default)
+#if (INST_PREC == 0 || INST_PREC == 2) && INST_KI == 32
+    // FP32 plans at 128 elements (in either form): 5 tiles
     case 5: return launch_ens_mt<5, false>(wcr, grid, lds, s, A);
 #endif
 #if INST_PREC == 3 && INST_KI == 32
@@ -237,7 +243,7 @@ hipError_t FN_LAUNCHER(INST_MODE, INST_KI, INST_PREC)(int mt, int wcr, int wct, 
 #endif
 
 #if !FN_WIDE
-// persistent batch launches: one kernel per class over the work items of many
+// persistent batch launches (FP32: the linear class only, as above): one kernel per class over the work items of many
 // plans (grid <= 0: only report the resident workgroups per CU in *occupancy)
 #define FN_PERSIST_LAUNCHER(m, k, p) FN_CAT6(launch_beamform_persistent_m, m, _k, k, _p, p)
 template <int MT, int WCR, int WCT>
@@ -264,12 +270,17 @@ static hipError_t launch_persist_wcr(int wcr, int grid, size_t lds, hipStream_t 
                                      const int4 *items, int n_items, int *counter, int *occ)
 {
     switch (wcr) {
-    case WC_RANGE: return launch_persist_one<MT, WC_RANGE, WCT>(grid, lds, s, jobs, items, n_items, counter, occ);
     case WC_LINEAR: return launch_persist_one<MT, WC_LINEAR, WCT>(grid, lds, s, jobs, items, n_items, counter, occ);
+#if INST_PREC == 0
+    default: return hipErrorInvalidValue;
+    }
+#else
+    case WC_RANGE: return launch_persist_one<MT, WC_RANGE, WCT>(grid, lds, s, jobs, items, n_items, counter, occ);
     case WC_COS_ALL: return launch_persist_one<MT, WC_COS_ALL, WCT>(grid, lds, s, jobs, items, n_items, counter, occ);
     case WC_COS_RF: return launch_persist_one<MT, WC_COS_RF, WCT>(grid, lds, s, jobs, items, n_items, counter, occ);
     default: return launch_persist_one<MT, WC_COS, WCT>(grid, lds, s, jobs, items, n_items, counter, occ);
     }
+#endif
 }
 
 hipError_t FN_PERSIST_LAUNCHER(INST_MODE, INST_KI, INST_PREC)(int mt, int wcr, int wct, int grid, size_t lds,

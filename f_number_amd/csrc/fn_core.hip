@@ -35,7 +35,7 @@ FN_DECL_LAUNCHERS(0, 64)
 FN_DECL_LAUNCHERS(1, 48)
 FN_DECL_LAUNCHERS(1, 64)
 #undef FN_DECL_LAUNCHERS
-#define FN_DECL_ENS(k)                                                                              \
+#define FN_DECL_ENS(k)                                                                                  \
     hipError_t launch_beamform_ens_k##k##_p0(int, int, dim3, size_t, hipStream_t, const BeamArgs &, int); \
     hipError_t launch_beamform_ens_k##k##_p1(int, int, dim3, size_t, hipStream_t, const BeamArgs &, int); \
     hipError_t launch_beamform_ens_k##k##_p2(int, int, dim3, size_t, hipStream_t, const BeamArgs &, int); \
@@ -46,7 +46,7 @@ FN_DECL_ENS(32)
 #undef FN_DECL_ENS
 // the last argument: 1 for a row stack (per-row transmit phases), 0 for an ensemble
 typedef hipError_t (*EnsLauncher)(int, int, dim3, size_t, hipStream_t, const BeamArgs &, int);
-// [KI = 8, 16, 32][precision]
+// [KI = 8, 16, 32][form of the contraction] (FP32: the windows the fp16 split is not for)
 static const EnsLauncher kEnsLaunchers[3][4] = {
     {launch_beamform_ens_k8_p0, launch_beamform_ens_k8_p1, launch_beamform_ens_k8_p2, launch_beamform_ens_k8_p3},
     {launch_beamform_ens_k16_p0, launch_beamform_ens_k16_p1, launch_beamform_ens_k16_p2, launch_beamform_ens_k16_p3},
@@ -146,7 +146,8 @@ struct fn_plan {
     float2 *d_sigF = nullptr;   // focused spectrum of the signal voxel [n_f]
     std::vector<double> h_px, h_pz, h_Frx, h_Ftx, h_sqf;  // host copies (signal voxel search)
     std::vector<double> h_delay;                          // delay offsets of the last set_tof (empty: zeros)
-    int precision = FN_PRECISION_FP32;
+    int precision = FN_PRECISION_FP32;  // as asked for
+    int kprec = FN_PRECISION_FP32;      // form of the forward contraction (kernel_precision)
     int verbosity = 0;
     fnk::BeamArgs args{};
     fnk::SpecArgs sargs{};
@@ -234,7 +235,7 @@ int select_device(int index)
 int setup_window(const fn_window &w, int semantics, fnk::WinCoef *c, int *wc, int *support)
 {
     const bool cpu = semantics == FN_SEMANTICS_CPU;
-    *c = fnk::WinCoef{-1.f, INFINITY, 0.f, 1.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    *c = fnk::WinCoef{-1.f, INFINITY, 0.f, 1.f, 0.f, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f};
     switch (w.id) {
     case FN_WINDOW_BOXCAR:
         *wc = fnk::WC_RANGE;
@@ -275,7 +276,7 @@ int setup_window(const fn_window &w, int semantics, fnk::WinCoef *c, int *wc, in
 // coefficients (|t|: flat part, A + C t + B cos(2 pi (t - t_off) s_half), cut)
 int taper_coef(const fn_window &w, fnk::WinCoef *c)
 {
-    *c = fnk::WinCoef{-1.f, INFINITY, 0.f, 1.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    *c = fnk::WinCoef{-1.f, INFINITY, 0.f, 1.f, 0.f, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f};
     switch (w.id) {
     case FN_WINDOW_BOXCAR: c->t_cut = 1.f; return FN_OK;                       // |t| < 1
     case FN_WINDOW_HANN: c->A = c->B = 0.5f; c->s_half = 0.5f; return FN_OK;   // untruncated
@@ -340,7 +341,6 @@ int wcr_general(int wcr) { return (wcr == fnk::WC_COS_ALL || wcr == fnk::WC_COS_
 
 // default transmit tiles per plane-wave workgroup that fit the register file:
 // ensembles hold per-row image accumulators, so 4; FP32 and fp16 at 128 elements 5
-// (FP32 with one 8-byte reload per bin from scratch in the full-array cosine class)
 int tile_cap(int n_frames, int precision, int KI)
 {
     if (n_frames <= 1) return 5;
@@ -350,6 +350,32 @@ int tile_cap(int n_frames, int precision, int KI)
 
 // transmit tiles per group of a row stack (its own kernel instances, per-row phases)
 int stack_tile_cap(int precision, int KI) { return (precision == FN_PRECISION_FP16 && KI == 32) ? 5 : 4; }
+
+// a receive window without a cut and not a cosine: its weights grow with the element distance
+bool unbounded_window(int wcr, const fnk::WinCoef &w) { return wcr == fnk::WC_LINEAR && std::isinf(w.t_cut); }
+
+// Form of the forward contraction.  FP32 plans run the fp16 hi + lo split: its operands
+// carry 22-23 bits and its products accumulate in FP32, so its error against 64 bits is that
+// of the FP32 products (11 angles, Tukey: 4.9e-7 both; 75 angles, Hann: 2.3e-7 and 2.2e-7;
+// synthetic aperture: 5.7e-7 and 5.6e-7), and it takes 12 matrix-core instructions of 16
+// cycles per 32 elements and tile against 24 of 32 (75 angles at 1024 x 512: 174.6 ms
+// against 422.5; 11 angles at 256 x 256: 3.1 against 4.5; synthetic aperture at 512 x 512:
+// 94 against 168).  The synthetic aperture beyond 128 elements keeps the FP32 kernel, which
+// is the faster there (192 elements, 128 x 256: 54 ms against 65); the windowed
+// normalization and line scans (no matrix product) have FP32 kernels only.
+int kernel_precision(const fn_plan *P, int precision)
+{
+    if (precision == FN_PRECISION_FP32 && !P->nw && !P->lbl && (P->KI <= 32 || P->mode == 0) &&
+        !unbounded_window(P->wcr, P->args.wrx))
+        return FN_PRECISION_FP16X3;
+    return precision;
+}
+
+int form_planes(int kprec) { return kprec == FN_PRECISION_FP16 ? 2 : 4; }
+
+// staged spectra bytes per M-tile and element step: FP32 interleaved complex, or 16-bit
+// planes (Xr, Xi and, for the split forms, their residuals)
+size_t form_step_bytes(int kprec) { return kprec == FN_PRECISION_FP32 ? 64 * sizeof(float2) : (size_t)form_planes(kprec) * 64 * 2; }
 
 // element steps per lane: 4 KI >= n_el elements in four lane groups
 int ki_of(int n_el)
@@ -411,8 +437,9 @@ static bool few_rows_pw(const fn_plan *P)
 
 // shared configuration of plan creation: tiling, launch shape and the scalar
 // arguments of the kernels; no device work and no allocation (the
-// no-allocation entry point runs it on a plan held on the stack)
-int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g)
+// no-allocation entry point runs it on a plan held on the stack, with plain_fp32 where its
+// scratch has no room for the split form's planes)
+int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, bool plain_fp32 = false)
 {
     if (c.precision < FN_PRECISION_FP32 || c.precision > FN_PRECISION_FP16)
         return fail(FN_ERR_ARGUMENT, "unknown precision %d", c.precision);
@@ -423,6 +450,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g)
     P->verbosity = c.verbosity;
     P->precision = c.precision;
     P->KI = ki_of(c.n_el);
+    P->kprec = plain_fp32 ? c.precision : kernel_precision(P, c.precision);
     if (!P->KI) return fail(FN_ERR_UNSUPPORTED, "at most 256 array elements are supported (got %d)", c.n_el);
     if (P->KI > 32) {
         // beyond 128 elements: the one-launch forward kernel of single-frame plans
@@ -443,7 +471,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g)
     } else if (P->mode == 0) {
         // at most 5 transmit tiles per group keep the LDS tile within 80 KiB
         // (ensembles: 4-5, for the per-row image accumulators)
-        const int max_tiles = P->nw ? 2 : std::min(tile_cap(P->n_frames, c.precision, P->KI), pw_mt_wide(P->KI));
+        const int max_tiles = P->nw ? 2 : std::min(tile_cap(P->n_frames, P->precision, P->KI), pw_mt_wide(P->KI));
         const int groups = (P->MT_all + max_tiles - 1) / max_tiles;
         P->MT_tmpl = (P->MT_all + groups - 1) / groups;
         P->n_groups = (P->MT_all + P->MT_tmpl - 1) / P->MT_tmpl;
@@ -451,10 +479,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g)
         P->MT_tmpl = sa_mt(P->KI);
         P->n_groups = (P->MT_all + P->MT_tmpl - 1) / P->MT_tmpl;
     }
-    // staged spectra per bin: FP32 interleaved complex (8 bytes per value) or
-    // 16-bit planes (Xr, Xi and, for the split forms, their residuals)
-    const int planes = c.precision == FN_PRECISION_FP16 ? 2 : 4;
-    const size_t step_bytes = c.precision == FN_PRECISION_FP32 ? 64 * sizeof(float2) : (size_t)planes * 64 * 2;
+    const size_t step_bytes = form_step_bytes(P->kprec);
     P->lds_beam = (size_t)P->MT_tmpl * P->KI * step_bytes;
     P->lds_spec = (size_t)g.N * sizeof(float2) + 64 * 65 * sizeof(float);
     if (P->lds_beam > kMaxLds) return fail(FN_ERR_UNSUPPORTED, "transmit tile exceeds LDS");
@@ -485,7 +510,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g)
     const int chunk = (g.n_f + split - 1) / split;
     P->bin_split = (g.n_f + chunk - 1) / chunk;
     P->x_bytes = (size_t)g.n_f * P->MT_all * P->KI * 64 * sizeof(float2);
-    if (c.precision != FN_PRECISION_FP32) P->xlp_bytes = (size_t)g.n_f * planes * P->MT_all * P->KI * 64 * 2;
+    P->xlp_bytes = P->kprec != FN_PRECISION_FP32 ? (size_t)g.n_f * form_planes(P->kprec) * P->MT_all * P->KI * 64 * 2 : 0;
 
     fnk::BeamArgs &A = P->args;
     A.ctof = c.c0;
@@ -541,7 +566,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     if ((s = upload(&P->d_tw, tw.data(), tw.size(), "twiddles"))) return s;
     HIP_CHECK(hipMalloc(&P->d_X, P->x_bytes), "spectra workspace");
     HIP_CHECK(hipMemset(P->d_X, 0, P->x_bytes), "spectra workspace");  // padding rows stay zero
-    if (c.precision != FN_PRECISION_FP32) {
+    if (P->kprec != FN_PRECISION_FP32) {
         HIP_CHECK(hipMalloc(&P->d_Xlp, P->xlp_bytes), "16-bit spectra planes");
         HIP_CHECK(hipMalloc(&P->d_xscale, (size_t)g.n_f * sizeof(float)), "spectra scales");
     }
@@ -614,8 +639,8 @@ hipError_t launch_beam(const fn_plan *P, dim3 grid, const fnk::BeamArgs &A, hipS
     const int kidx = ki_index(P->KI);  // ensembles, line scans and windowed plans stop at KI = 32
     if (P->lbl) return fnk::kLblLaunchers[kidx](P->wcr, grid, s, A);
     if (P->nw) return fnk::kNwLaunchers[P->mode][kidx](P->MT_tmpl, P->wcr, P->wct, grid, P->lds_beam, s, A);
-    if (P->n_frames > 1) return fnk::kEnsLaunchers[kidx][P->precision](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A, 0);
-    return fnk::kBeamLaunchers[P->mode][kidx][P->precision](P->MT_tmpl, P->wcr, P->wct, grid, P->lds_beam, s, A);
+    if (P->n_frames > 1) return fnk::kEnsLaunchers[kidx][P->kprec](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A, 0);
+    return fnk::kBeamLaunchers[P->mode][kidx][P->kprec](P->MT_tmpl, P->wcr, P->wct, grid, P->lds_beam, s, A);
 }
 
 // raise a kernel's dynamic-LDS limit once per process and size (no attribute
@@ -656,10 +681,25 @@ int launch_spectra(fn_plan *P, const void *d_rf, int dtype, hipStream_t s)
     return launch_spectra_into(P, d_rf, dtype, s, P->d_X, P->sargs);
 }
 
+// the arguments of the forward kernels: the fp16 split evaluates a bounded receive window
+// times an exact factor (SPLIT_PEAK)
+fnk::BeamArgs forward_args(const fn_plan *P)
+{
+    fnk::BeamArgs A = P->args;
+    if (P->kprec == FN_PRECISION_FP16X3 && !unbounded_window(P->wcr, A.wrx)) {
+        A.wrx.A *= fnk::SPLIT_PEAK;
+        A.wrx.B *= fnk::SPLIT_PEAK;
+        A.wrx.C *= fnk::SPLIT_PEAK;
+        A.wrx.peak = fnk::SPLIT_PEAK;
+        A.wrx.inv_peak = 1.0f / fnk::SPLIT_PEAK;
+    }
+    return A;
+}
+
 // the beamforming arguments of one execute (image and weight buffers)
 fnk::BeamArgs beam_args(const fn_plan *P, float *d_image, float *d_w, float *d_w_rx)
 {
-    fnk::BeamArgs A = P->args;
+    fnk::BeamArgs A = forward_args(P);
     A.image = reinterpret_cast<float2 *>(d_image);
     A.n_slots = beam_slots(P);
     A.slot_z = P->lbl ? 1 : P->n_groups;
@@ -718,7 +758,7 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
     }
     const fnk::SpecArgs &S = P->sargs;
     if (int st = launch_spectra(P, d_rf, dtype, s)) return st;
-    return launch_lowp_planes(P->precision, P->d_X, P->d_Xlp, P->d_xscale, S.n_f, S.MT, S.KI, s);
+    return launch_lowp_planes(P->kprec, P->d_X, P->d_Xlp, P->d_xscale, S.n_f, S.MT, S.KI, s);
 }
 
 int execute(fn_plan *P, const void *d_rf, int dtype, float *d_image, float *d_w, float *d_w_rx, hipStream_t user)
@@ -884,7 +924,7 @@ int max_tiles(const fn_plan *P)
     if (P->mode == 1) return sa_mt(P->KI);
     if (P->lbl) return 1;
     if (P->nw) return std::min(P->MT_all, 2);
-    if (P->n_frames > 1 && P->precision == FN_PRECISION_FP16 && P->KI == 32) return std::min(P->MT_all, 8);
+    if (P->n_frames > 1 && P->kprec == FN_PRECISION_FP16 && P->KI == 32) return std::min(P->MT_all, 8);
     return std::min(P->MT_all, std::min(tile_cap(P->n_frames, P->precision, P->KI), pw_mt_wide(P->KI)));
 }
 
@@ -899,9 +939,7 @@ int set_tiling(fn_plan *P, int mt, int split)
     const int n_f = P->g.n_f;
     if (split < 1 || split > n_f) return fail(FN_ERR_ARGUMENT, "bin_split must be in 1..%d", n_f);
     if (P->nw && split != 1) return fail(FN_ERR_ARGUMENT, "windowed normalization runs with bin_split 1");
-    const int planes = P->precision == FN_PRECISION_FP16 ? 2 : 4;
-    const size_t step_bytes = P->precision == FN_PRECISION_FP32 ? 64 * sizeof(float2) : (size_t)planes * 64 * 2;
-    const size_t lds = (size_t)mt * P->KI * step_bytes;
+    const size_t lds = (size_t)mt * P->KI * form_step_bytes(P->kprec);
     if (lds > kMaxLds) return fail(FN_ERR_ARGUMENT, "transmit tile exceeds LDS");
     const int chunk = (n_f + split - 1) / split;
     P->MT_tmpl = mt;
@@ -1466,28 +1504,36 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
     fn_plan P;
     Common c{};
     if ((st = configure_pw(&P, p, &c))) return st;
-    if ((st = configure_common(&P, c, g))) return st;
-    use_cos_all(&P);
     const int n_f = g.n_f, n_tx = c.n_tx, raw_per_tx = p->virtual_sources ? 2 : 1;
     Carve cv;
-    const size_t o_X = cv.take(P.x_bytes);
-    const size_t o_Xlp = cv.take(P.xlp_bytes);
-    const size_t o_xs = cv.take(P.precision != FN_PRECISION_FP32 ? (size_t)n_f * sizeof(float) : 0);
-    const size_t o_px = cv.take((size_t)c.n_x * sizeof(double));
-    const size_t o_pz = cv.take((size_t)c.n_z * sizeof(double));
-    const size_t o_F = cv.take((size_t)n_f * sizeof(double));
-    const size_t o_sqf = cv.take((size_t)n_f * sizeof(double));
-    const size_t o_raw = cv.take((size_t)n_tx * raw_per_tx * sizeof(double));
-    const size_t o_txp = cv.take((size_t)n_tx * 3 * sizeof(double));
-    const size_t o_tw = cv.take((size_t)g.N * sizeof(float2));
-    const size_t o_dl = cv.take((size_t)c.n_el * sizeof(double));
-    const int slots = beam_slots(&P);
-    const size_t o_pi = cv.take(slots > 1 ? (size_t)slots * P.n_vox * sizeof(float2) : 0);
+    size_t o_X = 0, o_Xlp = 0, o_xs = 0, o_px = 0, o_pz = 0, o_F = 0, o_sqf = 0, o_raw = 0, o_txp = 0, o_tw = 0, o_dl = 0,
+           o_pi = 0;
+    int slots = 1;
+    // an FP32 call whose split planes do not fit beside its spectra runs the FP32 kernels
+    for (bool plain_fp32 : {false, true}) {
+        if ((st = configure_common(&P, c, g, plain_fp32))) return st;
+        cv = Carve{};
+        o_X = cv.take(P.x_bytes);
+        o_Xlp = cv.take(P.xlp_bytes);
+        o_xs = cv.take(P.kprec != FN_PRECISION_FP32 ? (size_t)n_f * sizeof(float) : 0);
+        o_px = cv.take((size_t)c.n_x * sizeof(double));
+        o_pz = cv.take((size_t)c.n_z * sizeof(double));
+        o_F = cv.take((size_t)n_f * sizeof(double));
+        o_sqf = cv.take((size_t)n_f * sizeof(double));
+        o_raw = cv.take((size_t)n_tx * raw_per_tx * sizeof(double));
+        o_txp = cv.take((size_t)n_tx * 3 * sizeof(double));
+        o_tw = cv.take((size_t)g.N * sizeof(float2));
+        o_dl = cv.take((size_t)c.n_el * sizeof(double));
+        slots = beam_slots(&P);
+        o_pi = cv.take(slots > 1 ? (size_t)slots * P.n_vox * sizeof(float2) : 0);
+        if (cv.used <= kScratchBytes) break;
+    }
     if (cv.used > kScratchBytes)
         return fail(FN_ERR_UNSUPPORTED,
                     "fn_das_pw_noalloc: this call needs %zu bytes of device scratch, the entry point holds %zu "
                     "(spectra workspace %zu bytes); use a plan",
                     cv.used, kScratchBytes, P.x_bytes + P.xlp_bytes);
+    use_cos_all(&P);
     if ((st = select_device(p->index_gpu))) return st;
     unsigned char *base = nullptr;
     if ((st = scratch_on_device(p->index_gpu, &base))) return st;
@@ -1850,13 +1896,11 @@ static int batch_plan_stacks(fn_batch *b, float *const *d_images, std::vector<ch
         }
         const fn_plan *P0 = b->plans[i];
         r.MT_all = (r.rows + 15) / 16;
-        const int max_tiles = stack_tile_cap(P0->precision, P0->KI);  // the stack kernel's register budget
+        const int max_tiles = stack_tile_cap(P0->kprec, P0->KI);  // the stack kernel's register budget
         const int groups = (r.MT_all + max_tiles - 1) / max_tiles;
         r.MT_tmpl = (r.MT_all + groups - 1) / groups;
         r.n_groups = (r.MT_all + r.MT_tmpl - 1) / r.MT_tmpl;
-        const int planes = P0->precision == FN_PRECISION_FP16 ? 2 : 4;
-        const size_t step_bytes = P0->precision == FN_PRECISION_FP32 ? 64 * sizeof(float2) : (size_t)planes * 64 * 2;
-        r.lds_beam = (size_t)r.MT_tmpl * P0->KI * step_bytes;
+        r.lds_beam = (size_t)r.MT_tmpl * P0->KI * form_step_bytes(P0->kprec);
         // bin chunks: enough workgroups to fill the GPU several times over
         const long blocks = beam_tiles(P0) * r.n_groups;
         int split = 1;
@@ -1875,8 +1919,8 @@ static int batch_plan_stacks(fn_batch *b, float *const *d_images, std::vector<ch
         }
         hipError_t e = hipMalloc(&R.d_X, x_bytes);
         if (e == hipSuccess) e = hipMemset(R.d_X, 0, x_bytes);  // rows past the last plan stay zero
-        if (e == hipSuccess && P0->precision != FN_PRECISION_FP32) {
-            e = hipMalloc(&R.d_Xlp, n_f * planes * R.MT_all * P0->KI * 64 * 2);
+        if (e == hipSuccess && P0->kprec != FN_PRECISION_FP32) {
+            e = hipMalloc(&R.d_Xlp, n_f * form_planes(P0->kprec) * R.MT_all * P0->KI * 64 * 2);
             if (e == hipSuccess) e = hipMalloc(&R.d_xscale, n_f * sizeof(float));
         }
         if (e == hipSuccess) e = hipMalloc(&R.d_txp, 3 * sizeof(double) * R.rows);
@@ -1912,9 +1956,9 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
         S.write_pad = 0;
         if (int st = launch_spectra_into(P, d_rf[R.plans[m]], dtypes[R.plans[m]], s, R.d_X, S)) return st;
     }
-    if (int st = launch_lowp_planes(P0->precision, R.d_X, R.d_Xlp, R.d_xscale, P0->g.n_f, R.MT_all, P0->KI, s))
+    if (int st = launch_lowp_planes(P0->kprec, R.d_X, R.d_Xlp, R.d_xscale, P0->g.n_f, R.MT_all, P0->KI, s))
         return st;
-    fnk::BeamArgs A = P0->args;
+    fnk::BeamArgs A = forward_args(P0);
     A.X = R.d_X;
     A.Xlp = R.d_Xlp;
     A.xscale = R.d_xscale;
@@ -1933,7 +1977,7 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
     A.n_slots = 1;
     A.slot_z = R.n_groups;
     const dim3 grid((unsigned)beam_tiles(P0), (unsigned)R.bin_split, (unsigned)R.n_groups);
-    hipError_t e = fnk::kEnsLaunchers[ki_index(P0->KI)][P0->precision](R.MT_tmpl, P0->wcr, grid, R.lds_beam, s, A, 1);
+    hipError_t e = fnk::kEnsLaunchers[ki_index(P0->KI)][P0->kprec](R.MT_tmpl, P0->wcr, grid, R.lds_beam, s, A, 1);
     if (e != hipSuccess) return hip_fail(e, "beamform_kernel (row stack)");
     return FN_OK;
 }
@@ -1943,7 +1987,7 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
 static long batch_class_key(const fn_plan *P)
 {
     if (P->n_frames > 1 || P->nw || P->lbl || P->KI > 32) return -1;  // persistent kernels up to 128 elements
-    return ((((long)P->mode * 64 + P->KI) * 16 + P->MT_tmpl) * 8 + P->wcr) * 8 * 4 + P->wct * 4 + P->precision;
+    return ((((long)P->mode * 64 + P->KI) * 16 + P->MT_tmpl) * 8 + P->wcr) * 8 * 4 + P->wct * 4 + P->kprec;
 }
 
 // group the plans into classes, upload each class's job and work-item tables and
@@ -1999,7 +2043,7 @@ static int batch_plan_classes(fn_batch *b, float *const *d_images)
         const fn_plan *P0 = b->plans[c.plans[0]];
         const int kidx = P0->KI == 8 ? 0 : (P0->KI == 16 ? 1 : 2);
         int occ = 0;
-        hipError_t e = fnk::kPersistLaunchers[P0->mode][kidx][P0->precision](P0->MT_tmpl, P0->wcr, P0->wct, 0,
+        hipError_t e = fnk::kPersistLaunchers[P0->mode][kidx][P0->kprec](P0->MT_tmpl, P0->wcr, P0->wct, 0,
                                                                             P0->lds_beam, nullptr, nullptr, nullptr, 0,
                                                                             nullptr, &occ);
         if (e != hipSuccess) return hip_fail(e, "persistent kernel occupancy");
@@ -2121,7 +2165,7 @@ int32_t fn_batch_execute(fn_batch *b, const void *const *d_rf, const int32_t *dt
             if (e != hipSuccess || st) break;
             const fn_plan *P0 = b->plans[c.plans[0]];
             const int kidx = P0->KI == 8 ? 0 : (P0->KI == 16 ? 1 : 2);
-            e = fnk::kPersistLaunchers[P0->mode][kidx][P0->precision](P0->MT_tmpl, P0->wcr, P0->wct, c.grid,
+            e = fnk::kPersistLaunchers[P0->mode][kidx][P0->kprec](P0->MT_tmpl, P0->wcr, P0->wct, c.grid,
                                                                      P0->lds_beam, b->pstream, c.d_jobs, c.d_items,
                                                                      c.n_items, c.d_counter, nullptr);
             for (int i : c.plans) {

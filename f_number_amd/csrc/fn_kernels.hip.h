@@ -62,7 +62,14 @@ enum { MODE_PW = 0, MODE_SA = 1 };
 struct WinCoef {
     float t_flat, t_cut, t_off, A, B, C, s_half;  // cosine argument: (t - t_off) * s_half revolutions
     float q_s, q_o;  // WC_COS_RF: quarter-period argument t q_s + q_o = (t - t_off) s_half / 2
+    // value of the flat part (A, B and C carry the same factor), 1 or SPLIT_PEAK, and its inverse
+    float peak, inv_peak;
 };
+
+// fp16x3: a bounded receive window is evaluated times 2^10 (an exact factor, taken out with
+// the normalization), so that the low half of a small weight stays a normal fp16 number:
+// without it a tapered window's low halves reach the subnormal range (weights below 1/8).
+constexpr float SPLIT_PEAK = 1024.0f;
 
 // element support of a window for one aperture
 enum { SUPPORT_OPEN_H = 0,   // boxcar, CPU: |x_k - x| / h < 1 (das_pw.m:441)
@@ -151,6 +158,12 @@ __device__ __forceinline__ float rev_of(uint32_t P)
 {
     return __uint_as_float(__builtin_amdgcn_alignbit(0x7Fu, P, 9u));
 }
+
+// The truncation above lowers each phase by 2^-24 revolutions on average, the receive and
+// the transmit one together by 2^-23: a rotation of the whole image by 2 pi 2^-23, which
+// the epilogue takes back (first order: |r|^2 exceeds 1 by 6e-13).  It was most of the FP32
+// form's error against 64 bits (75 angles, Hann: 7.7e-7 with it, 2.2e-7 without).
+constexpr float PHASE_BACK = 7.4901e-7f;
 
 // Per (voxel, bin) aperture: das_pw.m:387, 399-411 (CPU) and
 // das_kernel_phase_shifts.cu:90-125 (MEX).  All bounds in FP64, as the oracle.
@@ -315,10 +328,10 @@ __device__ __forceinline__ float window_rf(float ad, float iw_q, float q_o)
 template <int WC>
 __device__ __forceinline__ float window_eval(float t, const WinCoef &w)
 {
-    if (WC == WC_RANGE) return 1.0f;
+    if (WC == WC_RANGE) return w.peak;
     if (WC == WC_COS_RF) {
         const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(fmaf(t, w.q_s, w.q_o), 0.f, 0.25f));
-        return c * c;
+        return w.peak * c * c;
     }
     float v;
     if (WC == WC_LINEAR) {
@@ -327,7 +340,7 @@ __device__ __forceinline__ float window_eval(float t, const WinCoef &w)
         const float u = __builtin_amdgcn_fractf((t - w.t_off) * w.s_half);  // revolutions, reduced to [0, 1)
         v = w.A + w.B * __builtin_amdgcn_cosf(u);
     }
-    v = (t <= w.t_flat) ? 1.0f : v;
+    v = (t <= w.t_flat) ? w.peak : v;
     v = (t < w.t_cut) ? v : 0.0f;
     return v;
 }
@@ -483,8 +496,9 @@ __global__ __launch_bounds__(256) void spectra_kernel(const T *__restrict__ rf, 
 // voxel l & 15).  K is the receive element:
 //   FP32  (v_mfma_f32_16x16x4f32):      lane group g supplies element 4j + g at step j
 //   16-bit (v_mfma_f32_16x16x32_{bf16,f16}): lane group g supplies elements
-//          32c + 8g + s, s = 0..7, of chunk c (8 packed values per lane)
-// Both give every lane KI elements j = 0..KI-1 (kelem()).
+//          4j + g, j = 8c .. 8c + 7, of chunk c (8 packed values per lane)
+// Both give every lane the KI elements 4j + g, so a step j outside the support of a
+// wave's voxels is skipped alike in both.
 enum { PREC_FP32 = 0, PREC_BF16X3 = 1, PREC_FP16X3 = 2, PREC_FP16 = 3 };
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -497,12 +511,6 @@ struct Prec {
     static constexpr bool split = (PREC == PREC_BF16X3 || PREC == PREC_FP16X3);
 };
 
-template <int PREC>
-__device__ __forceinline__ int kelem(int j, int g)
-{
-    return PREC == PREC_FP32 ? 4 * j + g : 32 * (j >> 3) + 8 * g + (j & 7);
-}
-
 // bytes of one bin of staged spectra per transmit M-tile and element step
 template <int PREC>
 __host__ __device__ constexpr int stage_bytes_per_tile_step()
@@ -510,33 +518,29 @@ __host__ __device__ constexpr int stage_bytes_per_tile_step()
     return PREC == PREC_FP32 ? 64 * 8 : Prec<PREC>::planes * 64 * 2;
 }
 
+// two operands a0 x0, a1 x1 as one packed word of 16-bit values, and (split forms) their
+// residuals as another.  The high word is opaque to the compiler, which would otherwise
+// form every high half a second time for its residual.
 template <int PREC>
-__device__ __forceinline__ void pack8(const float *v, u32x4 &hi, u32x4 &lo)
+__device__ __forceinline__ void pack2(float a0, float x0, float a1, float x1, uint32_t &hi, uint32_t &lo)
 {
+    const float v0 = a0 * x0, v1 = a1 * x1;
+    lo = 0u;
     if (PREC == PREC_BF16X3) {
-        // high parts rounded in pairs (one packed conversion), read back as floats from
-        // the packed word (a bf16 is the upper half of its float), low parts from the
-        // residuals
-        bf16x8 l;
-#pragma unroll
-        for (int s = 0; s < 8; s += 2) {
-            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-            const bf16x2 hp = bf16x2{(__bf16)v[s], (__bf16)v[s + 1]};
-            const uint32_t hw = __builtin_bit_cast(uint32_t, hp);
-            hi[s / 2] = hw;
-            l[s] = (__bf16)(v[s] - __uint_as_float(hw << 16));
-            l[s + 1] = (__bf16)(v[s + 1] - __uint_as_float(hw & 0xffff0000u));
-        }
-        lo = __builtin_bit_cast(u32x4, l);
+        // a bf16 is the upper half of its float
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        hi = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v0, (__bf16)v1});
+        lo = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)(v0 - __uint_as_float(hi << 16)),
+                                                 (__bf16)(v1 - __uint_as_float(hi & 0xffff0000u))});
     } else {
-        f16x8 h, l;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            h[s] = (_Float16)v[s];
-            if (PREC == PREC_FP16X3) l[s] = (_Float16)(v[s] - (float)h[s]);
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+        hi = __builtin_bit_cast(uint32_t, f16x2{(_Float16)v0, (_Float16)v1});
+        if (PREC == PREC_FP16X3) {
+            asm("" : "+v"(hi));
+            const f16x2 h = __builtin_bit_cast(f16x2, hi);
+            lo = __builtin_bit_cast(uint32_t, f16x2{(_Float16)fmaf(a0, x0, -(float)h[0]),
+                                                    (_Float16)fmaf(a1, x1, -(float)h[1])});
         }
-        hi = __builtin_bit_cast(u32x4, h);
-        if (PREC == PREC_FP16X3) lo = __builtin_bit_cast(u32x4, l);
     }
 }
 
@@ -681,7 +685,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     float Trx[TAN ? KI : 1];  // tangent: geometric receive time (s)
 #pragma unroll
     for (int j = 0; j < KI; ++j) {
-        const int k = kelem<PREC>(j, g);
+        const int k = 4 * j + g;
         const double lat = (((double)k - A.M) * A.pitch - x) / A.ctof;
         const double tg = sqrt(lat * lat + zc * zc);
         const double tau = tg + t_half + (k < A.n_el ? A.delay[k] : 0.0);
@@ -713,8 +717,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
         }
     // line scan: the phase increment of the block's own transmit row
     const uint32_t Qln = LBL ? frac32(A.f_s * (pw_tx_time(A, bz, x, z) + A.t0 / A.f_s) / A.N) : 0u;
-    const int k0 = kelem<PREC>(0, g);
-    const float dg = (float)(((double)k0 - A.M) * A.pitch - x);  // x_k - x of element j = 0
+    const float dg = (float)(((double)g - A.M) * A.pitch - x);  // x_k - x of element j = 0
     const float pf = (float)A.pitch;
     const float dg_tx = (float)((4.0 * g - A.M) * A.pitch - x);  // SA transmit rows, mt = r = 0
 
@@ -731,6 +734,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     // w_n = n * 2 pi f_s / N; the tangent factor -w_n / c_tof is applied per bin
     const float w_unit = (float)(2.0 * 3.141592653589793 * A.f_s / A.N);
     const float inv_c = (float)(1.0 / A.ctof);
+    const float inv_peak = PREC == PREC_FP16X3 ? A.wrx.inv_peak : 1.0f;
     const int b_begin = by * A.bin_chunk;
     const int b_end = min(b_begin + A.bin_chunk, A.n_f);
     const int MT_all = (A.n_tx + 15) >> 4;  // stride of the operand layout
@@ -1093,44 +1097,78 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 accR[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
                 accI[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
             }
-            const float ul = ap.inv_wl * A.wrx.s_half, ur = ap.inv_wr * A.wrx.s_half;
-            const float ql = ap.inv_wl * A.wrx.q_s, qr = ap.inv_wr * A.wrx.q_s;  // WC_COS_RF slopes
-            // WC_COS_ALL: |d| / (2 W_side) = max(d ur, -d ul), d = dgb + (k - k0) pitch
-            const float ar0 = dgb * ur, ar1 = pf * ur, al0 = -dgb * ul, al1 = -pf * ul;
+            // the window's argument of element step j as in the FP32 form: the larger of two
+            // linear functions of j, each the larger exactly on its own side
+            const float dstep = 4.0f * pf;
+            const float qo = WCR == WC_COS_RF ? A.wrx.q_o : 0.f;
+            const float wsc = WCR == WC_COS_ALL ? A.wrx.s_half : WCR == WC_COS_RF ? A.wrx.q_s : 1.f;
+            const float sr = ap.inv_wr * wsc, sl = ap.inv_wl * wsc;
+            const float tr0 = fmaf(dgb, sr, qo), tr1 = dstep * sr, tl0 = fmaf(-dgb, sl, qo), tl1 = -dstep * sl;
+            const int klo = ap.klo - g, khi = ap.khi - g;  // support in units of 4j
+            // element steps skipped together when no voxel of the wave has support there: pairs
+            // where the vector ALUs bound the loop and the window needs no support test (11
+            // angles, Tukey: 3.20 ms by pairs, 3.35 by chunks of 8), otherwise whole chunks,
+            // whose straight code interleaves better (75 angles, fp16: 4.12 against 4.61 ms;
+            // synthetic aperture, 128 x 256: 11.2 against 11.9 ms)
+            constexpr bool PAIRS = MODE == MODE_PW && MT <= (PREC == PREC_BF16X3 ? 2 : 3) &&
+                                   (WCR == WC_COS_RF || WCR == WC_RANGE);
+            constexpr int GRAN = PAIRS ? 2 : 8;
+            const int j_a = u_lo >> 2, j_b = min(u_hi >> 2, KI - 1);  // u_hi = -1: no step
+            auto weight = [&](const int j, float &cs, float &sn) __attribute__((always_inline)) {
+                const float jf = (float)j;
+                // (wide arrays keep the per-element side select: fewer live registers)
+                const float d = fmaf(jf, dstep, dgb);
+                const float t = KI <= 32 ? fmaxf(fmaf(jf, tr1, tr0), fmaf(jf, tl1, tl0))
+                                         : fmaf(fabsf(d), d < 0.f ? sl : sr, qo);
+                float a;
+                if (WCR == WC_COS_ALL) {
+                    a = fmaf(A.wrx.B, __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(t)), A.wrx.A);
+                } else if (WCR == WC_COS_RF) {
+                    const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(t, 0.f, 0.25f));
+                    a = (PREC == PREC_FP16X3 ? SPLIT_PEAK * c : c) * c;
+                } else {
+                    a = window_eval<WCR>(t, A.wrx);
+                    if (RTEST) a = (4 * j >= klo && 4 * j <= khi) ? a : 0.f;
+                }
+                const float rv = rev_of((uint32_t)n * Qrx[j]);
+                sn = __builtin_amdgcn_sinf(rv);
+                cs = __builtin_amdgcn_cosf(rv);
+                asum += a;
+                return a;
+            };
             auto chunk_lp = [&](auto cc_const) {
                 constexpr int cc = decltype(cc_const)::value;
                 if (pipe) chunk_begin(cc_const, b);
                 const u32x4 *xq;
                 if constexpr (LP_CHUNKED) xq = stage_chunk_lp<PREC, MT, cc>();
                 else xq = reinterpret_cast<const u32x4 *>(smem_raw) + cc * 64;
-                if (cc >= (u_lo >> 5) && cc <= (u_hi >> 5)) {  // elements 32 cc .. 32 cc + 31
-                float br[8], bi[8];
-#pragma unroll
-                for (int s = 0; s < 8; ++s) {
-                    const int j = 8 * cc + s;
-                    const int k = kelem<PREC>(j, g);
-                    const float d = fmaf((float)(k - k0), pf, dgb);
-                    float a;
-                    if (WCR == WC_COS_ALL) {
-                        const float e = (float)(k - k0);
-                        const float u = __builtin_amdgcn_fractf(fmaxf(fmaf(e, ar1, ar0), fmaf(e, al1, al0)));
-                        a = fmaf(A.wrx.B, __builtin_amdgcn_cosf(u), A.wrx.A);
-                    } else if (WCR == WC_COS_RF) {
-                        a = window_rf(fabsf(d), d < 0.f ? ql : qr, A.wrx.q_o);
-                    } else {
-                        const float t = fabsf(d) * (d < 0.f ? ap.inv_wl : ap.inv_wr);
-                        a = window_eval<WCR>(t, A.wrx);
-                        if (RTEST) a = (k >= ap.klo && k <= ap.khi) ? a : 0.f;
-                    }
-                    const float rv = rev_of((uint32_t)n * Qrx[j]);
-                    const float sn = __builtin_amdgcn_sinf(rv), cs = __builtin_amdgcn_cosf(rv);
-                    br[s] = a * cs;
-                    bi[s] = a * sn;
-                    asum += a;
-                }
+                if (8 * cc + 7 >= j_a && 8 * cc <= j_b) {  // element steps 8 cc .. 8 cc + 7
                 u32x4 brh, brl, bih, bil;
-                pack8<PREC>(br, brh, brl);
-                pack8<PREC>(bi, bih, bil);
+#pragma unroll
+                for (int p0 = 0; p0 < 4; p0 += GRAN / 2) {
+                    // GRAN element steps at a time, two per packed word; steps outside the
+                    // support of every voxel of the wave have zero weights.  (Where only some of
+                    // the GRAN meet the support, the others get zero weight from the support
+                    // test or the window's cut.)
+                    const int j0 = 8 * cc + 2 * p0;
+                    if (WCR == WC_COS_ALL || GRAN == 8 || (j0 + GRAN - 1 >= j_a && j0 <= j_b)) {
+#pragma unroll
+                        for (int p = p0; p < p0 + GRAN / 2; ++p) {
+                            float c0, s0, c1, s1;
+                            const float a0 = weight(8 * cc + 2 * p, c0, s0), a1 = weight(8 * cc + 2 * p + 1, c1, s1);
+                            uint32_t h, l;
+                            pack2<PREC>(a0, c0, a1, c1, h, l);
+                            brh[p] = h;
+                            brl[p] = l;
+                            pack2<PREC>(a0, s0, a1, s1, h, l);
+                            bih[p] = h;
+                            bil[p] = l;
+                        }
+                    } else {
+#pragma unroll
+                        for (int p = p0; p < p0 + GRAN / 2; ++p) brh[p] = brl[p] = bih[p] = bil[p] = 0u;
+                    }
+                }
                 const u32x4 nbih = neg16(bih);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
@@ -1182,7 +1220,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
         if (MODE == MODE_PW) {
             if (ap.valid) {
                 // v_rcp_f32 (1 ulp) instead of the correctly rounded division's ten instructions
-                const float sc = (A.norm_rx ? __builtin_amdgcn_rcpf(asum) : 1.0f) * xscale;
+                const float sc = (A.norm_rx ? __builtin_amdgcn_rcpf(asum) : inv_peak) * xscale;
                 // padded transmit rows have zero spectra, so every row is summed
                 float pr = 0.f, pi = 0.f;  // tangent: sum_rows T (tau_tx,g Y + Y')
                 if constexpr (LBL) {
@@ -1300,7 +1338,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                     }
             }
             if (ap.valid && at.valid) {
-                const float sc = (A.norm_rx ? __builtin_amdgcn_rcpf(asum) : 1.0f) *
+                const float sc = (A.norm_rx ? __builtin_amdgcn_rcpf(asum) : inv_peak) *
                                  (A.norm_tx ? __builtin_amdgcn_rcpf(tsum) : 1.0f) * xscale;
                 float pr = 0.f, pi = 0.f;
 #pragma unroll
@@ -1319,7 +1357,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             if (NW) nw_row += (ap.valid && at.valid) ? 1 : 0;
             if (b == A.n_f - 1) wtx_last = tsum;
         }
-        if (b == A.n_f - 1) w_last = asum;
+        if (b == A.n_f - 1) w_last = asum * inv_peak;
     }
     if (ENS) {
         // rows of this lane -> their frames; consecutive rows of one frame (row stacks) are
@@ -1344,8 +1382,8 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                     if (f != f_run) {
                         if (f_run >= 0) {
                             float2 *img = A.frame_image ? A.frame_image[f_run] : A.image + (size_t)f_run * n_vox;
-                            atomicAdd(&img[v].x, A.out_scale * sr);
-                            atomicAdd(&img[v].y, A.out_scale * si);
+                            atomicAdd(&img[v].x, A.out_scale * fmaf(-PHASE_BACK, si, sr));
+                            atomicAdd(&img[v].y, A.out_scale * fmaf(PHASE_BACK, sr, si));
                         }
                         f_run = f;
                         sr = si = 0.f;
@@ -1355,8 +1393,8 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 }
                 if (f_run >= 0) {
                     float2 *img = A.frame_image ? A.frame_image[f_run] : A.image + (size_t)f_run * n_vox;
-                    atomicAdd(&img[v].x, A.out_scale * sr);
-                    atomicAdd(&img[v].y, A.out_scale * si);
+                    atomicAdd(&img[v].x, A.out_scale * fmaf(-PHASE_BACK, si, sr));
+                    atomicAdd(&img[v].y, A.out_scale * fmaf(PHASE_BACK, sr, si));
                 }
             }
             if (g == 0 && b_end == A.n_f && bz == 0 && A.weights) A.weights[v] = w_last;
@@ -1374,15 +1412,16 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
         Di += __shfl_xor(Di, 32);
     }
     if (g == 0 && vok) {
-        const float2 val = make_float2(A.out_scale * Ir, A.out_scale * Ii);
+        const float2 val = make_float2(A.out_scale * fmaf(-PHASE_BACK, Ii, Ir), A.out_scale * fmaf(PHASE_BACK, Ir, Ii));
+        const float2 dval = make_float2(A.out_scale * fmaf(-PHASE_BACK, Di, Dr), A.out_scale * fmaf(PHASE_BACK, Dr, Di));
         float2 *dimg = reinterpret_cast<float2 *>(A.dimage);
         if (A.partial) {
             const long slot = (long)by * A.slot_z + (LBL ? 0 : bz);
             A.partial[slot * n_vox + v] = val;
-            if (TAN) A.partial[((long)A.n_slots + slot) * n_vox + v] = make_float2(A.out_scale * Dr, A.out_scale * Di);
+            if (TAN) A.partial[((long)A.n_slots + slot) * n_vox + v] = dval;
         } else {
             A.image[v] = val;
-            if (TAN) dimg[v] = make_float2(A.out_scale * Dr, A.out_scale * Di);
+            if (TAN) dimg[v] = dval;
         }
         if (b_end == A.n_f && (LBL || bz == 0)) {
             if (A.weights) A.weights[v] = w_last;
@@ -1470,7 +1509,7 @@ static __global__ __launch_bounds__(256) void reduce_partials_kernel(const float
 // One block per bin: reads the FP32 operand-ordered spectra of the bin, picks a
 // power-of-two scale (16-bit float variants: largest component in [2^14, 2^15)),
 // and writes planes [p][mt][c][64][8] (p: Xr hi, Xi hi, Xr lo, Xi lo) with
-// lane (a & 15) + 16 ((k & 31) >> 3), slot k & 7, chunk k >> 5.
+// lane (a & 15) + 16 (k & 3), slot (k >> 2) & 7, chunk k >> 5.
 template <int PREC>
 __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restrict__ X, void *__restrict__ Xlp,
                                                           float *__restrict__ xscale, int MT_all, int KI)
@@ -1495,7 +1534,8 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
     if (PREC != PREC_BF16X3 && mx > 0.f) {
         int e2;
         frexpf(mx, &e2);              // mx = f 2^e2, f in [0.5, 1)
-        scale = ldexpf(1.0f, e2 - 15);  // mx / scale in [2^14, 2^15)
+        // mx / scale in [2^14, 2^15); the scale and its reciprocal stay normal numbers
+        scale = ldexpf(1.0f, min(max(e2 - 15, -120), 112));
     }
     if (threadIdx.x == 0) xscale[b] = scale;
     const float inv = 1.0f / scale;
@@ -1507,8 +1547,7 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
         const int s = o & 7, ln = (o >> 3) & 63, q = o >> 9;  // q = mt * KC + c
         const int mt = q / KC, cc = q - mt * KC;
         const int row = ln & 15, gg = ln >> 4;
-        const int k = 32 * cc + 8 * gg + s;
-        const float2 v = Xb[(mt * KI + (k >> 2)) * 64 + row + 16 * (k & 3)];
+        const float2 v = Xb[(mt * KI + 8 * cc + s) * 64 + row + 16 * gg];  // element 32 cc + 4 s + gg
         const float vr = v.x * inv, vi = v.y * inv;
         if (PREC == PREC_BF16X3) {
             const __bf16 rh = (__bf16)vr, ih = (__bf16)vi;
