@@ -59,7 +59,7 @@ def autofocus(plan, rf, n_iter: int = 50, c0: float = 1480.0, delays0=None, weig
 
     dev = rf.device
     n_el = plan.n_elements
-    n_vox = plan.info()["n_voxels"]
+    n_vox = plan._n_voxels
     I = torch.empty(n_vox, dtype=torch.complex64, device=dev)
     dI = torch.empty_like(I)
     W = weights.reshape(-1).to(dev, torch.float32) if weights is not None else torch.ones(n_vox, device=dev)

@@ -152,6 +152,7 @@ struct fn_plan {
     fnk::BeamArgs args{};
     fnk::SpecArgs sargs{};
     size_t lds_beam = 0, lds_spec = 0;
+    unsigned char *d_block = nullptr;  // one allocation: the tables, the delay offsets, spectra, planes and scales
     double *d_px = nullptr, *d_pz = nullptr, *d_Frx = nullptr, *d_Ftx = nullptr, *d_txp = nullptr, *d_sqf = nullptr;
     float2 *d_tw = nullptr, *d_X = nullptr;
     void *d_Xlp = nullptr;    // 16-bit spectra planes (mixed precision)
@@ -180,7 +181,11 @@ struct fn_plan {
     std::vector<Run> pending, spare;
     double spec_ms = 0.0, beam_ms = 0.0;
     int runs = 0;
-    double flops = 0.0, useful_flops = 0.0;
+    double flops = 0.0;
+    // useful_flops: counted on the first fn_plan_info_get (n_f x up to 64 x 64 apertures, 15 ms
+    // at 250 bins), which executing a plan does not need
+    mutable std::once_flag useful_once;
+    mutable double useful_flops = 0.0;
 };
 
 namespace {
@@ -409,9 +414,7 @@ struct Common {
 void destroy(fn_plan *p)
 {
     if (!p) return;
-    hipFree(p->d_px); hipFree(p->d_pz); hipFree(p->d_Frx); hipFree(p->d_Ftx); hipFree(p->d_txp); hipFree(p->d_sqf);
-    hipFree(p->d_tw); hipFree(p->d_X); hipFree(p->d_Xlp); hipFree(p->d_xscale);
-    hipFree(p->d_delay); hipFree(p->d_P); hipFree(p->d_Z); hipFree(p->d_part); hipFree(p->d_qtab); hipFree(p->d_vsc); hipFree(p->d_nw);
+    hipFree(p->d_block); hipFree(p->d_P); hipFree(p->d_Z); hipFree(p->d_part); hipFree(p->d_qtab); hipFree(p->d_vsc); hipFree(p->d_nw);
     hipFree(p->d_sigF); hipFree(p->d_pimg); hipFree(p->d_ptan);
     for (auto &r : p->pending) { hipEventDestroy(r.e0); hipEventDestroy(r.e1); hipEventDestroy(r.e2); }
     for (auto &r : p->spare) { hipEventDestroy(r.e0); hipEventDestroy(r.e1); hipEventDestroy(r.e2); }
@@ -419,13 +422,16 @@ void destroy(fn_plan *p)
     delete p;
 }
 
-template <typename T>
-int upload(T **dst, const T *src, size_t n, const char *what)
-{
-    HIP_CHECK(hipMalloc(dst, sizeof(T) * n), what);
-    HIP_CHECK(hipMemcpy(*dst, src, sizeof(T) * n, hipMemcpyHostToDevice), what);
-    return FN_OK;
-}
+// sub-allocation of a device block: 256-byte aligned pieces
+struct Carve {
+    size_t used = 0;
+    size_t take(size_t bytes)
+    {
+        const size_t at = used;
+        used += (bytes + 255) & ~(size_t)255;
+        return at;
+    }
+};
 
 #ifndef FN_FEW_ROWS_BLOCKS
 #define FN_FEW_ROWS_BLOCKS 8192L
@@ -536,43 +542,65 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, bool plain
     return FN_OK;
 }
 
-// shared part of plan creation: configuration, then the device tables and workspace
-int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, const double *Ftx)
+// shared part of plan creation, after configure_common: the device tables and workspace.
+// One allocation and one copy: the tables (positions, F-numbers, sqrt(f_n), transmit rows
+// txp, twiddles, zero delay offsets) are laid out on the host first.  Every slot of the
+// spectra and their planes is written by each execute, padding as zeros.
+int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, const double *Ftx,
+                  const std::vector<double> &txp)
 {
-    int s = configure_common(P, c, g);
-    if (s) return s;
+    int s;
     if ((s = select_device(c.index_gpu))) return s;
 
     HIP_CHECK(hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking), "hipStreamCreate");
-    if ((s = upload(&P->d_px, c.px, c.n_x, "positions_x"))) return s;
-    if ((s = upload(&P->d_pz, c.pz, c.n_z, "positions_z"))) return s;
-    if ((s = upload(&P->d_Frx, Frx, g.n_f, "F-number"))) return s;
-    if (Ftx && (s = upload(&P->d_Ftx, Ftx, g.n_f, "F-number tx"))) return s;
-    // sqrt(f_n) per bin for the depth clamp of the F-number
-    std::vector<double> sqf(g.n_f);
-    for (int b = 0; b < g.n_f; ++b) sqf[b] = std::sqrt(c.f_s * (double)(g.n_lb + b) / g.N);
-    if ((s = upload(&P->d_sqf, sqf.data(), sqf.size(), "sqrt(f)"))) return s;
     P->h_px.assign(c.px, c.px + c.n_x);
     P->h_pz.assign(c.pz, c.pz + c.n_z);
     P->h_Frx.assign(Frx, Frx + g.n_f);
     if (Ftx) P->h_Ftx.assign(Ftx, Ftx + g.n_f);
-    P->h_sqf = sqf;
-    // twiddles e^{+j 2 pi m / N} rounded once from long double (conjugated in the kernel)
+    // sqrt(f_n) per bin for the depth clamp of the F-number
+    P->h_sqf.resize(g.n_f);
+    for (int b = 0; b < g.n_f; ++b) P->h_sqf[b] = std::sqrt(c.f_s * (double)(g.n_lb + b) / g.N);
+    // twiddles e^{+j 2 pi m / N} rounded once from long double (conjugated in the kernel);
+    // those of N - m are the conjugates
     std::vector<float2> tw(g.N);
-    for (int m = 0; m < g.N; ++m) {
+    for (int m = 0; m <= g.N / 2; ++m) {
         const long double ang = 2.0L * 3.141592653589793238462643383279502884L * (long double)m / (long double)g.N;
-        tw[m] = make_float2((float)cosl(ang), (float)sinl(ang));
+        long double sn, cs;
+        sincosl(ang, &sn, &cs);
+        tw[m] = make_float2((float)cs, (float)sn);
+        if (m) tw[g.N - m] = make_float2((float)cs, -(float)sn);
     }
-    if ((s = upload(&P->d_tw, tw.data(), tw.size(), "twiddles"))) return s;
-    HIP_CHECK(hipMalloc(&P->d_X, P->x_bytes), "spectra workspace");
-    HIP_CHECK(hipMemset(P->d_X, 0, P->x_bytes), "spectra workspace");  // padding rows stay zero
-    if (P->kprec != FN_PRECISION_FP32) {
-        HIP_CHECK(hipMalloc(&P->d_Xlp, P->xlp_bytes), "16-bit spectra planes");
-        HIP_CHECK(hipMalloc(&P->d_xscale, (size_t)g.n_f * sizeof(float)), "spectra scales");
-    }
-
-    HIP_CHECK(hipMalloc(&P->d_delay, (size_t)c.n_el * sizeof(double)), "delay offsets");
-    HIP_CHECK(hipMemset(P->d_delay, 0, (size_t)c.n_el * sizeof(double)), "delay offsets");
+    Carve cv;
+    const size_t o_px = cv.take(c.n_x * sizeof(double)), o_pz = cv.take(c.n_z * sizeof(double));
+    const size_t o_F = cv.take(g.n_f * sizeof(double)), o_Ft = cv.take(Ftx ? g.n_f * sizeof(double) : 0);
+    const size_t o_sqf = cv.take(g.n_f * sizeof(double)), o_txp = cv.take(txp.size() * sizeof(double));
+    const size_t o_tw = cv.take(tw.size() * sizeof(float2)), o_dl = cv.take(c.n_el * sizeof(double));
+    const size_t tables = cv.used;
+    const size_t o_X = cv.take(P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
+    const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
+    std::vector<unsigned char> h(tables, 0);
+    auto put = [&](size_t at, const void *src, size_t bytes) { if (bytes) std::memcpy(h.data() + at, src, bytes); };
+    put(o_px, c.px, c.n_x * sizeof(double));
+    put(o_pz, c.pz, c.n_z * sizeof(double));
+    put(o_F, Frx, g.n_f * sizeof(double));
+    if (Ftx) put(o_Ft, Ftx, g.n_f * sizeof(double));
+    put(o_sqf, P->h_sqf.data(), g.n_f * sizeof(double));
+    put(o_txp, txp.data(), txp.size() * sizeof(double));
+    put(o_tw, tw.data(), tw.size() * sizeof(float2));
+    HIP_CHECK(hipMalloc(&P->d_block, cv.used), "plan tables and spectra workspace");
+    HIP_CHECK(hipMemcpy(P->d_block, h.data(), tables, hipMemcpyHostToDevice), "plan tables");
+    auto at = [&](size_t o) { return reinterpret_cast<double *>(P->d_block + o); };
+    P->d_px = at(o_px);
+    P->d_pz = at(o_pz);
+    P->d_Frx = at(o_F);
+    P->d_Ftx = Ftx ? at(o_Ft) : nullptr;
+    P->d_sqf = at(o_sqf);
+    P->d_txp = txp.empty() ? nullptr : at(o_txp);
+    P->d_tw = reinterpret_cast<float2 *>(at(o_tw));
+    P->d_delay = at(o_dl);
+    P->d_X = reinterpret_cast<float2 *>(at(o_X));
+    P->d_Xlp = P->xlp_bytes ? at(o_Xlp) : nullptr;
+    P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
 
     fnk::BeamArgs &A = P->args;
     A.X = P->d_X;
@@ -607,9 +635,11 @@ int active_elements(double x, double z, double F, int support, double pitch, int
 // voxels and bins of the active receive elements times the transmit rows (plane
 // waves), or times the active transmitters (synthetic aperture), from a sample of
 // about 64 x 64 voxels and every bin, scaled to the grid.
-double useful_macs(const fn_plan *P, const double *px, int nx, const double *pz, int nz, const double *Frx,
-                   const double *Ftx, double f_s, double c0, double pitch)
+double useful_macs(const fn_plan *P)
 {
+    const int nx = P->n_x, nz = P->n_z;
+    const double *px = P->h_px.data(), *pz = P->h_pz.data(), *Frx = P->h_Frx.data(), *Ftx = P->h_Ftx.data();
+    const double f_s = P->args.f_s, c0 = P->args.c0, pitch = P->args.pitch;
     const fnh::Grid &g = P->g;
     const int sx = std::max(1, nx / 64), sz = std::max(1, nz / 64);
     double sum = 0.0;
@@ -847,7 +877,7 @@ int pw_plan(const fn_pw_params *p, fn_plan **out)
     if (!P) return fail(FN_ERR_OUT_OF_MEMORY, "host allocation");
     Common c{};
     if ((s = configure_pw(P, p, &c))) { destroy(P); return s; }
-    if ((s = create_common(P, c, g, p->f_number_values, nullptr))) { destroy(P); return s; }
+    if ((s = configure_common(P, c, g))) { destroy(P); return s; }
     const int n_rows = P->args.n_tx;  // operand rows (ensembles: frame slots)
     // steering geometry in FP64: das_pw.m:323-327 (x_ref = sign(e_x) x_0), or the
     // virtual sources (x_vs, z_vs, |r_vs|)
@@ -869,13 +899,10 @@ int pw_plan(const fn_pw_params *p, fn_plan **out)
         txp[3 * row + 1] = ez;
         txp[3 * row + 2] = sg * ((0 - M) * p->element_pitch);
     }
-    if ((s = upload(&P->d_txp, txp.data(), txp.size(), "steering"))) { destroy(P); return s; }
-    P->args.txp = P->d_txp;
+    if ((s = create_common(P, c, g, p->f_number_values, nullptr, txp))) { destroy(P); return s; }
     if (P->nw && (s = setup_windowed(P, true, p->window, p->normalization_window, false, p->window,
                                      p->normalization_window))) { destroy(P); return s; }
     use_cos_all(P);
-    P->useful_flops = 8.0 * useful_macs(P, p->positions_x, p->n_x, p->positions_z, p->n_z, p->f_number_values,
-                                        nullptr, p->f_s, p->c_0, p->element_pitch);
     *out = P;
     return FN_OK;
 }
@@ -903,9 +930,8 @@ int sa_plan(const fn_sa_params *p, fn_plan **out)
     Common c{p->positions_x, p->positions_z, p->n_x, p->n_z, p->n_samples, p->n_elements, p->n_elements,
              p->f_s, p->element_width, p->element_pitch, p->c_0, p->index_t0,
              p->semantics, p->precision, p->output_scale, p->index_gpu, p->verbosity};
-    if ((s = create_common(P, c, g, p->f_number_rx_values, p->f_number_tx_values))) { destroy(P); return s; }
-    P->useful_flops = 8.0 * useful_macs(P, p->positions_x, p->n_x, p->positions_z, p->n_z, p->f_number_rx_values,
-                                        p->f_number_tx_values, p->f_s, p->c_0, p->element_pitch);
+    if ((s = configure_common(P, c, g))) { destroy(P); return s; }
+    if ((s = create_common(P, c, g, p->f_number_rx_values, p->f_number_tx_values, {}))) { destroy(P); return s; }
     if (P->nw && (s = setup_windowed(P, nw_rx, p->window_rx, p->normalization_window_rx, nw_tx, p->window_tx,
                                      p->normalization_window_tx))) { destroy(P); return s; }
     use_cos_all(P);
@@ -1476,17 +1502,6 @@ int upload_chunked(double *dst, const double *src, long n, hipStream_t s)
     return FN_OK;
 }
 
-// sub-allocation of the scratch: 256-byte aligned pieces
-struct Carve {
-    size_t used = 0;
-    size_t take(size_t bytes)
-    {
-        const size_t at = used;
-        used += (bytes + 255) & ~(size_t)255;
-        return at;
-    }
-};
-
 int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_image, float *d_w, hipStream_t s)
 {
     fnh::Grid g;
@@ -1620,6 +1635,7 @@ int32_t fn_plan_info_get(const fn_plan *P, fn_plan_info *info)
     info->n_voxels = P->n_vox;
     info->workspace_bytes = (int64_t)P->x_bytes;
     info->flops_per_frame = P->flops;
+    std::call_once(P->useful_once, [P] { P->useful_flops = 8.0 * useful_macs(P); });
     info->useful_flops_per_frame = P->useful_flops;
     info->tile_voxels = 64;
     info->bin_split = P->bin_split;

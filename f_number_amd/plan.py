@@ -47,13 +47,12 @@ class _Plan:
             raise _lib.FNumberError(f"{self.prefix}:InvalidRFData", "RF must be float32 or float64")
         if image.dtype != torch.complex64:
             raise _lib.FNumberError(f"{self.prefix}:InvalidArgument", "image must be complex64")
-        inf = self.info()
-        if image.numel() != inf["n_voxels"] * getattr(self, "n_frames", 1):
+        if image.numel() != self._n_voxels * getattr(self, "n_frames", 1):
             raise _lib.FNumberError(f"{self.prefix}:InvalidArgument", "image size does not match the grid")
         if rf.numel() != self._rf_numel:
             raise _lib.FNumberError(f"{self.prefix}:InvalidRFData", "RF size does not match the plan")
         for w in (weights, weights_rx):
-            if w is not None and (w.dtype != torch.float32 or w.numel() != inf["n_voxels"] or not w.is_cuda):
+            if w is not None and (w.dtype != torch.float32 or w.numel() != self._n_voxels or not w.is_cuda):
                 raise _lib.FNumberError(f"{self.prefix}:InvalidArgument", "weights must be float32 device tensors")
         if stream is None:
             stream = torch.cuda.current_stream(rf.device)
@@ -76,7 +75,7 @@ class _Plan:
         import torch
 
         dev = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
-        out = torch.empty(self.info()["N_dft"], dtype=torch.complex64, device=dev)
+        out = torch.empty(self.grid["N_dft"], dtype=torch.complex64, device=dev)
         _lib.check(_lib.load().fn_plan_focused_signal(self._h, _ptr(out), _stream(stream, dev)), self.prefix)
         return out
 
@@ -161,6 +160,7 @@ class PwPlan(_Plan):
         _lib.check(_lib.load().fn_plan_pw_create(C.byref(P), C.byref(self._h)), self.prefix)
         self._keep = keep
         self.grid = info
+        self._n_voxels = keep[0].size * keep[1].size
         self.n_samples, self.n_elements, self.n_angles = int(n_samples), int(n_elements), len(keep[2])
         self.n_frames = max(1, int(n_frames))
         self.c_0 = float(c_0)
@@ -185,7 +185,7 @@ class PwPlan(_Plan):
         """image and dI/dc_tof (complex64 (N_x, N_z) each)."""
         import torch
 
-        n = self.info()["n_voxels"]
+        n = self._n_voxels
         _need(image, torch.complex64, n, "image", self.prefix)
         _need(dimage, torch.complex64, n, "dimage", self.prefix)
         if rf.numel() != self._rf_numel or not rf.is_cuda or not rf.is_contiguous():
@@ -200,7 +200,7 @@ class PwPlan(_Plan):
         """A^H y: y complex64 (N_x, N_z) -> float32 (N_a, N_el, N_t)."""
         import torch
 
-        _need(y, torch.complex64, self.info()["n_voxels"], "y", self.prefix)
+        _need(y, torch.complex64, self._n_voxels, "y", self.prefix)
         if rf_adj is None:
             rf_adj = torch.empty((self.n_angles, self.n_elements, self.n_samples), dtype=torch.float32,
                                  device=y.device)
@@ -214,7 +214,7 @@ class PwPlan(_Plan):
         (dJ = sum Re(conj(g) dI)); dJ/dc needs dimage from execute_tangent."""
         import torch
 
-        n = self.info()["n_voxels"]
+        n = self._n_voxels
         _need(g, torch.complex64, n, "g", self.prefix)
         if dimage is not None:
             _need(dimage, torch.complex64, n, "dimage", self.prefix)
@@ -249,6 +249,7 @@ class SaPlan(_Plan):
         _lib.check(_lib.load().fn_plan_sa_create(C.byref(P), C.byref(self._h)), self.prefix)
         self._keep = keep
         self.grid = info
+        self._n_voxels = keep[0].size * keep[1].size
         self._rf_numel = int(n_samples) * int(n_elements) * int(n_elements)
 
 
@@ -283,7 +284,7 @@ class Batch:
         for p, rf, img in zip(self.plans, rfs, images):
             if rf.numel() != p._rf_numel or not rf.is_cuda or not rf.is_contiguous():
                 raise _lib.FNumberError("fn_batch:InvalidRFData", "RF size does not match its plan")
-            if img.numel() != p.info()["n_voxels"] * getattr(p, "n_frames", 1) or not img.is_contiguous():
+            if img.numel() != p._n_voxels * getattr(p, "n_frames", 1) or not img.is_contiguous():
                 raise _lib.FNumberError("fn_batch:InvalidArgument", "image size does not match its plan")
         r = (C.c_void_p * n)(*[t.data_ptr() for t in rfs])
         d = (C.c_int32 * n)(*[_rf_dtype(t, "fn_batch") for t in rfs])
