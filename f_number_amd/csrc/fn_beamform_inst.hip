@@ -69,6 +69,42 @@ static hipError_t launch_mt(int wcr, dim3 grid, size_t lds, hipStream_t s, const
     }
 }
 
+#if INST_PREC == 2 && INST_KI <= 48
+// mirrored voxels: `mt` transmit tiles (1 or 2; beyond 128 elements 1), as many reversed
+template <int MT, int WCR>
+static hipError_t launch_mir_one(dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
+{
+    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, INST_PREC, false, false, false, false, false, true>;
+    static size_t lds_done = 0;
+    lds = dyn_lds(lds);
+    if (hipError_t e = set_lds_once(kern, lds, lds_done)) return e;
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, A);
+    return hipGetLastError();
+}
+
+template <int MT>
+static hipError_t launch_mir_mt(int wcr, dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
+{
+    switch (wcr) {
+    case WC_RANGE: return launch_mir_one<MT, WC_RANGE>(grid, lds, s, A);
+    case WC_LINEAR: return launch_mir_one<MT, WC_LINEAR>(grid, lds, s, A);
+    case WC_COS_ALL: return launch_mir_one<MT, WC_COS_ALL>(grid, lds, s, A);
+    case WC_COS_RF: return launch_mir_one<MT, WC_COS_RF>(grid, lds, s, A);
+    default: return launch_mir_one<MT, WC_COS>(grid, lds, s, A);
+    }
+}
+
+#define FN_MIR_LAUNCHER(k) FN_CAT6(launch_beamform_mir, _k, k, , , )
+hipError_t FN_MIR_LAUNCHER(INST_KI)(int mt, int wcr, dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
+{
+    if (mt == 1) return launch_mir_mt<2>(wcr, grid, 2 * lds, s, A);
+#if !FN_WIDE
+    if (mt == 2) return launch_mir_mt<4>(wcr, grid, 2 * lds, s, A);
+#endif
+    return hipErrorInvalidValue;
+}
+#endif
+
 #if INST_PREC == 0 && !FN_WIDE
 // tangent (dI / dc_tof) variant: groups of at most two transmit tiles
 #define FN_TAN_LAUNCHER(k) FN_CAT4(launch_beamform_tan, _k, k, )
@@ -224,6 +260,7 @@ static hipError_t launch_wct(int wct, dim3 grid, size_t lds, hipStream_t s, cons
     case WC_RANGE: return launch_one<SA_MT, WCR, WC_RANGE>(grid, lds, s, A);
     case WC_LINEAR: return launch_one<SA_MT, WCR, WC_LINEAR>(grid, lds, s, A);
     case WC_COS_RF: return launch_one<SA_MT, WCR, WC_COS_RF>(grid, lds, s, A);
+    case WC_COS_ALL: return launch_one<SA_MT, WCR, WC_COS_ALL>(grid, lds, s, A);
     default: return launch_one<SA_MT, WCR, WC_COS>(grid, lds, s, A);
     }
 }

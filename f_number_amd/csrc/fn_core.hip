@@ -44,6 +44,14 @@ FN_DECL_ENS(8)
 FN_DECL_ENS(16)
 FN_DECL_ENS(32)
 #undef FN_DECL_ENS
+// mirrored voxels (the fp16 split) [KI = 8 .. 48]
+hipError_t launch_beamform_mir_k8(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
+hipError_t launch_beamform_mir_k16(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
+hipError_t launch_beamform_mir_k32(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
+hipError_t launch_beamform_mir_k48(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
+typedef hipError_t (*MirLauncher)(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
+static const MirLauncher kMirLaunchers[4] = {launch_beamform_mir_k8, launch_beamform_mir_k16, launch_beamform_mir_k32,
+                                             launch_beamform_mir_k48};
 // the last argument: 1 for a row stack (per-row transmit phases), 0 for an ensemble
 typedef hipError_t (*EnsLauncher)(int, int, dim3, size_t, hipStream_t, const BeamArgs &, int);
 // [KI = 8, 16, 32][form of the contraction] (FP32: the windows the fp16 split is not for)
@@ -148,6 +156,8 @@ struct fn_plan {
     std::vector<double> h_delay;                          // delay offsets of the last set_tof (empty: zeros)
     int precision = FN_PRECISION_FP32;  // as asked for
     int kprec = FN_PRECISION_FP32;      // form of the forward contraction (kernel_precision)
+    int mirror = 0;         // lateral positions symmetric: planes hold the reversed elements too
+    int delays_even = 1;    // delay offsets symmetric about the array's centre
     int verbosity = 0;
     fnk::BeamArgs args{};
     fnk::SpecArgs sargs{};
@@ -190,8 +200,19 @@ struct fn_plan {
 
 namespace {
 
-// voxel tiles of 64 per beamforming group: the whole grid, or (line scan) one column
-long beam_tiles(const fn_plan *P) { return P->lbl ? (P->n_z + 63) / 64 : (P->n_vox + 63) / 64; }
+// the forward kernel whose lanes stand for a voxel and its mirror image (beamform_tile, MIR)
+bool use_mirror(const fn_plan *P) { return P->mirror && P->delays_even && P->n_groups == 1; }
+
+// M-tiles of the 16-bit planes: the transmit tiles and their mirrored ones, or whole groups
+int plane_tiles(const fn_plan *P) { return use_mirror(P) ? 2 * P->MT_all : P->n_groups * P->MT_tmpl; }
+
+// voxel tiles of 64 per beamforming group: the whole grid, half its columns (mirrored
+// voxels), or (line scan) one column
+long beam_tiles(const fn_plan *P)
+{
+    if (P->lbl) return (P->n_z + 63) / 64;
+    return ((use_mirror(P) ? (long)((P->n_x + 1) / 2) * P->n_z : P->n_vox) + 63) / 64;
+}
 
 // workgroups that share a voxel: bin chunks times transmit groups (a line scan's
 // groups are its columns, one per voxel); ensembles add their frames' rows atomically
@@ -327,19 +348,31 @@ void use_cos_all(fn_plan *P)
 {
     if (P->nw) return;
     const fnk::WinCoef &w = P->args.wrx;
+    // elements the kernel's loop runs over: the 16-bit forms run whole chunks of 32 elements
+    // that meet a support (some kernels of a plan skip finer steps), so 96 or 160 elements
+    // need no support test either, while their padding would be a part of a chunk otherwise
+    const bool lp = P->kprec != FN_PRECISION_FP32;
+    const int n_run = lp && P->n_el % 32 == 0 ? P->n_el : 4 * P->KI;
     if (P->wcr == fnk::WC_COS) {
-        if (P->args.support_rx == fnk::SUPPORT_ALL && P->n_el == 4 * P->KI && w.t_off == 0.f && w.t_flat < 0.f &&
-            std::isinf(w.t_cut))
+        if (P->args.support_rx == fnk::SUPPORT_ALL && P->n_el == n_run &&
+            w.t_off == 0.f && w.t_flat < 0.f && std::isinf(w.t_cut))
             P->wcr = fnk::WC_COS_ALL;
-        else if (fnk::cos_rf_window(P->args, P->args.support_rx, w, 4 * P->KI))
+        else if (fnk::cos_rf_window(P->args, P->args.support_rx, w, n_run))
             P->wcr = fnk::WC_COS_RF;
     }
     // the synthetic aperture's transmit side: the same cut-window class for its
     // transmitters (the SA kernels launch it; every other SA path evaluates the window
     // with its support test, which WC_COS_RF maps to)
-    if (P->mode == 1 && P->wct == fnk::WC_COS &&
-        fnk::cos_rf_window(P->args, P->args.support_tx, P->args.wtx, 4 * P->KI))
-        P->wct = fnk::WC_COS_RF;
+    // whole tiles of 16 transmitters: the padding tiles get no weight
+    const fnk::WinCoef &t = P->args.wtx;
+    const int n_tx = P->n_el % 16 == 0 ? P->n_el : 4 * P->KI;
+    if (P->mode == 1 && P->wct == fnk::WC_COS) {
+        if (P->args.support_tx == fnk::SUPPORT_ALL && P->n_el == n_tx && t.t_off == 0.f && t.t_flat < 0.f &&
+            std::isinf(t.t_cut))
+            P->wct = fnk::WC_COS_ALL;
+        else if (fnk::cos_rf_window(P->args, P->args.support_tx, t, n_tx))
+            P->wct = fnk::WC_COS_RF;
+    }
 }
 
 int wcr_general(int wcr) { return (wcr == fnk::WC_COS_ALL || wcr == fnk::WC_COS_RF) ? fnk::WC_COS : wcr; }
@@ -433,6 +466,17 @@ struct Carve {
     }
 };
 
+// transmit tiles per group the autotuner may try: the default cap, and for fp16
+// ensembles at 128 elements up to 8 (one wave per SIMD; each weight serves 128 rows)
+int max_tiles(const fn_plan *P)
+{
+    if (P->mode == 1) return sa_mt(P->KI);
+    if (P->lbl) return 1;
+    if (P->nw) return std::min(P->MT_all, 2);
+    if (P->n_frames > 1 && P->kprec == FN_PRECISION_FP16 && P->KI == 32) return std::min(P->MT_all, 8);
+    return std::min(P->MT_all, std::min(tile_cap(P->n_frames, P->precision, P->KI), pw_mt_wide(P->KI)));
+}
+
 #ifndef FN_FEW_ROWS_BLOCKS
 #define FN_FEW_ROWS_BLOCKS 8192L
 #endif
@@ -441,11 +485,32 @@ static bool few_rows_pw(const fn_plan *P)
     return P->mode == 0 && P->n_frames == 1 && !P->lbl && P->MT_tmpl <= 2;
 }
 
+// Plans whose lanes may stand for two mirrored voxels: single-frame plane waves in the fp16
+// split whose transmit rows fill one or two tiles (one at 129-192 elements), where the vector
+// work of the weights bounds the kernel, on lateral positions symmetric to 1e-12 pitches.  In
+// ms without / with (256 x 256): 11 angles 3.12 / 2.42, 31 angles 4.00 / 3.28, 192 elements
+// 5.96 / 4.42; from three tiles on the products bound it and twice the tiles have no room in
+// registers and LDS; 256 elements 7.27 / 9.59.  The one-pass fp16 form, whose operands' rounding
+// shows in the image, keeps one voxel a lane, so that a plan's image does not depend on whether
+// it runs alone or in a batch.  Not the boxcar window
+// at one F-number for every bin: its membership test has no taper, and its ties (a support
+// edge on an element for a whole band) would be broken by rounding.
+bool mirror_plan(const fn_plan *P, const Common &c, const double *Frx, int n_f)
+{
+    if (P->mode != 0 || P->n_frames > 1 || P->lbl || P->nw || P->kprec != FN_PRECISION_FP16X3 || !Frx) return false;
+    if (P->KI > 48 || P->MT_all > (P->KI <= 32 ? 2 : 1) || c.n_x < 2) return false;
+    if (P->wcr == fnk::WC_RANGE && std::all_of(Frx, Frx + n_f, [&](double F) { return F == Frx[0]; })) return false;
+    for (int i = 0; i < (c.n_x + 1) / 2; ++i)
+        if (!(std::fabs(c.px[i] + c.px[c.n_x - 1 - i]) <= 1e-12 * c.pitch)) return false;
+    return true;
+}
+
 // shared configuration of plan creation: tiling, launch shape and the scalar
 // arguments of the kernels; no device work and no allocation (the
 // no-allocation entry point runs it on a plan held on the stack, with plain_fp32 where its
 // scratch has no room for the split form's planes)
-int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, bool plain_fp32 = false)
+int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, bool plain_fp32 = false,
+                     bool mirror = true)
 {
     if (c.precision < FN_PRECISION_FP32 || c.precision > FN_PRECISION_FP16)
         return fail(FN_ERR_ARGUMENT, "unknown precision %d", c.precision);
@@ -485,6 +550,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, bool plain
         P->MT_tmpl = sa_mt(P->KI);
         P->n_groups = (P->MT_all + P->MT_tmpl - 1) / P->MT_tmpl;
     }
+    P->mirror = mirror && mirror_plan(P, c, Frx, g.n_f);
     const size_t step_bytes = form_step_bytes(P->kprec);
     P->lds_beam = (size_t)P->MT_tmpl * P->KI * step_bytes;
     P->lds_spec = (size_t)g.N * sizeof(float2) + 64 * 65 * sizeof(float);
@@ -516,7 +582,11 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, bool plain
     const int chunk = (g.n_f + split - 1) / split;
     P->bin_split = (g.n_f + chunk - 1) / chunk;
     P->x_bytes = (size_t)g.n_f * P->MT_all * P->KI * 64 * sizeof(float2);
-    P->xlp_bytes = P->kprec != FN_PRECISION_FP32 ? (size_t)g.n_f * form_planes(P->kprec) * P->MT_all * P->KI * 64 * 2 : 0;
+    // room for the planes of every tiling: groups of mt tiles hold up to mt - 1 zero tiles
+    const int xlp_tiles = P->mirror      ? 2 * P->MT_all
+                          : P->mode == 1 ? P->n_groups * P->MT_tmpl
+                                         : P->MT_all + std::max(P->MT_tmpl, max_tiles(P)) - 1;
+    P->xlp_bytes = P->kprec != FN_PRECISION_FP32 ? (size_t)g.n_f * form_planes(P->kprec) * xlp_tiles * P->KI * 64 * 2 : 0;
 
     fnk::BeamArgs &A = P->args;
     A.ctof = c.c0;
@@ -668,6 +738,7 @@ hipError_t launch_beam(const fn_plan *P, dim3 grid, const fnk::BeamArgs &A, hipS
 {
     const int kidx = ki_index(P->KI);  // ensembles, line scans and windowed plans stop at KI = 32
     if (P->lbl) return fnk::kLblLaunchers[kidx](P->wcr, grid, s, A);
+    if (use_mirror(P)) return fnk::kMirLaunchers[kidx](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A);
     if (P->nw) return fnk::kNwLaunchers[P->mode][kidx](P->MT_tmpl, P->wcr, P->wct, grid, P->lds_beam, s, A);
     if (P->n_frames > 1) return fnk::kEnsLaunchers[kidx][P->kprec](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A, 0);
     return fnk::kBeamLaunchers[P->mode][kidx][P->kprec](P->MT_tmpl, P->wcr, P->wct, grid, P->lds_beam, s, A);
@@ -716,6 +787,7 @@ int launch_spectra(fn_plan *P, const void *d_rf, int dtype, hipStream_t s)
 fnk::BeamArgs forward_args(const fn_plan *P)
 {
     fnk::BeamArgs A = P->args;
+    A.xlp_tiles = plane_tiles(P);
     if (P->kprec == FN_PRECISION_FP16X3 && !unbounded_window(P->wcr, A.wrx)) {
         A.wrx.A *= fnk::SPLIT_PEAK;
         A.wrx.B *= fnk::SPLIT_PEAK;
@@ -746,19 +818,24 @@ fnk::BeamArgs beam_args(const fn_plan *P, float *d_image, float *d_w, float *d_w
 
 // the 16-bit operand planes (and per-bin scales) of FP32 spectra X of MT tiles;
 // nothing for FP32 plans
-int launch_lowp_planes(int precision, const float2 *X, void *Xlp, float *xscale, int n_f, int MT, int KI, hipStream_t s)
+// MT_out, mirror_el: see lowp_planes_kernel
+int launch_lowp_planes(int precision, const float2 *X, void *Xlp, float *xscale, int n_f, int MT, int KI, int MT_out,
+                       int mirror_el, hipStream_t s)
 {
     if (precision == FN_PRECISION_FP32) return FN_OK;
     const dim3 cg((unsigned)n_f), cb(256);
     switch (precision) {
     case FN_PRECISION_BF16X3:
-        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_BF16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, KI);
+        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_BF16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, KI, MT_out,
+                           mirror_el);
         break;
     case FN_PRECISION_FP16X3:
-        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, KI);
+        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, KI, MT_out,
+                           mirror_el);
         break;
     default:
-        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16>, cg, cb, 0, s, X, Xlp, xscale, MT, KI);
+        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16>, cg, cb, 0, s, X, Xlp, xscale, MT, KI, MT_out,
+                           mirror_el);
         break;
     }
     HIP_CHECK(hipGetLastError(), "lowp_planes_kernel");
@@ -788,7 +865,8 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
     }
     const fnk::SpecArgs &S = P->sargs;
     if (int st = launch_spectra(P, d_rf, dtype, s)) return st;
-    return launch_lowp_planes(P->kprec, P->d_X, P->d_Xlp, P->d_xscale, S.n_f, S.MT, S.KI, s);
+    return launch_lowp_planes(P->kprec, P->d_X, P->d_Xlp, P->d_xscale, S.n_f, S.MT, S.KI, plane_tiles(P),
+                              use_mirror(P) ? P->n_el : 0, s);
 }
 
 int execute(fn_plan *P, const void *d_rf, int dtype, float *d_image, float *d_w, float *d_w_rx, hipStream_t user)
@@ -877,7 +955,7 @@ int pw_plan(const fn_pw_params *p, fn_plan **out)
     if (!P) return fail(FN_ERR_OUT_OF_MEMORY, "host allocation");
     Common c{};
     if ((s = configure_pw(P, p, &c))) { destroy(P); return s; }
-    if ((s = configure_common(P, c, g))) { destroy(P); return s; }
+    if ((s = configure_common(P, c, g, p->f_number_values))) { destroy(P); return s; }
     const int n_rows = P->args.n_tx;  // operand rows (ensembles: frame slots)
     // steering geometry in FP64: das_pw.m:323-327 (x_ref = sign(e_x) x_0), or the
     // virtual sources (x_vs, z_vs, |r_vs|)
@@ -930,7 +1008,7 @@ int sa_plan(const fn_sa_params *p, fn_plan **out)
     Common c{p->positions_x, p->positions_z, p->n_x, p->n_z, p->n_samples, p->n_elements, p->n_elements,
              p->f_s, p->element_width, p->element_pitch, p->c_0, p->index_t0,
              p->semantics, p->precision, p->output_scale, p->index_gpu, p->verbosity};
-    if ((s = configure_common(P, c, g))) { destroy(P); return s; }
+    if ((s = configure_common(P, c, g, p->f_number_rx_values))) { destroy(P); return s; }
     if ((s = create_common(P, c, g, p->f_number_rx_values, p->f_number_tx_values, {}))) { destroy(P); return s; }
     if (P->nw && (s = setup_windowed(P, nw_rx, p->window_rx, p->normalization_window_rx, nw_tx, p->window_tx,
                                      p->normalization_window_tx))) { destroy(P); return s; }
@@ -942,17 +1020,6 @@ int sa_plan(const fn_sa_params *p, fn_plan **out)
 size_t dtype_size(int dtype) { return dtype == FN_DTYPE_F64 ? 8 : 4; }
 
 // ---- tiling and autotuning ---------------------------------------------
-
-// transmit tiles per group the autotuner may try: the default cap, and for fp16
-// ensembles at 128 elements up to 8 (one wave per SIMD; each weight serves 128 rows)
-int max_tiles(const fn_plan *P)
-{
-    if (P->mode == 1) return sa_mt(P->KI);
-    if (P->lbl) return 1;
-    if (P->nw) return std::min(P->MT_all, 2);
-    if (P->n_frames > 1 && P->kprec == FN_PRECISION_FP16 && P->KI == 32) return std::min(P->MT_all, 8);
-    return std::min(P->MT_all, std::min(tile_cap(P->n_frames, P->precision, P->KI), pw_mt_wide(P->KI)));
-}
 
 int set_tiling(fn_plan *P, int mt, int split)
 {
@@ -1048,6 +1115,7 @@ int set_tof(fn_plan *P, double c_tof, const double *delays)
     HIP_CHECK(hipDeviceSynchronize(), "hipDeviceSynchronize");
     HIP_CHECK(hipMemcpy(P->d_delay, d.data(), d.size() * sizeof(double), hipMemcpyHostToDevice), "delay offsets");
     P->h_delay = d;
+    P->delays_even = std::equal(d.begin(), d.end(), d.rbegin());
     P->args.ctof = c_tof > 0 ? c_tof : P->args.c0;
     ++P->tof_serial;
     return FN_OK;
@@ -1524,9 +1592,10 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
     size_t o_X = 0, o_Xlp = 0, o_xs = 0, o_px = 0, o_pz = 0, o_F = 0, o_sqf = 0, o_raw = 0, o_txp = 0, o_tw = 0, o_dl = 0,
            o_pi = 0;
     int slots = 1;
-    // an FP32 call whose split planes do not fit beside its spectra runs the FP32 kernels
-    for (bool plain_fp32 : {false, true}) {
-        if ((st = configure_common(&P, c, g, plain_fp32))) return st;
+    // a call whose planes do not fit beside its spectra runs without the mirrored ones, an FP32
+    // call then without any, on the FP32 kernels
+    for (int lean = 0; lean < 3; ++lean) {
+        if ((st = configure_common(&P, c, g, p->f_number_values, lean == 2, lean == 0))) return st;
         cv = Carve{};
         o_X = cv.take(P.x_bytes);
         o_Xlp = cv.take(P.xlp_bytes);
@@ -1918,7 +1987,7 @@ static int batch_plan_stacks(fn_batch *b, float *const *d_images, std::vector<ch
         r.n_groups = (r.MT_all + r.MT_tmpl - 1) / r.MT_tmpl;
         r.lds_beam = (size_t)r.MT_tmpl * P0->KI * form_step_bytes(P0->kprec);
         // bin chunks: enough workgroups to fill the GPU several times over
-        const long blocks = beam_tiles(P0) * r.n_groups;
+        const long blocks = (P0->n_vox + 63) / 64 * r.n_groups;  // one voxel a lane
         int split = 1;
         if (blocks < 2048) split = (int)std::min<long>((2048 + blocks - 1) / blocks, std::max(1, P0->g.n_f / 8));
         r.chunk = (P0->g.n_f + split - 1) / split;
@@ -1936,7 +2005,7 @@ static int batch_plan_stacks(fn_batch *b, float *const *d_images, std::vector<ch
         hipError_t e = hipMalloc(&R.d_X, x_bytes);
         if (e == hipSuccess) e = hipMemset(R.d_X, 0, x_bytes);  // rows past the last plan stay zero
         if (e == hipSuccess && P0->kprec != FN_PRECISION_FP32) {
-            e = hipMalloc(&R.d_Xlp, n_f * form_planes(P0->kprec) * R.MT_all * P0->KI * 64 * 2);
+            e = hipMalloc(&R.d_Xlp, n_f * form_planes(P0->kprec) * R.n_groups * R.MT_tmpl * P0->KI * 64 * 2);
             if (e == hipSuccess) e = hipMalloc(&R.d_xscale, n_f * sizeof(float));
         }
         if (e == hipSuccess) e = hipMalloc(&R.d_txp, 3 * sizeof(double) * R.rows);
@@ -1972,7 +2041,8 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
         S.write_pad = 0;
         if (int st = launch_spectra_into(P, d_rf[R.plans[m]], dtypes[R.plans[m]], s, R.d_X, S)) return st;
     }
-    if (int st = launch_lowp_planes(P0->kprec, R.d_X, R.d_Xlp, R.d_xscale, P0->g.n_f, R.MT_all, P0->KI, s))
+    if (int st = launch_lowp_planes(P0->kprec, R.d_X, R.d_Xlp, R.d_xscale, P0->g.n_f, R.MT_all, P0->KI,
+                                    R.n_groups * R.MT_tmpl, 0, s))
         return st;
     fnk::BeamArgs A = forward_args(P0);
     A.X = R.d_X;
@@ -1981,6 +2051,7 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
     A.txp = R.d_txp;
     A.n_tx = R.rows;
     A.tx_group = R.MT_tmpl;
+    A.xlp_tiles = R.n_groups * R.MT_tmpl;
     A.bin_chunk = R.chunk;
     A.ens_frames = 0;
     A.ens_slots = 0;
@@ -1992,7 +2063,7 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
     A.partial = nullptr;
     A.n_slots = 1;
     A.slot_z = R.n_groups;
-    const dim3 grid((unsigned)beam_tiles(P0), (unsigned)R.bin_split, (unsigned)R.n_groups);
+    const dim3 grid((unsigned)((P0->n_vox + 63) / 64), (unsigned)R.bin_split, (unsigned)R.n_groups);
     hipError_t e = fnk::kEnsLaunchers[ki_index(P0->KI)][P0->kprec](R.MT_tmpl, P0->wcr, grid, R.lds_beam, s, A, 1);
     if (e != hipSuccess) return hip_fail(e, "beamform_kernel (row stack)");
     return FN_OK;

@@ -90,6 +90,7 @@ struct BeamArgs {
     int n_x, n_z, n_el, n_tx, n_f, n_lb, N;
     int bin_chunk;          // bins per blockIdx.y
     int tx_group;           // M-tiles per blockIdx.z group (PW angle groups)
+    int xlp_tiles;          // M-tiles per bin of the 16-bit planes (lowp_planes_kernel, MT_out)
     int clamp;              // CPU-semantics depth clamp of the PW F-number (das_pw.m:374-377)
     int support_rx, support_tx;        // SUPPORT_* of the receive / transmit window
     int norm_rx, norm_tx;
@@ -298,6 +299,8 @@ __device__ __forceinline__ int row_max16(int v)
 // aperture of a window cut at t = 1 when pitch > width / 2 (elements outside a
 // valid snapped aperture have t - 1 >= (pitch - width/2) / (h + width/2) > 0;
 // the 1e-3 margin keeps that far above float rounding).
+// n_full elements: n_el, or n_el rounded up where the padding has steps of its own, which no
+// support reaches and which are therefore never run.
 inline bool range_free_side(const BeamArgs &A, int support, const WinCoef &w, int n_full)
 {
     if (A.n_el != n_full) return false;
@@ -538,8 +541,10 @@ __device__ __forceinline__ void pack2(float a0, float x0, float a1, float x1, ui
         if (PREC == PREC_FP16X3) {
             asm("" : "+v"(hi));
             const f16x2 h = __builtin_bit_cast(f16x2, hi);
-            lo = __builtin_bit_cast(uint32_t, f16x2{(_Float16)fmaf(a0, x0, -(float)h[0]),
-                                                    (_Float16)fmaf(a1, x1, -(float)h[1])});
+            // v_fma_mix_f32 and one packed conversion: v_fma_mixlo_f16 takes twice as long
+            float l0 = fmaf(a0, x0, -(float)h[0]), l1 = fmaf(a1, x1, -(float)h[1]);
+            asm("" : "+v"(l0), "+v"(l1));
+            lo = __builtin_bit_cast(uint32_t, f16x2{(_Float16)l0, (_Float16)l1});
         }
     }
 }
@@ -648,17 +653,26 @@ struct PersistWavesPerEU {
 // images: a stack's rows are distinct angles, each row with its own transmit phase).
 // NW: windowed normalization (FP32, one bin chunk per block so that every lane
 // counts its voxel's valid rows from the first bin).
+// MIR (plane waves, 16-bit forms, one transmit group): lateral positions symmetric about the
+// array's centre.  Voxel (-x, z) sees element n_el - 1 - k as voxel (x, z) sees element k:
+// same delay, same window.  A lane's voxel stands for both; the upper half of the MT tiles
+// are the transmit rows with the elements in reverse order (planes written so), whose
+// products with the same weights are the mirrored voxel's.  The weights bound the kernel at
+// one or two transmit tiles, and half as many are formed per voxel.
 // One workgroup's share of a plan: voxel tile bx (64 voxels), bin chunk by,
 // transmit group bz.  beamform_kernel runs it for its block index; the
 // persistent batch kernel for every work item it claims.
 template <int MODE, int MT, int KI, int WCR, int WCT, int PREC, bool TAN = false, bool ENS = false, bool NW = false,
-          bool LBL = false, bool STK = false, typename Args = BeamArgs>
+          bool LBL = false, bool STK = false, bool MIR = false, typename Args = BeamArgs>
 __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by, const int bz, const int tid)
 {
     static_assert(!STK || ENS, "row stacks run the ensemble form");
     static_assert(!TAN || (MODE == MODE_PW && PREC == PREC_FP32), "tangent: plane waves, FP32");
     static_assert(!ENS || (MODE == MODE_PW && !TAN), "ensemble: plane waves");
     static_assert(!NW || (PREC == PREC_FP32 && !TAN && !ENS), "windowed normalization: FP32 forward");
+    static_assert(!MIR || (MODE == MODE_PW && PREC != PREC_FP32 && !TAN && !ENS && !NW && !LBL && MT % 2 == 0),
+                  "mirrored voxels: plane-wave forward, 16-bit forms");
+    constexpr int MTH = MIR ? MT / 2 : MT;  // tiles of transmit rows (the others: reversed elements)
     static_assert(!LBL || (MODE == MODE_PW && MT == 1 && !TAN && !ENS && !NW), "line scan: plane-wave forward, one tile");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     // the wave index is uniform: held in a scalar register, so the addresses of the
@@ -669,9 +683,11 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     // line scan: block bz covers depths of grid column bz, the line of transmit row bz
     const long v_loc = (long)bx * 64 + wave * 16 + c;
     const long v = LBL ? (long)bz * A.n_z + v_loc : v_loc;
-    const bool vok = LBL ? v_loc < A.n_z : v < n_vox;
-    const long vv = vok ? v : (LBL ? (long)bz * A.n_z + A.n_z - 1 : n_vox - 1);
+    const long n_own = MIR ? (long)((A.n_x + 1) >> 1) * A.n_z : n_vox;  // voxels with a lane of their own
+    const bool vok = LBL ? v_loc < A.n_z : v < n_own;
+    const long vv = vok ? v : (LBL ? (long)bz * A.n_z + A.n_z - 1 : n_own - 1);
     const int ix = (int)(vv / A.n_z), iz = (int)(vv - (long)ix * A.n_z);
+    const int ix2 = A.n_x - 1 - ix;  // MIR: the mirrored voxel's column
     const double x = A.px[ix], z = A.pz[iz];
     const double xp = x / A.pitch, zp = z / (2.0 * A.pitch);
     const double clamp_z = sqrt(z / (2.88 * A.c0));  // sqrt(f z / (2.88 c)) = sqrt(f) clamp_z (das_pw.m:374)
@@ -699,12 +715,12 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int a = 16 * (mt0 + mt) + 4 * g + r;
+            const int a = 16 * (mt0 + (MIR ? mt % MTH : mt)) + 4 * g + r;
             double tau = 0.0, tg = 0.0;
             if (a < A.n_tx) {
                 if (MODE == MODE_PW) {
                     // das_pw.m:336 (or a virtual source) + i_t0 / f_s
-                    tg = pw_tx_time(A, a, x, z);
+                    tg = pw_tx_time(A, a, MIR && mt >= MTH ? A.px[ix2] : x, z);
                     tau = tg + A.t0 / A.f_s;
                 } else {
                     // transmitting element a: its geometric delay and its delay offset
@@ -722,6 +738,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     const float dg_tx = (float)((4.0 * g - A.M) * A.pitch - x);  // SA transmit rows, mt = r = 0
 
     float Ir = 0.f, Ii = 0.f, w_last = 0.f, wtx_last = 0.f;
+    float Ir2 = 0.f, Ii2 = 0.f;  // MIR: the mirrored voxel
     int nw_row = 0;  // windowed normalization: valid rows of this voxel before the current bin
     float Dr = 0.f, Di = 0.f;  // tangent accumulators
     float Er[ENS ? MT : 1][4], Ei[ENS ? MT : 1][4];  // ensemble: per-row image accumulators
@@ -741,7 +758,8 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     // staged bytes per bin: this group's tiles of every plane
     constexpr int tile_bytes = stage_bytes_per_tile_step<PREC>() * KI;  // one M-tile, all elements
     constexpr int n_f4 = MT * tile_bytes / 16;
-    const int mt_here = min(MT, MT_all - mt0);
+    const int MT_lp = A.xlp_tiles;  // tile stride of the 16-bit planes
+    const int mt_here = min(MT, (PREC == PREC_FP32 ? MT_all : MT_lp) - mt0);
 
     // Staging pipeline: chunk c of bin b is copied by LDS-DMA (global_load_lds_dwordx4,
     // 1 KB per wave instruction: two element steps of one M-tile in FP32, one plane of
@@ -782,7 +800,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             }
         } else if constexpr (LP_CHUNKED) {
             // planes [p][mt][c][64] of 16-byte groups per bin; unit (p, mt) of chunk cq
-            const u32x4 *src = reinterpret_cast<const u32x4 *>(A.Xlp) + (size_t)bq * PL * MT_all * KC * 64;
+            const u32x4 *src = reinterpret_cast<const u32x4 *>(A.Xlp) + (size_t)bq * PL * MT_lp * KC * 64;
             u32x4 *dst = stage_chunk_lp<PREC, MT, cq>();
 #pragma unroll
             for (int i = 0; i < PIPE_LMAX; ++i) {
@@ -790,7 +808,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 if (PIPE_LMAX != PIPE_L && u >= UNITS) break;  // wave-uniform
                 const int pp = u / MT, mt = u - pp * MT;
                 __builtin_amdgcn_global_load_lds(
-                    (__attribute__((address_space(1))) const void *)(src + ((pp * MT_all + mt0 + mt) * KC + cq) * 64 + lane),
+                    (__attribute__((address_space(1))) const void *)(src + ((pp * MT_lp + mt0 + mt) * KC + cq) * 64 + lane),
                     (__attribute__((address_space(3))) void *)(dst + (pp * MT + mt) * 64), 16, 0, 0);
             }
         }
@@ -891,13 +909,13 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 }
             } else if constexpr (LP_CHUNKED) {
                 constexpr int tile4 = KC * 64;  // 16-byte groups per tile per plane
-                const u32x4 *src = reinterpret_cast<const u32x4 *>(A.Xlp) + (size_t)b * PL * MT_all * tile4;
+                const u32x4 *src = reinterpret_cast<const u32x4 *>(A.Xlp) + (size_t)b * PL * MT_lp * tile4;
                 for (int e = tid; e < PL * MT * tile4; e += 256) {
                     const int pp = e / (MT * tile4), rem = e - pp * (MT * tile4);
                     const int mt = rem / tile4, r2 = rem - mt * tile4, cq = r2 >> 6;
                     u32x4 *dst = stage_chunk_lp_at<PREC, MT>(cq);
                     dst[(pp * MT + mt) * 64 + (r2 & 63)] =
-                        (mt < mt_here) ? src[((size_t)pp * MT_all + mt0 + mt) * tile4 + r2] : u32x4{0u, 0u, 0u, 0u};
+                        (mt < mt_here) ? src[((size_t)pp * MT_lp + mt0 + mt) * tile4 + r2] : u32x4{0u, 0u, 0u, 0u};
                 }
             }
             __syncthreads();
@@ -907,11 +925,11 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             __syncthreads();
             float4 *dst = reinterpret_cast<float4 *>(smem_raw);
             constexpr int tile4 = tile_bytes / PL / 16;  // float4 per tile per plane
-            const float4 *src = reinterpret_cast<const float4 *>(A.Xlp) + (size_t)b * PL * MT_all * tile4;
+            const float4 *src = reinterpret_cast<const float4 *>(A.Xlp) + (size_t)b * PL * MT_lp * tile4;
             for (int e = tid; e < n_f4; e += 256) {
                 const int pp = e / (MT * tile4), rem = e - pp * (MT * tile4);
                 const int mt = rem / tile4;
-                dst[e] = (mt < mt_here) ? src[((size_t)pp * MT_all + mt0 + mt) * tile4 + (rem - mt * tile4)]
+                dst[e] = (mt < mt_here) ? src[((size_t)pp * MT_lp + mt0 + mt) * tile4 + (rem - mt * tile4)]
                                         : make_float4(0.f, 0.f, 0.f, 0.f);
             }
             __syncthreads();
@@ -1136,14 +1154,16 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 asum += a;
                 return a;
             };
-            auto chunk_lp = [&](auto cc_const) {
+            // the packed weights of a chunk (32 elements): real and imaginary parts, high and low
+            struct ChunkW {
+                u32x4 rh, rl, ih, il;
+            };
+            // (WC_COS_ALL: every element, in whole chunks)
+            auto active = [&](const int cc) {
+                return WCR == WC_COS_ALL ? cc == 0 || 32 * cc < A.n_el : 8 * cc + 7 >= j_a && 8 * cc <= j_b;
+            };
+            auto weights_lp = [&](auto cc_const, ChunkW &w) __attribute__((always_inline)) {
                 constexpr int cc = decltype(cc_const)::value;
-                if (pipe) chunk_begin(cc_const, b);
-                const u32x4 *xq;
-                if constexpr (LP_CHUNKED) xq = stage_chunk_lp<PREC, MT, cc>();
-                else xq = reinterpret_cast<const u32x4 *>(smem_raw) + cc * 64;
-                if (8 * cc + 7 >= j_a && 8 * cc <= j_b) {  // element steps 8 cc .. 8 cc + 7
-                u32x4 brh, brl, bih, bil;
 #pragma unroll
                 for (int p0 = 0; p0 < 4; p0 += GRAN / 2) {
                     // GRAN element steps at a time, two per packed word; steps outside the
@@ -1158,41 +1178,54 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                             const float a0 = weight(8 * cc + 2 * p, c0, s0), a1 = weight(8 * cc + 2 * p + 1, c1, s1);
                             uint32_t h, l;
                             pack2<PREC>(a0, c0, a1, c1, h, l);
-                            brh[p] = h;
-                            brl[p] = l;
+                            w.rh[p] = h;
+                            w.rl[p] = l;
                             pack2<PREC>(a0, s0, a1, s1, h, l);
-                            bih[p] = h;
-                            bil[p] = l;
+                            w.ih[p] = h;
+                            w.il[p] = l;
                         }
                     } else {
 #pragma unroll
-                        for (int p = p0; p < p0 + GRAN / 2; ++p) brh[p] = brl[p] = bih[p] = bil[p] = 0u;
+                        for (int p = p0; p < p0 + GRAN / 2; ++p) w.rh[p] = w.rl[p] = w.ih[p] = w.il[p] = 0u;
                     }
                 }
-                const u32x4 nbih = neg16(bih);
+            };
+            auto products_lp = [&](auto cc_const, const ChunkW &w) __attribute__((always_inline)) {
+                constexpr int cc = decltype(cc_const)::value;
+                const u32x4 *xq;
+                if constexpr (LP_CHUNKED) xq = stage_chunk_lp<PREC, MT, cc>();
+                else xq = reinterpret_cast<const u32x4 *>(smem_raw) + cc * 64;
+                const u32x4 nih = neg16(w.ih), nil = neg16(w.il);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     const u32x4 xrh = xq[(0 * MT + mt) * XS + lane];
                     const u32x4 xih = xq[(1 * MT + mt) * XS + lane];
-                    accR[mt] = mfma16<PREC>(xrh, brh, accR[mt]);
-                    accR[mt] = mfma16<PREC>(xih, nbih, accR[mt]);
-                    accI[mt] = mfma16<PREC>(xrh, bih, accI[mt]);
-                    accI[mt] = mfma16<PREC>(xih, brh, accI[mt]);
+                    accR[mt] = mfma16<PREC>(xrh, w.rh, accR[mt]);
+                    accI[mt] = mfma16<PREC>(xrh, w.ih, accI[mt]);
+                    accR[mt] = mfma16<PREC>(xih, nih, accR[mt]);
+                    accI[mt] = mfma16<PREC>(xih, w.rh, accI[mt]);
                     if (Prec<PREC>::split) {
                         const u32x4 xrl = xq[(2 * MT + mt) * XS + lane];
                         const u32x4 xil = xq[(3 * MT + mt) * XS + lane];
-                        const u32x4 nbil = neg16(bil);
-                        accR[mt] = mfma16<PREC>(xrh, brl, accR[mt]);
-                        accR[mt] = mfma16<PREC>(xrl, brh, accR[mt]);
-                        accR[mt] = mfma16<PREC>(xih, nbil, accR[mt]);
-                        accR[mt] = mfma16<PREC>(xil, nbih, accR[mt]);
-                        accI[mt] = mfma16<PREC>(xrh, bil, accI[mt]);
-                        accI[mt] = mfma16<PREC>(xrl, bih, accI[mt]);
-                        accI[mt] = mfma16<PREC>(xih, brl, accI[mt]);
-                        accI[mt] = mfma16<PREC>(xil, brh, accI[mt]);
+                        accR[mt] = mfma16<PREC>(xrh, w.rl, accR[mt]);
+                        accI[mt] = mfma16<PREC>(xrh, w.il, accI[mt]);
+                        accR[mt] = mfma16<PREC>(xrl, w.rh, accR[mt]);
+                        accI[mt] = mfma16<PREC>(xrl, w.ih, accI[mt]);
+                        accR[mt] = mfma16<PREC>(xih, nil, accR[mt]);
+                        accI[mt] = mfma16<PREC>(xih, w.rl, accI[mt]);
+                        accR[mt] = mfma16<PREC>(xil, nih, accR[mt]);
+                        accI[mt] = mfma16<PREC>(xil, w.rh, accI[mt]);
                     }
                 }
-                }  // chunk in the support
+            };
+            auto chunk_lp = [&](auto cc_const) {
+                constexpr int cc = decltype(cc_const)::value;
+                if (pipe) chunk_begin(cc_const, b);
+                if (active(cc)) {
+                    ChunkW w;
+                    weights_lp(cc_const, w);
+                    products_lp(cc_const, w);
+                }
                 if (pipe) chunk_end(cc_const, b);
             };  // chunk_lp
             // every chunk of 32 elements: KC = 1, 2, 4, 6 or 8
@@ -1232,6 +1265,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                     Ii += cs * yi + sn * yr;
                 } else {
                 float Sr = 0.f, Si = 0.f;  // sum over the rows of T Y, scaled once below
+                float Sr2 = 0.f, Si2 = 0.f;
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     // ensemble: the four rows of this lane in the tile share their angle
@@ -1258,10 +1292,9 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                         }
                         const float rv = rev_of((uint32_t)n * Qtx[mt][r]);
                         const float sn = __builtin_amdgcn_sinf(rv), cs = __builtin_amdgcn_cosf(rv);
-                        {
-                            Sr = fmaf(cs, accR[mt][r], fmaf(-sn, accI[mt][r], Sr));
-                            Si = fmaf(cs, accI[mt][r], fmaf(sn, accR[mt][r], Si));
-                        }
+                        float &tr = MIR && mt >= MTH ? Sr2 : Sr, &ti = MIR && mt >= MTH ? Si2 : Si;
+                        tr = fmaf(cs, accR[mt][r], fmaf(-sn, accI[mt][r], tr));
+                        ti = fmaf(cs, accI[mt][r], fmaf(sn, accR[mt][r], ti));
                         if (TAN) {
                             const float tt = Ttx[TAN ? mt : 0][r];
                             const float ur = fmaf(tt, accR[mt][r], tanR[TAN ? mt : 0][r]);
@@ -1274,6 +1307,10 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 if (!ENS) {
                     Ir = fmaf(sc, Sr, Ir);
                     Ii = fmaf(sc, Si, Ii);
+                    if (MIR) {
+                        Ir2 = fmaf(sc, Sr2, Ir2);
+                        Ii2 = fmaf(sc, Si2, Ii2);
+                    }
                 }
                 }
                 if (TAN) {
@@ -1292,39 +1329,54 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             float tsum = 0.f;
             // WC_COS_RF: cos^2 of the quarter-period argument max(k r1 + r0, k l1 + l0) for
             // transmitter offset k = 16 t + r from this lane's first row (each side's term
-            // is the larger exactly on its own side); the window's cut is the support test
-            const float sr = at.inv_wr * A.wtx.q_s, sl = at.inv_wl * A.wtx.q_s;
+            // is the larger exactly on its own side); the window's cut is the support test.
+            // WC_COS_ALL likewise, every transmitter.  Both also serve arrays of whole tiles
+            // below 4 KI elements: padding tiles get an argument beyond the cut, or zero.
+            const float wq = WCT == WC_COS_ALL ? A.wtx.s_half : A.wtx.q_s;
+            const float sr = at.inv_wr * wq, sl = at.inv_wl * wq;
+            const float qo = WCT == WC_COS_ALL ? 0.f : A.wtx.q_o;
             const float tr1 = pf * sr, tl1 = -pf * sl;
-            const float tr0 = fmaf(dg_tx, sr, A.wtx.q_o), tl0 = fmaf(-dg_tx, sl, A.wtx.q_o);
-            auto tx_weight = [&](int t, int r) __attribute__((always_inline)) {
-                const int i = 16 * t + 4 * g + r;
-                const float kf = (float)(16 * t + r);
-                if (WCT == WC_COS_RF) {
-                    const float c = __builtin_amdgcn_cosf(
-                        __builtin_amdgcn_fmed3f(fmaxf(fmaf(kf, tr1, tr0), fmaf(kf, tl1, tl0)), 0.f, 0.25f));
-                    return c * c;
-                }
-                const float d = fmaf(kf, pf, dg_tx);
-                const float tt = fabsf(d) * (d < 0.f ? at.inv_wl : at.inv_wr);
-                const float w = window_eval<WCT>(tt, A.wtx);
-                return (i >= at.klo && i <= at.khi) ? w : 0.f;
-            };
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+            const float tr0 = fmaf(dg_tx, sr, qo), tl0 = fmaf(-dg_tx, sl, qo);
+            auto tx_weights4 = [&](int t, float *w4) __attribute__((always_inline)) {
+                const float kt = (float)(16 * t);
+                const bool real = 16 * t < A.n_el;  // wave-uniform
+                const float past = real ? 0.f : 1e9f;
+                const float br = fmaf(kt, tr1, tr0 + past), bl = fmaf(kt, tl1, tl0 + past);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float w = tx_weight(mt0 + mt, r);
-                    wtx[mt][r] = w;
-                    tsum += w;
+                    const float u = r == 0 ? fmaxf(br, bl) : fmaxf(fmaf((float)r, tr1, br), fmaf((float)r, tl1, bl));
+                    if (WCT == WC_COS_RF) {
+                        const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(u, 0.f, 0.25f));
+                        w4[r] = c * c;
+                    } else if (WCT == WC_COS_ALL) {
+                        const float w = fmaf(A.wtx.B, __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(u)), A.wtx.A);
+                        w4[r] = real ? w : 0.f;
+                    } else {
+                        const int i = 16 * t + 4 * g + r;
+                        const float d = fmaf((float)(16 * t + r), pf, dg_tx);
+                        const float tt = fabsf(d) * (d < 0.f ? at.inv_wl : at.inv_wr);
+                        const float w = window_eval<WCT>(tt, A.wtx);
+                        w4[r] = (i >= at.klo && i <= at.khi) ? w : 0.f;
+                    }
                 }
+            };
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                tx_weights4(mt0 + mt, wtx[mt]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tsum += wtx[mt][r];
+            }
             if (MT_all > MT) {
                 // transmit rows split over groups (arrays beyond 128 elements): the
                 // normalization sums the window over every transmitter, not only this
                 // group's (das_sa.m:479)
                 tsum = 0.f;
-                for (int t = 0; t < MT_all; ++t)
+                for (int t = 0; t < MT_all; ++t) {
+                    float w4[4];
+                    tx_weights4(t, w4);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) tsum += tx_weight(t, r);
+                    for (int r = 0; r < 4; ++r) tsum += w4[r];
+                }
             }
             tsum += __shfl_xor(tsum, 16);
             tsum += __shfl_xor(tsum, 32);
@@ -1405,6 +1457,19 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     Ir += __shfl_xor(Ir, 32);
     Ii += __shfl_xor(Ii, 16);
     Ii += __shfl_xor(Ii, 32);
+    if (MIR) {
+        Ir2 += __shfl_xor(Ir2, 16);
+        Ir2 += __shfl_xor(Ir2, 32);
+        Ii2 += __shfl_xor(Ii2, 16);
+        Ii2 += __shfl_xor(Ii2, 32);
+        const long v2 = (long)ix2 * A.n_z + iz;
+        if (g == 0 && vok && ix2 != ix) {  // (the centre column of an odd grid is its own mirror)
+            const float2 val = make_float2(A.out_scale * fmaf(-PHASE_BACK, Ii2, Ir2), A.out_scale * fmaf(PHASE_BACK, Ir2, Ii2));
+            if (A.partial) A.partial[((long)by * A.slot_z + bz) * n_vox + v2] = val;
+            else A.image[v2] = val;
+            if (b_end == A.n_f && A.weights) A.weights[v2] = w_last;
+        }
+    }
     if (TAN) {
         Dr += __shfl_xor(Dr, 16);
         Dr += __shfl_xor(Dr, 32);
@@ -1431,7 +1496,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
 }
 
 template <int MODE, int MT, int KI, int WCR, int WCT, int PREC, bool TAN = false, bool ENS = false, bool NW = false,
-          bool LBL = false, bool STK = false>
+          bool LBL = false, bool STK = false, bool MIR = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BeamWavesPerEU<MT, KI, WCR, PREC, ENS>::value)))
 void beamform_kernel(BeamArgs A)
 {
@@ -1440,7 +1505,7 @@ void beamform_kernel(BeamArgs A)
     // reference form leaves the compiler the registers it schedules best with
     using Args =
         typename std::conditional<(MT * KI <= 64 || PREC != PREC_FP32), BeamArgs, const BeamArgs &>::type;
-    beamform_tile<MODE, MT, KI, WCR, WCT, PREC, TAN, ENS, NW, LBL, STK, Args>(A, blockIdx.x, blockIdx.y, blockIdx.z,
+    beamform_tile<MODE, MT, KI, WCR, WCT, PREC, TAN, ENS, NW, LBL, STK, MIR, Args>(A, blockIdx.x, blockIdx.y, blockIdx.z,
                                                                            threadIdx.x);
 }
 
@@ -1467,7 +1532,7 @@ void beamform_persistent_kernel(const BeamArgs *__restrict__ jobs, const int4 *_
         // recomputed per tile rather than hoisted out of the loop and held across tiles
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
-        beamform_tile<MODE, MT, KI, WCR, WCT, PREC, false, false, false, false, false, const BeamArgs &>(
+        beamform_tile<MODE, MT, KI, WCR, WCT, PREC, false, false, false, false, false, false, const BeamArgs &>(
             A, __builtin_amdgcn_readfirstlane(w.y),
                                                     __builtin_amdgcn_readfirstlane(w.z),
                                                     __builtin_amdgcn_readfirstlane(w.w), tid);
@@ -1509,10 +1574,13 @@ static __global__ __launch_bounds__(256) void reduce_partials_kernel(const float
 // One block per bin: reads the FP32 operand-ordered spectra of the bin, picks a
 // power-of-two scale (16-bit float variants: largest component in [2^14, 2^15)),
 // and writes planes [p][mt][c][64][8] (p: Xr hi, Xi hi, Xr lo, Xi lo) with
-// lane (a & 15) + 16 (k & 3), slot (k >> 2) & 7, chunk k >> 5.
+// lane (a & 15) + 16 (k & 3), slot (k >> 2) & 7, chunk k >> 5.  MT_out tiles are written:
+// those past MT_all are the first ones again with element mirror_el - 1 - k in the place of
+// element k (mirror_el > 0), or zeros, which fill the last transmit group of a launch.
 template <int PREC>
 __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restrict__ X, void *__restrict__ Xlp,
-                                                          float *__restrict__ xscale, int MT_all, int KI)
+                                                          float *__restrict__ xscale, int MT_all, int KI,
+                                                          int MT_out, int mirror_el)
 {
     __shared__ float red[256];
     const int b = blockIdx.x;
@@ -1541,13 +1609,15 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
     const float inv = 1.0f / scale;
     constexpr int pl = Prec<PREC>::planes;
     const int KC = KI / 8;
-    const int plane_elems = MT_all * KC * 64 * 8;  // 16-bit values per plane
+    const int plane_elems = MT_out * KC * 64 * 8;  // 16-bit values per plane
     unsigned short *out = reinterpret_cast<unsigned short *>(Xlp) + (size_t)b * pl * plane_elems;
     for (int o = threadIdx.x; o < plane_elems; o += 256) {
         const int s = o & 7, ln = (o >> 3) & 63, q = o >> 9;  // q = mt * KC + c
         const int mt = q / KC, cc = q - mt * KC;
         const int row = ln & 15, gg = ln >> 4;
-        const float2 v = Xb[(mt * KI + 8 * cc + s) * 64 + row + 16 * gg];  // element 32 cc + 4 s + gg
+        const int k = 32 * cc + 4 * s + gg;
+        const int km = mt < MT_all ? k : mirror_el - 1 - k, mx_t = mt < MT_all ? mt : mt - MT_all;
+        const float2 v = km >= 0 ? Xb[(mx_t * KI + (km >> 2)) * 64 + row + 16 * (km & 3)] : make_float2(0.f, 0.f);
         const float vr = v.x * inv, vi = v.y * inv;
         if (PREC == PREC_BF16X3) {
             const __bf16 rh = (__bf16)vr, ih = (__bf16)vi;

@@ -106,3 +106,35 @@ def test_noalloc_without_room_for_the_planes(fa):
     torch.cuda.synchronize()
     ref = _image(fa, w, rf.cpu().numpy(), "tukey", "cpu")
     assert rel_l2(img.cpu().numpy().T, ref) <= 2 * TOL
+
+
+@pytest.mark.parametrize("n_el,n_ang", [(128, 3), (128, 17), (100, 31), (192, 5)])
+@pytest.mark.parametrize("win", ["tukey", "hann", "boxcar"])
+def test_mirrored_voxels(fa, n_el, n_ang, win):
+    """a lateral grid symmetric about the array (one lane for two voxels) against its columns
+    on a grid that is not, with an odd and an even column count, and with delay offsets that
+    are not symmetric; each side within the bar of the same exact image"""
+    import torch
+
+    w = _workload(n_el, n_ang)
+    rf = torch.from_numpy(w.rf_host()).cuda()
+    d = np.linspace(-30e-9, 50e-9, n_el) ** 2 * 1e7
+    for n_x in (11, 12):
+        x = np.linspace(-15e-3, 15e-3, n_x)
+
+        def image(cols, delays):
+            plan = fa.PwPlan(cols, w.positions_z, w.n_samples, n_el, w.angles, w.f_s, w.width, w.pitch, w.c_0,
+                             w.f_bounds, 0.0, window=_window(fa, win),
+                             F_number=fa.f_numbers.grating.angle_lb(60, 1.5))
+            plan.set_tof(1500.0, delays)
+            img = torch.empty((cols.size, w.positions_z.size), dtype=torch.complex64, device="cuda")
+            wt = torch.empty((cols.size, w.positions_z.size), dtype=torch.float32, device="cuda")
+            plan.execute(rf, img, wt)
+            torch.cuda.synchronize()
+            return img.cpu().numpy(), wt.cpu().numpy()
+
+        print(f"case mirror {n_el} elements {n_ang} angles {win} n_x={n_x}", flush=True)
+        for delays in (None, d):
+            (a, wa), (b, wb) = image(x, delays), image(x[:-1], delays)
+            assert rel_l2(a[:-1], b) <= 2 * TOL
+            np.testing.assert_allclose(wa[:-1], wb, rtol=2e-5)
