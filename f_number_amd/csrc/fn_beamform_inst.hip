@@ -137,6 +137,45 @@ hipError_t FN_TAN_LAUNCHER(INST_KI)(int mt, int wcr, dim3 grid, size_t lds, hipS
     return hipErrorInvalidValue;
 }
 
+#endif
+
+#if INST_PREC == 2 && !FN_WIDE
+// tangent on the fp16 split: mt = 1 or 2 transmit tiles per group; mirror (mt = 1): one more
+// with reversed elements
+#define FN_TAN_LP_LAUNCHER(k) FN_CAT6(launch_beamform_tan, _k, k, _p2, , )
+template <int MT, int WCR, bool MIR>
+static hipError_t launch_tan_lp_one(dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
+{
+    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, 2, true, false, false, false, false, MIR>;
+    static size_t lds_done = 0;
+    lds = dyn_lds(lds);
+    if (hipError_t e = set_lds_once(kern, lds, lds_done)) return e;
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, A);
+    return hipGetLastError();
+}
+
+template <int MT, bool MIR>
+static hipError_t launch_tan_lp_mt(int wcr, dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
+{
+    switch (wcr) {
+    case WC_RANGE: return launch_tan_lp_one<MT, WC_RANGE, MIR>(grid, lds, s, A);
+    case WC_LINEAR: return launch_tan_lp_one<MT, WC_LINEAR, MIR>(grid, lds, s, A);
+    case WC_COS_ALL: return launch_tan_lp_one<MT, WC_COS_ALL, MIR>(grid, lds, s, A);
+    case WC_COS_RF: return launch_tan_lp_one<MT, WC_COS_RF, MIR>(grid, lds, s, A);
+    default: return launch_tan_lp_one<MT, WC_COS, MIR>(grid, lds, s, A);
+    }
+}
+
+hipError_t FN_TAN_LP_LAUNCHER(INST_KI)(int mt, int wcr, bool mirror, dim3 grid, size_t lds, hipStream_t s,
+                                       const BeamArgs &A)
+{
+    if (mt == 1) return mirror ? launch_tan_lp_mt<2, true>(wcr, grid, 2 * lds, s, A) : launch_tan_lp_mt<1, false>(wcr, grid, lds, s, A);
+    if (mt == 2 && !mirror) return launch_tan_lp_mt<2, false>(wcr, grid, lds, s, A);
+    return hipErrorInvalidValue;
+}
+#endif
+
+#if INST_PREC == 0 && !FN_WIDE
 // line scan: block z = grid column = its transmit row, one transmit tile
 #define FN_LBL_LAUNCHER(k) FN_CAT4(launch_beamform_lbl, _k, k, )
 template <int WCR>

@@ -91,6 +91,9 @@ hipError_t launch_focused_signal(const BeamArgs &A, int mode, int wcr, int wct, 
 hipError_t launch_beamform_tan_k8(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
 hipError_t launch_beamform_tan_k16(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
 hipError_t launch_beamform_tan_k32(int, int, dim3, size_t, hipStream_t, const BeamArgs &);
+hipError_t launch_beamform_tan_k8_p2(int, int, bool, dim3, size_t, hipStream_t, const BeamArgs &);
+hipError_t launch_beamform_tan_k16_p2(int, int, bool, dim3, size_t, hipStream_t, const BeamArgs &);
+hipError_t launch_beamform_tan_k32_p2(int, int, bool, dim3, size_t, hipStream_t, const BeamArgs &);
 hipError_t launch_beamform_lbl_k8(int, dim3, hipStream_t, const BeamArgs &);
 hipError_t launch_beamform_lbl_k16(int, dim3, hipStream_t, const BeamArgs &);
 hipError_t launch_beamform_lbl_k32(int, dim3, hipStream_t, const BeamArgs &);
@@ -98,7 +101,7 @@ typedef hipError_t (*LblLauncher)(int, dim3, hipStream_t, const BeamArgs &);
 static const LblLauncher kLblLaunchers[3] = {launch_beamform_lbl_k8, launch_beamform_lbl_k16, launch_beamform_lbl_k32};
 hipError_t launch_adjoint(int wcr, bool tables, bool scale, dim3 grid, hipStream_t s, const AdjArgs &S);
 hipError_t launch_adjoint_reduce(const float *P, float2 *Z, int n_vr, int n_f, int n_at, int n_tx, int n_el,
-                                 hipStream_t s);
+                                 const double *delay, double fs_over_N, int n_lb, hipStream_t s);
 hipError_t launch_adjoint_idft(const float2 *Z, const float2 *tw, float *out, int n_t, int n_ch, int N, int n_lb,
                                int n_f, hipStream_t s);
 hipError_t launch_vjp_delay(const float2 *X, const float2 *Z, double *out, int n_f, int n_tx, int n_el, int MT, int KI,
@@ -168,6 +171,7 @@ struct fn_plan {
     void *d_Xlp = nullptr;    // 16-bit spectra planes (mixed precision)
     float *d_xscale = nullptr;
     double *d_delay = nullptr;  // per-element delay offsets (zeros unless set)
+    double *d_zeros = nullptr;  // zeros in their place
     // adjoint / vector-Jacobian workspace (allocated on first use)
     float *d_P = nullptr;       // voxel-range partials of the voxel contraction
     float2 *d_Z = nullptr;      // reduced contraction [n_f][n_tx][n_el]
@@ -201,10 +205,16 @@ struct fn_plan {
 namespace {
 
 // the forward kernel whose lanes stand for a voxel and its mirror image (beamform_tile, MIR)
-bool use_mirror(const fn_plan *P) { return P->mirror && P->delays_even && P->n_groups == 1; }
+bool use_mirror(const fn_plan *P) { return P->mirror && P->n_groups == 1; }
 
 // M-tiles of the 16-bit planes: the transmit tiles and their mirrored ones, or whole groups
 int plane_tiles(const fn_plan *P) { return use_mirror(P) ? 2 * P->MT_all : P->n_groups * P->MT_tmpl; }
+
+// the tangent with mirrored voxels (mirrored plans run the fp16 split): one tile of rows
+bool tangent_mirror(const fn_plan *P) { return P->mirror && P->MT_all == 1; }
+
+// delay offsets of mirrored plans: taken into the planes unless they are symmetric
+const double *plane_delay(const fn_plan *P, bool mirror) { return mirror && !P->delays_even ? P->d_delay : nullptr; }
 
 // voxel tiles of 64 per beamforming group: the whole grid, half its columns (mirrored
 // voxels), or (line scan) one column
@@ -645,6 +655,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t o_F = cv.take(g.n_f * sizeof(double)), o_Ft = cv.take(Ftx ? g.n_f * sizeof(double) : 0);
     const size_t o_sqf = cv.take(g.n_f * sizeof(double)), o_txp = cv.take(txp.size() * sizeof(double));
     const size_t o_tw = cv.take(tw.size() * sizeof(float2)), o_dl = cv.take(c.n_el * sizeof(double));
+    const size_t o_zr = cv.take(c.n_el * sizeof(double));
     const size_t tables = cv.used;
     const size_t o_X = cv.take(P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
     const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
@@ -668,6 +679,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     P->d_txp = txp.empty() ? nullptr : at(o_txp);
     P->d_tw = reinterpret_cast<float2 *>(at(o_tw));
     P->d_delay = at(o_dl);
+    P->d_zeros = at(o_zr);
     P->d_X = reinterpret_cast<float2 *>(at(o_X));
     P->d_Xlp = P->xlp_bytes ? at(o_Xlp) : nullptr;
     P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
@@ -802,6 +814,7 @@ fnk::BeamArgs forward_args(const fn_plan *P)
 fnk::BeamArgs beam_args(const fn_plan *P, float *d_image, float *d_w, float *d_w_rx)
 {
     fnk::BeamArgs A = forward_args(P);
+    if (plane_delay(P, use_mirror(P))) A.delay = P->d_zeros;  // in the planes already
     A.image = reinterpret_cast<float2 *>(d_image);
     A.n_slots = beam_slots(P);
     A.slot_z = P->lbl ? 1 : P->n_groups;
@@ -816,26 +829,26 @@ fnk::BeamArgs beam_args(const fn_plan *P, float *d_image, float *d_w, float *d_w
     return A;
 }
 
-// the 16-bit operand planes (and per-bin scales) of FP32 spectra X of MT tiles;
-// nothing for FP32 plans
-// MT_out, mirror_el: see lowp_planes_kernel
-int launch_lowp_planes(int precision, const float2 *X, void *Xlp, float *xscale, int n_f, int MT, int KI, int MT_out,
-                       int mirror_el, hipStream_t s)
+// the 16-bit operand planes (and per-bin scales) of FP32 spectra X of MT tiles (MT_out,
+// mirror_el, delay: see lowp_planes_kernel); nothing for FP32 kernels
+int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xscale, int MT, int MT_out, int mirror_el,
+                       const double *delay, hipStream_t s)
 {
-    if (precision == FN_PRECISION_FP32) return FN_OK;
-    const dim3 cg((unsigned)n_f), cb(256);
-    switch (precision) {
+    const dim3 cg((unsigned)P->g.n_f), cb(256);
+    const double fs_over_N = P->args.f_s / P->g.N;
+    switch (P->kprec) {
+    case FN_PRECISION_FP32: return FN_OK;
     case FN_PRECISION_BF16X3:
-        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_BF16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, KI, MT_out,
-                           mirror_el);
+        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_BF16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el);
         break;
     case FN_PRECISION_FP16X3:
-        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, KI, MT_out,
-                           mirror_el);
+        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el);
         break;
     default:
-        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16>, cg, cb, 0, s, X, Xlp, xscale, MT, KI, MT_out,
-                           mirror_el);
+        hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el);
         break;
     }
     HIP_CHECK(hipGetLastError(), "lowp_planes_kernel");
@@ -865,8 +878,8 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
     }
     const fnk::SpecArgs &S = P->sargs;
     if (int st = launch_spectra(P, d_rf, dtype, s)) return st;
-    return launch_lowp_planes(P->kprec, P->d_X, P->d_Xlp, P->d_xscale, S.n_f, S.MT, S.KI, plane_tiles(P),
-                              use_mirror(P) ? P->n_el : 0, s);
+    return launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, S.MT, plane_tiles(P), use_mirror(P) ? P->n_el : 0,
+                              plane_delay(P, use_mirror(P)), s);
 }
 
 int execute(fn_plan *P, const void *d_rf, int dtype, float *d_image, float *d_w, float *d_w_rx, hipStream_t user)
@@ -1144,7 +1157,19 @@ int execute_tangent(fn_plan *P, const void *d_rf, int dtype, float *d_image, flo
     // groups of at most two transmit tiles keep the tangent accumulators in registers
     const int mt = std::min(P->MT_all, 2);
     const int groups = (P->MT_all + mt - 1) / mt;
-    fnk::BeamArgs A = P->args;
+    // plans whose forward runs the fp16 split contract the tangent on it too (11 angles, 384 x
+    // 384, 542 bins: 14.7 ms in FP32, 9.7 split, 6.8 mirrored), with mirrored voxels where one tile holds every row (four tiles of both
+    // accumulators would spill)
+    const bool split_form = P->kprec == FN_PRECISION_FP16X3;
+    const bool mirror = tangent_mirror(P);
+    if (split_form) {
+        if (int st = launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, P->MT_all, mirror ? 2 * P->MT_all : groups * mt,
+                                        mirror ? P->n_el : 0, plane_delay(P, mirror), s))
+            return st;
+    }
+    fnk::BeamArgs A = split_form ? forward_args(P) : P->args;
+    if (plane_delay(P, mirror)) A.delay = P->d_zeros;
+    A.xlp_tiles = mirror ? 2 * P->MT_all : groups * mt;
     A.image = reinterpret_cast<float2 *>(d_image);
     A.dimage = d_dimage;
     A.weights = d_w;
@@ -1153,7 +1178,7 @@ int execute_tangent(fn_plan *P, const void *d_rf, int dtype, float *d_image, flo
     // bin chunks: at least the plan's, and about 8192 workgroups (at most 8 chunks) when
     // the grid is smaller -- 11 angles, 384 x 384, 542 bins: 17.5 ms in one chunk,
     // 15.7-15.8 ms in 4 or 8
-    const long tiles = (P->n_vox + 63) / 64;
+    const long tiles = ((mirror ? (long)((P->n_x + 1) / 2) * P->n_z : P->n_vox) + 63) / 64;
     int split = P->bin_split;
     if (tiles * groups * split < 8192)
         split = std::max(split, (int)std::min<long>({(8192 + tiles * groups - 1) / (tiles * groups), 8L,
@@ -1176,12 +1201,19 @@ int execute_tangent(fn_plan *P, const void *d_rf, int dtype, float *d_image, flo
         }
         A.partial = P->d_ptan;
     }
-    const size_t lds = (size_t)mt * P->KI * 64 * sizeof(float2);
+    const size_t lds = (size_t)mt * P->KI * 64 * sizeof(float2);  // the split's planes are as large
     const dim3 grid((unsigned)tiles, (unsigned)split, (unsigned)groups);
-    const int wcr = wcr_general(P->wcr);
-    hipError_t e = P->KI == 8 ? fnk::launch_beamform_tan_k8(mt, wcr, grid, lds, s, A)
-                 : P->KI == 16 ? fnk::launch_beamform_tan_k16(mt, wcr, grid, lds, s, A)
-                               : fnk::launch_beamform_tan_k32(mt, wcr, grid, lds, s, A);
+    hipError_t e;
+    if (split_form) {
+        e = P->KI == 8    ? fnk::launch_beamform_tan_k8_p2(mt, P->wcr, mirror, grid, lds, s, A)
+            : P->KI == 16 ? fnk::launch_beamform_tan_k16_p2(mt, P->wcr, mirror, grid, lds, s, A)
+                          : fnk::launch_beamform_tan_k32_p2(mt, P->wcr, mirror, grid, lds, s, A);
+    } else {
+        const int wcr = wcr_general(P->wcr);
+        e = P->KI == 8    ? fnk::launch_beamform_tan_k8(mt, wcr, grid, lds, s, A)
+            : P->KI == 16 ? fnk::launch_beamform_tan_k16(mt, wcr, grid, lds, s, A)
+                          : fnk::launch_beamform_tan_k32(mt, wcr, grid, lds, s, A);
+    }
     if (e != hipSuccess) return hip_fail(e, "beamform tangent kernel");
     return finish_beam(P, A, s, reinterpret_cast<float2 *>(d_dimage));
 }
@@ -1215,16 +1247,23 @@ int contract_adjoint(fn_plan *P, const float *d_y, hipStream_t s)
         // phase words (128 + 16 n_at per voxel) followed by 4 doubles of aperture terms per voxel
         HIP_CHECK(hipMalloc(&P->d_qtab, (size_t)P->n_vox * (128 + 16 * P->adj_at + 8) * sizeof(uint32_t)),
                   "phase tables");
-        HIP_CHECK(hipMalloc(&P->d_vsc, (size_t)n_f * P->n_vox * sizeof(float)), "adjoint normalization");
+        // s / w_n(v) per bin and voxel, then two scale factors per bin
+        HIP_CHECK(hipMalloc(&P->d_vsc, ((size_t)n_f * P->n_vox + 2 * n_f) * sizeof(float)), "adjoint normalization");
     }
     fnk::AdjArgs S{};
     S.B = P->args;
+    // the delay offsets where the tangent has them: a gradient's real parts dwarf its imaginary
+    // ones, and cancel only between phases rounded alike (64 elements, 3 angles: d J / d delay
+    // 2.9e-6 from 64 bits with the offsets in the tangent's planes and the adjoint's words)
+    const double *delay = plane_delay(P, tangent_mirror(P));
+    if (delay) S.B.delay = P->d_zeros;
     S.y = reinterpret_cast<const float2 *>(d_y);
     S.P = P->d_P;
     S.qrx = P->d_qtab;
     S.qtx = P->d_qtab + (size_t)P->n_vox * 128;
     S.vgeo = reinterpret_cast<const double *>(P->d_qtab + (size_t)P->n_vox * (128 + 16 * P->adj_at));
     S.vsc = P->d_vsc;
+    S.us = P->d_vsc + (size_t)n_f * P->n_vox;
     S.vox_per_range = P->adj_vpr;
     S.n_at = P->adj_at;
     // bin quads fastest: the workgroups dispatched together share a voxel range, whose
@@ -1245,7 +1284,8 @@ int contract_adjoint(fn_plan *P, const float *d_y, hipStream_t s)
         P->adj_sc_stream = s;
     }
     if (e != hipSuccess) return hip_fail(e, "adjoint_kernel");
-    e = fnk::launch_adjoint_reduce(P->d_P, P->d_Z, P->adj_vr, n_f, P->adj_at, P->n_tx, P->n_el, s);
+    e = fnk::launch_adjoint_reduce(P->d_P, P->d_Z, P->adj_vr, n_f, P->adj_at, P->n_tx, P->n_el, delay,
+                                   P->args.f_s / P->g.N, P->g.n_lb, s);
     if (e != hipSuccess) return hip_fail(e, "adjoint_reduce_kernel");
     return FN_OK;
 }
@@ -2041,8 +2081,7 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
         S.write_pad = 0;
         if (int st = launch_spectra_into(P, d_rf[R.plans[m]], dtypes[R.plans[m]], s, R.d_X, S)) return st;
     }
-    if (int st = launch_lowp_planes(P0->kprec, R.d_X, R.d_Xlp, R.d_xscale, P0->g.n_f, R.MT_all, P0->KI,
-                                    R.n_groups * R.MT_tmpl, 0, s))
+    if (int st = launch_lowp_planes(P0, R.d_X, R.d_Xlp, R.d_xscale, R.MT_all, R.n_groups * R.MT_tmpl, 0, nullptr, s))
         return st;
     fnk::BeamArgs A = forward_args(P0);
     A.X = R.d_X;

@@ -129,6 +129,7 @@ struct AdjArgs {
     const uint32_t *qtx;    // transmit phase words [n_vox][16 n_at]
     const double *vgeo;     // per voxel: x, x / pitch, z / (2 pitch), sqrt(z / (2.88 c0))
     const float *vsc;       // per bin and voxel [n_f][n_vox]: s / w_n(v), 0 outside a valid aperture
+    const float *us;        // split contraction: per bin the cotangent's scale, then what takes it out
     long vox_per_range;     // multiple of 64
     int n_at;               // angle tiles of 16
 };
@@ -574,12 +575,13 @@ struct WavesPerEU {
 
 // One-launch-per-plan kernel: the smallest tiles (MT x KI <= 32) are held to 3
 // waves per SIMD where they fit without spilling (FP32, fp16, and the split forms
-// with the cosine windows WC_COS_ALL / WC_COS_RF; not the ensemble epilogue);
+// with the cosine windows WC_COS_ALL / WC_COS_RF; not the ensemble epilogue nor the
+// split's tangent);
 // otherwise WavesPerEU.
-template <int MT, int KI, int WCR, int PREC, bool ENS>
+template <int MT, int KI, int WCR, int PREC, bool ENS, bool TAN>
 struct BeamWavesPerEU {
     static constexpr bool fits3 =
-        !ENS && (PREC == PREC_FP32 || PREC == PREC_FP16 || WCR == WC_COS_ALL || WCR == WC_COS_RF);
+        !ENS && !(TAN && PREC != PREC_FP32) && (PREC == PREC_FP32 || PREC == PREC_FP16 || WCR == WC_COS_ALL || WCR == WC_COS_RF);
     static constexpr int value = (MT * KI <= 32 && fits3) ? 3 : WavesPerEU<MT, KI>::value;
 };
 
@@ -643,9 +645,10 @@ struct PersistWavesPerEU {
     static constexpr int value = (MODE == MODE_PW && MT <= 3 && MT * KI <= 64 && fits3) ? 3 : WavesPerEU<MT, KI>::value;
 };
 
-// TAN (plane waves, FP32): also accumulates the tangent dI/dc_tof.  Geometric
+// TAN (plane waves, FP32 or the fp16 split): also accumulates the tangent dI/dc_tof.  Geometric
 // delays scale as 1/c, so d/dc e^{j w tau} = j w (-(tau_tx,g + tau_rx,g) / c) e^{j w tau}:
-// a second contraction with B' = B tau_rx,g and the row factor tau_tx,g.
+// a second contraction with B' = B tau_rx,g and the row factor tau_tx,g (in seconds; the
+// split takes them in DFT periods N / f_s, so that its operands stay below 1).
 // ENS (plane waves): the transmit rows are (angle, frame slot) pairs of an ensemble
 // sharing one geometry, angle-major; every row keeps its own image accumulator over
 // the bins and is added to its frame's image at the end (frame = row % ens_slots when
@@ -667,11 +670,11 @@ template <int MODE, int MT, int KI, int WCR, int WCT, int PREC, bool TAN = false
 __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by, const int bz, const int tid)
 {
     static_assert(!STK || ENS, "row stacks run the ensemble form");
-    static_assert(!TAN || (MODE == MODE_PW && PREC == PREC_FP32), "tangent: plane waves, FP32");
+    static_assert(!TAN || (MODE == MODE_PW && (PREC == PREC_FP32 || PREC == PREC_FP16X3)), "tangent: plane waves");
     static_assert(!ENS || (MODE == MODE_PW && !TAN), "ensemble: plane waves");
     static_assert(!NW || (PREC == PREC_FP32 && !TAN && !ENS), "windowed normalization: FP32 forward");
-    static_assert(!MIR || (MODE == MODE_PW && PREC != PREC_FP32 && !TAN && !ENS && !NW && !LBL && MT % 2 == 0),
-                  "mirrored voxels: plane-wave forward, 16-bit forms");
+    static_assert(!MIR || (MODE == MODE_PW && PREC != PREC_FP32 && !ENS && !NW && !LBL && MT % 2 == 0),
+                  "mirrored voxels: plane waves, 16-bit forms");
     constexpr int MTH = MIR ? MT / 2 : MT;  // tiles of transmit rows (the others: reversed elements)
     static_assert(!LBL || (MODE == MODE_PW && MT == 1 && !TAN && !ENS && !NW), "line scan: plane-wave forward, one tile");
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -698,7 +701,8 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     const double zc = z / A.ctof;
     const double t_half = (MODE == MODE_SA) ? 0.5 * A.t0 / A.f_s : 0.0;  // das_sa.m:431
     uint32_t Qrx[KI];
-    float Trx[TAN ? KI : 1];  // tangent: geometric receive time (s)
+    float Trx[TAN ? KI : 1];  // tangent: geometric receive time
+    const double t_unit = PREC == PREC_FP32 ? 1.0 : A.f_s / A.N;
 #pragma unroll
     for (int j = 0; j < KI; ++j) {
         const int k = 4 * j + g;
@@ -706,11 +710,11 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
         const double tg = sqrt(lat * lat + zc * zc);
         const double tau = tg + t_half + (k < A.n_el ? A.delay[k] : 0.0);
         Qrx[j] = frac32(A.f_s * tau / A.N);
-        if (TAN) Trx[TAN ? j : 0] = (float)tg;
+        if (TAN) Trx[TAN ? j : 0] = (float)(tg * t_unit);
     }
     // transmit phase increments for the rows this lane holds
     uint32_t Qtx[MT][4];
-    float Ttx[TAN ? MT : 1][4];  // tangent: geometric transmit time (s)
+    float Ttx[TAN ? MT : 1][4];  // tangent: geometric transmit time
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -729,7 +733,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 }
             }
             Qtx[mt][r] = frac32(A.f_s * tau / A.N);
-            if (TAN) Ttx[TAN ? mt : 0][r] = (float)tg;
+            if (TAN) Ttx[TAN ? mt : 0][r] = (float)(tg * t_unit);
         }
     // line scan: the phase increment of the block's own transmit row
     const uint32_t Qln = LBL ? frac32(A.f_s * (pw_tx_time(A, bz, x, z) + A.t0 / A.f_s) / A.N) : 0u;
@@ -740,7 +744,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
     float Ir = 0.f, Ii = 0.f, w_last = 0.f, wtx_last = 0.f;
     float Ir2 = 0.f, Ii2 = 0.f;  // MIR: the mirrored voxel
     int nw_row = 0;  // windowed normalization: valid rows of this voxel before the current bin
-    float Dr = 0.f, Di = 0.f;  // tangent accumulators
+    float Dr = 0.f, Di = 0.f, Dr2 = 0.f, Di2 = 0.f;  // tangent accumulators (and the mirrored voxel's)
     float Er[ENS ? MT : 1][4], Ei[ENS ? MT : 1][4];  // ensemble: per-row image accumulators
     if (ENS) {
 #pragma unroll
@@ -749,7 +753,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             for (int r = 0; r < 4; ++r) Er[ENS ? mt : 0][r] = Ei[ENS ? mt : 0][r] = 0.f;
     }
     // w_n = n * 2 pi f_s / N; the tangent factor -w_n / c_tof is applied per bin
-    const float w_unit = (float)(2.0 * 3.141592653589793 * A.f_s / A.N);
+    const float w_unit = (float)(2.0 * 3.141592653589793 * (PREC == PREC_FP32 ? A.f_s / A.N : 1.0));
     const float inv_c = (float)(1.0 / A.ctof);
     const float inv_peak = PREC == PREC_FP16X3 ? A.wrx.inv_peak : 1.0f;
     const int b_begin = by * A.bin_chunk;
@@ -1114,6 +1118,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             for (int mt = 0; mt < MT; ++mt) {
                 accR[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
                 accI[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+                if (TAN) tanR[TAN ? mt : 0] = tanI[TAN ? mt : 0] = floatx4{0.f, 0.f, 0.f, 0.f};
             }
             // the window's argument of element step j as in the FP32 form: the larger of two
             // linear functions of j, each the larger exactly on its own side
@@ -1157,6 +1162,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             // the packed weights of a chunk (32 elements): real and imaginary parts, high and low
             struct ChunkW {
                 u32x4 rh, rl, ih, il;
+                u32x4 trh, trl, tih, til;  // tangent: times the receive time
             };
             // (WC_COS_ALL: every element, in whole chunks)
             auto active = [&](const int cc) {
@@ -1183,10 +1189,22 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                             pack2<PREC>(a0, s0, a1, s1, h, l);
                             w.ih[p] = h;
                             w.il[p] = l;
+                            if (TAN) {
+                                const float t0 = a0 * Trx[TAN ? 8 * cc + 2 * p : 0], t1 = a1 * Trx[TAN ? 8 * cc + 2 * p + 1 : 0];
+                                pack2<PREC>(t0, c0, t1, c1, h, l);
+                                w.trh[p] = h;
+                                w.trl[p] = l;
+                                pack2<PREC>(t0, s0, t1, s1, h, l);
+                                w.tih[p] = h;
+                                w.til[p] = l;
+                            }
                         }
                     } else {
 #pragma unroll
-                        for (int p = p0; p < p0 + GRAN / 2; ++p) w.rh[p] = w.rl[p] = w.ih[p] = w.il[p] = 0u;
+                        for (int p = p0; p < p0 + GRAN / 2; ++p) {
+                            w.rh[p] = w.rl[p] = w.ih[p] = w.il[p] = 0u;
+                            if (TAN) w.trh[p] = w.trl[p] = w.tih[p] = w.til[p] = 0u;
+                        }
                     }
                 }
             };
@@ -1196,6 +1214,11 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 if constexpr (LP_CHUNKED) xq = stage_chunk_lp<PREC, MT, cc>();
                 else xq = reinterpret_cast<const u32x4 *>(smem_raw) + cc * 64;
                 const u32x4 nih = neg16(w.ih), nil = neg16(w.il);
+                u32x4 ntih, ntil;
+                if (TAN) {
+                    ntih = neg16(w.tih);
+                    ntil = neg16(w.til);
+                }
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     const u32x4 xrh = xq[(0 * MT + mt) * XS + lane];
@@ -1215,6 +1238,21 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                         accI[mt] = mfma16<PREC>(xih, w.rl, accI[mt]);
                         accR[mt] = mfma16<PREC>(xil, nih, accR[mt]);
                         accI[mt] = mfma16<PREC>(xil, w.rh, accI[mt]);
+                        if (TAN) {
+                            floatx4 &tR = tanR[TAN ? mt : 0], &tI = tanI[TAN ? mt : 0];
+                            tR = mfma16<PREC>(xrh, w.trh, tR);
+                            tI = mfma16<PREC>(xrh, w.tih, tI);
+                            tR = mfma16<PREC>(xih, ntih, tR);
+                            tI = mfma16<PREC>(xih, w.trh, tI);
+                            tR = mfma16<PREC>(xrh, w.trl, tR);
+                            tI = mfma16<PREC>(xrh, w.til, tI);
+                            tR = mfma16<PREC>(xrl, w.trh, tR);
+                            tI = mfma16<PREC>(xrl, w.tih, tI);
+                            tR = mfma16<PREC>(xih, ntil, tR);
+                            tI = mfma16<PREC>(xih, w.trl, tI);
+                            tR = mfma16<PREC>(xil, ntih, tR);
+                            tI = mfma16<PREC>(xil, w.trh, tI);
+                        }
                     }
                 }
             };
@@ -1256,6 +1294,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 const float sc = (A.norm_rx ? __builtin_amdgcn_rcpf(asum) : inv_peak) * xscale;
                 // padded transmit rows have zero spectra, so every row is summed
                 float pr = 0.f, pi = 0.f;  // tangent: sum_rows T (tau_tx,g Y + Y')
+                float pr2 = 0.f, pi2 = 0.f;
                 if constexpr (LBL) {
                     // the lane's partial product over its elements, at the line's own transmit phase
                     const float rv = rev_of((uint32_t)n * Qln);
@@ -1299,8 +1338,9 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                             const float tt = Ttx[TAN ? mt : 0][r];
                             const float ur = fmaf(tt, accR[mt][r], tanR[TAN ? mt : 0][r]);
                             const float ui = fmaf(tt, accI[mt][r], tanI[TAN ? mt : 0][r]);
-                            pr += cs * ur - sn * ui;
-                            pi += cs * ui + sn * ur;
+                            float &qr = MIR && mt >= MTH ? pr2 : pr, &qi = MIR && mt >= MTH ? pi2 : pi;
+                            qr += cs * ur - sn * ui;
+                            qi += cs * ui + sn * ur;
                         }
                     }
                 }
@@ -1318,6 +1358,10 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                     const float f = -sc * (float)n * w_unit * inv_c;
                     Dr = fmaf(-f, pi, Dr);
                     Di = fmaf(f, pr, Di);
+                    if (MIR) {
+                        Dr2 = fmaf(-f, pi2, Dr2);
+                        Di2 = fmaf(f, pr2, Di2);
+                    }
                 }
             }
             if (NW) nw_row += ap.valid ? 1 : 0;
@@ -1462,11 +1506,24 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
         Ir2 += __shfl_xor(Ir2, 32);
         Ii2 += __shfl_xor(Ii2, 16);
         Ii2 += __shfl_xor(Ii2, 32);
+        if (TAN) {
+            Dr2 += __shfl_xor(Dr2, 16);
+            Dr2 += __shfl_xor(Dr2, 32);
+            Di2 += __shfl_xor(Di2, 16);
+            Di2 += __shfl_xor(Di2, 32);
+        }
         const long v2 = (long)ix2 * A.n_z + iz;
         if (g == 0 && vok && ix2 != ix) {  // (the centre column of an odd grid is its own mirror)
             const float2 val = make_float2(A.out_scale * fmaf(-PHASE_BACK, Ii2, Ir2), A.out_scale * fmaf(PHASE_BACK, Ir2, Ii2));
-            if (A.partial) A.partial[((long)by * A.slot_z + bz) * n_vox + v2] = val;
-            else A.image[v2] = val;
+            const float2 dval = make_float2(A.out_scale * fmaf(-PHASE_BACK, Di2, Dr2), A.out_scale * fmaf(PHASE_BACK, Dr2, Di2));
+            const long slot = (long)by * A.slot_z + bz;
+            if (A.partial) {
+                A.partial[slot * n_vox + v2] = val;
+                if (TAN) A.partial[((long)A.n_slots + slot) * n_vox + v2] = dval;
+            } else {
+                A.image[v2] = val;
+                if (TAN) reinterpret_cast<float2 *>(A.dimage)[v2] = dval;
+            }
             if (b_end == A.n_f && A.weights) A.weights[v2] = w_last;
         }
     }
@@ -1497,7 +1554,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
 
 template <int MODE, int MT, int KI, int WCR, int WCT, int PREC, bool TAN = false, bool ENS = false, bool NW = false,
           bool LBL = false, bool STK = false, bool MIR = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BeamWavesPerEU<MT, KI, WCR, PREC, ENS>::value)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BeamWavesPerEU<MT, KI, WCR, PREC, ENS, TAN>::value)))
 void beamform_kernel(BeamArgs A)
 {
     // small tiles take the arguments by value (their register count decides the
@@ -1577,10 +1634,13 @@ static __global__ __launch_bounds__(256) void reduce_partials_kernel(const float
 // lane (a & 15) + 16 (k & 3), slot (k >> 2) & 7, chunk k >> 5.  MT_out tiles are written:
 // those past MT_all are the first ones again with element mirror_el - 1 - k in the place of
 // element k (mirror_el > 0), or zeros, which fill the last transmit group of a launch.
+// delay: per-element delay offsets d_k taken into the spectra as e^{j w_n d_k} (null: left to
+// the kernels' phase words); the mirrored tiles' weights then stay alike on both sides.
 template <int PREC>
 __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restrict__ X, void *__restrict__ Xlp,
                                                           float *__restrict__ xscale, int MT_all, int KI,
-                                                          int MT_out, int mirror_el)
+                                                          int MT_out, int mirror_el, const double *__restrict__ delay,
+                                                          double fs_over_N, int n_lb, int n_el)
 {
     __shared__ float red[256];
     const int b = blockIdx.x;
@@ -1617,7 +1677,14 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
         const int row = ln & 15, gg = ln >> 4;
         const int k = 32 * cc + 4 * s + gg;
         const int km = mt < MT_all ? k : mirror_el - 1 - k, mx_t = mt < MT_all ? mt : mt - MT_all;
-        const float2 v = km >= 0 ? Xb[(mx_t * KI + (km >> 2)) * 64 + row + 16 * (km & 3)] : make_float2(0.f, 0.f);
+        float2 v = km >= 0 ? Xb[(mx_t * KI + (km >> 2)) * 64 + row + 16 * (km & 3)] : make_float2(0.f, 0.f);
+        if (delay && km >= 0 && km < n_el) {
+            // n frac(f_s d / N) mod 1 in units of 2^-32, then half revolutions
+            const uint32_t P = (uint32_t)(n_lb + b) * frac32(fs_over_N * delay[km]);
+            float sn, cs;
+            sincospif((float)(int32_t)P * (1.0f / 2147483648.0f), &sn, &cs);
+            v = make_float2(v.x * cs - v.y * sn, v.x * sn + v.y * cs);
+        }
         const float vr = v.x * inv, vi = v.y * inv;
         if (PREC == PREC_BF16X3) {
             const __bf16 rh = (__bf16)vr, ih = (__bf16)vi;
