@@ -104,6 +104,12 @@ hipError_t launch_adjoint_reduce(const float *P, float2 *Z, int n_vr, int n_f, i
                                  const double *delay, double fs_over_N, int n_lb, hipStream_t s);
 hipError_t launch_adjoint_idft(const float2 *Z, const float2 *tw, float *out, int n_t, int n_ch, int N, int n_lb,
                                int n_f, hipStream_t s);
+hipError_t launch_interp_tables(float2 *tw, float *ipsi, int M, int n_f, hipStream_t s);
+hipError_t launch_interp_samples(const float2 *X, const float2 *tw, const float *ipsi, float2 *G, int M, int n_f, int MT,
+                                 int KI, int n_tx, int n_el, hipStream_t s);
+hipError_t launch_interp_beamform(int wcr, const InterpArgs &S, hipStream_t s);
+size_t interp_table_floats2(int M, int n_tx, int n_el);
+int interp_groups(int n_tx);
 hipError_t launch_vjp_delay(const float2 *X, const float2 *Z, double *out, int n_f, int n_tx, int n_el, int MT, int KI,
                             int n_lb, double w_unit, hipStream_t s);
 hipError_t launch_dot_re(const float2 *g, const float2 *d, long n, double *part, int n_part, double *out, hipStream_t s);
@@ -119,6 +125,16 @@ static const BeamLauncher kBeamLaunchers[2][5][4] = {
     {FN_BEAM_ROW(0, 8), FN_BEAM_ROW(0, 16), FN_BEAM_ROW(0, 32), FN_BEAM_ROW(0, 48), FN_BEAM_ROW(0, 64)},
     {FN_BEAM_ROW(1, 8), FN_BEAM_ROW(1, 16), FN_BEAM_ROW(1, 32), FN_BEAM_ROW(1, 48), FN_BEAM_ROW(1, 64)}};
 #undef FN_BEAM_ROW
+// image (and weights, where given) of n_z depths per column into the first depths of columns of NZ
+__global__ void paste_depths_kernel(const float2 *img, const float *w, long n, int n_z, int NZ, float2 *out, float *w_out)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const long o = i / n_z * NZ + i % n_z;
+    out[o] = img[i];
+    if (w) w_out[o] = w[i];
+}
+
 // zero fill used instead of hipMemsetAsync so the launch sequence stays
 // capturable into a graph
 __global__ void fill_zero_kernel(float *p, long n)
@@ -161,6 +177,13 @@ struct fn_plan {
     int kprec = FN_PRECISION_FP32;      // form of the forward contraction (kernel_precision)
     int mirror = 0;         // lateral positions symmetric: planes hold the reversed elements too
     int delays_even = 1;    // delay offsets symmetric about the array's centre
+    int interp_M = 0;       // > 0: the forward image by interpolation of M samples per channel
+    float2 *d_ip = nullptr; // its channel samples, twiddles [M] and 1 / psi [n_f]
+    // interpolated plans with depths where the F-number clamp is at work: a plan of those
+    // leading depths (on this plan's spectra), its image and weights, pasted over the first rows
+    fn_plan *shallow = nullptr;
+    float2 *d_simg = nullptr;
+    float *d_sw = nullptr;
     int verbosity = 0;
     fnk::BeamArgs args{};
     fnk::SpecArgs sargs{};
@@ -205,7 +228,7 @@ struct fn_plan {
 namespace {
 
 // the forward kernel whose lanes stand for a voxel and its mirror image (beamform_tile, MIR)
-bool use_mirror(const fn_plan *P) { return P->mirror && P->n_groups == 1; }
+bool use_mirror(const fn_plan *P) { return P->mirror && P->n_groups == 1 && !P->interp_M; }
 
 // M-tiles of the 16-bit planes: the transmit tiles and their mirrored ones, or whole groups
 int plane_tiles(const fn_plan *P) { return use_mirror(P) ? 2 * P->MT_all : P->n_groups * P->MT_tmpl; }
@@ -226,7 +249,11 @@ long beam_tiles(const fn_plan *P)
 
 // workgroups that share a voxel: bin chunks times transmit groups (a line scan's
 // groups are its columns, one per voxel); ensembles add their frames' rows atomically
-int beam_slots(const fn_plan *P) { return P->n_frames > 1 ? 1 : P->bin_split * (P->lbl ? 1 : P->n_groups); }
+int beam_slots(const fn_plan *P)
+{
+    if (P->interp_M) return fnk::interp_groups(P->n_tx);
+    return P->n_frames > 1 ? 1 : P->bin_split * (P->lbl ? 1 : P->n_groups);
+}
 
 int hip_fail(hipError_t e, const char *what)
 {
@@ -457,7 +484,8 @@ struct Common {
 void destroy(fn_plan *p)
 {
     if (!p) return;
-    hipFree(p->d_block); hipFree(p->d_P); hipFree(p->d_Z); hipFree(p->d_part); hipFree(p->d_qtab); hipFree(p->d_vsc); hipFree(p->d_nw);
+    destroy(p->shallow);
+    hipFree(p->d_block); hipFree(p->d_ip); hipFree(p->d_simg); hipFree(p->d_sw); hipFree(p->d_P); hipFree(p->d_Z); hipFree(p->d_part); hipFree(p->d_qtab); hipFree(p->d_vsc); hipFree(p->d_nw);
     hipFree(p->d_sigF); hipFree(p->d_pimg); hipFree(p->d_ptan);
     for (auto &r : p->pending) { hipEventDestroy(r.e0); hipEventDestroy(r.e1); hipEventDestroy(r.e2); }
     for (auto &r : p->spare) { hipEventDestroy(r.e0); hipEventDestroy(r.e1); hipEventDestroy(r.e2); }
@@ -627,7 +655,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
 // txp, twiddles, zero delay offsets) are laid out on the host first.  Every slot of the
 // spectra and their planes is written by each execute, padding as zeros.
 int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, const double *Ftx,
-                  const std::vector<double> &txp)
+                  const std::vector<double> &txp, const fn_plan *spectra_of = nullptr)
 {
     int s;
     if ((s = select_device(c.index_gpu))) return s;
@@ -657,7 +685,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t o_tw = cv.take(tw.size() * sizeof(float2)), o_dl = cv.take(c.n_el * sizeof(double));
     const size_t o_zr = cv.take(c.n_el * sizeof(double));
     const size_t tables = cv.used;
-    const size_t o_X = cv.take(P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
+    const size_t o_X = cv.take(spectra_of ? 0 : P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
     const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
     std::vector<unsigned char> h(tables, 0);
     auto put = [&](size_t at, const void *src, size_t bytes) { if (bytes) std::memcpy(h.data() + at, src, bytes); };
@@ -680,7 +708,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     P->d_tw = reinterpret_cast<float2 *>(at(o_tw));
     P->d_delay = at(o_dl);
     P->d_zeros = at(o_zr);
-    P->d_X = reinterpret_cast<float2 *>(at(o_X));
+    P->d_X = spectra_of ? spectra_of->d_X : reinterpret_cast<float2 *>(at(o_X));
     P->d_Xlp = P->xlp_bytes ? at(o_Xlp) : nullptr;
     P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
 
@@ -746,8 +774,89 @@ double useful_macs(const fn_plan *P)
     return n ? sum / n * (double)P->n_vox : 0.0;
 }
 
+// interpolated plans: the two tables behind the channel samples
+size_t interp_samples(const fn_plan *P) { return fnk::interp_table_floats2(P->interp_M, P->n_tx, P->n_el); }
+float2 *interp_tw(const fn_plan *P) { return P->d_ip + interp_samples(P); }
+float *interp_ipsi(const fn_plan *P) { return reinterpret_cast<float *>(interp_tw(P) + P->interp_M); }
+
+// leading depths up to the last one where the clamp min(F, sqrt(f z / (2.88 c))) of the first
+// F-number bites at the lowest frequency (das_pw.m:374-377)
+int clamped_depths(const fn_plan *P)
+{
+    int n = 0;
+    for (int i = 0; P->args.clamp && i < P->n_z; ++i)
+        if (!(P->h_sqf[0] * std::sqrt(P->h_pz[i] / (2.88 * P->args.c0)) >= P->h_Frx[0])) n = i + 1;
+    return n;
+}
+
+// Samples per channel of a plan whose image can be interpolated (fn_interp.hip), 0 otherwise:
+// FP32 plane waves of one frame with one F-number for every bin; the depths where its clamp is
+// at work, at most half of them, have a plan of their own.  31 angles, boxcar, 512 x 384 (432
+// bins): 0.9 ms against 7.2 for the sum over the bins, and 0.23 for the samples; 75 angles,
+// 1024 x 512 (1455 bins, 14 % of the depths clamped): 27 ms against 118.  The samples cost the
+// same for any image, so the line is where both forms' estimated times cross: 8 n_f M flop per
+// padded channel at 100 TFLOP/s plus 75 ns per 64 voxels, element and angle, against 0.9 us +
+// 0.35 us per transmit tile for 16 voxels and a bin, each over 1024 SIMDs (100 x 77 voxels, 11
+// angles, 542 bins: 0.39 ms against 0.45; a quarter of these voxels: about even).  The samples
+// stay within 8 GiB and their twiddles within LDS.
+int interp_points(const fn_plan *P)
+{
+    const int n_f = P->g.n_f;
+    if (P->mode != 0 || P->n_frames > 1 || P->lbl || P->nw || P->precision != FN_PRECISION_FP32) return 0;
+    const double F = P->h_Frx[0];
+    if (!std::all_of(P->h_Frx.begin(), P->h_Frx.end(), [&](double f) { return f == F; })) return 0;
+    if (2 * clamped_depths(P) > P->n_z) return 0;
+    const long M = ((9L * n_f + 3) / 4 + 15) / 16 * 16;
+    if (M * 8 + (long)n_f * 4 > 131072) return 0;
+    if (fnk::interp_table_floats2((int)M, P->n_tx, P->n_el) * sizeof(float2) > ((size_t)8 << 30)) return 0;
+    const double t_samples = 8.0 * n_f * M * (16.0 * P->MT_all) * (4.0 * P->KI) / 1e14;
+    const double t_gather = P->n_vox / 64.0 * P->n_el * P->n_tx * 75e-9 / 1024.0;
+    const double t_sum = P->n_vox / 16.0 * n_f * (0.9 + 0.35 * P->MT_all) * (P->KI / 32.0) * 1e-6 / 1024.0;
+    if (t_samples + t_gather > t_sum) return 0;
+    return (int)M;
+}
+
+int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of = nullptr);
+
+int setup_interp(fn_plan *P, const fn_pw_params *p)
+{
+    P->interp_M = interp_points(P);
+    if (!P->interp_M) return FN_OK;
+    const int nz = clamped_depths(P);
+    if (nz > 0) {
+        fn_pw_params q = *p;
+        q.n_z = nz;
+        if (int st = pw_plan(&q, &P->shallow, P)) return st;
+        const fnh::Grid &a = P->g, &b = P->shallow->g;
+        if (a.N != b.N || a.n_lb != b.n_lb || a.n_f != b.n_f) {  // another DFT: the plan keeps the sum over the bins
+            destroy(P->shallow);
+            P->shallow = nullptr;
+            P->interp_M = 0;
+            return FN_OK;
+        }
+        HIP_CHECK(hipMalloc(&P->d_simg, (size_t)P->n_x * nz * sizeof(float2)), "clamped depths");
+        HIP_CHECK(hipMalloc(&P->d_sw, (size_t)P->n_x * nz * sizeof(float)), "clamped depths");
+    }
+    const size_t bytes = (interp_samples(P) + P->interp_M) * sizeof(float2) + P->g.n_f * sizeof(float);
+    HIP_CHECK(hipMalloc(&P->d_ip, bytes), "channel samples");
+    const hipError_t e = fnk::launch_interp_tables(interp_tw(P), interp_ipsi(P), P->interp_M, P->g.n_f, P->stream);
+    if (e != hipSuccess) return hip_fail(e, "interp_tables_kernel");
+    HIP_CHECK(hipStreamSynchronize(P->stream), "interp_tables_kernel");
+    return ensure_partials(P);
+}
+
 hipError_t launch_beam(const fn_plan *P, dim3 grid, const fnk::BeamArgs &A, hipStream_t s)
 {
+    if (P->interp_M) {
+        fnk::InterpArgs S{};
+        S.B = A;
+        S.B.wrx = P->args.wrx;  // FP32 weights
+        S.G = P->d_ip;
+        S.M = P->interp_M;
+        S.n_c = (uint32_t)(P->g.n_lb + P->g.n_f / 2);
+        S.empty_weight = P->wcr == fnk::WC_COS_ALL ? (float)P->n_el : 0.f;  // as the full-array class reports it
+        return fnk::launch_interp_beamform(wcr_general(P->wcr), S, s);
+    }
     const int kidx = ki_index(P->KI);  // ensembles, line scans and windowed plans stop at KI = 32
     if (P->lbl) return fnk::kLblLaunchers[kidx](P->wcr, grid, s, A);
     if (use_mirror(P)) return fnk::kMirLaunchers[kidx](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A);
@@ -855,15 +964,36 @@ int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xsca
     return FN_OK;
 }
 
-// after the beamforming launch: the partial images of a voxel's workgroups summed
-// in slot order into the image (nothing when one workgroup owns each voxel)
-int finish_beam(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s, float2 *dimage = nullptr)
+int finish_beam(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s, float2 *dimage = nullptr);
+
+// the clamped depths of an interpolated plan, from its spectra, pasted into its image
+int run_shallow(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s)
 {
-    if (!A.partial) return FN_OK;
-    hipLaunchKernelGGL(fnk::reduce_partials_kernel, dim3((unsigned)((P->n_vox + 255) / 256)), dim3(256), 0, s,
-                       A.partial, A.n_slots, P->n_vox, A.image, dimage);
-    HIP_CHECK(hipGetLastError(), "reduce_partials_kernel");
+    const fn_plan *C = P->shallow;
+    if (int st = launch_lowp_planes(C, C->d_X, C->d_Xlp, C->d_xscale, C->MT_all, plane_tiles(C), use_mirror(C) ? C->n_el : 0,
+                                    plane_delay(C, use_mirror(C)), s))
+        return st;
+    const fnk::BeamArgs B = beam_args(C, reinterpret_cast<float *>(P->d_simg), A.weights ? P->d_sw : nullptr, nullptr);
+    const hipError_t e = launch_beam(C, dim3((unsigned)beam_tiles(C), (unsigned)C->bin_split, (unsigned)C->n_groups), B, s);
+    if (e != hipSuccess) return hip_fail(e, "beamform_kernel");
+    if (int st = finish_beam(C, B, s)) return st;
+    hipLaunchKernelGGL(fnk::paste_depths_kernel, dim3((unsigned)((C->n_vox + 255) / 256)), dim3(256), 0, s, P->d_simg,
+                       A.weights ? P->d_sw : nullptr, C->n_vox, C->n_z, P->n_z, A.image, A.weights);
+    HIP_CHECK(hipGetLastError(), "paste_depths_kernel");
     return FN_OK;
+}
+
+// after the beamforming launch: the partial images of a voxel's workgroups summed
+// in slot order into the image (nothing when one workgroup owns each voxel), and the
+// clamped depths of an interpolated plan
+int finish_beam(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s, float2 *dimage)
+{
+    if (A.partial) {
+        hipLaunchKernelGGL(fnk::reduce_partials_kernel, dim3((unsigned)((P->n_vox + 255) / 256)), dim3(256), 0, s,
+                           A.partial, A.n_slots, P->n_vox, A.image, dimage);
+        HIP_CHECK(hipGetLastError(), "reduce_partials_kernel");
+    }
+    return P->shallow && !dimage ? run_shallow(P, A, s) : FN_OK;
 }
 
 // everything of an execute before the beamforming launch: the zeroed images of an
@@ -878,6 +1008,11 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
     }
     const fnk::SpecArgs &S = P->sargs;
     if (int st = launch_spectra(P, d_rf, dtype, s)) return st;
+    if (P->interp_M) {
+        const hipError_t e = fnk::launch_interp_samples(P->d_X, interp_tw(P), interp_ipsi(P), P->d_ip, P->interp_M, S.n_f,
+                                                        S.MT, S.KI, P->n_tx, P->n_el, s);
+        return e == hipSuccess ? FN_OK : hip_fail(e, "interp_samples_kernel");
+    }
     return launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, S.MT, plane_tiles(P), use_mirror(P) ? P->n_el : 0,
                               plane_delay(P, use_mirror(P)), s);
 }
@@ -959,7 +1094,8 @@ int configure_pw(fn_plan *P, const fn_pw_params *p, Common *c)
     return FN_OK;
 }
 
-int pw_plan(const fn_pw_params *p, fn_plan **out)
+// spectra_of: a plan of the same acquisition whose spectra this one reads (its clamped depths)
+int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of)
 {
     fnh::Grid g;
     int s = fnh::validate_pw(p, &g);
@@ -990,10 +1126,11 @@ int pw_plan(const fn_pw_params *p, fn_plan **out)
         txp[3 * row + 1] = ez;
         txp[3 * row + 2] = sg * ((0 - M) * p->element_pitch);
     }
-    if ((s = create_common(P, c, g, p->f_number_values, nullptr, txp))) { destroy(P); return s; }
+    if ((s = create_common(P, c, g, p->f_number_values, nullptr, txp, spectra_of))) { destroy(P); return s; }
     if (P->nw && (s = setup_windowed(P, true, p->window, p->normalization_window, false, p->window,
                                      p->normalization_window))) { destroy(P); return s; }
     use_cos_all(P);
+    if (!spectra_of && (s = setup_interp(P, p))) { destroy(P); return s; }
     *out = P;
     return FN_OK;
 }
@@ -1131,7 +1268,7 @@ int set_tof(fn_plan *P, double c_tof, const double *delays)
     P->delays_even = std::equal(d.begin(), d.end(), d.rbegin());
     P->args.ctof = c_tof > 0 ? c_tof : P->args.c0;
     ++P->tof_serial;
-    return FN_OK;
+    return P->shallow ? set_tof(P->shallow, c_tof, delays) : FN_OK;
 }
 
 int check_pw_fp32(const fn_plan *P, const char *what)
@@ -1982,8 +2119,9 @@ static void batch_release_graph(fn_batch *b)
 static bool row_stackable(const fn_plan *P)
 {
     // beyond three tiles of rows a plan fills its own transmit groups (the ensemble
-    // kernel holds at most four tiles per group against five of the plain kernel)
-    return P->mode == 0 && P->n_frames == 1 && !P->lbl && !P->nw && P->KI <= 32 && P->n_tx <= 48;
+    // kernel holds at most four tiles per group against five of the plain kernel); an
+    // interpolated plan has no weights per bin to share
+    return P->mode == 0 && P->n_frames == 1 && !P->lbl && !P->nw && P->KI <= 32 && P->n_tx <= 48 && !P->interp_M;
 }
 
 static bool same_receive_side(const fn_plan *a, const fn_plan *b)
@@ -2112,7 +2250,7 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
 // (ensembles, windowed normalization)
 static long batch_class_key(const fn_plan *P)
 {
-    if (P->n_frames > 1 || P->nw || P->lbl || P->KI > 32) return -1;  // persistent kernels up to 128 elements
+    if (P->n_frames > 1 || P->nw || P->lbl || P->interp_M || P->KI > 32) return -1;  // persistent kernels up to 128 elements
     return ((((long)P->mode * 64 + P->KI) * 16 + P->MT_tmpl) * 8 + P->wcr) * 8 * 4 + P->wct * 4 + P->kprec;
 }
 

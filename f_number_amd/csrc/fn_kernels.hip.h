@@ -29,6 +29,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include <type_traits>
@@ -132,6 +133,15 @@ struct AdjArgs {
     const float *us;        // split contraction: per bin the cotangent's scale, then what takes it out
     long vox_per_range;     // multiple of 64
     int n_at;               // angle tiles of 16
+};
+
+// interpolated images (fn_interp.hip)
+struct InterpArgs {
+    BeamArgs B;
+    const float2 *G;        // channel samples [n_el][n_tx][M + 7]
+    int M;                  // samples per DFT period
+    uint32_t n_c;           // the band's centre bin
+    float empty_weight;     // weight sum reported for an empty aperture
 };
 
 struct SpecArgs {
@@ -1224,19 +1234,19 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                     const u32x4 xrh = xq[(0 * MT + mt) * XS + lane];
                     const u32x4 xih = xq[(1 * MT + mt) * XS + lane];
                     accR[mt] = mfma16<PREC>(xrh, w.rh, accR[mt]);
-                    accI[mt] = mfma16<PREC>(xrh, w.ih, accI[mt]);
                     accR[mt] = mfma16<PREC>(xih, nih, accR[mt]);
+                    accI[mt] = mfma16<PREC>(xrh, w.ih, accI[mt]);
                     accI[mt] = mfma16<PREC>(xih, w.rh, accI[mt]);
                     if (Prec<PREC>::split) {
                         const u32x4 xrl = xq[(2 * MT + mt) * XS + lane];
                         const u32x4 xil = xq[(3 * MT + mt) * XS + lane];
                         accR[mt] = mfma16<PREC>(xrh, w.rl, accR[mt]);
-                        accI[mt] = mfma16<PREC>(xrh, w.il, accI[mt]);
                         accR[mt] = mfma16<PREC>(xrl, w.rh, accR[mt]);
-                        accI[mt] = mfma16<PREC>(xrl, w.ih, accI[mt]);
                         accR[mt] = mfma16<PREC>(xih, nil, accR[mt]);
-                        accI[mt] = mfma16<PREC>(xih, w.rl, accI[mt]);
                         accR[mt] = mfma16<PREC>(xil, nih, accR[mt]);
+                        accI[mt] = mfma16<PREC>(xrh, w.il, accI[mt]);
+                        accI[mt] = mfma16<PREC>(xrl, w.ih, accI[mt]);
+                        accI[mt] = mfma16<PREC>(xih, w.rl, accI[mt]);
                         accI[mt] = mfma16<PREC>(xil, w.rh, accI[mt]);
                         if (TAN) {
                             floatx4 &tR = tanR[TAN ? mt : 0], &tI = tanI[TAN ? mt : 0];
