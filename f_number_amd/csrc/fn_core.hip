@@ -807,7 +807,7 @@ int interp_points(const fn_plan *P)
     if (!std::all_of(P->h_Frx.begin(), P->h_Frx.end(), [&](double f) { return f == F; })) return 0;
     if (2 * clamped_depths(P) > P->n_z) return 0;
     const long M = ((9L * n_f + 3) / 4 + 15) / 16 * 16;
-    if (M * 8 + (long)n_f * 4 > 131072) return 0;
+    if (M * 8 + (long)n_f * 4 > fnk::INTERP_LDS_MAX) return 0;
     if (fnk::interp_table_floats2((int)M, P->n_tx, P->n_el) * sizeof(float2) > ((size_t)8 << 30)) return 0;
     const double t_samples = 8.0 * n_f * M * (16.0 * P->MT_all) * (4.0 * P->KI) / 1e14;
     const double t_gather = P->n_vox / 64.0 * P->n_el * P->n_tx * 75e-9 / 1024.0;
@@ -818,31 +818,44 @@ int interp_points(const fn_plan *P)
 
 int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of = nullptr);
 
+// the interpolated form's buffers (and the plan of its clamped depths); a plan without room for
+// them, or whose clamped depths have another DFT, keeps the sum over the bins
 int setup_interp(fn_plan *P, const fn_pw_params *p)
 {
     P->interp_M = interp_points(P);
     if (!P->interp_M) return FN_OK;
+    auto keep_sum = [&]() {
+        destroy(P->shallow);
+        hipFree(P->d_simg); hipFree(P->d_sw); hipFree(P->d_ip);
+        P->shallow = nullptr;
+        P->d_simg = P->d_ip = nullptr;
+        P->d_sw = nullptr;
+        P->interp_M = 0;
+        (void)hipGetLastError();
+        fnh::clear_error();
+        return FN_OK;
+    };
     const int nz = clamped_depths(P);
     if (nz > 0) {
         fn_pw_params q = *p;
         q.n_z = nz;
-        if (int st = pw_plan(&q, &P->shallow, P)) return st;
+        if (pw_plan(&q, &P->shallow, P) != FN_OK) return keep_sum();
         const fnh::Grid &a = P->g, &b = P->shallow->g;
-        if (a.N != b.N || a.n_lb != b.n_lb || a.n_f != b.n_f) {  // another DFT: the plan keeps the sum over the bins
-            destroy(P->shallow);
-            P->shallow = nullptr;
-            P->interp_M = 0;
-            return FN_OK;
-        }
-        HIP_CHECK(hipMalloc(&P->d_simg, (size_t)P->n_x * nz * sizeof(float2)), "clamped depths");
-        HIP_CHECK(hipMalloc(&P->d_sw, (size_t)P->n_x * nz * sizeof(float)), "clamped depths");
+        if (a.N != b.N || a.n_lb != b.n_lb || a.n_f != b.n_f) return keep_sum();
+        if (hipMalloc(&P->d_simg, (size_t)P->n_x * nz * sizeof(float2)) != hipSuccess ||
+            hipMalloc(&P->d_sw, (size_t)P->n_x * nz * sizeof(float)) != hipSuccess)
+            return keep_sum();
     }
     const size_t bytes = (interp_samples(P) + P->interp_M) * sizeof(float2) + P->g.n_f * sizeof(float);
-    HIP_CHECK(hipMalloc(&P->d_ip, bytes), "channel samples");
+    if (hipMalloc(&P->d_ip, bytes) != hipSuccess) return keep_sum();
+    if (ensure_partials(P) != FN_OK) {
+        keep_sum();
+        return ensure_partials(P);
+    }
     const hipError_t e = fnk::launch_interp_tables(interp_tw(P), interp_ipsi(P), P->interp_M, P->g.n_f, P->stream);
     if (e != hipSuccess) return hip_fail(e, "interp_tables_kernel");
     HIP_CHECK(hipStreamSynchronize(P->stream), "interp_tables_kernel");
-    return ensure_partials(P);
+    return FN_OK;
 }
 
 hipError_t launch_beam(const fn_plan *P, dim3 grid, const fnk::BeamArgs &A, hipStream_t s)

@@ -216,8 +216,13 @@ __global__ __launch_bounds__(256) void interp_beamform_kernel(InterpArgs S)
     if (blockIdx.y == 0 && A.weights) A.weights[v] = ap.valid ? asum : S.empty_weight;
 }
 
+// at plan creation: the tables, and the largest dynamic LDS a plan may ask of the samples kernel
+// (once for all sizes and here, so neither a capture nor another thread's launch meets it)
 hipError_t launch_interp_tables(float2 *tw, float *ipsi, int M, int n_f, hipStream_t s)
 {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(interp_samples_kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, INTERP_LDS_MAX);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(interp_tables_kernel, dim3((unsigned)((std::max(M, n_f) + 255) / 256)), dim3(256), 0, s, tw, ipsi,
                        M, n_f);
     return hipGetLastError();
@@ -227,13 +232,6 @@ hipError_t launch_interp_samples(const float2 *X, const float2 *tw, const float 
                                  int KI, int n_tx, int n_el, hipStream_t s)
 {
     const size_t lds = (size_t)M * sizeof(float2) + (size_t)n_f * sizeof(float);
-    static size_t lds_done = 0;  // raised once per process and size (graph capture issues no attribute calls)
-    if (lds > 65536 && lds > lds_done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(interp_samples_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        lds_done = lds;
-    }
     hipLaunchKernelGGL(interp_samples_kernel, dim3((unsigned)((M + IP_TAPS - 1 + 63) / 64), (unsigned)(MT * KI)), dim3(256),
                        lds, s, X, tw, ipsi, G, M, n_f, MT, KI, n_tx, n_el);
     return hipGetLastError();

@@ -135,7 +135,8 @@ struct AdjArgs {
     int n_at;               // angle tiles of 16
 };
 
-// interpolated images (fn_interp.hip)
+// interpolated images (fn_interp.hip); twiddles and bin weights of the samples in LDS
+constexpr int INTERP_LDS_MAX = 131072;
 struct InterpArgs {
     BeamArgs B;
     const float2 *G;        // channel samples [n_el][n_tx][M + 7]
