@@ -74,7 +74,7 @@ static hipError_t launch_mt(int wcr, dim3 grid, size_t lds, hipStream_t s, const
 template <int MT, int WCR>
 static hipError_t launch_mir_one(dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
 {
-    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, INST_PREC, false, false, false, false, false, true>;
+    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, INST_PREC, false, false, false, false, true>;
     static size_t lds_done = 0;
     lds = dyn_lds(lds);
     if (hipError_t e = set_lds_once(kern, lds, lds_done)) return e;
@@ -146,7 +146,7 @@ hipError_t FN_TAN_LAUNCHER(INST_KI)(int mt, int wcr, dim3 grid, size_t lds, hipS
 template <int MT, int WCR, bool MIR>
 static hipError_t launch_tan_lp_one(dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
 {
-    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, 2, true, false, false, false, false, MIR>;
+    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, 2, true, false, false, false, MIR>;
     static size_t lds_done = 0;
     lds = dyn_lds(lds);
     if (hipError_t e = set_lds_once(kern, lds, lds_done)) return e;
@@ -175,29 +175,6 @@ hipError_t FN_TAN_LP_LAUNCHER(INST_KI)(int mt, int wcr, bool mirror, dim3 grid, 
 }
 #endif
 
-#if INST_PREC == 0 && !FN_WIDE
-// line scan: block z = grid column = its transmit row, one transmit tile
-#define FN_LBL_LAUNCHER(k) FN_CAT4(launch_beamform_lbl, _k, k, )
-template <int WCR>
-static hipError_t launch_lbl_one(dim3 grid, hipStream_t s, const BeamArgs &A)
-{
-    auto kern = beamform_kernel<0, 1, INST_KI, WCR, WC_RANGE, 0, false, false, false, true>;
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, A);  // FP32: static LDS
-    return hipGetLastError();
-}
-
-hipError_t FN_LBL_LAUNCHER(INST_KI)(int wcr, dim3 grid, hipStream_t s, const BeamArgs &A)
-{
-    switch (wcr) {
-    case WC_RANGE: return launch_lbl_one<WC_RANGE>(grid, s, A);
-    case WC_LINEAR: return launch_lbl_one<WC_LINEAR>(grid, s, A);
-    case WC_COS_ALL: return launch_lbl_one<WC_COS_ALL>(grid, s, A);
-    case WC_COS_RF: return launch_lbl_one<WC_COS_RF>(grid, s, A);
-    default: return launch_lbl_one<WC_COS>(grid, s, A);
-    }
-}
-#endif
-
 #if INST_MODE == 0 && !FN_WIDE
 // ensemble variant: frames x angles as transmit rows, up to four tiles per group (FP32 and
 // the fp16 split at 128 elements five, fp16 eight).  FP32: the linear class only (FP32
@@ -206,7 +183,7 @@ hipError_t FN_LBL_LAUNCHER(INST_KI)(int wcr, dim3 grid, hipStream_t s, const Bea
 template <int MT, int WCR, bool STK>
 static hipError_t launch_ens_one(dim3 grid, size_t lds, hipStream_t s, const BeamArgs &A)
 {
-    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, INST_PREC, false, true, false, false, STK>;
+    auto kern = beamform_kernel<0, MT, INST_KI, WCR, WC_RANGE, INST_PREC, false, true, false, STK>;
     static size_t lds_done = 0;
     lds = dyn_lds(lds);
     if (hipError_t e = set_lds_once(kern, lds, lds_done)) return e;

@@ -94,16 +94,13 @@ hipError_t launch_beamform_tan_k32(int, int, dim3, size_t, hipStream_t, const Be
 hipError_t launch_beamform_tan_k8_p2(int, int, bool, dim3, size_t, hipStream_t, const BeamArgs &);
 hipError_t launch_beamform_tan_k16_p2(int, int, bool, dim3, size_t, hipStream_t, const BeamArgs &);
 hipError_t launch_beamform_tan_k32_p2(int, int, bool, dim3, size_t, hipStream_t, const BeamArgs &);
-hipError_t launch_beamform_lbl_k8(int, dim3, hipStream_t, const BeamArgs &);
-hipError_t launch_beamform_lbl_k16(int, dim3, hipStream_t, const BeamArgs &);
-hipError_t launch_beamform_lbl_k32(int, dim3, hipStream_t, const BeamArgs &);
-typedef hipError_t (*LblLauncher)(int, dim3, hipStream_t, const BeamArgs &);
-static const LblLauncher kLblLaunchers[3] = {launch_beamform_lbl_k8, launch_beamform_lbl_k16, launch_beamform_lbl_k32};
 hipError_t launch_adjoint(int wcr, bool tables, bool scale, dim3 grid, hipStream_t s, const AdjArgs &S);
 hipError_t launch_adjoint_reduce(const float *P, float2 *Z, int n_vr, int n_f, int n_at, int n_tx, int n_el,
                                  const double *delay, double fs_over_N, int n_lb, hipStream_t s);
 hipError_t launch_adjoint_idft(const float2 *Z, const float2 *tw, float *out, int n_t, int n_ch, int N, int n_lb,
                                int n_f, hipStream_t s);
+hipError_t launch_lines(int wcr, bool mirror, int tiles, int splits, const BeamArgs &A, const float2 *X, hipStream_t s);
+hipError_t launch_lines_spectra(const float2 *X, float2 *out, int n_f, int MT, int KI, int n_x, int n_el, hipStream_t s);
 hipError_t launch_interp_tables(float2 *tw, float *ipsi, int M, int n_f, hipStream_t s);
 hipError_t launch_interp_samples(const float2 *X, const float2 *tw, const float *ipsi, float2 *G, int M, int n_f, int MT,
                                  int KI, int n_tx, int n_el, hipStream_t s);
@@ -176,8 +173,10 @@ struct fn_plan {
     int precision = FN_PRECISION_FP32;  // as asked for
     int kprec = FN_PRECISION_FP32;      // form of the forward contraction (kernel_precision)
     int mirror = 0;         // lateral positions symmetric: planes hold the reversed elements too
+    int line_mirror = 0;    // line scan on symmetric lateral positions: two columns share their weights
     int delays_even = 1;    // delay offsets symmetric about the array's centre
     int interp_M = 0;       // > 0: the forward image by interpolation of M samples per channel
+    float2 *d_Xrow = nullptr;  // line scan: the spectra by rows [n_f][line][element]
     float2 *d_ip = nullptr; // its channel samples, twiddles [M] and 1 / psi [n_f]
     // interpolated plans with depths where the F-number clamp is at work: a plan of those
     // leading depths (on this plan's spectra), its image and weights, pasted over the first rows
@@ -523,24 +522,31 @@ static bool few_rows_pw(const fn_plan *P)
     return P->mode == 0 && P->n_frames == 1 && !P->lbl && P->MT_tmpl <= 2;
 }
 
-// Plans whose lanes may stand for two mirrored voxels: single-frame plane waves in the fp16
-// split whose transmit rows fill one or two tiles (one at 129-192 elements), where the vector
-// work of the weights bounds the kernel, on lateral positions symmetric to 1e-12 pitches.  In
-// ms without / with (256 x 256): 11 angles 3.12 / 2.42, 31 angles 4.00 / 3.28, 192 elements
-// 5.96 / 4.42; from three tiles on the products bound it and twice the tiles have no room in
-// registers and LDS; 256 elements 7.27 / 9.59.  The one-pass fp16 form, whose operands' rounding
-// shows in the image, keeps one voxel a lane, so that a plan's image does not depend on whether
-// it runs alone or in a batch.  Not the boxcar window
-// at one F-number for every bin: its membership test has no taper, and its ties (a support
-// edge on an element for a whole band) would be broken by rounding.
-bool mirror_plan(const fn_plan *P, const Common &c, const double *Frx, int n_f)
+// lateral positions symmetric about the array to 1e-12 pitches.  Not the boxcar window at one
+// F-number for every bin: its membership test has no taper, and its ties (a support edge on an
+// element for a whole band) would be broken by rounding.
+bool mirrored_positions(const fn_plan *P, const Common &c, const double *Frx, int n_f)
 {
-    if (P->mode != 0 || P->n_frames > 1 || P->lbl || P->nw || P->kprec != FN_PRECISION_FP16X3 || !Frx) return false;
-    if (P->KI > 48 || P->MT_all > (P->KI <= 32 ? 2 : 1) || c.n_x < 2) return false;
+    if (!Frx || c.n_x < 2) return false;
     if (P->wcr == fnk::WC_RANGE && std::all_of(Frx, Frx + n_f, [&](double F) { return F == Frx[0]; })) return false;
     for (int i = 0; i < (c.n_x + 1) / 2; ++i)
         if (!(std::fabs(c.px[i] + c.px[c.n_x - 1 - i]) <= 1e-12 * c.pitch)) return false;
     return true;
+}
+
+// Plans whose lanes may stand for two mirrored voxels: single-frame plane waves in the fp16
+// split whose transmit rows fill one or two tiles (one at 129-192 elements), where the vector
+// work of the weights bounds the kernel, on symmetric lateral positions.  In
+// ms without / with (256 x 256): 11 angles 3.12 / 2.42, 31 angles 4.00 / 3.28, 192 elements
+// 5.96 / 4.42; from three tiles on the products bound it and twice the tiles have no room in
+// registers and LDS; 256 elements 7.27 / 9.59.  The one-pass fp16 form, whose operands' rounding
+// shows in the image, keeps one voxel a lane, so that a plan's image does not depend on whether
+// it runs alone or in a batch.
+bool mirror_plan(const fn_plan *P, const Common &c, const double *Frx, int n_f)
+{
+    if (P->mode != 0 || P->n_frames > 1 || P->lbl || P->nw || P->kprec != FN_PRECISION_FP16X3) return false;
+    if (P->KI > 48 || P->MT_all > (P->KI <= 32 ? 2 : 1)) return false;
+    return mirrored_positions(P, c, Frx, n_f);
 }
 
 // shared configuration of plan creation: tiling, launch shape and the scalar
@@ -574,7 +580,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
     const int op_rows = P->n_frames > 1 ? P->ens_angles * P->args.ens_slots : c.n_tx;
     P->MT_all = (op_rows + 15) / 16;
     if (P->lbl) {
-        // line scan: one group per grid column, staging the M-tile of its transmit row
+        // line scan: one group per grid column (fn_lines.hip)
         P->MT_tmpl = 1;
         P->n_groups = c.n_x;
     } else if (P->mode == 0) {
@@ -589,6 +595,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
         P->n_groups = (P->MT_all + P->MT_tmpl - 1) / P->MT_tmpl;
     }
     P->mirror = mirror && mirror_plan(P, c, Frx, g.n_f);
+    P->line_mirror = P->lbl && mirrored_positions(P, c, Frx, g.n_f);
     const size_t step_bytes = form_step_bytes(P->kprec);
     P->lds_beam = (size_t)P->MT_tmpl * P->KI * step_bytes;
     P->lds_spec = (size_t)g.N * sizeof(float2) + 64 * 65 * sizeof(float);
@@ -600,9 +607,12 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
     const long blocks = tiles * P->n_groups;
     int split = 1;  // windowed normalization: every block walks all bins (valid-row counts)
     if (P->lbl) {
-        // line scans (vector-ALU bound, one column per group): about 8192 blocks below
-        // 4096, measured best over bin splits 1..64 at 64-256 lines x 256-1024 depths
-        if (blocks < 4096) split = (int)std::min<long>({(8192 + blocks - 1) / blocks, 16L, (long)std::max(1, g.n_f / 8)});
+        // line scans: about 3072 workgroups (two rounds of the 1280 that fit and some; mirrored
+        // columns share one), at most 12 chunks.  ms at 1 / 6 / 12 chunks: 128 lines x 512 depths
+        // 2.46 / 2.04 / 2.05, 64 x 256 1.71 / 0.81 / 0.84, 101 x 300 1.78 / 1.25 / 1.17; 256 x 1024
+        // at 1 / 2 / 12 7.46 / 7.23 / 7.70
+        const long wg = tiles * (P->line_mirror ? (c.n_x + 1) / 2 : c.n_x);
+        split = (int)std::min<long>({(3072 + wg - 1) / wg, 12L, (long)std::max(1, g.n_f / 16)});
     } else if (!P->nw && blocks < (few_rows_pw(P) ? FN_FEW_ROWS_BLOCKS : 2048L)) {
         // single-frame plane waves of one or two transmit tiles per group (vector-ALU
         // bound element loops): about FN_FEW_ROWS_BLOCKS blocks, otherwise about 2048
@@ -617,7 +627,8 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
         if (set > 32.0 * 1048576.0)
             split = (int)std::min<double>({16.0, std::ceil(set / (4.0 * 1048576.0)), (double)std::max(1, g.n_f / 8)});
     }
-    const int chunk = (g.n_f + split - 1) / split;
+    int chunk = (g.n_f + split - 1) / split;
+    if (P->lbl) chunk = (chunk + 15) / 16 * 16;  // whole rounds of its four waves, four bins each
     P->bin_split = (g.n_f + chunk - 1) / chunk;
     P->x_bytes = (size_t)g.n_f * P->MT_all * P->KI * 64 * sizeof(float2);
     // room for the planes of every tiling: groups of mt tiles hold up to mt - 1 zero tiles
@@ -687,6 +698,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t tables = cv.used;
     const size_t o_X = cv.take(spectra_of ? 0 : P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
     const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
+    const size_t o_xr = cv.take(P->lbl ? (size_t)g.n_f * c.n_x * c.n_el * sizeof(float2) : 0);
     std::vector<unsigned char> h(tables, 0);
     auto put = [&](size_t at, const void *src, size_t bytes) { if (bytes) std::memcpy(h.data() + at, src, bytes); };
     put(o_px, c.px, c.n_x * sizeof(double));
@@ -710,6 +722,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     P->d_zeros = at(o_zr);
     P->d_X = spectra_of ? spectra_of->d_X : reinterpret_cast<float2 *>(at(o_X));
     P->d_Xlp = P->xlp_bytes ? at(o_Xlp) : nullptr;
+    P->d_Xrow = P->lbl ? reinterpret_cast<float2 *>(at(o_xr)) : nullptr;
     P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
 
     fnk::BeamArgs &A = P->args;
@@ -871,7 +884,8 @@ hipError_t launch_beam(const fn_plan *P, dim3 grid, const fnk::BeamArgs &A, hipS
         return fnk::launch_interp_beamform(wcr_general(P->wcr), S, s);
     }
     const int kidx = ki_index(P->KI);  // ensembles, line scans and windowed plans stop at KI = 32
-    if (P->lbl) return fnk::kLblLaunchers[kidx](P->wcr, grid, s, A);
+    if (P->lbl)
+        return fnk::launch_lines(P->wcr, P->line_mirror && P->delays_even, (int)grid.x, (int)grid.y, A, P->d_Xrow, s);
     if (use_mirror(P)) return fnk::kMirLaunchers[kidx](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A);
     if (P->nw) return fnk::kNwLaunchers[P->mode][kidx](P->MT_tmpl, P->wcr, P->wct, grid, P->lds_beam, s, A);
     if (P->n_frames > 1) return fnk::kEnsLaunchers[kidx][P->kprec](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A, 0);
@@ -1021,6 +1035,10 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
     }
     const fnk::SpecArgs &S = P->sargs;
     if (int st = launch_spectra(P, d_rf, dtype, s)) return st;
+    if (P->lbl) {
+        const hipError_t e = fnk::launch_lines_spectra(P->d_X, P->d_Xrow, S.n_f, S.MT, S.KI, P->n_x, P->n_el, s);
+        return e == hipSuccess ? FN_OK : hip_fail(e, "lines_spectra_kernel");
+    }
     if (P->interp_M) {
         const hipError_t e = fnk::launch_interp_samples(P->d_X, interp_tw(P), interp_ipsi(P), P->d_ip, P->interp_M, S.n_f,
                                                         S.MT, S.KI, P->n_tx, P->n_el, s);

@@ -677,35 +677,32 @@ struct PersistWavesPerEU {
 // transmit group bz.  beamform_kernel runs it for its block index; the
 // persistent batch kernel for every work item it claims.
 template <int MODE, int MT, int KI, int WCR, int WCT, int PREC, bool TAN = false, bool ENS = false, bool NW = false,
-          bool LBL = false, bool STK = false, bool MIR = false, typename Args = BeamArgs>
+          bool STK = false, bool MIR = false, typename Args = BeamArgs>
 __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by, const int bz, const int tid)
 {
     static_assert(!STK || ENS, "row stacks run the ensemble form");
     static_assert(!TAN || (MODE == MODE_PW && (PREC == PREC_FP32 || PREC == PREC_FP16X3)), "tangent: plane waves");
     static_assert(!ENS || (MODE == MODE_PW && !TAN), "ensemble: plane waves");
     static_assert(!NW || (PREC == PREC_FP32 && !TAN && !ENS), "windowed normalization: FP32 forward");
-    static_assert(!MIR || (MODE == MODE_PW && PREC != PREC_FP32 && !ENS && !NW && !LBL && MT % 2 == 0),
+    static_assert(!MIR || (MODE == MODE_PW && PREC != PREC_FP32 && !ENS && !NW && MT % 2 == 0),
                   "mirrored voxels: plane waves, 16-bit forms");
     constexpr int MTH = MIR ? MT / 2 : MT;  // tiles of transmit rows (the others: reversed elements)
-    static_assert(!LBL || (MODE == MODE_PW && MT == 1 && !TAN && !ENS && !NW), "line scan: plane-wave forward, one tile");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     // the wave index is uniform: held in a scalar register, so the addresses of the
     // wave's tile copies are formed on the scalar unit
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, c = lane & 15;
     const long n_vox = (long)A.n_x * A.n_z;
-    // line scan: block bz covers depths of grid column bz, the line of transmit row bz
-    const long v_loc = (long)bx * 64 + wave * 16 + c;
-    const long v = LBL ? (long)bz * A.n_z + v_loc : v_loc;
+    const long v = (long)bx * 64 + wave * 16 + c;
     const long n_own = MIR ? (long)((A.n_x + 1) >> 1) * A.n_z : n_vox;  // voxels with a lane of their own
-    const bool vok = LBL ? v_loc < A.n_z : v < n_own;
-    const long vv = vok ? v : (LBL ? (long)bz * A.n_z + A.n_z - 1 : n_own - 1);
+    const bool vok = v < n_own;
+    const long vv = vok ? v : n_own - 1;
     const int ix = (int)(vv / A.n_z), iz = (int)(vv - (long)ix * A.n_z);
     const int ix2 = A.n_x - 1 - ix;  // MIR: the mirrored voxel's column
     const double x = A.px[ix], z = A.pz[iz];
     const double xp = x / A.pitch, zp = z / (2.0 * A.pitch);
     const double clamp_z = sqrt(z / (2.88 * A.c0));  // sqrt(f z / (2.88 c)) = sqrt(f) clamp_z (das_pw.m:374)
-    const int mt0 = LBL ? (bz >> 4) : bz * A.tx_group;  // first M-tile of this transmit group
+    const int mt0 = bz * A.tx_group;  // first M-tile of this transmit group
 
     // receive phase increments: tau_rx = sqrt(((x_k-x)/c)^2 + (z/c)^2) (das_pw.m:339-340,427)
     // plus the element's delay offset
@@ -746,8 +743,6 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             Qtx[mt][r] = frac32(A.f_s * tau / A.N);
             if (TAN) Ttx[TAN ? mt : 0][r] = (float)(tg * t_unit);
         }
-    // line scan: the phase increment of the block's own transmit row
-    const uint32_t Qln = LBL ? frac32(A.f_s * (pw_tx_time(A, bz, x, z) + A.t0 / A.f_s) / A.N) : 0u;
     const float dg = (float)(((double)g - A.M) * A.pitch - x);  // x_k - x of element j = 0
     const float pf = (float)A.pitch;
     const float dg_tx = (float)((4.0 * g - A.M) * A.pitch - x);  // SA transmit rows, mt = r = 0
@@ -977,11 +972,6 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             //   Re Y = K1 - K3, Im Y = K1 + K2
             floatx4 K1[MT], K2[MT], K3[MT];
             floatx4 T1[TAN ? MT : 1], T2[TAN ? MT : 1], T3[TAN ? MT : 1];
-            // line scan: one transmit row contributes, so the product runs on the vector ALUs
-            // (the lane's elements 4 j + g against row bz of the staged tile, read as a
-            // broadcast) instead of a 16-row matrix-core product of which one row is used
-            float Lr = 0.f, Li = 0.f;
-            const int lrow = bz & 15;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 K1[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -1040,14 +1030,6 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 }
                 const float br = a * cs, bi = a * sn;
                 const float bd = bi - br, bp = br + bi;
-                if constexpr (LBL) {
-                    const float2 xv = xs[(j - cc * SJC) * 64 + lrow + 16 * g];
-                    Lr = fmaf(xv.x, br, Lr);
-                    Lr = fmaf(-xv.y, bi, Lr);
-                    Li = fmaf(xv.x, bi, Li);
-                    Li = fmaf(xv.y, br, Li);
-                    return;
-                }
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     const float2 xv = xs[(mt * SJC + (j - cc * SJC)) * 64 + lane];
@@ -1064,12 +1046,12 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 }
                         };
             const int j_a = max(u_lo >> 2, cc * SJC), j_b = min(j_hi, cc * SJC + SJC - 1);
-            if constexpr (WCR == WC_COS_ALL && !LBL && !TAN && !NW) {
+            if constexpr (WCR == WC_COS_ALL && !TAN && !NW) {
                 // every element step (no support test): unrolled, so the phase words are
                 // read from fixed registers and the first step starts the accumulators
 #pragma unroll
                 for (int jj = 0; jj < SJC; ++jj) step(cc * SJC + jj);
-            } else if constexpr (KI > 32 && !LBL) {
+            } else if constexpr (KI > 32) {
                 // wide arrays: every step unrolled under its own uniform guard, so that the
                 // 48 / 64 phase words stay in registers (a runtime index would move them to
                 // scratch memory)
@@ -1078,7 +1060,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                     const int j = cc * SJC + jj;
                     if (j >= j_a && j <= j_b) step(j);
                 }
-            } else if constexpr (LBL || MT > 2) {
+            } else if constexpr (MT > 2) {
                 // (three or more tiles: a step's 9+ products keep the matrix cores busy)
 #pragma clang loop unroll(disable)
                 for (int j = j_a; j <= j_b; ++j) step(j);
@@ -1104,10 +1086,6 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             chunk_step(std::integral_constant<int, 1>{});
             chunk_step(std::integral_constant<int, 2>{});
             chunk_step(std::integral_constant<int, 3>{});
-            if constexpr (LBL) {
-                accR[0] = floatx4{Lr, 0.f, 0.f, 0.f};
-                accI[0] = floatx4{Li, 0.f, 0.f, 0.f};
-            } else
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
                 accR[mt] = K1[mt] - K3[mt];
@@ -1306,14 +1284,6 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                 // padded transmit rows have zero spectra, so every row is summed
                 float pr = 0.f, pi = 0.f;  // tangent: sum_rows T (tau_tx,g Y + Y')
                 float pr2 = 0.f, pi2 = 0.f;
-                if constexpr (LBL) {
-                    // the lane's partial product over its elements, at the line's own transmit phase
-                    const float rv = rev_of((uint32_t)n * Qln);
-                    const float sn = __builtin_amdgcn_sinf(rv), cs = __builtin_amdgcn_cosf(rv);
-                    const float yr = accR[0][0] * sc, yi = accI[0][0] * sc;
-                    Ir += cs * yr - sn * yi;
-                    Ii += cs * yi + sn * yr;
-                } else {
                 float Sr = 0.f, Si = 0.f;  // sum over the rows of T Y, scaled once below
                 float Sr2 = 0.f, Si2 = 0.f;
 #pragma unroll
@@ -1362,7 +1332,6 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                         Ir2 = fmaf(sc, Sr2, Ir2);
                         Ii2 = fmaf(sc, Si2, Ii2);
                     }
-                }
                 }
                 if (TAN) {
                     // dI += sc (j w_n) (-1 / c) P
@@ -1549,14 +1518,14 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
         const float2 dval = make_float2(A.out_scale * fmaf(-PHASE_BACK, Di, Dr), A.out_scale * fmaf(PHASE_BACK, Dr, Di));
         float2 *dimg = reinterpret_cast<float2 *>(A.dimage);
         if (A.partial) {
-            const long slot = (long)by * A.slot_z + (LBL ? 0 : bz);
+            const long slot = (long)by * A.slot_z + bz;
             A.partial[slot * n_vox + v] = val;
             if (TAN) A.partial[((long)A.n_slots + slot) * n_vox + v] = dval;
         } else {
             A.image[v] = val;
             if (TAN) dimg[v] = dval;
         }
-        if (b_end == A.n_f && (LBL || bz == 0)) {
+        if (b_end == A.n_f && bz == 0) {
             if (A.weights) A.weights[v] = w_last;
             if (MODE == MODE_SA && A.weights_tx) A.weights_tx[v] = wtx_last;
         }
@@ -1564,7 +1533,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
 }
 
 template <int MODE, int MT, int KI, int WCR, int WCT, int PREC, bool TAN = false, bool ENS = false, bool NW = false,
-          bool LBL = false, bool STK = false, bool MIR = false>
+          bool STK = false, bool MIR = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BeamWavesPerEU<MT, KI, WCR, PREC, ENS, TAN>::value)))
 void beamform_kernel(BeamArgs A)
 {
@@ -1573,7 +1542,7 @@ void beamform_kernel(BeamArgs A)
     // reference form leaves the compiler the registers it schedules best with
     using Args =
         typename std::conditional<(MT * KI <= 64 || PREC != PREC_FP32), BeamArgs, const BeamArgs &>::type;
-    beamform_tile<MODE, MT, KI, WCR, WCT, PREC, TAN, ENS, NW, LBL, STK, MIR, Args>(A, blockIdx.x, blockIdx.y, blockIdx.z,
+    beamform_tile<MODE, MT, KI, WCR, WCT, PREC, TAN, ENS, NW, STK, MIR, Args>(A, blockIdx.x, blockIdx.y, blockIdx.z,
                                                                            threadIdx.x);
 }
 
@@ -1600,7 +1569,7 @@ void beamform_persistent_kernel(const BeamArgs *__restrict__ jobs, const int4 *_
         // recomputed per tile rather than hoisted out of the loop and held across tiles
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
-        beamform_tile<MODE, MT, KI, WCR, WCT, PREC, false, false, false, false, false, false, const BeamArgs &>(
+        beamform_tile<MODE, MT, KI, WCR, WCT, PREC, false, false, false, false, false, const BeamArgs &>(
             A, __builtin_amdgcn_readfirstlane(w.y),
                                                     __builtin_amdgcn_readfirstlane(w.z),
                                                     __builtin_amdgcn_readfirstlane(w.w), tid);
