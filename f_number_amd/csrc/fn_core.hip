@@ -2117,6 +2117,7 @@ struct fn_batch {
     std::vector<const void *> rf;
     std::vector<int32_t> dtypes;
     std::vector<float *> images;
+    std::vector<long> tofs;            // every plan's tof_serial when the graph was captured
     int captures = 0;
     int64_t n_nodes = 0;
 };
@@ -2400,7 +2401,9 @@ int32_t fn_batch_execute(fn_batch *b, const void *const *d_rf, const int32_t *dt
     const bool same = b->exec && b->rf.size() == n &&
                       std::equal(b->rf.begin(), b->rf.end(), d_rf) &&
                       std::equal(b->dtypes.begin(), b->dtypes.end(), dtypes) &&
-                      std::equal(b->images.begin(), b->images.end(), d_images);
+                      std::equal(b->images.begin(), b->images.end(), d_images) &&
+                      std::equal(b->plans.begin(), b->plans.end(), b->tofs.begin(),
+                                 [](const fn_plan *P, long t) { return P->tof_serial == t; });
     if (!same) {
         batch_release_graph(b);
         // eager pass: validates every job and raises kernel LDS limits outside the capture
@@ -2489,6 +2492,8 @@ int32_t fn_batch_execute(fn_batch *b, const void *const *d_rf, const int32_t *dt
         b->rf.assign(d_rf, d_rf + n);
         b->dtypes.assign(dtypes, dtypes + n);
         b->images.assign(d_images, d_images + n);
+        b->tofs.clear();
+        for (const fn_plan *P : b->plans) b->tofs.push_back(P->tof_serial);
         b->captures += 1;
     }
     HIP_CHECK(hipGraphLaunch(b->exec, s), "hipGraphLaunch");

@@ -1,6 +1,7 @@
 """Line scans at the edges of their kernel: columns that share their weights with their mirror
 image (even and odd counts) and columns that cannot, ragged element counts, one and many
-depth tiles, bands shorter than a round of its waves; delay offsets that are not symmetric.
+depth tiles, bands shorter than a round of its waves; delay offsets that are not symmetric;
+and a captured batch whose plan gets other delays.
 
 Bars: the line scans' own (rel-L2 1e-4, peak -80 dB) against the FP64 oracle; against
 single-column plans, which round differently, 2e-6 (both are within 1e-6 of exact)."""
@@ -69,8 +70,15 @@ def test_delays_match_single_columns(fa, even):
     kw = dict(window=fa.windows.tukey(0.5), F_number=fa.f_numbers.grating.angle_lb(60, 1.5), output_scale="cpu")
     p = fa.LineScan(x, z, n_t, n_el, FS, WIDTH, PITCH, C0, band, 20e-3, **kw)
     img = torch.empty((n_lines, n_z), dtype=torch.complex64, device="cuda")
+    # a graph captured with no delays, then replayed with them
+    batch = fa.Batch([p.plan])
+    batch.execute([rf], [img])
     p.plan.set_tof(1500.0, d)
+    batch.execute([rf], [img])
+    torch.cuda.synchronize()
+    got = img.clone()
     p.execute(rf, img)
+    assert torch.equal(torch.view_as_real(got), torch.view_as_real(img))
     ref = torch.empty_like(img)
     for i in range(n_lines):
         q = fa.PwPlan(x[i:i + 1], z, n_t, n_el, np.zeros(1), FS, WIDTH, PITCH, C0, band, 0.0,
@@ -78,4 +86,27 @@ def test_delays_match_single_columns(fa, even):
         q.set_tof(1500.0, d)
         q.execute(rf[i:i + 1], ref[i:i + 1])
         torch.cuda.synchronize()
-    assert rel_l2(img.cpu().numpy(), ref.cpu().numpy()) <= 2e-6
+    assert rel_l2(got.cpu().numpy(), ref.cpu().numpy()) <= 2e-6
+    batch.close()
+
+
+def test_captured_mirrored_plan_gets_other_delays(fa):
+    """a plane-wave plan of mirrored voxels in a captured batch: delays that are not symmetric"""
+    import torch
+
+    n_el, n_t = 64, 900
+    x, z = np.linspace(-6e-3, 6e-3, 24), np.linspace(5e-3, 30e-3, 31)
+    p = fa.PwPlan(x, z, n_t, n_el, np.linspace(-0.2, 0.2, 3), FS, WIDTH, PITCH, C0, (2.25e6, 6.75e6), 0.0,
+                  window=fa.windows.tukey(0.5), F_number=fa.f_numbers.grating.angle_lb(60, 1.5))
+    rf = torch.randn((3, n_el, n_t), generator=torch.Generator().manual_seed(6)).cuda()
+    img = torch.empty((24, 31), dtype=torch.complex64, device="cuda")
+    batch = fa.Batch([p])
+    for d in (None, np.linspace(-25e-9, 40e-9, n_el), None):
+        p.set_tof(0.0, d)
+        batch.execute([rf], [img])
+        torch.cuda.synchronize()
+        got = img.clone()
+        p.execute(rf, img)
+        torch.cuda.synchronize()
+        assert rel_l2(got.cpu().numpy(), img.cpu().numpy()) <= 1e-6
+    batch.close()
