@@ -77,7 +77,7 @@ enum { FN_NORMALIZATION_OFF = 0, FN_NORMALIZATION_ON = 1, FN_NORMALIZATION_WINDO
  * truncated at |t| >= 1, element-snapped boxcar). */
 enum { FN_SEMANTICS_CPU = 0, FN_SEMANTICS_MEX = 1 };
 /* arithmetic of the element x transmit contraction */
-enum { FN_PRECISION_FP32 = 0,    /* FP32 MFMA operands, FP32 accumulation */
+enum { FN_PRECISION_FP32 = 0,    /* FP32 accuracy: FP32 operands or their fp16 hi + lo split, FP32 accumulation */
        FN_PRECISION_BF16X3 = 1,  /* BF16 hi+lo split operands, 3 MFMA passes, FP32 accumulation */
        FN_PRECISION_FP16X3 = 2,  /* FP16 hi+lo split operands, 3 passes */
        FN_PRECISION_FP16 = 3 };  /* FP16 operands, 1 pass */
