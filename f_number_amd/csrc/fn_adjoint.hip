@@ -11,8 +11,8 @@
 //   Z_n(k,a)      = s sum_v y(v) conj(T_n(v,a) a_nk(v) e^{j w_n tau_rx(v,k)}) / w_n(v)   (voxel contraction)
 //   (A^H y)[a][k][t] = Re sum_n Z_n(k,a) e^{+j 2 pi n t / N}                          (band-limited inverse DFT)
 //
-// Voxel contraction on the matrix cores (v_mfma_f32_16x16x4f32, Gauss three
-// multiplications): per bin, D[element][angle] += sum_v conj(B)[element][v] U[v][angle]
+// Voxel contraction on the matrix cores (fp16 hi + lo; the untruncated triangular window on
+// v_mfma_f32_16x16x4f32 with Gauss's three multiplications): per bin, D[element][angle] += sum_v conj(B)[element][v] U[v][angle]
 // with U = s y conj(T) / w.  The contraction index (voxels) is the MFMA K, so
 // lane l holds the pairs (voxel 4s + l/16 of a 16-voxel group, element
 // l%16 + 16 mt).  A block of 4 waves owns 4 consecutive bins (one per wave)

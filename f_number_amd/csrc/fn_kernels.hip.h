@@ -14,8 +14,8 @@
 //                   in registers (replaces das_kernel_phase_shifts.cu:8-147 /
 //                   saft_kernel_phase_shifts.cu:8-199, which wrote it to HBM),
 //                   contracts it against the transmit spectra X_n(k,a) on
-//                   v_mfma_f32_16x16x4f32 (replaces the cublasCgemm GEMV of
-//                   gpu_bf_das_pw_rf.cu:1034-1041), then applies the transmit
+//                   the matrix cores (FP32 plans as fp16 hi + lo; replaces the
+//                   cublasCgemm GEMV of gpu_bf_das_pw_rf.cu:1034-1041), then applies the transmit
 //                   phase / transmit apodization, the normalization
 //                   (das_kernel_normalization.cu:8-34) and accumulates the
 //                   image over bins in registers.
