@@ -192,6 +192,7 @@ struct fn_plan {
     float2 *d_tw = nullptr, *d_X = nullptr;
     void *d_Xlp = nullptr;    // 16-bit spectra planes (mixed precision)
     float *d_xscale = nullptr;
+    float *d_rowscale = nullptr;  // ensembles: scales of the rows and the peaks behind them (row_scales)
     double *d_delay = nullptr;  // per-element delay offsets (zeros unless set)
     double *d_zeros = nullptr;  // zeros in their place
     // adjoint / vector-Jacobian workspace (allocated on first use)
@@ -451,6 +452,12 @@ int form_planes(int kprec) { return kprec == FN_PRECISION_FP16 ? 2 : 4; }
 // planes (Xr, Xi and, for the split forms, their residuals)
 size_t form_step_bytes(int kprec) { return kprec == FN_PRECISION_FP32 ? 64 * sizeof(float2) : (size_t)form_planes(kprec) * 64 * 2; }
 
+// scales of MT tiles of transmit rows: [2][16 MT], and room for their peaks per chunk of bins
+constexpr int ROW_PEAK_CHUNKS = 64;
+size_t row_scale_bytes(int MT) { return (size_t)(2 + ROW_PEAK_CHUNKS) * 16 * MT * sizeof(float); }
+// (bf16 has the exponents of FP32)
+bool has_row_scales(int kprec) { return kprec == FN_PRECISION_FP16X3 || kprec == FN_PRECISION_FP16; }
+
 // element steps per lane: 4 KI >= n_el elements in four lane groups
 int ki_of(int n_el)
 {
@@ -698,6 +705,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t tables = cv.used;
     const size_t o_X = cv.take(spectra_of ? 0 : P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
     const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
+    const size_t o_rs = cv.take(P->n_frames > 1 && has_row_scales(P->kprec) ? row_scale_bytes(P->MT_all) : 0);
     const size_t o_xr = cv.take(P->lbl ? (size_t)g.n_f * c.n_x * c.n_el * sizeof(float2) : 0);
     std::vector<unsigned char> h(tables, 0);
     auto put = [&](size_t at, const void *src, size_t bytes) { if (bytes) std::memcpy(h.data() + at, src, bytes); };
@@ -722,6 +730,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     P->d_zeros = at(o_zr);
     P->d_X = spectra_of ? spectra_of->d_X : reinterpret_cast<float2 *>(at(o_X));
     P->d_Xlp = P->xlp_bytes ? at(o_Xlp) : nullptr;
+    P->d_rowscale = P->n_frames > 1 && has_row_scales(P->kprec) ? reinterpret_cast<float *>(at(o_rs)) : nullptr;
     P->d_Xrow = P->lbl ? reinterpret_cast<float2 *>(at(o_xr)) : nullptr;
     P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
 
@@ -730,6 +739,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     A.delay = P->d_delay;
     A.Xlp = P->d_Xlp;
     A.xscale = P->d_xscale;
+    A.row_scale = P->d_rowscale;
     A.px = P->d_px; A.pz = P->d_pz; A.Frx = P->d_Frx; A.Ftx = P->d_Ftx; A.txp = P->d_txp; A.sqrt_f = P->d_sqf;
     return ensure_partials(P);
 }
@@ -965,26 +975,42 @@ fnk::BeamArgs beam_args(const fn_plan *P, float *d_image, float *d_w, float *d_w
     return A;
 }
 
-// the 16-bit operand planes (and per-bin scales) of FP32 spectra X of MT tiles (MT_out,
-// mirror_el, delay: see lowp_planes_kernel); nothing for FP32 kernels
-int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xscale, int MT, int MT_out, int mirror_el,
-                       const double *delay, hipStream_t s)
+int launch_row_scales(const float2 *X, float *scale, int MT, int KI, int n_f, hipStream_t s)
 {
+    const int rows = 16 * MT, chunk = (n_f + ROW_PEAK_CHUNKS - 1) / ROW_PEAK_CHUNKS, n = (n_f + chunk - 1) / chunk;
+    hipLaunchKernelGGL(fnk::row_peak_kernel, dim3((unsigned)MT, (unsigned)n), dim3(256), 0, s, X, scale + 2 * rows, MT, KI,
+                       n_f, chunk);
+    HIP_CHECK(hipGetLastError(), "row_peak_kernel");
+    hipLaunchKernelGGL(fnk::row_scale_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, scale + 2 * rows, scale,
+                       rows, n);
+    HIP_CHECK(hipGetLastError(), "row_scale_kernel");
+    return FN_OK;
+}
+
+// the 16-bit operand planes (and per-bin scales) of FP32 spectra X of MT tiles (MT_out,
+// mirror_el, delay: see lowp_planes_kernel; rowscale: launch_row_scales, null: none); nothing
+// for FP32 kernels
+int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xscale, int MT, int MT_out, int mirror_el,
+                       const double *delay, hipStream_t s, float *rowscale = nullptr)
+{
+    const float *row_inv = rowscale ? rowscale + 16 * MT : nullptr;
+    if (rowscale)
+        if (int st = launch_row_scales(X, rowscale, MT, P->KI, P->g.n_f, s)) return st;
     const dim3 cg((unsigned)P->g.n_f), cb(256);
     const double fs_over_N = P->args.f_s / P->g.N;
     switch (P->kprec) {
     case FN_PRECISION_FP32: return FN_OK;
     case FN_PRECISION_BF16X3:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_BF16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el);
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv);
         break;
     case FN_PRECISION_FP16X3:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el);
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv);
         break;
     default:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el);
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv);
         break;
     }
     HIP_CHECK(hipGetLastError(), "lowp_planes_kernel");
@@ -1045,7 +1071,7 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
         return e == hipSuccess ? FN_OK : hip_fail(e, "interp_samples_kernel");
     }
     return launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, S.MT, plane_tiles(P), use_mirror(P) ? P->n_el : 0,
-                              plane_delay(P, use_mirror(P)), s);
+                              plane_delay(P, use_mirror(P)), s, P->d_rowscale);
 }
 
 int execute(fn_plan *P, const void *d_rf, int dtype, float *d_image, float *d_w, float *d_w_rx, hipStream_t user)
@@ -2093,7 +2119,7 @@ struct RowStack {
     size_t lds_beam = 0;
     float2 *d_X = nullptr;
     void *d_Xlp = nullptr;
-    float *d_xscale = nullptr;
+    float *d_xscale = nullptr, *d_rowscale = nullptr;
     double *d_txp = nullptr;
     int *d_row_frame = nullptr;
     float2 **d_frame_image = nullptr;
@@ -2137,6 +2163,7 @@ static void batch_release_graph(fn_batch *b)
         hipFree(r.d_X);
         hipFree(r.d_Xlp);
         hipFree(r.d_xscale);
+        hipFree(r.d_rowscale);
         hipFree(r.d_txp);
         hipFree(r.d_row_frame);
         hipFree(r.d_frame_image);
@@ -2217,6 +2244,7 @@ static int batch_plan_stacks(fn_batch *b, float *const *d_images, std::vector<ch
         if (e == hipSuccess && P0->kprec != FN_PRECISION_FP32) {
             e = hipMalloc(&R.d_Xlp, n_f * form_planes(P0->kprec) * R.n_groups * R.MT_tmpl * P0->KI * 64 * 2);
             if (e == hipSuccess) e = hipMalloc(&R.d_xscale, n_f * sizeof(float));
+            if (e == hipSuccess && has_row_scales(P0->kprec)) e = hipMalloc(&R.d_rowscale, row_scale_bytes(R.MT_all));
         }
         if (e == hipSuccess) e = hipMalloc(&R.d_txp, 3 * sizeof(double) * R.rows);
         for (size_t m = 0; m < R.plans.size() && e == hipSuccess; ++m) {
@@ -2251,12 +2279,14 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
         S.write_pad = 0;
         if (int st = launch_spectra_into(P, d_rf[R.plans[m]], dtypes[R.plans[m]], s, R.d_X, S)) return st;
     }
-    if (int st = launch_lowp_planes(P0, R.d_X, R.d_Xlp, R.d_xscale, R.MT_all, R.n_groups * R.MT_tmpl, 0, nullptr, s))
+    if (int st = launch_lowp_planes(P0, R.d_X, R.d_Xlp, R.d_xscale, R.MT_all, R.n_groups * R.MT_tmpl, 0, nullptr, s,
+                                    R.d_rowscale))
         return st;
     fnk::BeamArgs A = forward_args(P0);
     A.X = R.d_X;
     A.Xlp = R.d_Xlp;
     A.xscale = R.d_xscale;
+    A.row_scale = R.d_rowscale;
     A.txp = R.d_txp;
     A.n_tx = R.rows;
     A.tx_group = R.MT_tmpl;

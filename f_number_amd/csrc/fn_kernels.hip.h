@@ -81,6 +81,7 @@ struct BeamArgs {
     const float2 *X;        // spectra in operand order [n_f][MT][KI][64]
     const void *Xlp;        // 16-bit spectra planes (mixed precision) [n_f][planes][MT][KI/8][64][8]
     const float *xscale;    // per-bin scale of the 16-bit planes
+    const float *row_scale; // ensembles, row stacks: per transmit row a scale beside it (null: none)
     const double *px, *pz;  // voxel positions
     const double *Frx;      // F-number per band bin (receive)
     const double *Ftx;      // F-number per band bin (transmit, SA)
@@ -1464,8 +1465,9 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                         f_run = f;
                         sr = si = 0.f;
                     }
-                    sr += Er[ENS ? mt : 0][r];
-                    si += Ei[ENS ? mt : 0][r];
+                    const float rs = A.row_scale ? A.row_scale[row] : 1.0f;
+                    sr = fmaf(rs, Er[ENS ? mt : 0][r], sr);
+                    si = fmaf(rs, Ei[ENS ? mt : 0][r], si);
                 }
                 if (f_run >= 0) {
                     float2 *img = A.frame_image ? A.frame_image[f_run] : A.image + (size_t)f_run * n_vox;
@@ -1608,8 +1610,45 @@ static __global__ __launch_bounds__(256) void reduce_partials_kernel(const float
 // -------------------------------------------------------------------------
 // 16-bit spectra planes for the mixed-precision contraction
 // -------------------------------------------------------------------------
+// Transmit rows of an ensemble or a row stack are other frames or jobs, whose samples may be
+// of any size: each has a power of two of its own over the whole band, so that the planes'
+// exponent range (2^-39 of a bin's largest value) holds row by row.  Constant over the bins,
+// it is taken out where a row's image is added to its frame's.  One block per M-tile and chunk
+// of bins: the rows' largest components, peak[chunk][16 MT].  Bound by reading the spectra.
+static __global__ __launch_bounds__(256) void row_peak_kernel(const float2 *__restrict__ X, float *__restrict__ peak, int MT,
+                                                              int KI, int n_f, int chunk)
+{
+    __shared__ float red[256];
+    const int mt = blockIdx.x, tid = threadIdx.x, b1 = min((int)(blockIdx.y + 1) * chunk, n_f);
+    float m = 0.f;
+    for (int b = blockIdx.y * chunk; b < b1; ++b) {
+        const float2 *Xb = X + ((size_t)b * MT + mt) * KI * 64;
+        for (int e = tid; e < KI * 64; e += 256) m = fmaxf(m, fmaxf(fabsf(Xb[e].x), fabsf(Xb[e].y)));  // row e & 15
+    }
+    red[tid] = m;
+    __syncthreads();
+    if (tid >= 16) return;
+    for (int w = 16 + tid; w < 256; w += 16) m = fmaxf(m, red[w]);
+    peak[(size_t)blockIdx.y * 16 * MT + 16 * mt + tid] = m;
+}
+
+// scale[row] = 2^e with the row's largest component in [2^(e-1), 2^e), then 1 / scale[row]
+static __global__ void row_scale_kernel(const float *__restrict__ peak, float *__restrict__ scale, int n_rows, int n_chunks)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= n_rows) return;
+    float m = 0.f;
+    for (int c = 0; c < n_chunks; ++c) m = fmaxf(m, peak[(size_t)c * n_rows + r]);
+    int e2 = 0;
+    if (m > 0.f) frexpf(m, &e2);
+    e2 = min(max(e2, -120), 120);
+    scale[r] = ldexpf(1.0f, e2);
+    scale[n_rows + r] = ldexpf(1.0f, -e2);
+}
+
 // One block per bin: reads the FP32 operand-ordered spectra of the bin, picks a
-// power-of-two scale (16-bit float variants: largest component in [2^14, 2^15)),
+// power-of-two scale (16-bit float variants: largest component in [2^14, 2^15), of the rows
+// divided by their own scale where row_inv gives one),
 // and writes planes [p][mt][c][64][8] (p: Xr hi, Xi hi, Xr lo, Xi lo) with
 // lane (a & 15) + 16 (k & 3), slot (k >> 2) & 7, chunk k >> 5.  MT_out tiles are written:
 // those past MT_all are the first ones again with element mirror_el - 1 - k in the place of
@@ -1620,7 +1659,8 @@ template <int PREC>
 __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restrict__ X, void *__restrict__ Xlp,
                                                           float *__restrict__ xscale, int MT_all, int KI,
                                                           int MT_out, int mirror_el, const double *__restrict__ delay,
-                                                          double fs_over_N, int n_lb, int n_el)
+                                                          double fs_over_N, int n_lb, int n_el,
+                                                          const float *__restrict__ row_inv)
 {
     __shared__ float red[256];
     const int b = blockIdx.x;
@@ -1629,7 +1669,8 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
     float m = 0.f;
     for (int e = threadIdx.x; e < n_pairs; e += 256) {
         const float2 v = Xb[e];
-        m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)));
+        const float ri = row_inv ? row_inv[16 * (e / (KI * 64)) + (e & 15)] : 1.0f;
+        m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)) * ri);
     }
     red[threadIdx.x] = m;
     __syncthreads();
@@ -1664,6 +1705,10 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
             float sn, cs;
             sincospif((float)(int32_t)P * (1.0f / 2147483648.0f), &sn, &cs);
             v = make_float2(v.x * cs - v.y * sn, v.x * sn + v.y * cs);
+        }
+        if (row_inv && mt < MT_all) {
+            const float ri = row_inv[16 * mt + row];
+            v = make_float2(v.x * ri, v.y * ri);
         }
         const float vr = v.x * inv, vi = v.y * inv;
         if (PREC == PREC_BF16X3) {
