@@ -192,6 +192,7 @@ struct fn_plan {
     float2 *d_tw = nullptr, *d_X = nullptr;
     void *d_Xlp = nullptr;    // 16-bit spectra planes (mixed precision)
     float *d_xscale = nullptr;
+    uint32_t *d_bad = nullptr;    // elements that are not finite, beside the planes
     float *d_rowscale = nullptr;  // ensembles: scales of the rows and the peaks behind them (row_scales)
     double *d_delay = nullptr;  // per-element delay offsets (zeros unless set)
     double *d_zeros = nullptr;  // zeros in their place
@@ -458,6 +459,11 @@ size_t row_scale_bytes(int MT) { return (size_t)(2 + ROW_PEAK_CHUNKS) * 16 * MT 
 // (bf16 has the exponents of FP32)
 bool has_row_scales(int kprec) { return kprec == FN_PRECISION_FP16X3 || kprec == FN_PRECISION_FP16; }
 
+// words of a mask of 4 KI elements, and bytes of the masks beside n_f bins of planes (each of
+// `rows` operand rows has its own where they are other frames or jobs)
+int bad_words(int KI) { return KI / 8; }
+size_t bad_bytes(int n_f, int rows, int KI) { return (size_t)n_f * rows * bad_words(KI) * sizeof(uint32_t); }
+
 // element steps per lane: 4 KI >= n_el elements in four lane groups
 int ki_of(int n_el)
 {
@@ -705,6 +711,9 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t tables = cv.used;
     const size_t o_X = cv.take(spectra_of ? 0 : P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
     const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
+    P->args.bad_rows = P->n_frames > 1 ? 16 * P->MT_all : 1;
+    P->args.bad_words = bad_words(P->KI);
+    const size_t o_bad = cv.take(P->xlp_bytes ? bad_bytes(g.n_f, P->args.bad_rows, P->KI) : 0);
     const size_t o_rs = cv.take(P->n_frames > 1 && has_row_scales(P->kprec) ? row_scale_bytes(P->MT_all) : 0);
     const size_t o_xr = cv.take(P->lbl ? (size_t)g.n_f * c.n_x * c.n_el * sizeof(float2) : 0);
     std::vector<unsigned char> h(tables, 0);
@@ -730,6 +739,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     P->d_zeros = at(o_zr);
     P->d_X = spectra_of ? spectra_of->d_X : reinterpret_cast<float2 *>(at(o_X));
     P->d_Xlp = P->xlp_bytes ? at(o_Xlp) : nullptr;
+    P->d_bad = P->xlp_bytes ? reinterpret_cast<uint32_t *>(at(o_bad)) : nullptr;
     P->d_rowscale = P->n_frames > 1 && has_row_scales(P->kprec) ? reinterpret_cast<float *>(at(o_rs)) : nullptr;
     P->d_Xrow = P->lbl ? reinterpret_cast<float2 *>(at(o_xr)) : nullptr;
     P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
@@ -739,6 +749,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     A.delay = P->d_delay;
     A.Xlp = P->d_Xlp;
     A.xscale = P->d_xscale;
+    A.bad = P->d_bad;
     A.row_scale = P->d_rowscale;
     A.px = P->d_px; A.pz = P->d_pz; A.Frx = P->d_Frx; A.Ftx = P->d_Ftx; A.txp = P->d_txp; A.sqrt_f = P->d_sqf;
     return ensure_partials(P);
@@ -960,6 +971,7 @@ fnk::BeamArgs forward_args(const fn_plan *P)
 fnk::BeamArgs beam_args(const fn_plan *P, float *d_image, float *d_w, float *d_w_rx)
 {
     fnk::BeamArgs A = forward_args(P);
+    if (P->interp_M || P->lbl) A.bad = nullptr;               // no planes
     if (plane_delay(P, use_mirror(P))) A.delay = P->d_zeros;  // in the planes already
     A.image = reinterpret_cast<float2 *>(d_image);
     A.n_slots = beam_slots(P);
@@ -988,10 +1000,10 @@ int launch_row_scales(const float2 *X, float *scale, int MT, int KI, int n_f, hi
 }
 
 // the 16-bit operand planes (and per-bin scales) of FP32 spectra X of MT tiles (MT_out,
-// mirror_el, delay: see lowp_planes_kernel; rowscale: launch_row_scales, null: none); nothing
+// mirror_el, delay, bad: see lowp_planes_kernel; rowscale: launch_row_scales, null: none); nothing
 // for FP32 kernels
-int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xscale, int MT, int MT_out, int mirror_el,
-                       const double *delay, hipStream_t s, float *rowscale = nullptr)
+int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xscale, uint32_t *bad, int bad_rows, int MT,
+                       int MT_out, int mirror_el, const double *delay, hipStream_t s, float *rowscale = nullptr)
 {
     const float *row_inv = rowscale ? rowscale + 16 * MT : nullptr;
     if (rowscale)
@@ -1002,15 +1014,15 @@ int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xsca
     case FN_PRECISION_FP32: return FN_OK;
     case FN_PRECISION_BF16X3:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_BF16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv);
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI));
         break;
     case FN_PRECISION_FP16X3:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv);
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI));
         break;
     default:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv);
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI));
         break;
     }
     HIP_CHECK(hipGetLastError(), "lowp_planes_kernel");
@@ -1023,7 +1035,7 @@ int finish_beam(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s, float2 
 int run_shallow(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s)
 {
     const fn_plan *C = P->shallow;
-    if (int st = launch_lowp_planes(C, C->d_X, C->d_Xlp, C->d_xscale, C->MT_all, plane_tiles(C), use_mirror(C) ? C->n_el : 0,
+    if (int st = launch_lowp_planes(C, C->d_X, C->d_Xlp, C->d_xscale, C->d_bad, 1, C->MT_all, plane_tiles(C), use_mirror(C) ? C->n_el : 0,
                                     plane_delay(C, use_mirror(C)), s))
         return st;
     const fnk::BeamArgs B = beam_args(C, reinterpret_cast<float *>(P->d_simg), A.weights ? P->d_sw : nullptr, nullptr);
@@ -1037,14 +1049,17 @@ int run_shallow(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s)
 }
 
 // after the beamforming launch: the partial images of a voxel's workgroups summed
-// in slot order into the image (nothing when one workgroup owns each voxel), and the
-// clamped depths of an interpolated plan
+// in slot order into the image (none when one workgroup owns each voxel), the voxels that meet
+// values that are not finite (16-bit forms), and the clamped depths of an interpolated plan
 int finish_beam(const fn_plan *P, const fnk::BeamArgs &A, hipStream_t s, float2 *dimage)
 {
     if (A.partial) {
-        hipLaunchKernelGGL(fnk::reduce_partials_kernel, dim3((unsigned)((P->n_vox + 255) / 256)), dim3(256), 0, s,
-                           A.partial, A.n_slots, P->n_vox, A.image, dimage);
+        hipLaunchKernelGGL(fnk::reduce_partials_kernel, dim3((unsigned)((P->n_vox + 255) / 256)), dim3(256), 0, s, A, A.image,
+                           dimage);
         HIP_CHECK(hipGetLastError(), "reduce_partials_kernel");
+    } else if (A.bad) {
+        hipLaunchKernelGGL(fnk::nonfinite_kernel, dim3((unsigned)((P->n_vox + 255) / 256)), dim3(256), 0, s, A);
+        HIP_CHECK(hipGetLastError(), "nonfinite_kernel");
     }
     return P->shallow && !dimage ? run_shallow(P, A, s) : FN_OK;
 }
@@ -1070,8 +1085,8 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
                                                         S.MT, S.KI, P->n_tx, P->n_el, s);
         return e == hipSuccess ? FN_OK : hip_fail(e, "interp_samples_kernel");
     }
-    return launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, S.MT, plane_tiles(P), use_mirror(P) ? P->n_el : 0,
-                              plane_delay(P, use_mirror(P)), s, P->d_rowscale);
+    return launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, P->d_bad, P->args.bad_rows, S.MT, plane_tiles(P),
+                              use_mirror(P) ? P->n_el : 0, plane_delay(P, use_mirror(P)), s, P->d_rowscale);
 }
 
 int execute(fn_plan *P, const void *d_rf, int dtype, float *d_image, float *d_w, float *d_w_rx, hipStream_t user)
@@ -1357,7 +1372,7 @@ int execute_tangent(fn_plan *P, const void *d_rf, int dtype, float *d_image, flo
     const bool split_form = P->kprec == FN_PRECISION_FP16X3;
     const bool mirror = tangent_mirror(P);
     if (split_form) {
-        if (int st = launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, P->MT_all, mirror ? 2 * P->MT_all : groups * mt,
+        if (int st = launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, P->d_bad, 1, P->MT_all, mirror ? 2 * P->MT_all : groups * mt,
                                         mirror ? P->n_el : 0, plane_delay(P, mirror), s))
             return st;
     }
@@ -1716,7 +1731,7 @@ int one_shot(fn_plan *P, const void *rf, int dtype, float *image, float *w0, flo
 // and then uses exclusively (the array's name in host code is only a stand-in).
 // Calls on one device share the array and race if they overlap.
 namespace {
-constexpr size_t kScratchBytes = (size_t)32 << 20;
+constexpr size_t kScratchBytes = ((size_t)32 << 20) + ((size_t)64 << 10);  // (the masks take 32 KiB at most)
 constexpr int kMaxDevices = 64;
 }  // namespace
 
@@ -1824,7 +1839,7 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
     const int n_f = g.n_f, n_tx = c.n_tx, raw_per_tx = p->virtual_sources ? 2 : 1;
     Carve cv;
     size_t o_X = 0, o_Xlp = 0, o_xs = 0, o_px = 0, o_pz = 0, o_F = 0, o_sqf = 0, o_raw = 0, o_txp = 0, o_tw = 0, o_dl = 0,
-           o_pi = 0;
+           o_pi = 0, o_bad = 0;
     int slots = 1;
     // a call whose planes do not fit beside its spectra runs without the mirrored ones, an FP32
     // call then without any, on the FP32 kernels
@@ -1834,6 +1849,7 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
         o_X = cv.take(P.x_bytes);
         o_Xlp = cv.take(P.xlp_bytes);
         o_xs = cv.take(P.kprec != FN_PRECISION_FP32 ? (size_t)n_f * sizeof(float) : 0);
+        o_bad = cv.take(P.kprec != FN_PRECISION_FP32 ? bad_bytes(n_f, 1, P.KI) : 0);
         o_px = cv.take((size_t)c.n_x * sizeof(double));
         o_pz = cv.take((size_t)c.n_z * sizeof(double));
         o_F = cv.take((size_t)n_f * sizeof(double));
@@ -1858,6 +1874,9 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
     P.d_X = reinterpret_cast<float2 *>(base + o_X);
     P.d_Xlp = P.xlp_bytes ? base + o_Xlp : nullptr;
     P.d_xscale = P.xlp_bytes ? reinterpret_cast<float *>(base + o_xs) : nullptr;
+    P.d_bad = P.xlp_bytes ? reinterpret_cast<uint32_t *>(base + o_bad) : nullptr;
+    P.args.bad_rows = 1;
+    P.args.bad_words = bad_words(P.KI);
     P.d_px = reinterpret_cast<double *>(base + o_px);
     P.d_pz = reinterpret_cast<double *>(base + o_pz);
     P.d_Frx = reinterpret_cast<double *>(base + o_F);
@@ -1882,6 +1901,7 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
     A.X = P.d_X;
     A.Xlp = P.d_Xlp;
     A.xscale = P.d_xscale;
+    A.bad = P.d_bad;
     A.px = P.d_px; A.pz = P.d_pz; A.Frx = P.d_Frx; A.Ftx = nullptr; A.txp = P.d_txp; A.sqrt_f = P.d_sqf;
     A.delay = P.d_delay;
     // spectra (every operand slot of the workspace is written, padding as zeros) and
@@ -2120,6 +2140,7 @@ struct RowStack {
     float2 *d_X = nullptr;
     void *d_Xlp = nullptr;
     float *d_xscale = nullptr, *d_rowscale = nullptr;
+    uint32_t *d_bad = nullptr;
     double *d_txp = nullptr;
     int *d_row_frame = nullptr;
     float2 **d_frame_image = nullptr;
@@ -2164,6 +2185,7 @@ static void batch_release_graph(fn_batch *b)
         hipFree(r.d_Xlp);
         hipFree(r.d_xscale);
         hipFree(r.d_rowscale);
+        hipFree(r.d_bad);
         hipFree(r.d_txp);
         hipFree(r.d_row_frame);
         hipFree(r.d_frame_image);
@@ -2244,6 +2266,7 @@ static int batch_plan_stacks(fn_batch *b, float *const *d_images, std::vector<ch
         if (e == hipSuccess && P0->kprec != FN_PRECISION_FP32) {
             e = hipMalloc(&R.d_Xlp, n_f * form_planes(P0->kprec) * R.n_groups * R.MT_tmpl * P0->KI * 64 * 2);
             if (e == hipSuccess) e = hipMalloc(&R.d_xscale, n_f * sizeof(float));
+            if (e == hipSuccess) e = hipMalloc(&R.d_bad, bad_bytes((int)n_f, 16 * R.MT_all, P0->KI));
             if (e == hipSuccess && has_row_scales(P0->kprec)) e = hipMalloc(&R.d_rowscale, row_scale_bytes(R.MT_all));
         }
         if (e == hipSuccess) e = hipMalloc(&R.d_txp, 3 * sizeof(double) * R.rows);
@@ -2279,7 +2302,7 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
         S.write_pad = 0;
         if (int st = launch_spectra_into(P, d_rf[R.plans[m]], dtypes[R.plans[m]], s, R.d_X, S)) return st;
     }
-    if (int st = launch_lowp_planes(P0, R.d_X, R.d_Xlp, R.d_xscale, R.MT_all, R.n_groups * R.MT_tmpl, 0, nullptr, s,
+    if (int st = launch_lowp_planes(P0, R.d_X, R.d_Xlp, R.d_xscale, R.d_bad, 16 * R.MT_all, R.MT_all, R.n_groups * R.MT_tmpl, 0, nullptr, s,
                                     R.d_rowscale))
         return st;
     fnk::BeamArgs A = forward_args(P0);
@@ -2287,6 +2310,8 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
     A.Xlp = R.d_Xlp;
     A.xscale = R.d_xscale;
     A.row_scale = R.d_rowscale;
+    A.bad = R.d_bad;
+    A.bad_rows = 16 * R.MT_all;
     A.txp = R.d_txp;
     A.n_tx = R.rows;
     A.tx_group = R.MT_tmpl;
@@ -2305,6 +2330,9 @@ static int batch_run_stack(fn_batch *b, const RowStack &R, const void *const *d_
     const dim3 grid((unsigned)((P0->n_vox + 63) / 64), (unsigned)R.bin_split, (unsigned)R.n_groups);
     hipError_t e = fnk::kEnsLaunchers[ki_index(P0->KI)][P0->kprec](R.MT_tmpl, P0->wcr, grid, R.lds_beam, s, A, 1);
     if (e != hipSuccess) return hip_fail(e, "beamform_kernel (row stack)");
+    if (!A.bad) return FN_OK;
+    hipLaunchKernelGGL(fnk::nonfinite_kernel, dim3((unsigned)((P0->n_vox + 255) / 256)), dim3(256), 0, s, A);
+    HIP_CHECK(hipGetLastError(), "nonfinite_kernel (row stack)");
     return FN_OK;
 }
 

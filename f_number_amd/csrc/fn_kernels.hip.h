@@ -80,7 +80,11 @@ enum { SUPPORT_OPEN_H = 0,   // boxcar, CPU: |x_k - x| / h < 1 (das_pw.m:441)
 struct BeamArgs {
     const float2 *X;        // spectra in operand order [n_f][MT][KI][64]
     const void *Xlp;        // 16-bit spectra planes (mixed precision) [n_f][planes][MT][KI/8][64][8]
-    const float *xscale;    // per-bin scale of the 16-bit planes
+    const float *xscale;    // per-bin scale of the 16-bit planes, negative where the bin has values that are not finite
+    // 16-bit forms: elements whose spectra are not finite, one bit each, [n_f][bad_rows][bad_words]
+    // (written and read at the bins of negative xscale alone; bad_rows 1: of any row)
+    const uint32_t *bad;
+    int bad_rows, bad_words;
     const float *row_scale; // ensembles, row stacks: per transmit row a scale beside it (null: none)
     const double *px, *pz;  // voxel positions
     const double *Frx;      // F-number per band bin (receive)
@@ -1276,7 +1280,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
         }
         asum += __shfl_xor(asum, 16);
         asum += __shfl_xor(asum, 32);
-        const float xscale = (PREC == PREC_FP32) ? 1.0f : A.xscale[b];  // spectra were stored / xscale
+        const float xscale = (PREC == PREC_FP32) ? 1.0f : fabsf(A.xscale[b]);  // spectra were stored / xscale
 
         if (MODE == MODE_PW) {
             if (ap.valid) {
@@ -1580,30 +1584,101 @@ void beamform_persistent_kernel(const BeamArgs *__restrict__ jobs, const int4 *_
 
 static __global__ void reset_counter_kernel(int *c) { *c = 0; }
 
+// Spectra that are not finite (a NaN, Inf or overflowing sample).  The matrix forms multiply
+// every element of a chunk, those outside a voxel's support by zero, and 0 x NaN would reach
+// voxels that never meet the element.  The planes hold zeros in their place, and the voxels
+// whose receive support holds such an element, at a bin where it is not finite, get NaN here:
+// put(row), row = operand row where every row has its own elements (bad_rows > 1).  Nothing but
+// a look at the bins' signs where every value is finite.  One voxel a thread, v >= n_vox: none.
+template <typename Put>
+__device__ __forceinline__ void spread_nonfinite(const BeamArgs &A, const long v, Put put)
+{
+    const int tid = threadIdx.x;
+    bool any = false;
+    for (int b = tid; b < A.n_f; b += blockDim.x) any |= A.xscale[b] < 0.f;
+    if (!__syncthreads_or(any)) return;
+    __shared__ uint32_t m[8];
+    int lo = 0x7fff, hi = -1;  // the voxel's support over these bins (each surrounds the voxel)
+    if (v < (long)A.n_x * A.n_z) {
+        const int ix = (int)(v / A.n_z), iz = (int)(v - (long)ix * A.n_z);
+        const double x = A.px[ix], z = A.pz[iz];
+        const double clamp_z = sqrt(z / (2.88 * A.c0));
+        for (int b = 0; b < A.n_f; ++b) {
+            if (!(A.xscale[b] < 0.f)) continue;
+            double Fr = A.Frx[b];
+            if (A.clamp) Fr = fmin(Fr, A.sqrt_f[b] * clamp_z);
+            const Aperture ap = make_aperture(x, x / A.pitch, z / (2.0 * A.pitch), Fr, A, A.support_rx);
+            if (!ap.valid || ap.klo > ap.khi) continue;
+            lo = min(lo, ap.klo);
+            hi = max(hi, ap.khi);
+        }
+    }
+    for (int r = 0; r < A.bad_rows; ++r) {
+        __syncthreads();
+        if (tid < 8) m[tid] = 0u;
+        __syncthreads();
+        for (int b = tid; b < A.n_f; b += blockDim.x)
+            for (int j = 0; A.xscale[b] < 0.f && j < A.bad_words; ++j)
+                atomicOr(&m[j], A.bad[((size_t)b * A.bad_rows + r) * A.bad_words + j]);
+        __syncthreads();
+        bool hit = false;
+        for (int j = 0; j < A.bad_words; ++j) {
+            const int b0 = max(lo - 32 * j, 0), b1 = min(hi - 32 * j, 31);  // bits b0 .. b1 of the word
+            if (b0 <= b1) hit |= (m[j] & (0xffffffffu << b0) & (0xffffffffu >> (31 - b1))) != 0u;
+        }
+        if (hit) put(r);
+    }
+}
+
+static __global__ __launch_bounds__(256) void nonfinite_kernel(BeamArgs A)
+{
+    const long v = (long)blockIdx.x * blockDim.x + threadIdx.x, n_vox = (long)A.n_x * A.n_z;
+    const float2 nan2 = make_float2(__builtin_nanf(""), __builtin_nanf(""));
+    spread_nonfinite(A, v, [&](int r) {
+        float2 *img = A.image;
+        if (A.bad_rows > 1) {
+            if (r >= A.n_tx) return;
+            const int f = A.row_frame ? A.row_frame[r] : r % A.ens_slots;
+            if (f < 0 || (!A.row_frame && f >= A.ens_frames)) return;
+            img = A.frame_image ? A.frame_image[f] : A.image + (size_t)f * n_vox;
+        }
+        img[v] = nan2;
+        if (A.dimage) reinterpret_cast<float2 *>(A.dimage)[v] = nan2;
+    });
+}
+
 // sum of the partial images of every (bin chunk, transmit group) slot in slot
 // order: out[v] = sum_s P[s][v]; dout (tangent) from slots n_slots .. 2 n_slots - 1
-static __global__ __launch_bounds__(256) void reduce_partials_kernel(const float2 *__restrict__ P, int n_slots,
-                                                                     long n_vox, float2 *__restrict__ out,
+static __global__ __launch_bounds__(256) void reduce_partials_kernel(BeamArgs A, float2 *__restrict__ out,
                                                                      float2 *__restrict__ dout)
 {
-    const long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n_vox) return;
-    float2 a = P[v];
-    for (int k = 1; k < n_slots; ++k) {
-        const float2 q = P[(long)k * n_vox + v];
-        a.x += q.x;
-        a.y += q.y;
-    }
-    out[v] = a;
-    if (dout) {
-        float2 d = P[(long)n_slots * n_vox + v];
+    const float2 *__restrict__ const P = A.partial;
+    const int n_slots = A.n_slots;
+    const long v = (long)blockIdx.x * blockDim.x + threadIdx.x, n_vox = (long)A.n_x * A.n_z;
+    if (v < n_vox) {
+        float2 a = P[v];
         for (int k = 1; k < n_slots; ++k) {
-            const float2 q = P[(long)(n_slots + k) * n_vox + v];
-            d.x += q.x;
-            d.y += q.y;
+            const float2 q = P[(long)k * n_vox + v];
+            a.x += q.x;
+            a.y += q.y;
         }
-        dout[v] = d;
+        out[v] = a;
+        if (dout) {
+            float2 d = P[(long)n_slots * n_vox + v];
+            for (int k = 1; k < n_slots; ++k) {
+                const float2 q = P[(long)(n_slots + k) * n_vox + v];
+                d.x += q.x;
+                d.y += q.y;
+            }
+            dout[v] = d;
+        }
     }
+    if (A.bad)
+        spread_nonfinite(A, v, [&](int) {
+            const float2 nan2 = make_float2(__builtin_nanf(""), __builtin_nanf(""));
+            out[v] = nan2;
+            if (dout) dout[v] = nan2;
+        });
 }
 
 
@@ -1623,7 +1698,10 @@ static __global__ __launch_bounds__(256) void row_peak_kernel(const float2 *__re
     float m = 0.f;
     for (int b = blockIdx.y * chunk; b < b1; ++b) {
         const float2 *Xb = X + ((size_t)b * MT + mt) * KI * 64;
-        for (int e = tid; e < KI * 64; e += 256) m = fmaxf(m, fmaxf(fabsf(Xb[e].x), fabsf(Xb[e].y)));  // row e & 15
+        for (int e = tid; e < KI * 64; e += 256) {  // row e & 15
+            const float a = fmaxf(fabsf(Xb[e].x), fabsf(Xb[e].y));
+            m = a < INFINITY ? fmaxf(m, a) : m;
+        }
     }
     red[tid] = m;
     __syncthreads();
@@ -1655,20 +1733,29 @@ static __global__ void row_scale_kernel(const float *__restrict__ peak, float *_
 // element k (mirror_el > 0), or zeros, which fill the last transmit group of a launch.
 // delay: per-element delay offsets d_k taken into the spectra as e^{j w_n d_k} (null: left to
 // the kernels' phase words); the mirrored tiles' weights then stay alike on both sides.
+// Values that are not finite are left out of the scale and written as zeros; the bin's scale is
+// then negative and their elements are noted in bad (spread_nonfinite).
 template <int PREC>
 __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restrict__ X, void *__restrict__ Xlp,
                                                           float *__restrict__ xscale, int MT_all, int KI,
                                                           int MT_out, int mirror_el, const double *__restrict__ delay,
                                                           double fs_over_N, int n_lb, int n_el,
-                                                          const float *__restrict__ row_inv)
+                                                          const float *__restrict__ row_inv,
+                                                          uint32_t *__restrict__ bad, int bad_rows, int bad_words)
 {
+    auto finite = [](float2 v) { return fabsf(v.x) < INFINITY && fabsf(v.y) < INFINITY; };
     __shared__ float red[256];
     const int b = blockIdx.x;
     const int n_pairs = MT_all * KI * 64;
     const float2 *Xb = X + (size_t)b * n_pairs;
     float m = 0.f;
+    bool nf = false;
     for (int e = threadIdx.x; e < n_pairs; e += 256) {
         const float2 v = Xb[e];
+        if (!finite(v)) {
+            nf = true;
+            continue;
+        }
         const float ri = row_inv ? row_inv[16 * (e / (KI * 64)) + (e & 15)] : 1.0f;
         m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)) * ri);
     }
@@ -1684,9 +1771,21 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
         int e2;
         frexpf(mx, &e2);              // mx = f 2^e2, f in [0.5, 1)
         // mx / scale in [2^14, 2^15); the scale and its reciprocal stay normal numbers
-        scale = ldexpf(1.0f, min(max(e2 - 15, -120), 112));
+        scale = ldexpf(1.0f, min(max(e2 - 15, -120), 113));
     }
-    if (threadIdx.x == 0) xscale[b] = scale;
+    const bool any_nf = __syncthreads_or(nf);
+    if (any_nf) {
+        uint32_t *w = bad + (size_t)b * bad_rows * bad_words;
+        for (int i = threadIdx.x; i < bad_rows * bad_words; i += 256) atomicExch(&w[i], 0u);
+        __threadfence();
+        __syncthreads();
+        for (int e = threadIdx.x; e < n_pairs; e += 256) {
+            if (finite(Xb[e])) continue;
+            const int q = e >> 6, k = 4 * (q % KI) + ((e & 63) >> 4), row = 16 * (q / KI) + (e & 15);
+            atomicOr(&w[(bad_rows > 1 ? row * bad_words : 0) + (k >> 5)], 1u << (k & 31));
+        }
+    }
+    if (threadIdx.x == 0) xscale[b] = any_nf ? -scale : scale;
     const float inv = 1.0f / scale;
     constexpr int pl = Prec<PREC>::planes;
     const int KC = KI / 8;
@@ -1699,6 +1798,7 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
         const int k = 32 * cc + 4 * s + gg;
         const int km = mt < MT_all ? k : mirror_el - 1 - k, mx_t = mt < MT_all ? mt : mt - MT_all;
         float2 v = km >= 0 ? Xb[(mx_t * KI + (km >> 2)) * 64 + row + 16 * (km & 3)] : make_float2(0.f, 0.f);
+        if (any_nf && !finite(v)) v = make_float2(0.f, 0.f);
         if (delay && km >= 0 && km < n_el) {
             // n frac(f_s d / N) mod 1 in units of 2^-32, then half revolutions
             const uint32_t P = (uint32_t)(n_lb + b) * frac32(fs_over_N * delay[km]);
