@@ -99,8 +99,10 @@ hipError_t launch_adjoint_reduce(const float *P, float2 *Z, int n_vr, int n_f, i
                                  const double *delay, double fs_over_N, int n_lb, hipStream_t s);
 hipError_t launch_adjoint_idft(const float2 *Z, const float2 *tw, float *out, int n_t, int n_ch, int N, int n_lb,
                                int n_f, hipStream_t s);
-hipError_t launch_lines(int wcr, bool mirror, int tiles, int splits, const BeamArgs &A, const float2 *X, hipStream_t s);
-hipError_t launch_lines_spectra(const float2 *X, float2 *out, int n_f, int MT, int KI, int n_x, int n_el, hipStream_t s);
+hipError_t launch_lines(int wcr, bool mirror, int tiles, int splits, const BeamArgs &A, const float2 *X, const uint32_t *flag,
+                        const uint32_t *bad, int KW, hipStream_t s);
+hipError_t launch_lines_spectra(const float2 *X, float2 *out, int n_f, int MT, int KI, int n_x, int n_el, uint32_t *flag,
+                                uint32_t *bad, hipStream_t s);
 hipError_t launch_interp_tables(float2 *tw, float *ipsi, int M, int n_f, hipStream_t s);
 hipError_t launch_interp_samples(const float2 *X, const float2 *tw, const float *ipsi, float2 *G, int M, int n_f, int MT,
                                  int KI, int n_tx, int n_el, hipStream_t s);
@@ -177,6 +179,7 @@ struct fn_plan {
     int delays_even = 1;    // delay offsets symmetric about the array's centre
     int interp_M = 0;       // > 0: the forward image by interpolation of M samples per channel
     float2 *d_Xrow = nullptr;  // line scan: the spectra by rows [n_f][line][element]
+    uint32_t *d_lflag = nullptr;  // its tiles' flags and masks of elements that are not finite (fn_lines.hip)
     float2 *d_ip = nullptr; // its channel samples, twiddles [M] and 1 / psi [n_f]
     // interpolated plans with depths where the F-number clamp is at work: a plan of those
     // leading depths (on this plan's spectra), its image and weights, pasted over the first rows
@@ -464,6 +467,9 @@ bool has_row_scales(int kprec) { return kprec == FN_PRECISION_FP16X3 || kprec ==
 int bad_words(int KI) { return KI / 8; }
 size_t bad_bytes(int n_f, int rows, int KI) { return (size_t)n_f * rows * bad_words(KI) * sizeof(uint32_t); }
 
+// words of a line scan's flags, before its masks
+size_t lines_flags(const fn_plan *P) { return (size_t)P->MT_all * P->g.n_f; }
+
 // element steps per lane: 4 KI >= n_el elements in four lane groups
 int ki_of(int n_el)
 {
@@ -716,6 +722,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t o_bad = cv.take(P->xlp_bytes ? bad_bytes(g.n_f, P->args.bad_rows, P->KI) : 0);
     const size_t o_rs = cv.take(P->n_frames > 1 && has_row_scales(P->kprec) ? row_scale_bytes(P->MT_all) : 0);
     const size_t o_xr = cv.take(P->lbl ? (size_t)g.n_f * c.n_x * c.n_el * sizeof(float2) : 0);
+    const size_t o_lf = cv.take(P->lbl ? lines_flags(P) * sizeof(uint32_t) + bad_bytes(g.n_f, c.n_x, P->KI) : 0);
     std::vector<unsigned char> h(tables, 0);
     auto put = [&](size_t at, const void *src, size_t bytes) { if (bytes) std::memcpy(h.data() + at, src, bytes); };
     put(o_px, c.px, c.n_x * sizeof(double));
@@ -742,6 +749,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     P->d_bad = P->xlp_bytes ? reinterpret_cast<uint32_t *>(at(o_bad)) : nullptr;
     P->d_rowscale = P->n_frames > 1 && has_row_scales(P->kprec) ? reinterpret_cast<float *>(at(o_rs)) : nullptr;
     P->d_Xrow = P->lbl ? reinterpret_cast<float2 *>(at(o_xr)) : nullptr;
+    P->d_lflag = P->lbl ? reinterpret_cast<uint32_t *>(at(o_lf)) : nullptr;
     P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
 
     fnk::BeamArgs &A = P->args;
@@ -906,7 +914,8 @@ hipError_t launch_beam(const fn_plan *P, dim3 grid, const fnk::BeamArgs &A, hipS
     }
     const int kidx = ki_index(P->KI);  // ensembles, line scans and windowed plans stop at KI = 32
     if (P->lbl)
-        return fnk::launch_lines(P->wcr, P->line_mirror && P->delays_even, (int)grid.x, (int)grid.y, A, P->d_Xrow, s);
+        return fnk::launch_lines(P->wcr, P->line_mirror && P->delays_even, (int)grid.x, (int)grid.y, A, P->d_Xrow,
+                                 P->d_lflag, P->d_lflag + lines_flags(P), bad_words(P->KI), s);
     if (use_mirror(P)) return fnk::kMirLaunchers[kidx](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A);
     if (P->nw) return fnk::kNwLaunchers[P->mode][kidx](P->MT_tmpl, P->wcr, P->wct, grid, P->lds_beam, s, A);
     if (P->n_frames > 1) return fnk::kEnsLaunchers[kidx][P->kprec](P->MT_tmpl, P->wcr, grid, P->lds_beam, s, A, 0);
@@ -1077,7 +1086,8 @@ int prepare(fn_plan *P, const void *d_rf, int dtype, float *d_image, hipStream_t
     const fnk::SpecArgs &S = P->sargs;
     if (int st = launch_spectra(P, d_rf, dtype, s)) return st;
     if (P->lbl) {
-        const hipError_t e = fnk::launch_lines_spectra(P->d_X, P->d_Xrow, S.n_f, S.MT, S.KI, P->n_x, P->n_el, s);
+        const hipError_t e = fnk::launch_lines_spectra(P->d_X, P->d_Xrow, S.n_f, S.MT, S.KI, P->n_x, P->n_el, P->d_lflag,
+                                                       P->d_lflag + lines_flags(P), s);
         return e == hipSuccess ? FN_OK : hip_fail(e, "lines_spectra_kernel");
     }
     if (P->interp_M) {

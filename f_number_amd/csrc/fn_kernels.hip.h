@@ -1584,6 +1584,17 @@ void beamform_persistent_kernel(const BeamArgs *__restrict__ jobs, const int4 *_
 
 static __global__ void reset_counter_kernel(int *c) { *c = 0; }
 
+// does a mask of elements hold one of lo .. hi (none where lo > hi)
+__device__ __forceinline__ bool mask_meets(const uint32_t *m, const int words, const int lo, const int hi)
+{
+    bool hit = false;
+    for (int j = 0; j < words; ++j) {
+        const int b0 = max(lo - 32 * j, 0), b1 = min(hi - 32 * j, 31);  // bits b0 .. b1 of the word
+        if (b0 <= b1) hit |= (m[j] & (0xffffffffu << b0) & (0xffffffffu >> (31 - b1))) != 0u;
+    }
+    return hit;
+}
+
 // Spectra that are not finite (a NaN, Inf or overflowing sample).  The matrix forms multiply
 // every element of a chunk, those outside a voxel's support by zero, and 0 x NaN would reach
 // voxels that never meet the element.  The planes hold zeros in their place, and the voxels
@@ -1621,12 +1632,7 @@ __device__ __forceinline__ void spread_nonfinite(const BeamArgs &A, const long v
             for (int j = 0; A.xscale[b] < 0.f && j < A.bad_words; ++j)
                 atomicOr(&m[j], A.bad[((size_t)b * A.bad_rows + r) * A.bad_words + j]);
         __syncthreads();
-        bool hit = false;
-        for (int j = 0; j < A.bad_words; ++j) {
-            const int b0 = max(lo - 32 * j, 0), b1 = min(hi - 32 * j, 31);  // bits b0 .. b1 of the word
-            if (b0 <= b1) hit |= (m[j] & (0xffffffffu << b0) & (0xffffffffu >> (31 - b1))) != 0u;
-        }
-        if (hit) put(r);
+        if (mask_meets(m, A.bad_words, lo, hi)) put(r);
     }
 }
 

@@ -21,16 +21,38 @@ constexpr int LN_BINS = 4;  // bins a wave walks together: one phase word read a
 
 // The spectra [n_f][MT][KI][64] by rows, [n_f][line][element]: a wave's scalar loads then take
 // four elements of a line at once (in operand order each element's 8 bytes are a cache line of
-// their own: 2.76 ms a frame of 128 x 512 against 2.13).
+// their own: 2.76 ms a frame of 128 x 512 against 2.13).  Values that are not finite are written
+// as zeros: flag [MT][n_f] says whether the 16 lines of a tile hold any at a bin, and their
+// elements are then noted in bad [n_f][line][KI / 8], one bit each.
 __global__ __launch_bounds__(256) void lines_spectra_kernel(const float2 *__restrict__ X, float2 *__restrict__ out, int MT,
-                                                            int KI, int n_x, int n_el)
+                                                            int KI, int n_x, int n_el, uint32_t *__restrict__ flag,
+                                                            uint32_t *__restrict__ bad)
 {
     __shared__ float2 t[32 * 66];  // one M-tile, element steps padded apart
-    const int b = blockIdx.y, mt = blockIdx.x;
+    __shared__ uint32_t m[16 * 4];
+    const int b = blockIdx.y, mt = blockIdx.x, KW = KI / 8;
     const float2 *src = X + ((size_t)b * MT + mt) * KI * 64;
-    for (int e = threadIdx.x; e < KI * 64; e += 256) t[(e >> 6) * 66 + (e & 63)] = src[e];
-    __syncthreads();
+    if (threadIdx.x < 64) m[threadIdx.x] = 0u;
+    bool nf = false;
+    for (int e = threadIdx.x; e < KI * 64; e += 256) {
+        const float2 v = src[e];
+        t[(e >> 6) * 66 + (e & 63)] = v;
+        nf |= !(fabsf(v.x) < INFINITY && fabsf(v.y) < INFINITY);
+    }
+    const bool any = __syncthreads_or(nf);
     const int rows = min(16, n_x - 16 * mt);
+    if (threadIdx.x == 0) flag[(size_t)mt * gridDim.y + b] = any;
+    if (any) {
+        for (int e = threadIdx.x; e < KI * 64; e += 256) {
+            float2 &v = t[(e >> 6) * 66 + (e & 63)];
+            if (fabsf(v.x) < INFINITY && fabsf(v.y) < INFINITY) continue;
+            const int k = 4 * (e >> 6) + ((e & 63) >> 4);
+            atomicOr(&m[(e & 15) * KW + (k >> 5)], 1u << (k & 31));
+            v = make_float2(0.f, 0.f);
+        }
+        __syncthreads();
+        if (threadIdx.x < rows * KW) bad[((size_t)b * n_x + 16 * mt) * KW + threadIdx.x] = m[threadIdx.x];
+    }
     float2 *dst = out + ((size_t)b * n_x + 16 * mt) * n_el;
     for (int e = threadIdx.x; e < rows * n_el; e += 256) {
         const int r = e / n_el, k = e - r * n_el;
@@ -38,16 +60,19 @@ __global__ __launch_bounds__(256) void lines_spectra_kernel(const float2 *__rest
     }
 }
 
-hipError_t launch_lines_spectra(const float2 *X, float2 *out, int n_f, int MT, int KI, int n_x, int n_el, hipStream_t s)
+hipError_t launch_lines_spectra(const float2 *X, float2 *out, int n_f, int MT, int KI, int n_x, int n_el, uint32_t *flag,
+                                uint32_t *bad, hipStream_t s)
 {
-    hipLaunchKernelGGL(lines_spectra_kernel, dim3((unsigned)MT, (unsigned)n_f), dim3(256), 0, s, X, out, MT, KI, n_x, n_el);
+    hipLaunchKernelGGL(lines_spectra_kernel, dim3((unsigned)MT, (unsigned)n_f), dim3(256), 0, s, X, out, MT, KI, n_x, n_el,
+                       flag, bad);
     return hipGetLastError();
 }
 
 // Workgroup (depth tile of 64, bin chunk, column or column pair); its waves take blocks of
 // LN_BINS bins in turn and add up through LDS in a fixed order.
 template <int WCR, bool MIR>
-__global__ __launch_bounds__(256) void lines_kernel(BeamArgs A, const float2 *__restrict__ X)
+__global__ __launch_bounds__(256) void lines_kernel(BeamArgs A, const float2 *__restrict__ X,
+                                                    const uint32_t *__restrict__ flag, const uint32_t *__restrict__ bad, int KW)
 {
     extern __shared__ uint32_t qs[];  // receive phase words [n_el][64]
     __shared__ float red[4][4][64];
@@ -179,6 +204,24 @@ __global__ __launch_bounds__(256) void lines_kernel(BeamArgs A, const float2 *__
             }
         }
     }
+    // depths whose aperture holds an element that is not finite at a bin of this chunk (the bins'
+    // flags alone are read where every value is finite)
+    bool any = false;
+    for (int b = b_begin + (int)threadIdx.x; b < b_end; b += 256)
+        any |= flag[(size_t)(col >> 4) * A.n_f + b] || (MIR && flag[(size_t)(col2 >> 4) * A.n_f + b]);
+    if (__syncthreads_or(any)) {
+        for (int b = b_begin; b < b_end; ++b) {
+            const bool f1 = flag[(size_t)(col >> 4) * A.n_f + b], f2 = MIR && flag[(size_t)(col2 >> 4) * A.n_f + b];
+            if (!f1 && !f2) continue;
+            double Fr = A.Frx[b];
+            if (A.clamp) Fr = fmin(Fr, A.sqrt_f[b] * clamp_z);
+            const Aperture ap = make_aperture(x, xp, zp, Fr, A, A.support_rx);
+            if (!ap.valid) continue;
+            if (f1 && mask_meets(bad + ((size_t)b * A.n_x + col) * KW, KW, ap.klo, ap.khi)) Ir = Ii = __builtin_nanf("");
+            if (f2 && mask_meets(bad + ((size_t)b * A.n_x + col2) * KW, KW, A.n_el - 1 - ap.khi, A.n_el - 1 - ap.klo))
+                Ir2 = Ii2 = __builtin_nanf("");
+        }
+    }
     red[wave][0][lane] = Ir;
     red[wave][1][lane] = Ii;
     red[wave][2][lane] = Ir2;
@@ -200,24 +243,26 @@ __global__ __launch_bounds__(256) void lines_kernel(BeamArgs A, const float2 *__
 }
 
 template <bool MIR>
-static void launch(int wcr, dim3 grid, const BeamArgs &A, const float2 *X, hipStream_t s)
+static void launch(int wcr, dim3 grid, const BeamArgs &A, const float2 *X, const uint32_t *flag, const uint32_t *bad, int KW,
+                   hipStream_t s)
 {
     const size_t lds = (size_t)A.n_el * 64 * sizeof(uint32_t);  // 32 KiB at most
     switch (wcr) {
-    case WC_RANGE: hipLaunchKernelGGL((lines_kernel<WC_RANGE, MIR>), grid, dim3(256), lds, s, A, X); break;
-    case WC_LINEAR: hipLaunchKernelGGL((lines_kernel<WC_LINEAR, MIR>), grid, dim3(256), lds, s, A, X); break;
-    case WC_COS_ALL: hipLaunchKernelGGL((lines_kernel<WC_COS_ALL, MIR>), grid, dim3(256), lds, s, A, X); break;
-    case WC_COS_RF: hipLaunchKernelGGL((lines_kernel<WC_COS_RF, MIR>), grid, dim3(256), lds, s, A, X); break;
-    default: hipLaunchKernelGGL((lines_kernel<WC_COS, MIR>), grid, dim3(256), lds, s, A, X); break;
+    case WC_RANGE: hipLaunchKernelGGL((lines_kernel<WC_RANGE, MIR>), grid, dim3(256), lds, s, A, X, flag, bad, KW); break;
+    case WC_LINEAR: hipLaunchKernelGGL((lines_kernel<WC_LINEAR, MIR>), grid, dim3(256), lds, s, A, X, flag, bad, KW); break;
+    case WC_COS_ALL: hipLaunchKernelGGL((lines_kernel<WC_COS_ALL, MIR>), grid, dim3(256), lds, s, A, X, flag, bad, KW); break;
+    case WC_COS_RF: hipLaunchKernelGGL((lines_kernel<WC_COS_RF, MIR>), grid, dim3(256), lds, s, A, X, flag, bad, KW); break;
+    default: hipLaunchKernelGGL((lines_kernel<WC_COS, MIR>), grid, dim3(256), lds, s, A, X, flag, bad, KW); break;
     }
 }
 
 // grid: (depth tiles of 64, bin chunks, columns, or pairs of mirrored columns)
-hipError_t launch_lines(int wcr, bool mirror, int tiles, int splits, const BeamArgs &A, const float2 *X, hipStream_t s)
+hipError_t launch_lines(int wcr, bool mirror, int tiles, int splits, const BeamArgs &A, const float2 *X, const uint32_t *flag,
+                        const uint32_t *bad, int KW, hipStream_t s)
 {
     const dim3 grid((unsigned)tiles, (unsigned)splits, (unsigned)(mirror ? (A.n_x + 1) / 2 : A.n_x));
-    if (mirror) launch<true>(wcr, grid, A, X, s);
-    else launch<false>(wcr, grid, A, X, s);
+    if (mirror) launch<true>(wcr, grid, A, X, flag, bad, KW, s);
+    else launch<false>(wcr, grid, A, X, flag, bad, KW, s);
     return hipGetLastError();
 }
 

@@ -201,3 +201,39 @@ def test_frames_and_jobs_stay_apart(fa, oracle, precision, value):
     torch.cuda.synchronize()
     assert all(torch.isfinite(torch.view_as_real(o)).all() for o in outs)
     batch.close()
+
+
+@pytest.mark.parametrize("shift", [0.0, 1e-3])
+@pytest.mark.parametrize("win,value", [("tukey", np.nan), ("boxcar", np.inf)])
+def test_line_scan(fa, oracle, shift, win, value):
+    """mirrored columns and columns that are not: only the bad transmit's own column, at the depths
+    whose aperture holds the element"""
+    import torch
+
+    x, rf, n_z = np.linspace(-9e-3, 9e-3, 19) + shift, _rf(19, 8), 150
+    z, chan = np.linspace(3e-3, 40e-3, n_z), (4, 30)
+    p = fa.LineScan(x, z, N_T, N_EL, FS, WIDTH, PITCH, C0, BAND, 15e-3, window=_window(fa, win),
+                    F_number=_F(fa, "angle_lb"), output_scale="cpu")
+    print(f"case lines shift {shift} {win} {value}", flush=True)
+    imgs = []
+    for v in (value, None):
+        r = rf.copy()
+        if v is None:
+            r[chan] = 0.0
+        else:
+            r[chan + (99,)] = v
+        img = torch.empty((19, n_z), dtype=torch.complex64, device="cuda")
+        p.execute(torch.from_numpy(r).cuda(), img)
+        torch.cuda.synchronize()
+        imgs.append(img)
+    met = np.zeros((19, n_z), dtype=bool)
+    cols = []
+    for seed in (1, 2):
+        r = rf[chan[0]:chan[0] + 1].copy()
+        r[0, chan[1]] = np.random.default_rng(seed).standard_normal(N_T)
+        col, _ = oracle.das_pw(x[chan[0]:chan[0] + 1], z, r, FS, np.zeros(1), WIDTH, PITCH, C0, BAND, 0.0,
+                               (win, 0.5 if win == "tukey" else 0.0), _oracle_F(oracle, "angle_lb"), "on",
+                               virtual_sources=[[x[chan[0]], 15e-3]])
+        cols.append(np.asarray(col).reshape(-1))
+    met[chan[0]] = cols[0] != cols[1]
+    _check(imgs[0], imgs[1], met, 1e-5)
