@@ -175,7 +175,8 @@ __global__ __launch_bounds__(256) void interp_beamform_kernel(InterpArgs S)
         const double dk = ((double)k - A.M) * A.pitch - x;
         const float d = (float)dk;
         float a = window_eval<WCR>(fabsf(d) * (d < 0.f ? ap.inv_wl : ap.inv_wr), A.wrx);
-        a = (k >= ap.klo && k <= ap.khi) ? a : 0.f;
+        const bool own = k >= ap.klo && k <= ap.khi;
+        a = own ? a : 0.f;
         asum += a;
         const double lat = dk / A.ctof;
         const uint32_t Qk = frac32(A.f_s * (sqrt(lat * lat + zc * zc) + A.delay[k]) / A.N);
@@ -194,8 +195,9 @@ __global__ __launch_bounds__(256) void interp_beamform_kernel(InterpArgs S)
         }
         const float rv = rev_of(S.n_c * Qk);
         const float er = a * __builtin_amdgcn_cosf(rv), ei = a * __builtin_amdgcn_sinf(rv);
-        Ir = fmaf(er, sr, fmaf(-ei, si, Ir));
-        Ii = fmaf(er, si, fmaf(ei, sr, Ii));
+        // (a channel whose samples are not finite stays with the voxels that hold its element)
+        Ir = own ? fmaf(er, sr, fmaf(-ei, si, Ir)) : Ir;
+        Ii = own ? fmaf(er, si, fmaf(ei, sr, Ii)) : Ii;
     }
     red[0][wave][lane] = Ir;
     red[1][wave][lane] = Ii;

@@ -237,3 +237,32 @@ def test_line_scan(fa, oracle, shift, win, value):
         cols.append(np.asarray(col).reshape(-1))
     met[chan[0]] = cols[0] != cols[1]
     _check(imgs[0], imgs[1], met, 1e-5)
+
+
+@pytest.mark.parametrize("win", ["tukey", "boxcar"])
+def test_one_f_number(fa, oracle, win):
+    """one F-number for every bin: the interpolated form"""
+    import torch
+
+    rf, chan, x, z = _rf(2, 10), (1, 20), np.linspace(-9e-3, 9e-3, 90), np.linspace(4e-3, 22e-3, 130)
+    plan = fa.PwPlan(x, z, N_T, N_EL, np.linspace(-0.2, 0.2, 2), FS, WIDTH, PITCH, C0, BAND, 0.0, window=_window(fa, win),
+                     F_number=_F(fa, "constant"), output_scale="cpu")
+    imgs = []
+    for v in (np.nan, None):
+        r = rf.copy()
+        if v is None:
+            r[chan] = 0.0
+        else:
+            r[chan + (99,)] = v
+        img = torch.empty((90, 130), dtype=torch.complex64, device="cuda")
+        plan.execute(torch.from_numpy(r).cuda(), img)
+        torch.cuda.synchronize()
+        imgs.append(img)
+    o = []
+    for seed in (1, 2):
+        r = rf.copy()
+        r[chan] = np.random.default_rng(seed).standard_normal(N_T)
+        img, _ = oracle.das_pw(x, z, r, FS, np.linspace(-0.2, 0.2, 2), WIDTH, PITCH, C0, BAND, 0.0,
+                               (win, 0.5 if win == "tukey" else 0.0), _oracle_F(oracle, "constant"), "on")
+        o.append(np.asarray(img).T)
+    _check(imgs[0], imgs[1], o[0] != o[1], 1e-5)
