@@ -273,32 +273,87 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(
         }
 }
 
-// Scale of the split contraction's cotangent operand per bin: a power of two that brings
-// max_v |s y(v) / w_n(v)| into [2^13, 2^14) (NaN left out), so that its fp16 halves neither
-// overflow nor lose a voxel 2^-25 below the largest; us[n_f + b] is the factor that takes it
-// and the window's (SPLIT_PEAK) out of the sums.  Bound by reading vsc once (4 bytes per bin
-// and voxel).
-__global__ __launch_bounds__(1024) void adjoint_uscale_kernel(const float *__restrict__ vsc,
-                                                              const float2 *__restrict__ y, long n_vox, int n_f,
-                                                              float inv_peak, float *__restrict__ us)
+// Units of the split contraction's cotangent operand: per bin and 64 consecutive voxels a power
+// of two that brings their max |s y / w| into [2^7, 2^15), kept from one block to the next where
+// it can be (each change costs the contraction 64 multiplications), or 0 where they are all
+// zero; and whether any of them is far below that (UNIT_FAR) or not finite (UNIT_BAD: left out
+// of the rest), which *rest then says.  A wave walks the blocks of one bin and voxel range.
+// Bound by reading vsc once (4 bytes per bin and voxel).
+constexpr uint32_t UNIT_FAR = 1u, UNIT_BAD = 2u;
+constexpr int UNIT_DEPTH = 16;   // exponents below the unit that keep 22 bits in two fp16 halves
+constexpr int UNIT_SPREAD = 64;  // the sums may be moved to a unit this far below the largest before it
+
+// x = f 2^e, f in [0.5, 1), of the bits of x >= 0 (a subnormal's e is taken as 2^-100's: the
+// factors below stay normal numbers)
+__device__ __forceinline__ int exponent_of(int bits) { return max((bits >> 23) - 126, -100); }
+
+__device__ __forceinline__ int wave_max(int v)
 {
-    __shared__ float red[16];
-    const int b = blockIdx.x;
-    float m = 0.f;
-    for (long v = threadIdx.x; v < n_vox; v += 1024) {
-        const float2 q = y[v];
-        m = fmaxf(m, fabsf(vsc[(size_t)b * n_vox + v]) * fmaxf(fabsf(q.x), fabsf(q.y)));
-    }
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; ++w) m = fmaxf(m, red[w]);
-        int e2 = 0;
-        if (m > 0.f) frexpf(m, &e2);  // m = f 2^e2, f in [0.5, 1)
-        const int k = min(max(14 - e2, -100), 100);
-        us[b] = ldexpf(1.0f, k);
-        us[n_f + b] = ldexpf(inv_peak, -k);
+    v = row_max16(v);
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+// 2^(14 - e), -100 <= e <= 128
+__device__ __forceinline__ float unit_factor(int e) { return __int_as_float((127 + 14 - e) << 23); }
+
+// a finite magnitude in its unit that keeps 22 bits there (NaN: no)
+__device__ __forceinline__ bool near_unit(float m)
+{
+    const uint32_t least = (uint32_t)(127 + 14 - UNIT_DEPTH - 1) << 23;
+    return __float_as_uint(m) - least < 0x7f800000u - least;
+}
+
+__device__ __forceinline__ bool finite2(float2 v) { return fabsf(v.x) < INFINITY && fabsf(v.y) < INFINITY; }
+
+constexpr int UNIT_BINS = 4;  // bins a wave walks together (y read once)
+__global__ __launch_bounds__(64) void adjoint_units_kernel(const float *__restrict__ vsc, const float2 *__restrict__ y,
+                                                           long n_vox, int n_f, long vox_per_range, int n_blocks,
+                                                           float *__restrict__ units, uint32_t *__restrict__ flags,
+                                                           uint32_t *__restrict__ rest)
+{
+    const int lane = threadIdx.x, b0 = blockIdx.x * UNIT_BINS;
+    const long v0 = (long)blockIdx.y * vox_per_range, v1 = min(v0 + vox_per_range, n_vox);
+    int e_use[UNIT_BINS];
+#pragma unroll
+    for (int i = 0; i < UNIT_BINS; ++i) e_use[i] = -1000;
+    float sc[UNIT_BINS];
+    float2 q;
+    auto load = [&](long base) {
+        const long u = min(base + lane, n_vox - 1);
+        q = y[u];
+#pragma unroll
+        for (int i = 0; i < UNIT_BINS; ++i) sc[i] = vsc[(size_t)min(b0 + i, n_f - 1) * n_vox + u];
+    };
+    load(v0);
+    for (long at = v0; at < v1; at += 64) {
+        float2 v[UNIT_BINS];
+#pragma unroll
+        for (int i = 0; i < UNIT_BINS; ++i) v[i] = at + lane < v1 ? make_float2(sc[i] * q.x, sc[i] * q.y) : make_float2(0.f, 0.f);
+        load(at + 64);  // the next block, while this one is looked at
+#pragma unroll
+        for (int i = 0; i < UNIT_BINS; ++i) {
+            const bool ok = finite2(v[i]);
+            const int bits = ok ? __float_as_int(fmaxf(fabsf(v[i].x), fabsf(v[i].y))) : 0;  // (floats >= 0 in integer order)
+            const int hi = wave_max(bits), lo = -wave_max(bits ? -bits : -0x7f800000);
+            uint32_t w = __ballot(!ok) ? UNIT_BAD : 0u;
+            float us = 0.f;
+            if (hi) {
+                const int e = exponent_of(hi);
+                const float least = __int_as_float(lo);
+                if (e > e_use[i] + 1 || e < e_use[i] - 6 ||
+                    (!near_unit(least * unit_factor(e_use[i])) && near_unit(least * unit_factor(e))))
+                    e_use[i] = e;
+                us = unit_factor(e_use[i]);
+                w |= near_unit(least * us) ? 0u : UNIT_FAR;
+            }
+            if (lane == 0 && b0 + i < n_f) {
+                const size_t o = (size_t)(b0 + i) * n_blocks + (at >> 6);
+                units[o] = us;
+                flags[o] = w;
+                if (w) atomicOr(rest, 1u);
+            }
+        }
     }
 }
 
@@ -308,8 +363,16 @@ __global__ __launch_bounds__(1024) void adjoint_uscale_kernel(const float *__res
 // kernel above; a group of 32 voxels is one MFMA K, lane group q holding its voxels 4 s + q.
 // Per element tile and 32 voxels: 12 matrix-core instructions of 16 cycles against 24 of 32,
 // beside 8 weights a lane; bound by the vector work of the weights.
-template <int WCR, bool FULL>
-__global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void adjoint_split_kernel(AdjArgs S)
+// The cotangent operand is in the unit of its 64 voxels (adjoint_units_kernel); the FP32 sums
+// move to the next block's unit by 64 multiplications where it differs (neighbouring depths
+// seldom need it), so elements that meet no loud voxel keep their bits.
+// REST: what that leaves, added to its partials.  Voxels far below their unit, band by band in
+// units of their own; blocks 2^64 below an earlier one, which the sums' exponents have no room
+// for; and NaN for the elements of a voxel that is not finite.  A launch without such a
+// block ends at once (*rest, which the reduction of the partials clears again).
+template <int WCR, bool FULL, bool REST>
+__global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(REST ? 1 : 2))) void
+adjoint_split_kernel(AdjArgs S)
 {
     static_assert(ADJ_GV == 32, "a group is one MFMA K");
     __shared__ __align__(16) uint32_t q_rx[2][ADJ_GV * ADJ_QS];  // [voxel i][mt][cidx]: element cidx + 16 mt
@@ -325,8 +388,11 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(
     const int b = blockIdx.x * ADJ_WAVES + wave;
     const bool active = b < A.n_f;
     const int at = blockIdx.z;
-    const long vr0 = (long)blockIdx.y * S.vox_per_range;
-    const long vr1 = min(vr0 + S.vox_per_range, n_vox);
+    long vr0 = (long)blockIdx.y * S.vox_per_range;
+    long vr1 = min(vr0 + S.vox_per_range, n_vox);
+    const int n_blocks = (int)((n_vox + 63) >> 6);
+    // (the factors' bits: biased exponents, 0 where there is none)
+    const uint32_t *const units = reinterpret_cast<const uint32_t *>(S.units) + (size_t)(active ? b : 0) * n_blocks;
     const float c16 = (float)cidx * 0.0625f;  // element cidx in units of 16 elements
     const uint32_t n = (uint32_t)(A.n_lb + (active ? b : 0));
     const double Fb = active ? A.Frx[b] : 0.0, sqf = active ? A.sqrt_f[b] : 0.0;
@@ -341,9 +407,10 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(
         uint4 rx[RX4];
         uint32_t tx[TX1];
         float2 ys;
+        float us;
     };
     const int bs = blockIdx.x * ADJ_WAVES + tid / ADJ_GV;  // (threads below ADJ_WAVES x ADJ_GV)
-    const float us_own = tid < ADJ_WAVES * ADJ_GV && bs < A.n_f ? S.us[bs] : 0.f;
+    const uint32_t us_row = (uint32_t)bs * (uint32_t)n_blocks;  // (n_f n_vox / 64 words: vsc holds n_f n_vox floats)
     auto fetch_group = [&](long base) {
         GroupRegs r;
 #pragma unroll
@@ -360,12 +427,14 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(
             r.tx[h] = uv < n_vox ? S.qtx[(size_t)uv * qtx_stride + 16 * at + col] : 0u;
         }
         r.ys = make_float2(0.f, 0.f);
+        r.us = 0.f;
         if (tid < ADJ_WAVES * ADJ_GV) {
             const long u3 = base + tid % ADJ_GV;
             if (bs < A.n_f && u3 < vr1) {
-                const float sc = S.vsc[(size_t)bs * n_vox + u3] * us_own;
+                const float sc = S.vsc[(size_t)bs * n_vox + u3];
                 const float2 y = S.y[u3];
                 r.ys = make_float2(sc * y.x, sc * y.y);
+                if (!REST) r.us = S.units[us_row + (uint32_t)(base >> 6)];
             }
         }
         return r;
@@ -378,7 +447,14 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(
         }
 #pragma unroll
         for (int h = 0; h < TX1; ++h) q_tx[buf][tid + 256 * h] = r.tx[h];
-        if (tid < ADJ_WAVES * ADJ_GV) ys[buf][tid / ADJ_GV][tid % ADJ_GV] = r.ys;
+        if (tid < ADJ_WAVES * ADJ_GV) {
+            float2 v = r.ys;
+            if (!REST) {
+                v = make_float2(v.x * r.us, v.y * r.us);
+                if (!near_unit(fabsf(v.x) + fabsf(v.y))) v = make_float2(0.f, 0.f);  // left to REST, or zero
+            }
+            ys[buf][tid / ADJ_GV][tid % ADJ_GV] = v;
+        }
     };
     // per-voxel aperture terms of voxel `base + lane` (clamped into the grid)
     auto load_geo = [&](long base) {
@@ -387,6 +463,183 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(
     };
     const bool a_ok = 16 * at + cidx < A.n_tx;
     const double x0 = -A.M * A.pitch;
+    // apertures of this wave's bin for the 64 voxels of `geo`, one per lane (forward formulas)
+    auto apertures = [&](const double4 geo) __attribute__((always_inline)) {
+        double Fr = Fb;
+        if (A.clamp) Fr = fmin(Fr, sqf * geo.w);  // das_pw.m:374-377
+        const Aperture ap = make_aperture(geo.x, geo.y, geo.z, Fr, A, A.support_rx);
+        // d = x_e - x = (x_0 - x) + e pitch; right side d / W_R, left side -d / W_L, times
+        // the window's argument scale, plus its offset
+        const double sl = WCR == WC_COS_RF ? (double)A.wrx.q_s : WCR == WC_COS_ALL ? (double)A.wrx.s_half : 1.0;
+        const double qo = WCR == WC_COS_RF ? (double)A.wrx.q_o : 0.0;
+        const double wr = (double)ap.inv_wr * sl, wl = (double)ap.inv_wl * sl, dx = x0 - geo.x;
+        akk[wave][lane] = (uint32_t)ap.klo | ((uint32_t)ap.khi << 16);
+        apx[wave][lane] = make_uint4(__float_as_uint((float)(16.0 * A.pitch * wr)),
+                                     __float_as_uint((float)(-16.0 * A.pitch * wl)),
+                                     __float_as_uint((float)(dx * wr + qo)), __float_as_uint((float)(qo - dx * wl)));
+    };
+    // the group of 32 voxels in buffer `cur`, half gh of apx
+    auto contract = [&](const int cur, const int gh) __attribute__((always_inline)) {
+        // element tiles [t_lo, t_hi] of 16 that meet the support of some voxel of the
+        // group (wave-uniform): every other tile has zero window for all 32 voxels
+        int t_lo, t_hi;
+        {
+            const uint32_t kk = akk[wave][32 * gh + (lane & 31)];
+            const int kl = (int)(kk & 0xffffu), kh = (int)(kk >> 16);
+            const int lo = row_min16(kl <= kh ? kl : 0x7fff), hi = row_max16(kl <= kh ? kh : -1);
+            t_lo = min(__builtin_amdgcn_readlane(lo, 0), __builtin_amdgcn_readlane(lo, 16)) >> 4;
+            t_hi = max(__builtin_amdgcn_readlane(hi, 0), __builtin_amdgcn_readlane(hi, 16)) >> 4;  // -1: none
+        }
+        // per voxel step s (voxel 4 s + q): the window argument as max(mt R1 + R0, mt L1 + L0)
+        // over the element tile mt, and the cotangent operand U = s y conj(T) / w
+        float R0[8], R1[8], L0[8], L1[8];
+        uint32_t kk[8];
+        u32x4 urh, url, uih, uil;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            float ur[2], ui[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int sv = 2 * p + h, i = 4 * sv + q;
+                const uint4 apv = apx[wave][32 * gh + i];  // written by this wave (LDS operations of a wave are ordered)
+                if (!FULL) kk[sv] = akk[wave][32 * gh + i];
+                R1[sv] = __uint_as_float(apv.x);
+                L1[sv] = __uint_as_float(apv.y);
+                R0[sv] = fmaf(c16, R1[sv], __uint_as_float(apv.z));  // element cidx of tile 0
+                L0[sv] = fmaf(c16, L1[sv], __uint_as_float(apv.w));
+                const float2 yv = a_ok ? ys[cur][wave][i] : make_float2(0.f, 0.f);
+                const float rt = rev_of(n * q_tx[cur][i * 16 + cidx]);
+                const float st = __builtin_amdgcn_sinf(rt), ct = __builtin_amdgcn_cosf(rt);
+                ur[h] = fmaf(yv.x, ct, yv.y * st);
+                ui[h] = fmaf(yv.y, ct, -(yv.x * st));
+            }
+            uint32_t hi, lo;
+            pack2<PREC_FP16X3>(ur[0], 1.f, ur[1], 1.f, hi, lo);
+            urh[p] = hi;
+            url[p] = lo;
+            pack2<PREC_FP16X3>(ui[0], 1.f, ui[1], 1.f, hi, lo);
+            uih[p] = hi;
+            uil[p] = lo;
+        }
+        const u32x4 nurh = neg16(urh), nurl = neg16(url);
+#pragma unroll
+        for (int mt = 0; mt < ADJ_ET; ++mt) {
+            if (mt < t_lo || mt > t_hi) continue;
+            const int e = cidx + 16 * mt;
+            u32x4 brh, brl, bih, bil;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                float w[2], sn[2], cs[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int sv = 2 * p + h;
+                    const uint32_t Qv = q_rx[cur][(4 * sv + q) * ADJ_QS + cidx + 16 * mt];
+                    const float ta = mt == 0 ? R0[sv] : fmaf((float)mt, R1[sv], R0[sv]);
+                    const float tb = mt == 0 ? L0[sv] : fmaf((float)mt, L1[sv], L0[sv]);
+                    // max(ta, tb) as an integer max of the bit patterns (one of the two is >= 0,
+                    // where the integer order is the float order; fmaxf would canonicalize both)
+                    const float tm = __int_as_float(max(__float_as_int(ta), __float_as_int(tb)));
+                    if (WCR == WC_COS_RF) {
+                        const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(tm, 0.f, 0.25f));
+                        w[h] = SPLIT_PEAK * c * c;
+                    } else if (WCR == WC_COS_ALL) {
+                        w[h] = fmaf(A.wrx.B, __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(tm)), A.wrx.A);
+                    } else {
+                        w[h] = window_eval<WCR>(tm, A.wrx);
+                    }
+                    if (!FULL) w[h] = (e >= (int)(kk[sv] & 0xffffu) && e <= (int)(kk[sv] >> 16)) ? w[h] : 0.f;
+                    const float rv = rev_of(n * Qv);
+                    sn[h] = __builtin_amdgcn_sinf(rv);
+                    cs[h] = __builtin_amdgcn_cosf(rv);
+                }
+                uint32_t hi, lo;
+                pack2<PREC_FP16X3>(w[0], cs[0], w[1], cs[1], hi, lo);
+                brh[p] = hi;
+                brl[p] = lo;
+                pack2<PREC_FP16X3>(w[0], sn[0], w[1], sn[1], hi, lo);
+                bih[p] = hi;
+                bil[p] = lo;
+            }
+            ZR[mt] = mfma16<PREC_FP16X3>(brh, urh, ZR[mt]);
+            ZI[mt] = mfma16<PREC_FP16X3>(brh, uih, ZI[mt]);
+            ZR[mt] = mfma16<PREC_FP16X3>(bih, uih, ZR[mt]);
+            ZI[mt] = mfma16<PREC_FP16X3>(bih, nurh, ZI[mt]);
+            ZR[mt] = mfma16<PREC_FP16X3>(brh, url, ZR[mt]);
+            ZI[mt] = mfma16<PREC_FP16X3>(brh, uil, ZI[mt]);
+            ZR[mt] = mfma16<PREC_FP16X3>(bih, uil, ZR[mt]);
+            ZI[mt] = mfma16<PREC_FP16X3>(bih, nurl, ZI[mt]);
+            ZR[mt] = mfma16<PREC_FP16X3>(brl, urh, ZR[mt]);
+            ZI[mt] = mfma16<PREC_FP16X3>(brl, uih, ZI[mt]);
+            ZR[mt] = mfma16<PREC_FP16X3>(bil, uih, ZR[mt]);
+            ZI[mt] = mfma16<PREC_FP16X3>(bil, nurh, ZI[mt]);
+        }
+    };
+    const int per_bin = 2 * ADJ_ET * 256;
+    // lane holds D[4q + r][cidx] = Z(element 16 mt + 4q + r, angle column cidx) of the range
+    auto partial = [&](int range) { return S.P + (((size_t)range * A.n_f + b) * S.n_at + at) * per_bin; };
+    if constexpr (REST) {
+        if (!*S.rest) return;
+        for (int range = blockIdx.y; range < S.n_vr; range += gridDim.y) {
+            vr0 = (long)range * S.vox_per_range;
+            vr1 = min(vr0 + S.vox_per_range, n_vox);
+            const int k0 = (int)(vr0 >> 6), k1 = (int)((vr1 + 63) >> 6);
+            int e_min = 0x7fff;  // as the other form walks the units
+            for (int k = k0; k < k1; ++k) {
+                const int eu = active ? (int)(units[k] >> 23) : 0;
+                e_min = eu ? min(e_min, eu) : e_min;
+                const bool skipped = eu > e_min + UNIT_SPREAD;
+                const uint32_t w = active ? S.flags[(size_t)b * n_blocks + k] : 0u;
+                if (!__syncthreads_or(w != 0u || skipped)) continue;
+                for (int gh = 0; gh < 2; ++gh) {
+                    const long base = 64L * k + 32 * gh;
+                    if (base >= vr1) break;
+                    __syncthreads();  // buffer 0 is free
+                    store_group(fetch_group(base), 0);
+                    __syncthreads();
+                    if (!active) continue;
+                    if (gh == 0) apertures(load_geo(base));
+                    float *const dst = partial(range);
+                    float2 v = make_float2(0.f, 0.f);  // what is left of voxel base + lane
+                    if (lane < ADJ_GV) v = ys[0][wave][lane];
+                    uint64_t nf = __ballot(!finite2(v));
+                    if (!finite2(v)) v = make_float2(0.f, 0.f);
+                    for (; nf; nf &= nf - 1) {
+                        const uint32_t k2 = akk[wave][32 * gh + __builtin_ctzll(nf)];
+                        for (int i = 0; i < 4 * ADJ_ET; ++i) {  // (the elements whose sums this lane holds)
+                            const int e = 16 * (i >> 2) + 4 * q + (i & 3), o = e * 16 + cidx;
+                            if (e >= (int)(k2 & 0xffffu) && e <= (int)(k2 >> 16))
+                                dst[o] = dst[ADJ_ET * 256 + o] = __builtin_nanf("");
+                        }
+                    }
+                    const float us0 = __uint_as_float((uint32_t)eu << 23);
+                    if (!skipped && near_unit(fabsf(v.x * us0) + fabsf(v.y * us0))) v = make_float2(0.f, 0.f);  // the other form's
+                    int bits = __float_as_int(fmaxf(fabsf(v.x), fabsf(v.y)));
+                    for (;;) {
+                        const int m = wave_max(bits);
+                        if (m == 0) break;
+                        const int e = exponent_of(m);
+                        const bool in = exponent_of(bits) >= e - UNIT_DEPTH;
+                        const float us = unit_factor(e);
+                        if (lane < ADJ_GV) ys[0][wave][lane] = in ? make_float2(v.x * us, v.y * us) : make_float2(0.f, 0.f);
+                        bits = in ? 0 : bits;
+#pragma unroll
+                        for (int mt = 0; mt < ADJ_ET; ++mt) ZR[mt] = ZI[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+                        contract(0, gh);
+                        const float inv = ldexpf(A.wrx.inv_peak, e - 14);
+#pragma unroll
+                        for (int mt = 0; mt < ADJ_ET; ++mt)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const int o = (16 * mt + 4 * q + r) * 16 + cidx;
+                                dst[o] += ZR[mt][r] * inv;
+                                dst[ADJ_ET * 256 + o] += ZI[mt][r] * inv;
+                            }
+                    }
+                }
+            }
+        }
+        return;
+    }
     double4 geo = make_double4(0.0, 0.0, 0.0, 0.0);
     if (vr0 < vr1) {
         store_group(fetch_group(vr0), 0);
@@ -394,131 +647,45 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) __attribute__((amdgpu_waves_per_eu(
     }
     __syncthreads();
     int cur = 0;
+    // biased exponents of the sums' factor and of the smallest so far (the largest unit); 0: none
+    int e_acc = 0, e_min = 0x7fff;
+    uint32_t w_next = vr0 < vr1 ? units[vr0 >> 6] : 0u;
+    bool skip = false;
     for (long base = vr0; base < vr1; base += ADJ_GV, cur ^= 1) {
         const bool more = base + ADJ_GV < vr1;
         GroupRegs next{};
         if (more) next = fetch_group(base + ADJ_GV);
         const int gh = (int)((base - vr0) >> 5) & 1;  // half of the 64 voxels of apx
+        if (gh == 0) {
+            const int eu = (int)(__builtin_amdgcn_readfirstlane(w_next) >> 23);
+            e_min = eu ? min(e_min, eu) : e_min;
+            skip = eu == 0 || eu > e_min + UNIT_SPREAD;
+            if (skip && eu && lane == 0) atomicOr(const_cast<uint32_t *>(S.rest), 1u);
+            if (!skip && eu != e_acc) {
+                const float f = ldexpf(1.0f, e_acc ? max(eu - e_acc, -126) : 0);
+#pragma unroll
+                for (int mt = 0; mt < ADJ_ET; ++mt) {
+                    ZR[mt] *= f;
+                    ZI[mt] *= f;
+                }
+                e_acc = eu;
+            }
+            if (base + 64 < vr1) w_next = units[(base + 64) >> 6];
+        }
         if (active) {
             if (gh == 0) {
-                // apertures of this wave's bin for voxels base .. base + 63, one per lane (forward formulas)
-                double Fr = Fb;
-                if (A.clamp) Fr = fmin(Fr, sqf * geo.w);  // das_pw.m:374-377
-                const Aperture ap = make_aperture(geo.x, geo.y, geo.z, Fr, A, A.support_rx);
-                // d = x_e - x = (x_0 - x) + e pitch; right side d / W_R, left side -d / W_L, times
-                // the window's argument scale, plus its offset
-                const double sl = WCR == WC_COS_RF ? (double)A.wrx.q_s : WCR == WC_COS_ALL ? (double)A.wrx.s_half : 1.0;
-                const double qo = WCR == WC_COS_RF ? (double)A.wrx.q_o : 0.0;
-                const double wr = (double)ap.inv_wr * sl, wl = (double)ap.inv_wl * sl, dx = x0 - geo.x;
-                akk[wave][lane] = (uint32_t)ap.klo | ((uint32_t)ap.khi << 16);
-                apx[wave][lane] = make_uint4(__float_as_uint((float)(16.0 * A.pitch * wr)),
-                                             __float_as_uint((float)(-16.0 * A.pitch * wl)),
-                                             __float_as_uint((float)(dx * wr + qo)), __float_as_uint((float)(qo - dx * wl)));
+                apertures(geo);
                 if (base + 64 < vr1) geo = load_geo(base + 64);  // consumed two groups later
             }
-            // element tiles [t_lo, t_hi] of 16 that meet the support of some voxel of the
-            // group (wave-uniform): every other tile has zero window for all 32 voxels
-            int t_lo, t_hi;
-            {
-                const uint32_t kk = akk[wave][32 * gh + (lane & 31)];
-                const int kl = (int)(kk & 0xffffu), kh = (int)(kk >> 16);
-                const int lo = row_min16(kl <= kh ? kl : 0x7fff), hi = row_max16(kl <= kh ? kh : -1);
-                t_lo = min(__builtin_amdgcn_readlane(lo, 0), __builtin_amdgcn_readlane(lo, 16)) >> 4;
-                t_hi = max(__builtin_amdgcn_readlane(hi, 0), __builtin_amdgcn_readlane(hi, 16)) >> 4;  // -1: none
-            }
-            // per voxel step s (voxel 4 s + q): the window argument as max(mt R1 + R0, mt L1 + L0)
-            // over the element tile mt, and the cotangent operand U = s y conj(T) / w
-            float R0[8], R1[8], L0[8], L1[8];
-            uint32_t kk[8];
-            u32x4 urh, url, uih, uil;
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                float ur[2], ui[2];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int sv = 2 * p + h, i = 4 * sv + q;
-                    const uint4 apv = apx[wave][32 * gh + i];  // written by this wave (LDS operations of a wave are ordered)
-                    if (!FULL) kk[sv] = akk[wave][32 * gh + i];
-                    R1[sv] = __uint_as_float(apv.x);
-                    L1[sv] = __uint_as_float(apv.y);
-                    R0[sv] = fmaf(c16, R1[sv], __uint_as_float(apv.z));  // element cidx of tile 0
-                    L0[sv] = fmaf(c16, L1[sv], __uint_as_float(apv.w));
-                    const float2 yv = a_ok ? ys[cur][wave][i] : make_float2(0.f, 0.f);
-                    const float rt = rev_of(n * q_tx[cur][i * 16 + cidx]);
-                    const float st = __builtin_amdgcn_sinf(rt), ct = __builtin_amdgcn_cosf(rt);
-                    ur[h] = fmaf(yv.x, ct, yv.y * st);
-                    ui[h] = fmaf(yv.y, ct, -(yv.x * st));
-                }
-                uint32_t hi, lo;
-                pack2<PREC_FP16X3>(ur[0], 1.f, ur[1], 1.f, hi, lo);
-                urh[p] = hi;
-                url[p] = lo;
-                pack2<PREC_FP16X3>(ui[0], 1.f, ui[1], 1.f, hi, lo);
-                uih[p] = hi;
-                uil[p] = lo;
-            }
-            const u32x4 nurh = neg16(urh), nurl = neg16(url);
-#pragma unroll
-            for (int mt = 0; mt < ADJ_ET; ++mt) {
-                if (mt < t_lo || mt > t_hi) continue;
-                const int e = cidx + 16 * mt;
-                u32x4 brh, brl, bih, bil;
-#pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    float w[2], sn[2], cs[2];
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const int sv = 2 * p + h;
-                        const uint32_t Qv = q_rx[cur][(4 * sv + q) * ADJ_QS + cidx + 16 * mt];
-                        const float ta = mt == 0 ? R0[sv] : fmaf((float)mt, R1[sv], R0[sv]);
-                        const float tb = mt == 0 ? L0[sv] : fmaf((float)mt, L1[sv], L0[sv]);
-                        // max(ta, tb) as an integer max of the bit patterns (one of the two is >= 0,
-                        // where the integer order is the float order; fmaxf would canonicalize both)
-                        const float tm = __int_as_float(max(__float_as_int(ta), __float_as_int(tb)));
-                        if (WCR == WC_COS_RF) {
-                            const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(tm, 0.f, 0.25f));
-                            w[h] = SPLIT_PEAK * c * c;
-                        } else if (WCR == WC_COS_ALL) {
-                            w[h] = fmaf(A.wrx.B, __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(tm)), A.wrx.A);
-                        } else {
-                            w[h] = window_eval<WCR>(tm, A.wrx);
-                        }
-                        if (!FULL) w[h] = (e >= (int)(kk[sv] & 0xffffu) && e <= (int)(kk[sv] >> 16)) ? w[h] : 0.f;
-                        const float rv = rev_of(n * Qv);
-                        sn[h] = __builtin_amdgcn_sinf(rv);
-                        cs[h] = __builtin_amdgcn_cosf(rv);
-                    }
-                    uint32_t hi, lo;
-                    pack2<PREC_FP16X3>(w[0], cs[0], w[1], cs[1], hi, lo);
-                    brh[p] = hi;
-                    brl[p] = lo;
-                    pack2<PREC_FP16X3>(w[0], sn[0], w[1], sn[1], hi, lo);
-                    bih[p] = hi;
-                    bil[p] = lo;
-                }
-                ZR[mt] = mfma16<PREC_FP16X3>(brh, urh, ZR[mt]);
-                ZI[mt] = mfma16<PREC_FP16X3>(brh, uih, ZI[mt]);
-                ZR[mt] = mfma16<PREC_FP16X3>(bih, uih, ZR[mt]);
-                ZI[mt] = mfma16<PREC_FP16X3>(bih, nurh, ZI[mt]);
-                ZR[mt] = mfma16<PREC_FP16X3>(brh, url, ZR[mt]);
-                ZI[mt] = mfma16<PREC_FP16X3>(brh, uil, ZI[mt]);
-                ZR[mt] = mfma16<PREC_FP16X3>(bih, uil, ZR[mt]);
-                ZI[mt] = mfma16<PREC_FP16X3>(bih, nurl, ZI[mt]);
-                ZR[mt] = mfma16<PREC_FP16X3>(brl, urh, ZR[mt]);
-                ZI[mt] = mfma16<PREC_FP16X3>(brl, uih, ZI[mt]);
-                ZR[mt] = mfma16<PREC_FP16X3>(bil, uih, ZR[mt]);
-                ZI[mt] = mfma16<PREC_FP16X3>(bil, nurh, ZI[mt]);
-            }
+            if (!skip) contract(cur, gh);
         }  // active
         // buffer cur ^ 1 was last read two groups ago (before the previous barrier)
         if (more) store_group(next, cur ^ 1);
         __syncthreads();  // group `base` consumed, group `base + ADJ_GV` stored
     }
     if (!active) return;
-    // lane holds D[4q + r][cidx] = Z(element 16 mt + 4q + r, angle column cidx) of the range
-    const int per_bin = 2 * ADJ_ET * 256;
-    const float inv = S.us[A.n_f + b];
-    float *dst = S.P + (((size_t)blockIdx.y * A.n_f + b) * S.n_at + at) * per_bin;
+    const float inv = e_acc ? ldexpf(A.wrx.inv_peak, 127 - e_acc) : 0.f;
+    float *dst = partial(blockIdx.y);
 #pragma unroll
     for (int mt = 0; mt < ADJ_ET; ++mt)
 #pragma unroll
@@ -570,8 +737,10 @@ __global__ __launch_bounds__(256) void adjoint_tables_kernel(BeamArgs A, uint32_
 // (null: none), with the rounding of the spectra planes that hold them in the forward kernels
 __global__ __launch_bounds__(256) void adjoint_reduce_kernel(const float *__restrict__ P, float2 *__restrict__ Z,
                                                              int n_vr, int n_f, int n_at, int n_tx, int n_el,
-                                                             const double *__restrict__ delay, double fs_over_N, int n_lb)
+                                                             const double *__restrict__ delay, double fs_over_N, int n_lb,
+                                                             uint32_t *__restrict__ rest)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *rest = 0u;  // for the next contraction
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     const long total = (long)n_f * n_at * 16 * ADJ_ET * 16;
     if (i >= total) return;
@@ -804,9 +973,14 @@ static void launch_adjoint_class(bool scale, bool split, dim3 grid, hipStream_t 
             return;
         }
     }
-    hipLaunchKernelGGL(adjoint_uscale_kernel, dim3((unsigned)B.n_f), dim3(1024), 0, s, S.vsc, S.y, n_vox, B.n_f,
-                       S.B.wrx.inv_peak, const_cast<float *>(S.us));
-    hipLaunchKernelGGL((adjoint_split_kernel<WCR, FULL>), grid, dim3(64 * ADJ_WAVES), 0, s, S);
+    const int n_blocks = (int)((n_vox + 63) / 64);
+    hipLaunchKernelGGL(adjoint_units_kernel, dim3((unsigned)((B.n_f + UNIT_BINS - 1) / UNIT_BINS), grid.y), dim3(64), 0, s, S.vsc, S.y,
+                       n_vox, B.n_f,
+                       S.vox_per_range, n_blocks, const_cast<float *>(S.units), const_cast<uint32_t *>(S.flags),
+                       const_cast<uint32_t *>(S.rest));
+    hipLaunchKernelGGL((adjoint_split_kernel<WCR, FULL, false>), grid, dim3(64 * ADJ_WAVES), 0, s, S);
+    hipLaunchKernelGGL((adjoint_split_kernel<WCR, FULL, true>), dim3(grid.x, std::min(grid.y, 8u), grid.z),
+                       dim3(64 * ADJ_WAVES), 0, s, S);
 }
 
 // The contraction runs on the fp16 split, but for the untruncated triangular window, whose
@@ -853,11 +1027,11 @@ hipError_t launch_adjoint(int wcr, bool tables, bool scale, dim3 grid, hipStream
 }
 
 hipError_t launch_adjoint_reduce(const float *P, float2 *Z, int n_vr, int n_f, int n_at, int n_tx, int n_el,
-                                 const double *delay, double fs_over_N, int n_lb, hipStream_t s)
+                                 const double *delay, double fs_over_N, int n_lb, uint32_t *rest, hipStream_t s)
 {
     const long total = (long)n_f * n_at * 16 * ADJ_ET * 16;
     hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, P, Z, n_vr, n_f,
-                       n_at, n_tx, n_el, delay, fs_over_N, n_lb);
+                       n_at, n_tx, n_el, delay, fs_over_N, n_lb, rest);
     return hipGetLastError();
 }
 

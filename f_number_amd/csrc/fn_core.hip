@@ -96,7 +96,7 @@ hipError_t launch_beamform_tan_k16_p2(int, int, bool, dim3, size_t, hipStream_t,
 hipError_t launch_beamform_tan_k32_p2(int, int, bool, dim3, size_t, hipStream_t, const BeamArgs &);
 hipError_t launch_adjoint(int wcr, bool tables, bool scale, dim3 grid, hipStream_t s, const AdjArgs &S);
 hipError_t launch_adjoint_reduce(const float *P, float2 *Z, int n_vr, int n_f, int n_at, int n_tx, int n_el,
-                                 const double *delay, double fs_over_N, int n_lb, hipStream_t s);
+                                 const double *delay, double fs_over_N, int n_lb, uint32_t *rest, hipStream_t s);
 hipError_t launch_adjoint_idft(const float2 *Z, const float2 *tw, float *out, int n_t, int n_ch, int N, int n_lb,
                                int n_f, hipStream_t s);
 hipError_t launch_lines(int wcr, bool mirror, int tiles, int splits, const BeamArgs &A, const float2 *X, const uint32_t *flag,
@@ -1466,8 +1466,11 @@ int contract_adjoint(fn_plan *P, const float *d_y, hipStream_t s)
         // phase words (128 + 16 n_at per voxel) followed by 4 doubles of aperture terms per voxel
         HIP_CHECK(hipMalloc(&P->d_qtab, (size_t)P->n_vox * (128 + 16 * P->adj_at + 8) * sizeof(uint32_t)),
                   "phase tables");
-        // s / w_n(v) per bin and voxel, then two scale factors per bin
-        HIP_CHECK(hipMalloc(&P->d_vsc, ((size_t)n_f * P->n_vox + 2 * n_f) * sizeof(float)), "adjoint normalization");
+        // s / w_n(v) per bin and voxel, then the cotangent's units and flags per bin and 64 voxels, and a flag for all
+        const size_t vsc_bytes = ((size_t)n_f * (P->n_vox + 2 * groups64) + 1) * sizeof(float);
+        HIP_CHECK(hipMalloc(&P->d_vsc, vsc_bytes), "adjoint normalization");
+        hipLaunchKernelGGL(fnk::fill_zero_kernel, dim3(1), dim3(256), 0, s, P->d_vsc + vsc_bytes / sizeof(float) - 1, 1L);
+        HIP_CHECK(hipGetLastError(), "fill_zero_kernel");
     }
     fnk::AdjArgs S{};
     S.B = P->args;
@@ -1482,7 +1485,10 @@ int contract_adjoint(fn_plan *P, const float *d_y, hipStream_t s)
     S.qtx = P->d_qtab + (size_t)P->n_vox * 128;
     S.vgeo = reinterpret_cast<const double *>(P->d_qtab + (size_t)P->n_vox * (128 + 16 * P->adj_at));
     S.vsc = P->d_vsc;
-    S.us = P->d_vsc + (size_t)n_f * P->n_vox;
+    S.units = P->d_vsc + (size_t)n_f * P->n_vox;
+    S.flags = reinterpret_cast<const uint32_t *>(S.units + (size_t)n_f * ((P->n_vox + 63) / 64));
+    S.rest = S.flags + (size_t)n_f * ((P->n_vox + 63) / 64);
+    S.n_vr = P->adj_vr;
     S.vox_per_range = P->adj_vpr;
     S.n_at = P->adj_at;
     // bin quads fastest: the workgroups dispatched together share a voxel range, whose
@@ -1504,7 +1510,7 @@ int contract_adjoint(fn_plan *P, const float *d_y, hipStream_t s)
     }
     if (e != hipSuccess) return hip_fail(e, "adjoint_kernel");
     e = fnk::launch_adjoint_reduce(P->d_P, P->d_Z, P->adj_vr, n_f, P->adj_at, P->n_tx, P->n_el, delay,
-                                   P->args.f_s / P->g.N, P->g.n_lb, s);
+                                   P->args.f_s / P->g.N, P->g.n_lb, const_cast<uint32_t *>(S.rest), s);
     if (e != hipSuccess) return hip_fail(e, "adjoint_reduce_kernel");
     return FN_OK;
 }

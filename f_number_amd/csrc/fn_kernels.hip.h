@@ -135,7 +135,10 @@ struct AdjArgs {
     const uint32_t *qtx;    // transmit phase words [n_vox][16 n_at]
     const double *vgeo;     // per voxel: x, x / pitch, z / (2 pitch), sqrt(z / (2.88 c0))
     const float *vsc;       // per bin and voxel [n_f][n_vox]: s / w_n(v), 0 outside a valid aperture
-    const float *us;        // split contraction: per bin the cotangent's scale, then what takes it out
+    const float *units;     // split contraction: the cotangent's unit per bin and 64 voxels [n_f][ceil(n_vox / 64)]
+    const uint32_t *flags;  // and its exceptions (adjoint_units_kernel)
+    const uint32_t *rest;   // split contraction: is anything left for its second launch
+    int n_vr;               // voxel ranges
     long vox_per_range;     // multiple of 64
     int n_at;               // angle tiles of 16
 };
