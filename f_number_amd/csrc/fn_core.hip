@@ -124,6 +124,19 @@ static const BeamLauncher kBeamLaunchers[2][5][4] = {
     {FN_BEAM_ROW(0, 8), FN_BEAM_ROW(0, 16), FN_BEAM_ROW(0, 32), FN_BEAM_ROW(0, 48), FN_BEAM_ROW(0, 64)},
     {FN_BEAM_ROW(1, 8), FN_BEAM_ROW(1, 16), FN_BEAM_ROW(1, 32), FN_BEAM_ROW(1, 48), FN_BEAM_ROW(1, 64)}};
 #undef FN_BEAM_ROW
+// One thread per voxel of the left half and chunk of bins; bound by a division and eight roundings
+// in FP64 per voxel and bin (128 x 96, 240 bins: 7 us).
+constexpr int MIRROR_BINS = 8;
+__global__ __launch_bounds__(256) void mirror_check_kernel(MirrorArgs m)
+{
+    const long v = (long)blockIdx.x * 256 + threadIdx.x;
+    if (v >= (long)(m.n_x / 2) * m.n_z) return;
+    const int b0 = blockIdx.y * MIRROR_BINS, b1 = min(b0 + MIRROR_BINS, m.n_f);
+    bool off = false;
+    for (int b = b0; b < b1; ++b) off |= mirror_off(m, v, b);
+    if (off) *m.tie = 1u;
+}
+
 // image (and weights, where given) of n_z depths per column into the first depths of columns of NZ
 __global__ void paste_depths_kernel(const float2 *img, const float *w, long n, int n_z, int NZ, float2 *out, float *w_out)
 {
@@ -176,6 +189,8 @@ struct fn_plan {
     int kprec = FN_PRECISION_FP32;      // form of the forward contraction (kernel_precision)
     int mirror = 0;         // lateral positions symmetric: planes hold the reversed elements too
     int line_mirror = 0;    // line scan on symmetric lateral positions: two columns share their weights
+    uint32_t *d_tie = nullptr;  // plans that may mirror: the check's answer (mirror_off)
+    int tie_later = 0;          // a one-shot call's plan: its own kernels look (Mirror::later)
     int delays_even = 1;    // delay offsets symmetric about the array's centre
     int interp_M = 0;       // > 0: the forward image by interpolation of M samples per channel
     float2 *d_Xrow = nullptr;  // line scan: the spectra by rows [n_f][line][element]
@@ -541,9 +556,9 @@ static bool few_rows_pw(const fn_plan *P)
     return P->mode == 0 && P->n_frames == 1 && !P->lbl && P->MT_tmpl <= 2;
 }
 
-// lateral positions symmetric about the array to 1e-12 pitches.  Not the boxcar window at one
-// F-number for every bin: its membership test has no taper, and its ties (a support edge on an
-// element for a whole band) would be broken by rounding.
+// lateral positions symmetric about the array to 1e-12 pitches (create_common then looks at
+// every aperture: mirror_check_kernel).  Not the boxcar window at one F-number for every bin, whose
+// images of some size are interpolated; what is left of them is small.
 bool mirrored_positions(const fn_plan *P, const Common &c, const double *Frx, int n_f)
 {
     if (!Frx || c.n_x < 2) return false;
@@ -567,6 +582,12 @@ bool mirror_plan(const fn_plan *P, const Common &c, const double *Frx, int n_f)
     if (P->KI > 48 || P->MT_all > (P->KI <= 32 ? 2 : 1)) return false;
     return mirrored_positions(P, c, Frx, n_f);
 }
+
+// Plans that may mirror: look at the apertures on the device and wait for the answer; leave the
+// look to the planes kernel of a one-shot call, which finds the answer in its image and runs
+// again in the rare case (one more launch or copy there is 20 to 70 us of 750); or one voxel a
+// lane.
+enum class Mirror { check, later, no };
 
 // shared configuration of plan creation: tiling, launch shape and the scalar
 // arguments of the kernels; no device work and no allocation (the
@@ -614,7 +635,7 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
         P->n_groups = (P->MT_all + P->MT_tmpl - 1) / P->MT_tmpl;
     }
     P->mirror = mirror && mirror_plan(P, c, Frx, g.n_f);
-    P->line_mirror = P->lbl && mirrored_positions(P, c, Frx, g.n_f);
+    P->line_mirror = mirror && P->lbl && mirrored_positions(P, c, Frx, g.n_f);
     const size_t step_bytes = form_step_bytes(P->kprec);
     P->lds_beam = (size_t)P->MT_tmpl * P->KI * step_bytes;
     P->lds_spec = (size_t)g.N * sizeof(float2) + 64 * 65 * sizeof(float);
@@ -680,12 +701,18 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
     return FN_OK;
 }
 
+fnk::MirrorArgs mirror_args(const fn_plan *P)
+{
+    const fnk::BeamArgs &A = P->args;
+    return {P->d_tie, A.px, A.pz, A.Frx, A.sqrt_f, A.M, A.pitch, A.c0, A.n_x, A.n_z, A.n_el, A.n_f, A.clamp};
+}
+
 // shared part of plan creation, after configure_common: the device tables and workspace.
 // One allocation and one copy: the tables (positions, F-numbers, sqrt(f_n), transmit rows
 // txp, twiddles, zero delay offsets) are laid out on the host first.  Every slot of the
 // spectra and their planes is written by each execute, padding as zeros.
 int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, const double *Ftx,
-                  const std::vector<double> &txp, const fn_plan *spectra_of = nullptr)
+                  const std::vector<double> &txp, const fn_plan *spectra_of = nullptr, Mirror how = Mirror::check)
 {
     int s;
     if ((s = select_device(c.index_gpu))) return s;
@@ -714,6 +741,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t o_sqf = cv.take(g.n_f * sizeof(double)), o_txp = cv.take(txp.size() * sizeof(double));
     const size_t o_tw = cv.take(tw.size() * sizeof(float2)), o_dl = cv.take(c.n_el * sizeof(double));
     const size_t o_zr = cv.take(c.n_el * sizeof(double));
+    const size_t o_tie = cv.take(sizeof(uint32_t));
     const size_t tables = cv.used;
     const size_t o_X = cv.take(spectra_of ? 0 : P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
     const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
@@ -760,6 +788,21 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     A.bad = P->d_bad;
     A.row_scale = P->d_rowscale;
     A.px = P->d_px; A.pz = P->d_pz; A.Frx = P->d_Frx; A.Ftx = P->d_Ftx; A.txp = P->d_txp; A.sqrt_f = P->d_sqf;
+    if (P->mirror || P->line_mirror) {
+        P->d_tie = reinterpret_cast<uint32_t *>(P->d_block + o_tie);
+        P->tie_later = how == Mirror::later && !P->lbl;  // (line scans have no planes)
+        if (!P->tie_later) {
+            uint32_t tie = 0;
+            const dim3 grid((unsigned)(((long)(c.n_x / 2) * c.n_z + 255) / 256),
+                            (unsigned)((g.n_f + fnk::MIRROR_BINS - 1) / fnk::MIRROR_BINS));
+            hipLaunchKernelGGL(fnk::mirror_check_kernel, grid, dim3(256), 0, P->stream, mirror_args(P));
+            HIP_CHECK(hipGetLastError(), "mirror_check_kernel");
+            HIP_CHECK(hipMemcpyAsync(&tie, P->d_tie, sizeof(tie), hipMemcpyDeviceToHost, P->stream), "mirror_check_kernel");
+            HIP_CHECK(hipStreamSynchronize(P->stream), "mirror_check_kernel");
+            // one voxel a lane: the planes of either tiling fit the mirrored ones' room
+            if (tie && (s = configure_common(P, c, g, Frx, false, false))) return s;
+        }
+    }
     return ensure_partials(P);
 }
 
@@ -858,7 +901,7 @@ int interp_points(const fn_plan *P)
     return (int)M;
 }
 
-int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of = nullptr);
+int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of = nullptr, Mirror how = Mirror::check);
 
 // the interpolated form's buffers (and the plan of its clamped depths); a plan without room for
 // them, or whose clamped depths have another DFT, keeps the sum over the bins
@@ -981,6 +1024,7 @@ fnk::BeamArgs beam_args(const fn_plan *P, float *d_image, float *d_w, float *d_w
 {
     fnk::BeamArgs A = forward_args(P);
     if (P->interp_M || P->lbl) A.bad = nullptr;               // no planes
+    A.tie = P->tie_later && use_mirror(P) ? P->d_tie : nullptr;
     if (plane_delay(P, use_mirror(P))) A.delay = P->d_zeros;  // in the planes already
     A.image = reinterpret_cast<float2 *>(d_image);
     A.n_slots = beam_slots(P);
@@ -1015,6 +1059,7 @@ int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xsca
                        int MT_out, int mirror_el, const double *delay, hipStream_t s, float *rowscale = nullptr)
 {
     const float *row_inv = rowscale ? rowscale + 16 * MT : nullptr;
+    const fnk::MirrorArgs look = P->tie_later && use_mirror(P) ? mirror_args(P) : fnk::MirrorArgs{};
     if (rowscale)
         if (int st = launch_row_scales(X, rowscale, MT, P->KI, P->g.n_f, s)) return st;
     const dim3 cg((unsigned)P->g.n_f), cb(256);
@@ -1023,15 +1068,15 @@ int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xsca
     case FN_PRECISION_FP32: return FN_OK;
     case FN_PRECISION_BF16X3:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_BF16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI));
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI), look);
         break;
     case FN_PRECISION_FP16X3:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16X3>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI));
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI), look);
         break;
     default:
         hipLaunchKernelGGL(fnk::lowp_planes_kernel<fnk::PREC_FP16>, cg, cb, 0, s, X, Xlp, xscale, MT, P->KI, MT_out,
-                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI));
+                           mirror_el, delay, fs_over_N, P->g.n_lb, P->n_el, row_inv, bad, bad_rows, bad_words(P->KI), look);
         break;
     }
     HIP_CHECK(hipGetLastError(), "lowp_planes_kernel");
@@ -1177,7 +1222,7 @@ int configure_pw(fn_plan *P, const fn_pw_params *p, Common *c)
 }
 
 // spectra_of: a plan of the same acquisition whose spectra this one reads (its clamped depths)
-int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of)
+int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of, Mirror how)
 {
     fnh::Grid g;
     int s = fnh::validate_pw(p, &g);
@@ -1186,7 +1231,7 @@ int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of)
     if (!P) return fail(FN_ERR_OUT_OF_MEMORY, "host allocation");
     Common c{};
     if ((s = configure_pw(P, p, &c))) { destroy(P); return s; }
-    if ((s = configure_common(P, c, g, p->f_number_values))) { destroy(P); return s; }
+    if ((s = configure_common(P, c, g, p->f_number_values, false, how != Mirror::no))) { destroy(P); return s; }
     const int n_rows = P->args.n_tx;  // operand rows (ensembles: frame slots)
     // steering geometry in FP64: das_pw.m:323-327 (x_ref = sign(e_x) x_0), or the
     // virtual sources (x_vs, z_vs, |r_vs|)
@@ -1208,7 +1253,7 @@ int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of)
         txp[3 * row + 1] = ez;
         txp[3 * row + 2] = sg * ((0 - M) * p->element_pitch);
     }
-    if ((s = create_common(P, c, g, p->f_number_values, nullptr, txp, spectra_of))) { destroy(P); return s; }
+    if ((s = create_common(P, c, g, p->f_number_values, nullptr, txp, spectra_of, how))) { destroy(P); return s; }
     if (P->nw && (s = setup_windowed(P, true, p->window, p->normalization_window, false, p->window,
                                      p->normalization_window))) { destroy(P); return s; }
     use_cos_all(P);
@@ -1692,8 +1737,9 @@ void compose_report(const fn_plan *P, size_t rf_bytes, size_t img_bytes, size_t 
 }
 
 // one-shot: H2D, execute, D2H (gpu_bf_das_pw_rf.cu:730-1122); with verbosity >= 1
-// the stages are timed with HIP events and reported
-int one_shot(fn_plan *P, const void *rf, int dtype, float *image, float *w0, float *w1)
+// the stages are timed with HIP events and reported.  *unmirror: the image is not to be used, a
+// plan of Mirror::no is
+int one_shot(fn_plan *P, const void *rf, int dtype, float *image, float *w0, float *w1, bool *unmirror = nullptr)
 {
     const size_t rf_bytes = (size_t)P->n_t * P->n_el * P->n_tx * dtype_size(dtype);
     const size_t img_bytes = (size_t)P->n_vox * 2 * sizeof(float) * P->n_frames;
@@ -1735,6 +1781,7 @@ int one_shot(fn_plan *P, const void *rf, int dtype, float *image, float *w0, flo
     for (auto &x : ev)
         if (x) hipEventDestroy(x);
     hipFree(d_rf); hipFree(d_img); hipFree(d_w0); hipFree(d_w1);
+    if (unmirror) *unmirror = !s && std::memcmp(image, &fnk::TIE_MARK, sizeof(fnk::TIE_MARK)) == 0;
     return s;
 }
 
@@ -1857,10 +1904,11 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
     size_t o_X = 0, o_Xlp = 0, o_xs = 0, o_px = 0, o_pz = 0, o_F = 0, o_sqf = 0, o_raw = 0, o_txp = 0, o_tw = 0, o_dl = 0,
            o_pi = 0, o_bad = 0;
     int slots = 1;
-    // a call whose planes do not fit beside its spectra runs without the mirrored ones, an FP32
-    // call then without any, on the FP32 kernels
-    for (int lean = 0; lean < 3; ++lean) {
-        if ((st = configure_common(&P, c, g, p->f_number_values, lean == 2, lean == 0))) return st;
+    // one voxel a lane: whether the grid's apertures mirror is only known after a look at them on
+    // the device, which this call may not wait for.  An FP32 call whose planes do not fit beside
+    // its spectra runs on the FP32 kernels.
+    for (int lean = 0; lean < 2; ++lean) {
+        if ((st = configure_common(&P, c, g, p->f_number_values, lean == 1, false))) return st;
         cv = Carve{};
         o_X = cv.take(P.x_bytes);
         o_Xlp = cv.take(P.xlp_bytes);
@@ -2075,8 +2123,13 @@ int32_t fn_das_pw(const fn_pw_params *p, const void *data_rf, int32_t rf_dtype, 
     if (!image) return fail(FN_ERR_ARGUMENT, "image buffer missing");
     if (rf_dtype != FN_DTYPE_F32 && rf_dtype != FN_DTYPE_F64) return fail(FN_ERR_RF_DATA, "RF data must be float32 or float64");
     fn_plan *P = nullptr;
-    int s = pw_plan(p, &P);
+    int s = pw_plan(p, &P, nullptr, Mirror::later);
     if (s) return s;
+    bool unmirror = false;
+    s = one_shot(P, data_rf, rf_dtype, image, weights, nullptr, &unmirror);
+    destroy(P);
+    if (s || !unmirror) return s;
+    if ((s = pw_plan(p, &P, nullptr, Mirror::no))) return s;
     s = one_shot(P, data_rf, rf_dtype, image, weights, nullptr);
     destroy(P);
     return s;

@@ -85,6 +85,7 @@ struct BeamArgs {
     // (written and read at the bins of negative xscale alone; bad_rows 1: of any row)
     const uint32_t *bad;
     int bad_rows, bad_words;
+    const uint32_t *tie;    // one-shot calls: does the grid not mirror after all (mirror_off; null: settled)
     const float *row_scale; // ensembles, row stacks: per transmit row a scale beside it (null: none)
     const double *px, *pz;  // voxel positions
     const double *Frx;      // F-number per band bin (receive)
@@ -231,6 +232,32 @@ __device__ __forceinline__ Aperture make_aperture(double x, double xp, double zp
         }
     }
     return ap;
+}
+
+// Does a lateral grid mirror about the array: the aperture bounds of columns i and n_x - 1 - i
+// (make_aperture's roundings, each at its own position) are each other's mirror image.  Where a
+// bound falls on an element rounding decides, and not alike on both sides: *tie is then set.
+struct MirrorArgs {
+    uint32_t *tie;
+    const double *px, *pz, *Frx, *sqrt_f;
+    double M, pitch, c0;
+    int n_x, n_z, n_el, n_f, clamp;
+};
+
+// first value (both parts) of a one-shot image whose grid does not mirror: a NaN of its own
+constexpr uint32_t TIE_MARK = 0x7fc071e5u;
+
+__device__ __forceinline__ bool mirror_off(const MirrorArgs &m, long v, int b)
+{
+    const int ix = (int)(v / m.n_z), iz = (int)(v - (long)ix * m.n_z);
+    const double z = m.pz[iz], last = m.n_el - 1;
+    double F = m.Frx[b];
+    if (m.clamp) F = fmin(F, m.sqrt_f[b] * sqrt(z / (2.88 * m.c0)));
+    const double hp = z / (2.0 * m.pitch) / F, x1 = m.px[ix] / m.pitch, x2 = m.px[m.n_x - 1 - ix] / m.pitch;
+    const double ua = m.M + (x1 - hp), ub = m.M + (x1 + hp), va = m.M + (x2 - hp), vb = m.M + (x2 + hp);
+    return fmax(ceil(ua), 0.0) + fmin(floor(vb), last) != last || fmax(ceil(va), 0.0) + fmin(floor(ub), last) != last ||
+           fmax(floor(ua) + 1.0, 0.0) + fmin(ceil(vb) - 1.0, last) != last ||
+           fmax(floor(va) + 1.0, 0.0) + fmin(ceil(ub) - 1.0, last) != last;
 }
 
 // An aperture in three words, for moving it between lanes: klo | valid << 15 | khi << 16
@@ -1654,6 +1681,7 @@ static __global__ __launch_bounds__(256) void nonfinite_kernel(BeamArgs A)
         img[v] = nan2;
         if (A.dimage) reinterpret_cast<float2 *>(A.dimage)[v] = nan2;
     });
+    if (A.tie && v == 0 && *A.tie) A.image[0] = make_float2(__uint_as_float(TIE_MARK), __uint_as_float(TIE_MARK));
 }
 
 // sum of the partial images of every (bin chunk, transmit group) slot in slot
@@ -1688,6 +1716,7 @@ static __global__ __launch_bounds__(256) void reduce_partials_kernel(BeamArgs A,
             out[v] = nan2;
             if (dout) dout[v] = nan2;
         });
+    if (A.tie && v == 0 && *A.tie) out[0] = make_float2(__uint_as_float(TIE_MARK), __uint_as_float(TIE_MARK));
 }
 
 
@@ -1743,14 +1772,16 @@ static __global__ void row_scale_kernel(const float *__restrict__ peak, float *_
 // delay: per-element delay offsets d_k taken into the spectra as e^{j w_n d_k} (null: left to
 // the kernels' phase words); the mirrored tiles' weights then stay alike on both sides.
 // Values that are not finite are left out of the scale and written as zeros; the bin's scale is
-// then negative and their elements are noted in bad (spread_nonfinite).
+// then negative and their elements are noted in bad (spread_nonfinite).  look: whether the grid
+// mirrors at this bin, for one-shot calls (null tie: known).
 template <int PREC>
 __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restrict__ X, void *__restrict__ Xlp,
                                                           float *__restrict__ xscale, int MT_all, int KI,
                                                           int MT_out, int mirror_el, const double *__restrict__ delay,
                                                           double fs_over_N, int n_lb, int n_el,
                                                           const float *__restrict__ row_inv,
-                                                          uint32_t *__restrict__ bad, int bad_rows, int bad_words)
+                                                          uint32_t *__restrict__ bad, int bad_rows, int bad_words,
+                                                          MirrorArgs look)
 {
     auto finite = [](float2 v) { return fabsf(v.x) < INFINITY && fabsf(v.y) < INFINITY; };
     __shared__ float red[256];
@@ -1795,6 +1826,11 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
         }
     }
     if (threadIdx.x == 0) xscale[b] = any_nf ? -scale : scale;
+    if (look.tie) {
+        bool off = false;
+        for (long v = threadIdx.x; v < (long)(look.n_x / 2) * look.n_z; v += 256) off |= mirror_off(look, v, b);
+        if (off) *look.tie = 1u;
+    }
     const float inv = 1.0f / scale;
     constexpr int pl = Prec<PREC>::planes;
     const int KC = KI / 8;
