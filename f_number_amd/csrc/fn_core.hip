@@ -168,6 +168,10 @@ struct Run {
 
 }  // namespace
 
+// room for 16-bit planes: of every tiling a plan may be given, of its own, of its own without the
+// zero tiles of a last group, or none (an FP32 call then runs the FP32 kernels)
+enum class Planes { any, own, bare, none };
+
 struct fn_plan {
     int mode = 0;  // 0: plane waves, 1: synthetic aperture
     int device = 0;
@@ -187,6 +191,7 @@ struct fn_plan {
     std::vector<double> h_delay;                          // delay offsets of the last set_tof (empty: zeros)
     int precision = FN_PRECISION_FP32;  // as asked for
     int kprec = FN_PRECISION_FP32;      // form of the forward contraction (kernel_precision)
+    Planes planes = Planes::any;
     int mirror = 0;         // lateral positions symmetric: planes hold the reversed elements too
     int line_mirror = 0;    // line scan on symmetric lateral positions: two columns share their weights
     uint32_t *d_tie = nullptr;  // plans that may mirror: the check's answer (mirror_off)
@@ -249,8 +254,13 @@ namespace {
 // the forward kernel whose lanes stand for a voxel and its mirror image (beamform_tile, MIR)
 bool use_mirror(const fn_plan *P) { return P->mirror && P->n_groups == 1 && !P->interp_M; }
 
-// M-tiles of the 16-bit planes: the transmit tiles and their mirrored ones, or whole groups
-int plane_tiles(const fn_plan *P) { return use_mirror(P) ? 2 * P->MT_all : P->n_groups * P->MT_tmpl; }
+// M-tiles of the 16-bit planes: the transmit tiles and their mirrored ones, or whole groups (a
+// no-allocation call without room for a last group's zero tiles: the transmit tiles alone)
+int plane_tiles(const fn_plan *P)
+{
+    if (use_mirror(P)) return 2 * P->MT_all;
+    return P->planes == Planes::bare ? P->MT_all : P->n_groups * P->MT_tmpl;
+}
 
 // the tangent with mirrored voxels (mirrored plans run the fp16 split): one tile of rows
 bool tangent_mirror(const fn_plan *P) { return P->mirror && P->MT_all == 1; }
@@ -591,10 +601,9 @@ enum class Mirror { check, later, no };
 
 // shared configuration of plan creation: tiling, launch shape and the scalar
 // arguments of the kernels; no device work and no allocation (the
-// no-allocation entry point runs it on a plan held on the stack, with plain_fp32 where its
-// scratch has no room for the split form's planes)
-int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, bool plain_fp32 = false,
-                     bool mirror = true)
+// no-allocation entry point runs it on a plan held on the stack)
+int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, bool mirror = true,
+                     Planes planes = Planes::any)
 {
     if (c.precision < FN_PRECISION_FP32 || c.precision > FN_PRECISION_FP16)
         return fail(FN_ERR_ARGUMENT, "unknown precision %d", c.precision);
@@ -605,7 +614,8 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
     P->verbosity = c.verbosity;
     P->precision = c.precision;
     P->KI = ki_of(c.n_el);
-    P->kprec = plain_fp32 ? c.precision : kernel_precision(P, c.precision);
+    P->planes = planes;
+    P->kprec = planes == Planes::none ? c.precision : kernel_precision(P, c.precision);
     if (!P->KI) return fail(FN_ERR_UNSUPPORTED, "at most 256 array elements are supported (got %d)", c.n_el);
     if (P->KI > 32) {
         // beyond 128 elements: the one-launch forward kernel of single-frame plans
@@ -671,10 +681,10 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
     if (P->lbl) chunk = (chunk + 15) / 16 * 16;  // whole rounds of its four waves, four bins each
     P->bin_split = (g.n_f + chunk - 1) / chunk;
     P->x_bytes = (size_t)g.n_f * P->MT_all * P->KI * 64 * sizeof(float2);
-    // room for the planes of every tiling: groups of mt tiles hold up to mt - 1 zero tiles
-    const int xlp_tiles = P->mirror      ? 2 * P->MT_all
-                          : P->mode == 1 ? P->n_groups * P->MT_tmpl
-                                         : P->MT_all + std::max(P->MT_tmpl, max_tiles(P)) - 1;
+    // (groups of mt tiles hold up to mt - 1 zero tiles)
+    const int xlp_tiles = P->mirror                                      ? 2 * P->MT_all
+                          : P->mode == 1 || P->planes != Planes::any     ? plane_tiles(P)
+                                                                         : P->MT_all + std::max(P->MT_tmpl, max_tiles(P)) - 1;
     P->xlp_bytes = P->kprec != FN_PRECISION_FP32 ? (size_t)g.n_f * form_planes(P->kprec) * xlp_tiles * P->KI * 64 * 2 : 0;
 
     fnk::BeamArgs &A = P->args;
@@ -800,7 +810,7 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
             HIP_CHECK(hipMemcpyAsync(&tie, P->d_tie, sizeof(tie), hipMemcpyDeviceToHost, P->stream), "mirror_check_kernel");
             HIP_CHECK(hipStreamSynchronize(P->stream), "mirror_check_kernel");
             // one voxel a lane: the planes of either tiling fit the mirrored ones' room
-            if (tie && (s = configure_common(P, c, g, Frx, false, false))) return s;
+            if (tie && (s = configure_common(P, c, g, Frx, false))) return s;
         }
     }
     return ensure_partials(P);
@@ -1231,7 +1241,7 @@ int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of, Mir
     if (!P) return fail(FN_ERR_OUT_OF_MEMORY, "host allocation");
     Common c{};
     if ((s = configure_pw(P, p, &c))) { destroy(P); return s; }
-    if ((s = configure_common(P, c, g, p->f_number_values, false, how != Mirror::no))) { destroy(P); return s; }
+    if ((s = configure_common(P, c, g, p->f_number_values, how != Mirror::no))) { destroy(P); return s; }
     const int n_rows = P->args.n_tx;  // operand rows (ensembles: frame slots)
     // steering geometry in FP64: das_pw.m:323-327 (x_ref = sign(e_x) x_0), or the
     // virtual sources (x_vs, z_vs, |r_vs|)
@@ -1905,10 +1915,11 @@ int das_pw_noalloc(const fn_pw_params *p, const void *d_rf, int dtype, float *d_
            o_pi = 0, o_bad = 0;
     int slots = 1;
     // one voxel a lane: whether the grid's apertures mirror is only known after a look at them on
-    // the device, which this call may not wait for.  An FP32 call whose planes do not fit beside
-    // its spectra runs on the FP32 kernels.
-    for (int lean = 0; lean < 2; ++lean) {
-        if ((st = configure_common(&P, c, g, p->f_number_values, lean == 1, false))) return st;
+    // the device, which this call may not wait for.  A call whose planes do not fit beside its
+    // spectra leaves out their zero tiles, then an FP32 call runs the FP32 kernels.
+    for (const Planes room : {Planes::own, Planes::bare, Planes::none}) {
+        if (room == Planes::none && p->precision != FN_PRECISION_FP32) break;
+        if ((st = configure_common(&P, c, g, p->f_number_values, false, room))) return st;
         cv = Carve{};
         o_X = cv.take(P.x_bytes);
         o_Xlp = cv.take(P.xlp_bytes);
