@@ -168,9 +168,10 @@ struct Run {
 
 }  // namespace
 
-// room for 16-bit planes: of every tiling a plan may be given, of its own, of its own without the
-// zero tiles of a last group, or none (an FP32 call then runs the FP32 kernels)
-enum class Planes { any, own, bare, none };
+// room for 16-bit planes: of a plan's own tiling and the tangent's (others: ensure_planes), of its
+// own, of its own without the zero tiles of a last group, or none (an FP32 call then runs the
+// FP32 kernels)
+enum class Planes { plan, own, bare, none };
 
 struct fn_plan {
     int mode = 0;  // 0: plane waves, 1: synthetic aperture
@@ -191,7 +192,7 @@ struct fn_plan {
     std::vector<double> h_delay;                          // delay offsets of the last set_tof (empty: zeros)
     int precision = FN_PRECISION_FP32;  // as asked for
     int kprec = FN_PRECISION_FP32;      // form of the forward contraction (kernel_precision)
-    Planes planes = Planes::any;
+    Planes planes = Planes::plan;
     int mirror = 0;         // lateral positions symmetric: planes hold the reversed elements too
     int line_mirror = 0;    // line scan on symmetric lateral positions: two columns share their weights
     uint32_t *d_tie = nullptr;  // plans that may mirror: the check's answer (mirror_off)
@@ -233,6 +234,8 @@ struct fn_plan {
     hipStream_t adj_sc_stream = nullptr;
     long adj_vpr = 0;
     size_t x_bytes = 0, xlp_bytes = 0;
+    int xlp_tiles = 0;          // tiles that d_Xlp has room for
+    void *d_xlp_own = nullptr;  // planes beyond those of the block (ensure_planes)
     float2 *d_pimg = nullptr;   // partial images [slot][n_vox] (several workgroups per voxel)
     size_t pimg_cap = 0;        // float2 capacity of d_pimg
     float2 *d_ptan = nullptr;   // tangent partials: image slots, then dI/dc slots
@@ -487,6 +490,8 @@ size_t row_scale_bytes(int MT) { return (size_t)(2 + ROW_PEAK_CHUNKS) * 16 * MT 
 // (bf16 has the exponents of FP32)
 bool has_row_scales(int kprec) { return kprec == FN_PRECISION_FP16X3 || kprec == FN_PRECISION_FP16; }
 
+size_t plane_bytes(const fn_plan *P, int tiles) { return (size_t)P->g.n_f * form_planes(P->kprec) * tiles * P->KI * 64 * 2; }
+
 // words of a mask of 4 KI elements, and bytes of the masks beside n_f bins of planes (each of
 // `rows` operand rows has its own where they are other frames or jobs)
 int bad_words(int KI) { return KI / 8; }
@@ -528,7 +533,7 @@ void destroy(fn_plan *p)
 {
     if (!p) return;
     destroy(p->shallow);
-    hipFree(p->d_block); hipFree(p->d_ip); hipFree(p->d_simg); hipFree(p->d_sw); hipFree(p->d_P); hipFree(p->d_Z); hipFree(p->d_part); hipFree(p->d_qtab); hipFree(p->d_vsc); hipFree(p->d_nw);
+    hipFree(p->d_block); hipFree(p->d_xlp_own); hipFree(p->d_ip); hipFree(p->d_simg); hipFree(p->d_sw); hipFree(p->d_P); hipFree(p->d_Z); hipFree(p->d_part); hipFree(p->d_qtab); hipFree(p->d_vsc); hipFree(p->d_nw);
     hipFree(p->d_sigF); hipFree(p->d_pimg); hipFree(p->d_ptan);
     for (auto &r : p->pending) { hipEventDestroy(r.e0); hipEventDestroy(r.e1); hipEventDestroy(r.e2); }
     for (auto &r : p->spare) { hipEventDestroy(r.e0); hipEventDestroy(r.e1); hipEventDestroy(r.e2); }
@@ -603,7 +608,7 @@ enum class Mirror { check, later, no };
 // arguments of the kernels; no device work and no allocation (the
 // no-allocation entry point runs it on a plan held on the stack)
 int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double *Frx, bool mirror = true,
-                     Planes planes = Planes::any)
+                     Planes planes = Planes::plan)
 {
     if (c.precision < FN_PRECISION_FP32 || c.precision > FN_PRECISION_FP16)
         return fail(FN_ERR_ARGUMENT, "unknown precision %d", c.precision);
@@ -681,11 +686,14 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
     if (P->lbl) chunk = (chunk + 15) / 16 * 16;  // whole rounds of its four waves, four bins each
     P->bin_split = (g.n_f + chunk - 1) / chunk;
     P->x_bytes = (size_t)g.n_f * P->MT_all * P->KI * 64 * sizeof(float2);
-    // (groups of mt tiles hold up to mt - 1 zero tiles)
-    const int xlp_tiles = P->mirror                                      ? 2 * P->MT_all
-                          : P->mode == 1 || P->planes != Planes::any     ? plane_tiles(P)
-                                                                         : P->MT_all + std::max(P->MT_tmpl, max_tiles(P)) - 1;
-    P->xlp_bytes = P->kprec != FN_PRECISION_FP32 ? (size_t)g.n_f * form_planes(P->kprec) * xlp_tiles * P->KI * 64 * 2 : 0;
+    P->xlp_tiles = 0;
+    if (P->kprec != FN_PRECISION_FP32 && !P->lbl) {
+        P->xlp_tiles = P->mirror ? 2 * P->MT_all : plane_tiles(P);
+        // (the tangent runs pairs of tiles)
+        if (P->planes == Planes::plan && P->mode == 0 && P->n_frames == 1 && P->KI <= 32 && P->precision == FN_PRECISION_FP32)
+            P->xlp_tiles = std::max(P->xlp_tiles, P->MT_all > 1 ? (P->MT_all + 1) / 2 * 2 : 1);
+    }
+    P->xlp_bytes = plane_bytes(P, P->xlp_tiles);
 
     fnk::BeamArgs &A = P->args;
     A.ctof = c.c0;
@@ -715,6 +723,23 @@ fnk::MirrorArgs mirror_args(const fn_plan *P)
 {
     const fnk::BeamArgs &A = P->args;
     return {P->d_tie, A.px, A.pz, A.Frx, A.sqrt_f, A.M, A.pitch, A.c0, A.n_x, A.n_z, A.n_el, A.n_f, A.clamp};
+}
+
+int interp_points(const fn_plan *P);
+
+// planes of `tiles` tiles and more: of every tiling a plan may be given, once, beside those of its
+// block (which a captured graph may still read)
+int ensure_planes(fn_plan *P, int tiles)
+{
+    if (P->kprec == FN_PRECISION_FP32 || P->lbl || tiles <= P->xlp_tiles) return FN_OK;
+    const int most = std::max(tiles, P->MT_all + std::max(P->MT_tmpl, max_tiles(P)) - 1);
+    HIP_CHECK(hipSetDevice(P->device), "hipSetDevice");
+    HIP_CHECK(hipMalloc(&P->d_xlp_own, plane_bytes(P, most)), "16-bit spectra planes");
+    P->xlp_tiles = most;
+    P->xlp_bytes += plane_bytes(P, most);
+    P->d_Xlp = P->d_xlp_own;
+    P->args.Xlp = P->d_Xlp;
+    return FN_OK;
 }
 
 // shared part of plan creation, after configure_common: the device tables and workspace.
@@ -753,11 +778,15 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     const size_t o_zr = cv.take(c.n_el * sizeof(double));
     const size_t o_tie = cv.take(sizeof(uint32_t));
     const size_t tables = cv.used;
+    // (an interpolated image takes no planes: only its plan's tangent does)
+    const bool lp = P->xlp_tiles > 0;
+    if (!spectra_of && interp_points(P)) P->xlp_tiles = 0;
+    P->xlp_bytes = plane_bytes(P, P->xlp_tiles);
     const size_t o_X = cv.take(spectra_of ? 0 : P->x_bytes), o_Xlp = cv.take(P->xlp_bytes);
-    const size_t o_xs = cv.take(P->xlp_bytes ? g.n_f * sizeof(float) : 0);
+    const size_t o_xs = cv.take(lp ? g.n_f * sizeof(float) : 0);
     P->args.bad_rows = P->n_frames > 1 ? 16 * P->MT_all : 1;
     P->args.bad_words = bad_words(P->KI);
-    const size_t o_bad = cv.take(P->xlp_bytes ? bad_bytes(g.n_f, P->args.bad_rows, P->KI) : 0);
+    const size_t o_bad = cv.take(lp ? bad_bytes(g.n_f, P->args.bad_rows, P->KI) : 0);
     const size_t o_rs = cv.take(P->n_frames > 1 && has_row_scales(P->kprec) ? row_scale_bytes(P->MT_all) : 0);
     const size_t o_xr = cv.take(P->lbl ? (size_t)g.n_f * c.n_x * c.n_el * sizeof(float2) : 0);
     const size_t o_lf = cv.take(P->lbl ? lines_flags(P) * sizeof(uint32_t) + bad_bytes(g.n_f, c.n_x, P->KI) : 0);
@@ -784,11 +813,11 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
     P->d_zeros = at(o_zr);
     P->d_X = spectra_of ? spectra_of->d_X : reinterpret_cast<float2 *>(at(o_X));
     P->d_Xlp = P->xlp_bytes ? at(o_Xlp) : nullptr;
-    P->d_bad = P->xlp_bytes ? reinterpret_cast<uint32_t *>(at(o_bad)) : nullptr;
+    P->d_bad = lp ? reinterpret_cast<uint32_t *>(at(o_bad)) : nullptr;
     P->d_rowscale = P->n_frames > 1 && has_row_scales(P->kprec) ? reinterpret_cast<float *>(at(o_rs)) : nullptr;
     P->d_Xrow = P->lbl ? reinterpret_cast<float2 *>(at(o_xr)) : nullptr;
     P->d_lflag = P->lbl ? reinterpret_cast<uint32_t *>(at(o_lf)) : nullptr;
-    P->d_xscale = P->xlp_bytes ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
+    P->d_xscale = lp ? reinterpret_cast<float *>(at(o_xs)) : nullptr;
 
     fnk::BeamArgs &A = P->args;
     A.X = P->d_X;
@@ -810,7 +839,10 @@ int create_common(fn_plan *P, const Common &c, const fnh::Grid &g, const double 
             HIP_CHECK(hipMemcpyAsync(&tie, P->d_tie, sizeof(tie), hipMemcpyDeviceToHost, P->stream), "mirror_check_kernel");
             HIP_CHECK(hipStreamSynchronize(P->stream), "mirror_check_kernel");
             // one voxel a lane: the planes of either tiling fit the mirrored ones' room
+            const int tiles = P->xlp_tiles;
             if (tie && (s = configure_common(P, c, g, Frx, false))) return s;
+            P->xlp_tiles = tiles;
+            P->xlp_bytes = plane_bytes(P, tiles);
         }
     }
     return ensure_partials(P);
@@ -893,7 +925,7 @@ int clamped_depths(const fn_plan *P)
 // padded channel at 100 TFLOP/s plus 75 ns per 64 voxels, element and angle, against 0.9 us +
 // 0.35 us per transmit tile for 16 voxels and a bin, each over 1024 SIMDs (100 x 77 voxels, 11
 // angles, 542 bins: 0.39 ms against 0.45; a quarter of these voxels: about even).  The samples
-// stay within 8 GiB and their twiddles within LDS.
+// stay within 2 GiB (a hundredth of the card's memory) and their twiddles within LDS.
 int interp_points(const fn_plan *P)
 {
     const int n_f = P->g.n_f;
@@ -903,7 +935,7 @@ int interp_points(const fn_plan *P)
     if (2 * clamped_depths(P) > P->n_z) return 0;
     const long M = ((9L * n_f + 3) / 4 + 15) / 16 * 16;
     if (M * 8 + (long)n_f * 4 > fnk::INTERP_LDS_MAX) return 0;
-    if (fnk::interp_table_floats2((int)M, P->n_tx, P->n_el) * sizeof(float2) > ((size_t)8 << 30)) return 0;
+    if (fnk::interp_table_floats2((int)M, P->n_tx, P->n_el) * sizeof(float2) > ((size_t)2 << 30)) return 0;
     const double t_samples = 8.0 * n_f * M * (16.0 * P->MT_all) * (4.0 * P->KI) / 1e14;
     const double t_gather = P->n_vox / 64.0 * P->n_el * P->n_tx * 75e-9 / 1024.0;
     const double t_sum = P->n_vox / 16.0 * n_f * (0.9 + 0.35 * P->MT_all) * (P->KI / 32.0) * 1e-6 / 1024.0;
@@ -928,7 +960,7 @@ int setup_interp(fn_plan *P, const fn_pw_params *p)
         P->interp_M = 0;
         (void)hipGetLastError();
         fnh::clear_error();
-        return FN_OK;
+        return ensure_planes(P, plane_tiles(P));
     };
     const int nz = clamped_depths(P);
     if (nz > 0) {
@@ -944,7 +976,7 @@ int setup_interp(fn_plan *P, const fn_pw_params *p)
     const size_t bytes = (interp_samples(P) + P->interp_M) * sizeof(float2) + P->g.n_f * sizeof(float);
     if (hipMalloc(&P->d_ip, bytes) != hipSuccess) return keep_sum();
     if (ensure_partials(P) != FN_OK) {
-        keep_sum();
+        if (int s = keep_sum()) return s;
         return ensure_partials(P);
     }
     const hipError_t e = fnk::launch_interp_tables(interp_tw(P), interp_ipsi(P), P->interp_M, P->g.n_f, P->stream);
@@ -952,6 +984,21 @@ int setup_interp(fn_plan *P, const fn_pw_params *p)
     HIP_CHECK(hipStreamSynchronize(P->stream), "interp_tables_kernel");
     return FN_OK;
 }
+
+// device bytes of interpolated channel samples, their tables and the plan of the clamped depths
+size_t interp_bytes(const fn_plan *P)
+{
+    if (!P->interp_M) return 0;
+    size_t n = (interp_samples(P) + P->interp_M) * sizeof(float2) + P->g.n_f * sizeof(float);
+    if (P->shallow) n += P->shallow->xlp_bytes + (size_t)P->shallow->n_vox * (sizeof(float2) + sizeof(float));
+    return n;
+}
+
+// device bytes of a line scan's spectra by rows
+size_t row_bytes(const fn_plan *P) { return P->lbl ? (size_t)P->g.n_f * P->n_x * P->n_el * sizeof(float2) : 0; }
+
+// the spectra and everything that is laid out from them
+size_t workspace_bytes(const fn_plan *P) { return P->x_bytes + P->xlp_bytes + interp_bytes(P) + row_bytes(P); }
 
 hipError_t launch_beam(const fn_plan *P, dim3 grid, const fnk::BeamArgs &A, hipStream_t s)
 {
@@ -1328,6 +1375,8 @@ int set_tiling(fn_plan *P, int mt, int split)
     P->lds_beam = lds;
     P->args.tx_group = mt;
     P->args.bin_chunk = chunk;
+    if (!P->interp_M)
+        if (int st = ensure_planes(P, plane_tiles(P))) return st;
     return ensure_partials(P);
 }
 
@@ -1437,6 +1486,7 @@ int execute_tangent(fn_plan *P, const void *d_rf, int dtype, float *d_image, flo
     const bool split_form = P->kprec == FN_PRECISION_FP16X3;
     const bool mirror = tangent_mirror(P);
     if (split_form) {
+        if (int st = ensure_planes(P, mirror ? 2 * P->MT_all : groups * mt)) return st;
         if (int st = launch_lowp_planes(P, P->d_X, P->d_Xlp, P->d_xscale, P->d_bad, 1, P->MT_all, mirror ? 2 * P->MT_all : groups * mt,
                                         mirror ? P->n_el : 0, plane_delay(P, mirror), s))
             return st;
@@ -1718,7 +1768,7 @@ void compose_report(const fn_plan *P, size_t rf_bytes, size_t img_bytes, size_t 
     const double b_pos = 8.0 * (P->n_x + P->n_z);
     const double b_tab = 8.0 * P->g.n_f * (P->d_Ftx ? 3 : 2) + (P->d_txp ? 24.0 * P->n_tx : 0.0) + 8.0 * P->g.N +
                          8.0 * P->n_el;
-    const double b_spec = (double)P->x_bytes + (double)P->xlp_bytes + (P->xlp_bytes ? 4.0 * P->g.n_f : 0.0);
+    const double b_spec = (double)workspace_bytes(P) + (P->d_xscale ? 4.0 * P->g.n_f : 0.0);
     const double b_part = 8.0 * (double)P->pimg_cap;
     const double b_tot = b_pos + b_tab + rf_bytes + b_spec + b_part + img_bytes + (double)w_bytes * n_w;
     r += kRule;
@@ -2031,7 +2081,7 @@ int32_t fn_plan_info_get(const fn_plan *P, fn_plan_info *info)
     info->n_f = P->g.n_f;
     info->n_tx = P->n_tx;
     info->n_voxels = P->n_vox;
-    info->workspace_bytes = (int64_t)P->x_bytes;
+    info->workspace_bytes = (int64_t)workspace_bytes(P);
     info->flops_per_frame = P->flops;
     std::call_once(P->useful_once, [P] { P->useful_flops = 8.0 * useful_macs(P); });
     info->useful_flops_per_frame = P->useful_flops;

@@ -252,7 +252,7 @@ typedef struct fn_plan_info {
     int32_t N_dft, n_lb, n_ub, n_f;
     int32_t n_tx;                 /* angles (PW) or elements (SA) */
     int64_t n_voxels;
-    int64_t workspace_bytes;
+    int64_t workspace_bytes;      /* spectra, their 16-bit planes and what else is laid out from them */
     double flops_per_frame;       /* 8 * n_f * n_voxels * n_elements * n_tx */
     double useful_flops_per_frame;/* same over the elements whose weight can be nonzero (the aperture
                                      bounds; every element of an untruncated window) and, for the

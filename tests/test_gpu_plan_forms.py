@@ -1,0 +1,81 @@
+"""Workspaces that are laid out on demand.
+
+Images (relative L2): 1e-5 between two forms or tilings, each within 5e-6 of exact.
+"""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+PITCH, WIDTH, C0, FS = 0.3048e-3, 0.27e-3, 1540.0, 20.832e6
+
+
+@pytest.fixture(scope="module")
+def fa():
+    import f_number_amd as fa
+
+    fa.load()
+    return fa
+
+
+SYM, OFF = np.linspace(-8e-3, 8e-3, 80), np.linspace(-8e-3, 8e-3, 80) + 1e-3
+DEPTHS = np.linspace(5e-3, 30e-3, 90)
+
+
+def _plan(fa, n_ang, x=OFF, n_el=128, F=None, **kw):
+    return fa.PwPlan(x, DEPTHS, 700, n_el, np.linspace(-0.2, 0.2, n_ang), FS, WIDTH, PITCH, C0, (4e6, 6e6), 0.0,
+                     window=fa.windows.tukey(0.5), F_number=F if F is not None else fa.f_numbers.grating.angle_lb(60, 1.5),
+                     **kw)
+
+
+@pytest.mark.parametrize("n_ang,precision", [(75, "fp32"), (75, "bf16x3"), (40, "fp16"), (100, "fp32")])
+def test_tilings_beyond_the_default_one(fa, n_ang, precision):
+    """planes for a tiling that a plan was not created with are laid out on demand, and the memory
+    of a plan says so"""
+    import torch
+
+    plan = _plan(fa, n_ang, precision=precision)
+    rf = torch.randn((n_ang, 128, 700), generator=torch.Generator().manual_seed(3)).cuda()
+    ref = torch.empty((80, 90), dtype=torch.complex64, device="cuda")
+    plan.execute(rf, ref)
+    info = plan.info()
+    tiles = -(-n_ang // 16)
+    bins = info["n_f"]
+    planes = {"fp32": 16384, "bf16x3": 16384, "fp16": 8192}[precision] * bins
+    assert info["workspace_bytes"] <= tiles * 16384 * bins + (tiles + 1) * planes
+    img = torch.empty_like(ref)
+    batch = fa.Batch([plan])
+    batch.execute([rf], [img])  # captured with the first planes
+    for mt in range(1, min(tiles, 5) + 1):
+        plan.set_tiling(mt, 3)
+        plan.execute(rf, img)
+        torch.cuda.synchronize()
+        print(f"case tiling {n_ang} angles {precision} {mt}", flush=True)
+        assert rel_l2(img.cpu().numpy(), ref.cpu().numpy()) <= (1e-3 if precision == "fp16" else 1e-5)
+    batch.execute([rf], [img])
+    torch.cuda.synchronize()
+    assert rel_l2(img.cpu().numpy(), ref.cpu().numpy()) <= (1e-3 if precision == "fp16" else 1e-5)
+    batch.close()
+
+
+@pytest.mark.parametrize("n_ang", [3, 20, 70])
+def test_interpolated_plans_tangent(fa, n_ang):
+    """an interpolated plan holds no planes until its tangent asks"""
+    import torch
+
+    F = fa.f_numbers.constant(1.5)
+    plan, other = _plan(fa, n_ang, F=F), _plan(fa, n_ang, F=F, precision="fp16x3")
+    rf = torch.randn((n_ang, 128, 700), generator=torch.Generator().manual_seed(5)).cuda()
+    ref, img, d = (torch.empty((80, 90), dtype=torch.complex64, device="cuda") for _ in range(3))
+    other.execute(rf, ref)
+    plan.execute(rf, img)
+    before = plan.info()["workspace_bytes"]
+    plan.execute_tangent(rf, img, d)
+    torch.cuda.synchronize()
+    assert plan.info()["workspace_bytes"] > before
+    assert rel_l2(img.cpu().numpy(), ref.cpu().numpy()) <= 1e-5
+    plan.execute(rf, img)
+    torch.cuda.synchronize()
+    assert rel_l2(img.cpu().numpy(), ref.cpu().numpy()) <= 1e-5
