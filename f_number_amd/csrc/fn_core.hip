@@ -1388,7 +1388,8 @@ int autotune(fn_plan *P, const void *d_rf, int dtype, float *d_image, int reps, 
     std::vector<std::pair<int, int>> cand;
     const int n_f = P->g.n_f;
     const int mt_lo = P->mode == 1 ? sa_mt(P->KI) : 1, mt_hi = max_tiles(P);
-    for (int mt = mt_lo; mt <= mt_hi; ++mt) {
+    if (P->interp_M) cand.emplace_back(mt0, split0);  // (an interpolated image has no tiling)
+    for (int mt = mt_lo; mt <= mt_hi && !P->interp_M; ++mt) {
         // distinct group counts only: the tile count of a balanced split
         if (P->mode == 0) {
             const int groups = (P->MT_all + mt - 1) / mt;
@@ -1753,18 +1754,39 @@ void compose_report(const fn_plan *P, size_t rf_bytes, size_t img_bytes, size_t 
                 (double)prop.maxSharedMemoryPerMultiProcessor / 1024.0);
     report_line(r, "  %-20s: %-18d %-22s: %d.%d / %d.%d\n", "registers per block", prop.regsPerBlock,
                 "driver / runtime", drv / 10000000, (drv / 100000) % 100, rt / 10000000, (rt / 100000) % 100);
-    report_line(r, "  %-20s: %-18s %-22s: %s\n", "contraction", kPrec[P->precision], "mode",
-                P->mode == 0 ? (P->n_frames > 1 ? "plane waves, ensemble" : "plane waves") : "synthetic aperture");
+    std::string form = kPrec[P->precision];
+    if (P->interp_M) form += ", interpolated";
+    else if (P->lbl ? P->line_mirror && P->delays_even : use_mirror(P)) form += P->lbl ? ", mirrored columns" : ", mirrored voxels";
+    report_line(r, "  %-20s: %-22s %-22s: %s\n", "contraction", form.c_str(), "mode",
+                P->lbl         ? "line scan"
+                : P->mode == 1 ? "synthetic aperture"
+                : P->n_frames > 1 ? "plane waves, ensemble" : "plane waves");
     r += kRule;
     r += " launch parameters\n";
     r += kRule;
-    const long tiles = beam_tiles(P);
-    report_line(r, "  %-20s: %-6ld x 64 voxels %-11s %-22s: %d x %d of 16 rows\n", "voxel tiles", tiles, "",
-                "transmit groups x tiles", P->n_groups, P->MT_tmpl);
-    report_line(r, "  %-20s: %-3d of %-5d bins %-8s %-22s: %d (4 elements each)\n", "bin chunks", P->bin_split,
-                P->args.bin_chunk, "", "element steps / lane", P->KI);
-    report_line(r, "  %-20s: %-18ld %-22s: %s\n", "workgroups", tiles * P->bin_split * P->n_groups, "receive window class",
-                kWin[P->wcr]);
+    const long tiles = P->interp_M ? (P->n_vox + 63) / 64 : beam_tiles(P);
+    if (P->interp_M) {
+        report_line(r, "  %-20s: %-6ld x 64 voxels %-11s %-22s: %d of up to 32 angles\n", "voxel tiles", tiles, "",
+                    "transmit groups", beam_slots(P));
+        report_line(r, "  %-20s: %-18d %-22s: %d of %d\n", "samples per channel", P->interp_M, "clamped depths (summed)",
+                    P->shallow ? P->shallow->n_z : 0, P->n_z);
+        report_line(r, "  %-20s: %-18ld %-22s: %s\n", "workgroups", tiles * beam_slots(P), "receive window class",
+                    kWin[wcr_general(P->wcr)]);
+    } else if (P->lbl) {
+        const int cols = P->line_mirror && P->delays_even ? (P->n_x + 1) / 2 : P->n_x;
+        report_line(r, "  %-20s: %-6ld x 64 depths %-11s %-22s: %d of %d lines\n", "depth tiles", tiles, "", "column groups", cols,
+                    P->n_x);
+        report_line(r, "  %-20s: %-3d of %-5d bins\n", "bin chunks", P->bin_split, P->args.bin_chunk);
+        report_line(r, "  %-20s: %-18ld %-22s: %s\n", "workgroups", tiles * P->bin_split * cols, "receive window class",
+                    kWin[P->wcr]);
+    } else {
+        report_line(r, "  %-20s: %-6ld x 64 voxels %-11s %-22s: %d x %d of 16 rows\n", "voxel tiles", tiles, "",
+                    "transmit groups x tiles", P->n_groups, P->MT_tmpl);
+        report_line(r, "  %-20s: %-3d of %-5d bins %-8s %-22s: %d (4 elements each)\n", "bin chunks", P->bin_split,
+                    P->args.bin_chunk, "", "element steps / lane", P->KI);
+        report_line(r, "  %-20s: %-18ld %-22s: %s\n", "workgroups", tiles * P->bin_split * P->n_groups,
+                    "receive window class", kWin[P->wcr]);
+    }
     const double b_pos = 8.0 * (P->n_x + P->n_z);
     const double b_tab = 8.0 * P->g.n_f * (P->d_Ftx ? 3 : 2) + (P->d_txp ? 24.0 * P->n_tx : 0.0) + 8.0 * P->g.N +
                          8.0 * P->n_el;

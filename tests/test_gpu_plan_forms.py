@@ -1,4 +1,5 @@
-"""Workspaces that are laid out on demand.
+"""Which form of the beamformer a call takes, from its report, on both sides of each rule; and the
+workspaces that are laid out on demand.
 
 Images (relative L2): 1e-5 between two forms or tilings, each within 5e-6 of exact.
 """
@@ -20,8 +21,42 @@ def fa():
     return fa
 
 
+def _report(fa, x, z, n_el=64, n_ang=3, win="boxcar", F=None, band=(2.25e6, 6.75e6), n_t=700, precision="fp32"):
+    from f_number_amd import _lib
+
+    window = fa.windows.tukey(0.5) if win == "tukey" else getattr(fa.windows, win)()
+    rf = np.random.default_rng(1).standard_normal((n_t, n_el, n_ang)).astype(np.float32)
+    fa.das_pw(x, z, np.asfortranarray(rf), FS, np.linspace(-0.2, 0.2, n_ang), WIDTH, PITCH, C0, band, 0, window,
+              F if F is not None else fa.f_numbers.grating.angle_lb(60, 1.5), precision=precision, verbosity=1)
+    return _lib.load().fn_last_report().decode()
+
+
+def _line(report, what):
+    return [l for l in report.splitlines() if what in l][0]
+
+
 SYM, OFF = np.linspace(-8e-3, 8e-3, 80), np.linspace(-8e-3, 8e-3, 80) + 1e-3
 DEPTHS = np.linspace(5e-3, 30e-3, 90)
+
+
+def test_one_f_number_is_interpolated_where_it_pays(fa):
+    F = fa.f_numbers.constant(1.5)
+    r = _report(fa, SYM, DEPTHS, F=F)
+    assert "fp32, interpolated" in _line(r, "contraction") and " 0 of 90" in _line(r, "samples per channel")
+    # 1 MHz upwards from 3 mm: the clamp is at work above 10 mm
+    r = _report(fa, SYM, np.linspace(3e-3, 30e-3, 90), F=F, band=(1e6, 6e6))
+    assert "fp32, interpolated" in _line(r, "contraction") and " 0 of 90" not in _line(r, "samples per channel")
+    # few voxels; another precision; an F-number per bin
+    for kw in (dict(x=SYM[:5], z=DEPTHS[:4], F=F), dict(x=SYM, z=DEPTHS, F=F, precision="fp16x3"), dict(x=SYM, z=DEPTHS)):
+        assert "interpolated" not in _line(_report(fa, **kw), "contraction")
+
+
+def test_symmetric_grids_are_mirrored(fa):
+    for n_ang, mirrored in ((1, True), (16, True), (32, True), (33, False)):
+        r = _report(fa, SYM, DEPTHS, n_ang=n_ang, win="tukey")
+        assert ("fp32, mirrored voxels" in _line(r, "contraction")) == mirrored, n_ang
+    assert "mirrored" not in _line(_report(fa, OFF, DEPTHS, win="tukey"), "contraction")
+    assert "mirrored" not in _line(_report(fa, SYM, DEPTHS, win="tukey", precision="fp16"), "contraction")
 
 
 def _plan(fa, n_ang, x=OFF, n_el=128, F=None, **kw):
@@ -61,8 +96,8 @@ def test_tilings_beyond_the_default_one(fa, n_ang, precision):
 
 
 @pytest.mark.parametrize("n_ang", [3, 20, 70])
-def test_interpolated_plans_tangent(fa, n_ang):
-    """an interpolated plan holds no planes until its tangent asks"""
+def test_interpolated_plans_tangent_and_autotune(fa, n_ang):
+    """an interpolated plan holds no planes until its tangent asks; its tiling changes nothing"""
     import torch
 
     F = fa.f_numbers.constant(1.5)
@@ -70,6 +105,8 @@ def test_interpolated_plans_tangent(fa, n_ang):
     rf = torch.randn((n_ang, 128, 700), generator=torch.Generator().manual_seed(5)).cuda()
     ref, img, d = (torch.empty((80, 90), dtype=torch.complex64, device="cuda") for _ in range(3))
     other.execute(rf, ref)
+    r = plan.autotune(rf, img, repetitions=2)
+    assert r["n_candidates"] == 1
     plan.execute(rf, img)
     before = plan.info()["workspace_bytes"]
     plan.execute_tangent(rf, img, d)
