@@ -916,15 +916,27 @@ int clamped_depths(const fn_plan *P)
     return n;
 }
 
+// Estimated seconds of the two forms of an image: the sum over the bins of MT transmit tiles
+// (0.9 us + 0.35 us per tile for 16 voxels and a bin) and the interpolation of M samples per
+// channel (8 n_f M flop per padded channel at 100 TFLOP/s, then 75 ns per 64 voxels, element and
+// angle), each over 1024 SIMDs.
+double sum_seconds(const fn_plan *P, int MT)
+{
+    return P->n_vox / 16.0 * P->g.n_f * (0.9 + 0.35 * MT) * (P->KI / 32.0) * 1e-6 / 1024.0;
+}
+double interp_seconds(const fn_plan *P, long M)
+{
+    return 8.0 * P->g.n_f * M * (16.0 * P->MT_all) * (4.0 * P->KI) / 1e14 +
+           P->n_vox / 64.0 * P->n_el * P->n_tx * 75e-9 / 1024.0;
+}
+
 // Samples per channel of a plan whose image can be interpolated (fn_interp.hip), 0 otherwise:
 // FP32 plane waves of one frame with one F-number for every bin; the depths where its clamp is
 // at work, at most half of them, have a plan of their own.  31 angles, boxcar, 512 x 384 (432
 // bins): 0.9 ms against 7.2 for the sum over the bins, and 0.23 for the samples; 75 angles,
 // 1024 x 512 (1455 bins, 14 % of the depths clamped): 27 ms against 118.  The samples cost the
-// same for any image, so the line is where both forms' estimated times cross: 8 n_f M flop per
-// padded channel at 100 TFLOP/s plus 75 ns per 64 voxels, element and angle, against 0.9 us +
-// 0.35 us per transmit tile for 16 voxels and a bin, each over 1024 SIMDs (100 x 77 voxels, 11
-// angles, 542 bins: 0.39 ms against 0.45; a quarter of these voxels: about even).  The samples
+// same for any image, so the line is where both forms' estimated times cross (100 x 77 voxels,
+// 11 angles, 542 bins: 0.39 ms against 0.45; a quarter of these voxels: about even).  The samples
 // stay within 2 GiB (a hundredth of the card's memory) and their twiddles within LDS.
 int interp_points(const fn_plan *P)
 {
@@ -936,11 +948,7 @@ int interp_points(const fn_plan *P)
     const long M = ((9L * n_f + 3) / 4 + 15) / 16 * 16;
     if (M * 8 + (long)n_f * 4 > fnk::INTERP_LDS_MAX) return 0;
     if (fnk::interp_table_floats2((int)M, P->n_tx, P->n_el) * sizeof(float2) > ((size_t)2 << 30)) return 0;
-    const double t_samples = 8.0 * n_f * M * (16.0 * P->MT_all) * (4.0 * P->KI) / 1e14;
-    const double t_gather = P->n_vox / 64.0 * P->n_el * P->n_tx * 75e-9 / 1024.0;
-    const double t_sum = P->n_vox / 16.0 * n_f * (0.9 + 0.35 * P->MT_all) * (P->KI / 32.0) * 1e-6 / 1024.0;
-    if (t_samples + t_gather > t_sum) return 0;
-    return (int)M;
+    return interp_seconds(P, M) > sum_seconds(P, P->MT_all) ? 0 : (int)M;
 }
 
 int pw_plan(const fn_pw_params *p, fn_plan **out, const fn_plan *spectra_of = nullptr, Mirror how = Mirror::check);
@@ -2352,9 +2360,25 @@ static void batch_release_graph(fn_batch *b)
 static bool row_stackable(const fn_plan *P)
 {
     // beyond three tiles of rows a plan fills its own transmit groups (the ensemble
-    // kernel holds at most four tiles per group against five of the plain kernel); an
-    // interpolated plan has no weights per bin to share
-    return P->mode == 0 && P->n_frames == 1 && !P->lbl && !P->nw && P->KI <= 32 && P->n_tx <= 48 && !P->interp_M;
+    // kernel holds at most four tiles per group against five of the plain kernel)
+    return P->mode == 0 && P->n_frames == 1 && !P->lbl && !P->nw && P->KI <= 32 && P->n_tx <= 48;
+}
+
+// Interpolated plans join a stack where its one sum over the bins is estimated below their
+// images: 0.12 ms for a stack and 0.03 ms a plan beside the two estimates.  ms stacked / apart
+// (128 elements, 367 bins): 16 plans of 1 angle at 64 x 64 1.64 / 2.46, 128 x 128 2.03 / 2.49,
+// 256 x 256 3.50 / 2.58; 4 at 64 x 64 0.60 / 0.70, 128 x 128 0.97 / 0.70; 16 of 3 angles at 128 x
+// 128 2.54 / 2.55; 4 of 11 at 256 x 256 4.00 / 0.97.
+static bool stack_interpolated(const fn_batch *b, const std::vector<int> &plans)
+{
+    int rows = 0;
+    double apart = 0.0;
+    for (int i : plans) {
+        const fn_plan *P = b->plans[i];
+        rows += P->n_tx;
+        apart += (P->interp_M ? interp_seconds(P, P->interp_M) : sum_seconds(P, P->MT_all)) + 30e-6;
+    }
+    return sum_seconds(b->plans[plans[0]], (rows + 15) / 16) + 120e-6 < apart;
 }
 
 static bool same_receive_side(const fn_plan *a, const fn_plan *b)
@@ -2384,13 +2408,16 @@ static int batch_plan_stacks(fn_batch *b, float *const *d_images, std::vector<ch
         for (int j = i; j < n; ++j)
             if (!taken[j] && row_stackable(b->plans[j]) && same_receive_side(b->plans[i], b->plans[j]))
                 r.plans.push_back(j);
+        auto interpolated = [&](int j) { return b->plans[j]->interp_M > 0; };
+        if (std::any_of(r.plans.begin(), r.plans.end(), interpolated) && !stack_interpolated(b, r.plans))
+            r.plans.erase(std::remove_if(r.plans.begin(), r.plans.end(), interpolated), r.plans.end());
         if (r.plans.size() < 2) continue;
         for (int j : r.plans) {
             r.row0.push_back(r.rows);
             r.rows += b->plans[j]->n_tx;
             taken[j] = 1;
         }
-        const fn_plan *P0 = b->plans[i];
+        const fn_plan *P0 = b->plans[r.plans[0]];
         r.MT_all = (r.rows + 15) / 16;
         const int max_tiles = stack_tile_cap(P0->kprec, P0->KI);  // the stack kernel's register budget
         const int groups = (r.MT_all + max_tiles - 1) / max_tiles;

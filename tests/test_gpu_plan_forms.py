@@ -116,3 +116,28 @@ def test_interpolated_plans_tangent_and_autotune(fa, n_ang):
     plan.execute(rf, img)
     torch.cuda.synchronize()
     assert rel_l2(img.cpu().numpy(), ref.cpu().numpy()) <= 1e-5
+
+
+@pytest.mark.parametrize("n,n_ang,nx,nz,stacked", [(16, 1, 64, 64, 16), (4, 1, 64, 64, 4), (8, 3, 160, 180, 0),
+                                                   (2, 1, 128, 128, 0)])
+def test_interpolated_plans_in_a_batch(fa, n, n_ang, nx, nz, stacked):
+    """plans of one F-number share one sum over the bins where that is the faster; either way each
+    image is its own plan's"""
+    import torch
+
+    x, z = np.linspace(-19e-3, 19e-3, nx), np.linspace(5e-3, 40e-3, nz)
+    plans = [fa.PwPlan(x, z, 1536, 128, np.linspace(-0.2, 0.2, n_ang) + 0.01 * i, FS, WIDTH, PITCH, C0, (2.25e6, 6.75e6),
+                       0.0, window=fa.windows.tukey(0.5), F_number=fa.f_numbers.constant(1.5)) for i in range(n)]
+    rfs = [torch.randn((n_ang, 128, 1536), generator=torch.Generator().manual_seed(i)).cuda() for i in range(n)]
+    imgs = [torch.empty((nx, nz), dtype=torch.complex64, device="cuda") for _ in range(n)]
+    batch = fa.Batch(plans)
+    for _ in range(2):
+        batch.execute(rfs, imgs)
+    torch.cuda.synchronize()
+    assert batch.info()["stacked_plans"] == stacked
+    ref = torch.empty_like(imgs[0])
+    for p, r, g in zip(plans, rfs, imgs):
+        p.execute(r, ref)
+        torch.cuda.synchronize()
+        assert rel_l2(g.cpu().numpy(), ref.cpu().numpy()) <= 1e-5
+    batch.close()
