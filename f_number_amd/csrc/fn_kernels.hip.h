@@ -375,13 +375,14 @@ __device__ __forceinline__ float window_rf(float ad, float iw_q, float q_o)
     return c * c;
 }
 
-template <int WC>
+template <int WC, bool PEAK = true>
 __device__ __forceinline__ float window_eval(float t, const WinCoef &w)
 {
-    if (WC == WC_RANGE) return w.peak;
+    const float peak = PEAK ? w.peak : 1.0f;
+    if (WC == WC_RANGE) return peak;
     if (WC == WC_COS_RF) {
         const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(fmaf(t, w.q_s, w.q_o), 0.f, 0.25f));
-        return w.peak * c * c;
+        return peak * c * c;
     }
     float v;
     if (WC == WC_LINEAR) {
@@ -390,7 +391,7 @@ __device__ __forceinline__ float window_eval(float t, const WinCoef &w)
         const float u = __builtin_amdgcn_fractf((t - w.t_off) * w.s_half);  // revolutions, reduced to [0, 1)
         v = w.A + w.B * __builtin_amdgcn_cosf(u);
     }
-    v = (t <= w.t_flat) ? w.peak : v;
+    v = (t <= w.t_flat) ? peak : v;
     v = (t < w.t_cut) ? v : 0.0f;
     return v;
 }
@@ -1052,7 +1053,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                         const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(t, 0.f, 0.25f));
                         a = c * c;
                     } else {
-                        a = window_eval<WCR>(t, A.wrx);
+                        a = window_eval<WCR, false>(t, A.wrx);
                         if (RTEST) a = (4 * j >= klo && 4 * j <= khi) ? a : 0.f;
                     }
                 }
@@ -1151,7 +1152,12 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             const float wsc = WCR == WC_COS_ALL ? A.wrx.s_half : WCR == WC_COS_RF ? A.wrx.q_s : 1.f;
             const float sr = ap.inv_wr * wsc, sl = ap.inv_wl * wsc;
             const float tr0 = fmaf(dgb, sr, qo), tr1 = dstep * sr, tl0 = fmaf(-dgb, sl, qo), tl1 = -dstep * sl;
-            const int klo = ap.klo - g, khi = ap.khi - g;  // support in units of 4j
+            // support in units of 4j; beyond 128 elements, whose kernels run alone on their SIMD, one
+            // unsigned comparison instead of two (256 elements, boxcar, fp16: synthetic aperture 32.6
+            // -> 31.2 ms at 128 x 128, 11 angles 5.00 -> 4.80 at 256 x 256); an empty one starts past
+            // every element
+            const int khi = ap.khi - g, klo = KI > 32 && ap.klo > ap.khi ? 0x10000 : ap.klo - g;
+            const uint32_t rspan = (uint32_t)max(ap.khi - ap.klo, 0);
             // element steps skipped together when no voxel of the wave has support there: pairs
             // where the vector ALUs bound the loop and the window needs no support test (11
             // angles, Tukey: 3.20 ms by pairs, 3.35 by chunks of 8), otherwise whole chunks,
@@ -1163,10 +1169,12 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             const int j_a = u_lo >> 2, j_b = min(u_hi >> 2, KI - 1);  // u_hi = -1: no step
             auto weight = [&](const int j, float &cs, float &sn) __attribute__((always_inline)) {
                 const float jf = (float)j;
-                // (wide arrays keep the per-element side select: fewer live registers)
+                // (wide synthetic apertures keep the per-element side select: 256 elements, bf16x3,
+                // Tukey, 192 x 192: 138.8 ms against 140.7; plane waves do not: 256 elements, 11
+                // angles, fp16, Hann: 6.98 against 6.74)
                 const float d = fmaf(jf, dstep, dgb);
-                const float t = KI <= 32 ? fmaxf(fmaf(jf, tr1, tr0), fmaf(jf, tl1, tl0))
-                                         : fmaf(fabsf(d), d < 0.f ? sl : sr, qo);
+                const float t = KI <= 32 || MODE == MODE_PW ? fmaxf(fmaf(jf, tr1, tr0), fmaf(jf, tl1, tl0))
+                                                            : fmaf(fabsf(d), d < 0.f ? sl : sr, qo);
                 float a;
                 if (WCR == WC_COS_ALL) {
                     a = fmaf(A.wrx.B, __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(t)), A.wrx.A);
@@ -1174,8 +1182,8 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                     const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fmed3f(t, 0.f, 0.25f));
                     a = (PREC == PREC_FP16X3 ? SPLIT_PEAK * c : c) * c;
                 } else {
-                    a = window_eval<WCR>(t, A.wrx);
-                    if (RTEST) a = (4 * j >= klo && 4 * j <= khi) ? a : 0.f;
+                    a = window_eval<WCR, PREC == PREC_FP16X3>(t, A.wrx);
+                    if (RTEST) a = (KI > 32 ? (uint32_t)(4 * j - klo) <= rspan : 4 * j >= klo && 4 * j <= khi) ? a : 0.f;
                 }
                 const float rv = rev_of((uint32_t)n * Qrx[j]);
                 sn = __builtin_amdgcn_sinf(rv);
@@ -1414,7 +1422,7 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
                         const int i = 16 * t + 4 * g + r;
                         const float d = fmaf((float)(16 * t + r), pf, dg_tx);
                         const float tt = fabsf(d) * (d < 0.f ? at.inv_wl : at.inv_wr);
-                        const float w = window_eval<WCT>(tt, A.wtx);
+                        const float w = window_eval<WCT, false>(tt, A.wtx);
                         w4[r] = (i >= at.klo && i <= at.khi) ? w : 0.f;
                     }
                 }
