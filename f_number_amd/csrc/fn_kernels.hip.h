@@ -1169,12 +1169,13 @@ __device__ __forceinline__ void beamform_tile(Args A, const int bx, const int by
             const int j_a = u_lo >> 2, j_b = min(u_hi >> 2, KI - 1);  // u_hi = -1: no step
             auto weight = [&](const int j, float &cs, float &sn) __attribute__((always_inline)) {
                 const float jf = (float)j;
-                // (wide synthetic apertures keep the per-element side select: 256 elements, bf16x3,
-                // Tukey, 192 x 192: 138.8 ms against 140.7; plane waves do not: 256 elements, 11
-                // angles, fp16, Hann: 6.98 against 6.74)
+                // (wide arrays keep the per-element side select, which rounds less and needs fewer live
+                // registers; not the one-pass fp16 form of the full-array window, 256 elements, 11
+                // angles: 6.98 ms with it, 6.74 without)
                 const float d = fmaf(jf, dstep, dgb);
-                const float t = KI <= 32 || MODE == MODE_PW ? fmaxf(fmaf(jf, tr1, tr0), fmaf(jf, tl1, tl0))
-                                                            : fmaf(fabsf(d), d < 0.f ? sl : sr, qo);
+                const float t = KI <= 32 || (PREC == PREC_FP16 && MODE == MODE_PW && WCR == WC_COS_ALL)
+                                    ? fmaxf(fmaf(jf, tr1, tr0), fmaf(jf, tl1, tl0))
+                                    : fmaf(fabsf(d), d < 0.f ? sl : sr, qo);
                 float a;
                 if (WCR == WC_COS_ALL) {
                     a = fmaf(A.wrx.B, __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(t)), A.wrx.A);
