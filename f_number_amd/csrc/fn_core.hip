@@ -257,12 +257,14 @@ namespace {
 // the forward kernel whose lanes stand for a voxel and its mirror image (beamform_tile, MIR)
 bool use_mirror(const fn_plan *P) { return P->mirror && P->n_groups == 1 && !P->interp_M; }
 
-// M-tiles of the 16-bit planes: the transmit tiles and their mirrored ones, or whole groups (a
-// no-allocation call without room for a last group's zero tiles: the transmit tiles alone)
+// M-tiles of the 16-bit planes: the transmit tiles and their mirrored ones, or whole groups, which
+// the kernels at 65-128 elements copy ahead of their products (the others fill in a last group's
+// zero tiles themselves: synthetic aperture of 224 elements, bf16x3, 14 tiles in groups of 4: 83.1
+// ms with zero tiles to read, 77.3 without); a no-allocation call short of room leaves them out too
 int plane_tiles(const fn_plan *P)
 {
     if (use_mirror(P)) return 2 * P->MT_all;
-    return P->planes == Planes::bare ? P->MT_all : P->n_groups * P->MT_tmpl;
+    return P->KI != 32 || P->planes == Planes::bare ? P->MT_all : P->n_groups * P->MT_tmpl;
 }
 
 // the tangent with mirrored voxels (mirrored plans run the fp16 split): one tile of rows
