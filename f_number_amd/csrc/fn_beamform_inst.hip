@@ -286,12 +286,18 @@ hipError_t FN_LAUNCHER(INST_MODE, INST_KI, INST_PREC)(int mt, int wcr, int wct, 
 {
     if (mt != SA_MT) return hipErrorInvalidValue;
     switch (wcr) {
-    case WC_RANGE: return launch_wct<WC_RANGE>(wct, grid, lds, s, A);
     case WC_LINEAR: return launch_wct<WC_LINEAR>(wct, grid, lds, s, A);
+#if INST_PREC == 0 && !FN_WIDE
+    // (FP32 plans of every other receive window run the fp16 split)
+    default: return hipErrorInvalidValue;
+    }
+#else
+    case WC_RANGE: return launch_wct<WC_RANGE>(wct, grid, lds, s, A);
     case WC_COS_ALL: return launch_wct<WC_COS_ALL>(wct, grid, lds, s, A);
     case WC_COS_RF: return launch_wct<WC_COS_RF>(wct, grid, lds, s, A);
     default: return launch_wct<WC_COS>(wct, grid, lds, s, A);
     }
+#endif
 }
 #endif
 
