@@ -28,6 +28,8 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_TFLOPS = 157.3   # MI355X dense FP32 matrix
 PEAK_16BIT_TFLOPS = 2500.0  # MI355X dense BF16 / FP16 matrix
+PEAK_FP32_VECTOR_TFLOPS = 157.3  # MI355X FP32 vector
+INTERP_FLOP = 104.0  # interpolated images: 52 FMAs per (voxel, active element, angle)
 PEAK_HBM_GBS = 8000.0
 CPU_LABEL = "reference CPU path (FP64 C restatement of das_pw.m / das_sa.m; MATLAB unavailable)"
 
@@ -685,6 +687,44 @@ def main():
     value = w.n_voxels / (head["ms_per_step"] / 1e3) / 1e6
     flops = head["info"]["useful_flops_per_frame"]
     achieved = flops / (head["beamform_ms"] / 1e3) / 1e12
+    one_f = head_key != "hann_angle_lb"
+    roofline = {
+        "kernel": "beamform_kernel",
+        "bound": "mfma",
+        "achieved": achieved,
+        "peak": PEAK_16BIT_TFLOPS,
+        "unit": "TFLOP/s",
+        "frac": achieved / PEAK_16BIT_TFLOPS,
+        "executed_frac": 3.0 * achieved / PEAK_16BIT_TFLOPS,
+        "contraction": "FP32 operands as fp16 hi + lo: three passes on the 16-bit matrix instructions, "
+                       "FP32 accumulation",
+        "traffic": measured_traffic(w.name),
+        "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated)",
+        "flops_per_launch": flops,
+        "flops_dense_per_launch": head["info"]["flops_per_frame"],
+        "flops_note": "8 flop per complex multiply-add over the elements whose weight can be nonzero "
+                      "(aperture bounds; every element for an untruncated window such as the CPU Hann)",
+        "avg_launch_ms": head["beamform_ms"],
+    }
+    if one_f:
+        # one F-number for every bin: channel samples interpolated at one time per (voxel, active
+        # element, angle), no product over the bins
+        points = flops / (8.0 * head["info"]["n_f"])
+        achieved = INTERP_FLOP * points / (head["beamform_ms"] / 1e3) / 1e12
+        roofline = {
+            "kernel": "interp_beamform_kernel",
+            "bound": "valu and the L1 rate of the gathers",
+            "achieved": achieved,
+            "peak": PEAK_FP32_VECTOR_TFLOPS,
+            "unit": "TFLOP/s",
+            "frac": achieved / PEAK_FP32_VECTOR_TFLOPS,
+            "flops_per_launch": INTERP_FLOP * points,
+            "flops_note": f"{INTERP_FLOP:.0f} flop per (voxel, active element, angle): 32 FMAs for the eight taps' "
+                          "weights, 16 for their sums, 4 for the transmit phase; the duration includes the sum "
+                          "over the bins at the depths whose F-number is clamped",
+            "flops_of_the_sum_over_the_bins": flops,
+            "avg_launch_ms": head["beamform_ms"],
+        }
     out = {
         "metric": "Mvoxel*frames/s",
         "value": value,
@@ -707,24 +747,7 @@ def main():
             "f_bounds_hz": list(w.f_bounds), "N_dft": head["info"]["N_dft"], "n_f": head["info"]["n_f"],
             "precision": "fp32", "semantics": "cpu",
         },
-        "roofline": {
-            "kernel": "beamform_kernel",
-            "bound": "mfma",
-            "achieved": achieved,
-            "peak": PEAK_16BIT_TFLOPS,
-            "unit": "TFLOP/s",
-            "frac": achieved / PEAK_16BIT_TFLOPS,
-            "executed_frac": 3.0 * achieved / PEAK_16BIT_TFLOPS,
-            "contraction": "FP32 operands as fp16 hi + lo: three passes on the 16-bit matrix instructions, "
-                           "FP32 accumulation",
-            "traffic": measured_traffic(w.name),
-            "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated)",
-            "flops_per_launch": flops,
-            "flops_dense_per_launch": head["info"]["flops_per_frame"],
-            "flops_note": "8 flop per complex multiply-add over the elements whose weight can be nonzero "
-                          "(aperture bounds; every element for an untruncated window such as the CPU Hann)",
-            "avg_launch_ms": head["beamform_ms"],
-        },
+        "roofline": roofline,
         "stages_ms": {"spectra": head["spectra_ms"], "beamform": head["beamform_ms"]},
         "spectra_roofline": spectra_roofline(w, head["info"]["n_f"], head["spectra_ms"]),
         "arms": {k: {"value": w.n_voxels / (v["ms_per_step"] / 1e3) / 1e6, "ms_per_step": v["ms_per_step"],

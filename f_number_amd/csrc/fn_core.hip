@@ -413,8 +413,8 @@ int setup_windowed(fn_plan *P, bool rx, const fn_window &wrx, const fn_window &n
 
 // forward element loops without per-element support tests: the raised cosine
 // over every element of a full array (CPU Hann) takes WC_COS_ALL, a cosine
-// window whose cut implies the support takes WC_COS_RF; tangent and adjoint
-// launch the general classes
+// window whose cut implies the support takes WC_COS_RF.  The tangent and the adjoint have
+// instances of both on the fp16 split; a tangent on FP32 instructions runs the general class
 void use_cos_all(fn_plan *P)
 {
     if (P->nw) return;
@@ -676,10 +676,12 @@ int configure_common(fn_plan *P, const Common &c, const fnh::Grid &g, const doub
         const long target = few_rows_pw(P) ? FN_FEW_ROWS_BLOCKS : 2048L;
         split = (int)std::min<long>((target + blocks - 1) / blocks, std::max(1, g.n_f / 8));
     } else if (P->mode == 0 && !P->nw && P->n_frames == 1) {
-        // a group's band spectra beyond 32 MiB (many transmit tiles, a long band): the bins
-        // are split so that the workgroups running together walk about 4 MiB of them (an
-        // XCD's L2); at 75 angles x 1455 bins this cut the fetches beyond L2 from 152-179 GB
-        // to 74-93 GB per launch at the same duration
+        // a group's band spectra beyond 32 MiB (many transmit tiles, a long band): about 4 MiB
+        // (an XCD's L2) to a chunk of bins, at most 16.  The kernels on FP32 instructions, whose
+        // workgroups kept in step, fetched half as much beyond L2 with it.  The present ones drift
+        // apart within a chunk and the count hardly matters; it stays, with the sums' order, where it
+        // was.  ms at 1 / 2 / 4 / 8 / 16 / 32 chunks: 75 angles x 1455 bins 179.0 / 178.4 / 179.1 /
+        // 179.7 / 179.9 / 177.9, bf16x3 x 542 bins 32.1 / 31.9 / 31.9 / 32.2 / 32.9 / 34.3
         const double set = (double)g.n_f * (double)P->lds_beam;
         if (set > 32.0 * 1048576.0)
             split = (int)std::min<double>({16.0, std::ceil(set / (4.0 * 1048576.0)), (double)std::max(1, g.n_f / 8)});

@@ -77,7 +77,10 @@ enum { FN_NORMALIZATION_OFF = 0, FN_NORMALIZATION_ON = 1, FN_NORMALIZATION_WINDO
  * truncated at |t| >= 1, element-snapped boxcar). */
 enum { FN_SEMANTICS_CPU = 0, FN_SEMANTICS_MEX = 1 };
 /* arithmetic of the element x transmit contraction */
-enum { FN_PRECISION_FP32 = 0,    /* FP32 accuracy: FP32 operands or their fp16 hi + lo split, FP32 accumulation */
+enum { FN_PRECISION_FP32 = 0,    /* FP32 samples, phases, sums and results; the operands of the products
+                                    as FP32 or as fp16 hi + lo halves of 22-23 bits (down to 2^-17 of
+                                    the largest of their bin in one frame), whichever is the faster at
+                                    an error against 64 bits no larger */
        FN_PRECISION_BF16X3 = 1,  /* BF16 hi+lo split operands, 3 MFMA passes, FP32 accumulation */
        FN_PRECISION_FP16X3 = 2,  /* FP16 hi+lo split operands, 3 passes */
        FN_PRECISION_FP16 = 3 };  /* FP16 operands, 1 pass */
@@ -228,12 +231,13 @@ int32_t fn_das_sa(const fn_sa_params *p, const void *data_rf, int32_t rf_dtype, 
  * layout of fn_plan_execute, d_image complex float [n_x][n_z], d_weights (may
  * be NULL) float [n_x][n_z] -- enqueued on `stream` (NULL: the default stream)
  * without host synchronisation.  The plan tables and the spectra workspace live
- * in a fixed 32 MiB device array of the library (one per GPU, held until the
+ * in a fixed device array of 32 MiB (and 64 KiB) of the library (one per GPU, held until the
  * process ends); a call that needs more returns FN_ERR_UNSUPPORTED before any
  * device work (the FP32 spectra take 16 KiB per band bin and group of 16 angles
  * at 128 elements, so about 2000 (bin, angle group) pairs fit: 11 angles over
- * 542 bins take 8.9 MB, 75 angles over 1455 bins would take 119 MB; the 16-bit
- * forms need twice that per pair).  Ensembles, line scans and windowed normalization (CPU
+ * 542 bins take 8.9 MB, 75 angles over 1455 bins would take 119 MB; the split
+ * forms need twice that per pair and fp16 half as much again; an FP32 call
+ * without room for its split planes runs on FP32 products).  Ensembles, line scans and windowed normalization (CPU
  * semantics) also return FN_ERR_UNSUPPORTED.  The host arrays of p are read
  * before the call returns.  Every call on one GPU uses that GPU's array, so
  * calls that overlap on one GPU (other host threads, or other streams still
