@@ -81,12 +81,6 @@ struct BeamArgs {
     const float2 *X;        // spectra in operand order [n_f][MT][KI][64]
     const void *Xlp;        // 16-bit spectra planes (mixed precision) [n_f][planes][MT][KI/8][64][8]
     const float *xscale;    // per-bin scale of the 16-bit planes, negative where the bin has values that are not finite
-    // 16-bit forms: elements whose spectra are not finite, one bit each, [n_f][bad_rows][bad_words]
-    // (written and read at the bins of negative xscale alone; bad_rows 1: of any row)
-    const uint32_t *bad;
-    int bad_rows, bad_words;
-    const uint32_t *tie;    // one-shot calls: does the grid not mirror after all (mirror_off; null: settled)
-    const float *row_scale; // ensembles, row stacks: per transmit row a scale beside it (null: none)
     const double *px, *pz;  // voxel positions
     const double *Frx;      // F-number per band bin (receive)
     const double *Ftx;      // F-number per band bin (transmit, SA)
@@ -125,6 +119,12 @@ struct BeamArgs {
     // L / 2 per (voxel, element), receive and (SA) transmit, and the taper windows
     const float *nw_rx, *nw_tx;  // [n_vox][n_el]; 0 where L = 0
     WinCoef wn_rx, wn_tx;
+    // 16-bit forms: elements whose spectra are not finite, one bit each, [n_f][bad_rows][bad_words]
+    // (written and read at the bins of negative xscale alone; bad_rows 1: of any row)
+    const uint32_t *bad;
+    int bad_rows, bad_words;
+    const uint32_t *tie;    // one-shot calls: does the grid not mirror after all (mirror_off; null: settled)
+    const float *row_scale; // ensembles, row stacks: per transmit row a scale beside it (null: none)
 };
 
 // adjoint voxel contraction (fn_adjoint.hip)
@@ -1797,16 +1797,23 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
     const int b = blockIdx.x;
     const int n_pairs = MT_all * KI * 64;
     const float2 *Xb = X + (size_t)b * n_pairs;
-    float m = 0.f;
-    bool nf = false;
+    // largest magnitude as an integer (of floats >= 0 the order is the same, and what is not finite
+    // comes last)
+    uint32_t mi = 0u;
     for (int e = threadIdx.x; e < n_pairs; e += 256) {
         const float2 v = Xb[e];
-        if (!finite(v)) {
-            nf = true;
-            continue;
+        mi = max(mi, max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu));
+    }
+    const bool any_nf = __syncthreads_or(mi >= 0x7f800000u);
+    float m = __uint_as_float(mi);
+    if (any_nf || row_inv) {
+        const int tile_log2 = 31 - __builtin_clz(KI * 64);  // (rows have scales up to 128 elements: KI = 8, 16, 32)
+        m = 0.f;
+        for (int e = threadIdx.x; e < n_pairs; e += 256) {
+            const float2 v = Xb[e];
+            const float ri = row_inv ? row_inv[16 * (e >> tile_log2) + (e & 15)] : 1.0f;
+            m = finite(v) ? fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)) * ri) : m;
         }
-        const float ri = row_inv ? row_inv[16 * (e / (KI * 64)) + (e & 15)] : 1.0f;
-        m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)) * ri);
     }
     red[threadIdx.x] = m;
     __syncthreads();
@@ -1822,7 +1829,6 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
         // mx / scale in [2^14, 2^15); the scale and its reciprocal stay normal numbers
         scale = ldexpf(1.0f, min(max(e2 - 15, -120), 113));
     }
-    const bool any_nf = __syncthreads_or(nf);
     if (any_nf) {
         uint32_t *w = bad + (size_t)b * bad_rows * bad_words;
         for (int i = threadIdx.x; i < bad_rows * bad_words; i += 256) atomicExch(&w[i], 0u);
