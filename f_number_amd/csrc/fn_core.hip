@@ -1506,6 +1506,7 @@ int execute_tangent(fn_plan *P, const void *d_rf, int dtype, float *d_image, flo
             return st;
     }
     fnk::BeamArgs A = split_form ? forward_args(P) : P->args;
+    if (!split_form) A.bad = nullptr;  // no planes in this call
     if (plane_delay(P, mirror)) A.delay = P->d_zeros;
     A.xlp_tiles = mirror ? 2 * P->MT_all : groups * mt;
     A.image = reinterpret_cast<float2 *>(d_image);

@@ -266,3 +266,20 @@ def test_one_f_number(fa, oracle, win):
                                (win, 0.5 if win == "tukey" else 0.0), _oracle_F(oracle, "constant"), "on")
         o.append(np.asarray(img).T)
     _check(imgs[0], imgs[1], o[0] != o[1], 1e-5)
+
+
+@pytest.mark.parametrize("precision", ["bf16x3", "fp16"])
+def test_tangent_beside_another_precision(fa, oracle, precision):
+    """a tangent on FP32 products after a forward call whose samples were not finite"""
+    import torch
+
+    plan, rf = _plan(fa, 3, precision=precision), _rf(3, 12)
+    img, d = (torch.empty((NX, NZ), dtype=torch.complex64, device="cuda") for _ in range(2))
+    bad = rf.copy()
+    bad[1, 30, 40] = np.nan
+    plan.execute(torch.from_numpy(bad).cuda(), img)
+    plan.execute_tangent(torch.from_numpy(rf).cuda(), img, d)
+    torch.cuda.synchronize()
+    ref, _ = oracle.das_pw(X, Z, rf, FS, np.linspace(-0.2, 0.2, 3), WIDTH, PITCH, C0, BAND, 0.0, ("tukey", 0.5),
+                           _oracle_F(oracle, "angle_lb"), "on")
+    assert torch.isfinite(torch.view_as_real(d)).all() and rel_l2(img.cpu().numpy().T, ref) <= 5e-6

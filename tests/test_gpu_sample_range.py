@@ -85,3 +85,22 @@ def test_jobs_of_a_row_stack(fa, n_el, n_ang, win):
             assert rel_l2(g, _eager(p, r)) <= TOL
     assert batch.info()["stacked_plans"] == n
     batch.close()
+
+
+@pytest.mark.parametrize("n_ang", [3, 40])
+def test_channels_of_one_frame(fa, n_ang):
+    """a channel 1e5 louder than the others of its frame (100 dB, below 2^17): the voxels that do
+    not meet its element keep their bits"""
+    import torch
+
+    n_el, n_t, k = 128, 700, 5
+    plan = _plan(fa, n_el, np.linspace(-0.2, 0.2, n_ang), n_t, "tukey")
+    rf = _rf(1, n_ang, n_el, n_t, 6)[0]
+    quiet, only = rf.clone(), torch.zeros_like(rf)
+    quiet[:, k] = 0
+    only[:, k] = rf[:, k] * 1e5
+    apart = np.abs(_eager(plan, only)) == 0
+    assert 0 < apart.sum() < apart.size
+    print(f"case loud channel {n_ang} angles", flush=True)
+    a, b = _eager(plan, quiet + only), _eager(plan, quiet)
+    assert rel_l2(a[apart], b[apart]) <= TOL
