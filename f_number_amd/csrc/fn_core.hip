@@ -227,6 +227,7 @@ struct fn_plan {
     double *d_part = nullptr;   // reduction partials
     int adj_vr = 0, adj_at = 0;
     long tof_serial = 1;                // bumped by every set_tof
+    long tiling_serial = 1;             // bumped by every set_tiling (whose buffers may be others)
     long adj_tab_serial = 0;            // tof_serial the phase tables were built for
     hipStream_t adj_tab_stream = nullptr;  // stream that built them (reuse is ordered only there)
     float *d_vsc = nullptr;                // adjoint normalization s / w_n(v) [n_f][n_vox]
@@ -1388,6 +1389,7 @@ int set_tiling(fn_plan *P, int mt, int split)
     P->lds_beam = lds;
     P->args.tx_group = mt;
     P->args.bin_chunk = chunk;
+    ++P->tiling_serial;
     if (!P->interp_M)
         if (int st = ensure_planes(P, plane_tiles(P))) return st;
     return ensure_partials(P);
@@ -2330,7 +2332,7 @@ struct fn_batch {
     std::vector<const void *> rf;
     std::vector<int32_t> dtypes;
     std::vector<float *> images;
-    std::vector<long> tofs;            // every plan's tof_serial when the graph was captured
+    std::vector<std::pair<long, long>> serials;  // every plan's tof_serial and tiling_serial when the graph was captured
     int captures = 0;
     int64_t n_nodes = 0;
 };
@@ -2645,8 +2647,9 @@ int32_t fn_batch_execute(fn_batch *b, const void *const *d_rf, const int32_t *dt
                       std::equal(b->rf.begin(), b->rf.end(), d_rf) &&
                       std::equal(b->dtypes.begin(), b->dtypes.end(), dtypes) &&
                       std::equal(b->images.begin(), b->images.end(), d_images) &&
-                      std::equal(b->plans.begin(), b->plans.end(), b->tofs.begin(),
-                                 [](const fn_plan *P, long t) { return P->tof_serial == t; });
+                      std::equal(b->plans.begin(), b->plans.end(), b->serials.begin(), [](const fn_plan *P, auto &t) {
+                          return P->tof_serial == t.first && P->tiling_serial == t.second;
+                      });
     if (!same) {
         batch_release_graph(b);
         // eager pass: validates every job and raises kernel LDS limits outside the capture
@@ -2735,8 +2738,8 @@ int32_t fn_batch_execute(fn_batch *b, const void *const *d_rf, const int32_t *dt
         b->rf.assign(d_rf, d_rf + n);
         b->dtypes.assign(dtypes, dtypes + n);
         b->images.assign(d_images, d_images + n);
-        b->tofs.clear();
-        for (const fn_plan *P : b->plans) b->tofs.push_back(P->tof_serial);
+        b->serials.clear();
+        for (const fn_plan *P : b->plans) b->serials.push_back({P->tof_serial, P->tiling_serial});
         b->captures += 1;
     }
     HIP_CHECK(hipGraphLaunch(b->exec, s), "hipGraphLaunch");

@@ -294,7 +294,8 @@ int32_t fn_plan_set_tiling(fn_plan *plan, int32_t m_tiles, int32_t bin_split);
 /* A batch executes many plans (same device) as one hipGraph: the launch
  * sequences of all plans are captured once, spread over n_streams forked
  * streams, and replayed by one graph launch per fn_batch_execute.  The graph
- * is captured again when any buffer pointer differs from the captured ones.
+ * is captured again when any buffer pointer differs from the captured ones,
+ * and after fn_plan_set_tof or fn_plan_set_tiling of any plan.
  * Arrays have one entry per plan; rf_dtypes FN_DTYPE_*; weights may be NULL. */
 typedef struct fn_batch fn_batch;
 int32_t fn_batch_create(fn_plan *const *plans, int32_t n_plans, int32_t n_streams, fn_batch **batch);

@@ -141,3 +141,26 @@ def test_interpolated_plans_in_a_batch(fa, n, n_ang, nx, nz, stacked):
         torch.cuda.synchronize()
         assert rel_l2(g.cpu().numpy(), ref.cpu().numpy()) <= 1e-5
     batch.close()
+
+
+@pytest.mark.parametrize("n_ang,stacking", [(11, False), (40, True)])
+def test_batches_follow_a_new_tiling(fa, n_ang, stacking):
+    """partial images grow with the bin split, in a buffer of their own: a graph that holds the old
+    one is captured again"""
+    import torch
+
+    plan, other = _plan(fa, n_ang), _plan(fa, n_ang)
+    rf = [torch.randn((n_ang, 128, 700), generator=torch.Generator().manual_seed(k)).cuda() for k in (7, 8)]
+    img = [torch.empty((80, 90), dtype=torch.complex64, device="cuda") for _ in range(2)]
+    ref = torch.empty_like(img[0])
+    batch = fa.Batch([plan, other], stacking=stacking)
+    for k, (mt, split) in enumerate([(1, 1), (1, 24), (1, 48), (1, 2)]):
+        plan.set_tiling(mt, split)
+        plan.execute(rf[0], ref)
+        for _ in range(3):
+            img[0].zero_()
+            batch.execute(rf, img)
+            torch.cuda.synchronize()
+            assert rel_l2(img[0].cpu().numpy(), ref.cpu().numpy()) <= 1e-5
+        assert batch.info()["captures"] == k + 1
+    batch.close()
