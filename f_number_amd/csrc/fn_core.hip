@@ -292,7 +292,10 @@ int beam_slots(const fn_plan *P)
 
 int hip_fail(hipError_t e, const char *what)
 {
-    if (e == hipErrorOutOfMemory) return fail(FN_ERR_OUT_OF_MEMORY, "%s: out of device memory", what);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // reported here, not by the next launch
+        return fail(FN_ERR_OUT_OF_MEMORY, "%s: out of device memory", what);
+    }
     return fail(FN_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
@@ -302,17 +305,18 @@ int hip_fail(hipError_t e, const char *what)
         if (e_ != hipSuccess) return hip_fail(e_, what); \
     } while (0)
 
-// partial-image buffer of the plan's tiling (grown, never shrunk; freed with the plan)
+// partial-image buffer of the plan's tiling (grown, never shrunk; freed with the plan); where
+// there is no memory for a larger one the old one stays
 int ensure_partials(fn_plan *P)
 {
     const int slots = beam_slots(P);
     const size_t need = slots > 1 ? (size_t)slots * P->n_vox : 0;
     if (need <= P->pimg_cap) return FN_OK;
     HIP_CHECK(hipSetDevice(P->device), "hipSetDevice");
-    if (P->d_pimg) HIP_CHECK(hipFree(P->d_pimg), "hipFree");  // synchronizes: no launch still reads it
-    P->d_pimg = nullptr;
-    P->pimg_cap = 0;
-    HIP_CHECK(hipMalloc(&P->d_pimg, need * sizeof(float2)), "partial images");
+    float2 *grown = nullptr;
+    HIP_CHECK(hipMalloc(&grown, need * sizeof(float2)), "partial images");
+    hipFree(P->d_pimg);  // synchronizes: no launch still reads it
+    P->d_pimg = grown;
     P->pimg_cap = need;
     return FN_OK;
 }
@@ -1380,19 +1384,22 @@ int set_tiling(fn_plan *P, int mt, int split)
     const int n_f = P->g.n_f;
     if (split < 1 || split > n_f) return fail(FN_ERR_ARGUMENT, "bin_split must be in 1..%d", n_f);
     if (P->nw && split != 1) return fail(FN_ERR_ARGUMENT, "windowed normalization runs with bin_split 1");
-    const size_t lds = (size_t)mt * P->KI * form_step_bytes(P->kprec);
-    if (lds > kMaxLds) return fail(FN_ERR_ARGUMENT, "transmit tile exceeds LDS");
-    const int chunk = (n_f + split - 1) / split;
-    P->MT_tmpl = mt;
-    P->n_groups = P->lbl ? P->n_x : (P->MT_all + mt - 1) / mt;
-    P->bin_split = (n_f + chunk - 1) / chunk;
-    P->lds_beam = lds;
-    P->args.tx_group = mt;
-    P->args.bin_chunk = chunk;
-    ++P->tiling_serial;
-    if (!P->interp_M)
-        if (int st = ensure_planes(P, plane_tiles(P))) return st;
-    return ensure_partials(P);
+    if ((size_t)mt * P->KI * form_step_bytes(P->kprec) > kMaxLds) return fail(FN_ERR_ARGUMENT, "transmit tile exceeds LDS");
+    const int chunk0 = P->args.bin_chunk, mt0 = P->MT_tmpl;
+    auto apply = [P, n_f](int tiles, int chunk) {
+        P->MT_tmpl = tiles;
+        P->n_groups = P->lbl ? P->n_x : (P->MT_all + tiles - 1) / tiles;
+        P->bin_split = (n_f + chunk - 1) / chunk;
+        P->lds_beam = (size_t)tiles * P->KI * form_step_bytes(P->kprec);
+        P->args.tx_group = tiles;
+        P->args.bin_chunk = chunk;
+        ++P->tiling_serial;
+    };
+    apply(mt, (n_f + split - 1) / split);
+    int st = P->interp_M ? FN_OK : ensure_planes(P, plane_tiles(P));
+    if (st == FN_OK) st = ensure_partials(P);
+    if (st != FN_OK) apply(mt0, chunk0);  // no memory: the tiling before, whose buffers are there
+    return st;
 }
 
 int autotune(fn_plan *P, const void *d_rf, int dtype, float *d_image, int reps, fn_tune_result *res, hipStream_t s)

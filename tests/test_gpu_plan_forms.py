@@ -164,3 +164,37 @@ def test_batches_follow_a_new_tiling(fa, n_ang, stacking):
             assert rel_l2(img[0].cpu().numpy(), ref.cpu().numpy()) <= 1e-5
         assert batch.info()["captures"] == k + 1
     batch.close()
+
+
+def test_a_tiling_without_memory_leaves_the_old_one(fa):
+    """planes (476 MB) or partial images that the device has no room for (256 MiB left) refuse the
+    tiling, and the plan goes on with the one it has, bit for bit"""
+    import torch
+
+    n_ang, n_t = 96, 8192
+    x, z = np.linspace(-8e-3, 8e-3, 192) + 1e-3, np.linspace(5e-3, 30e-3, 256)
+    plan = fa.PwPlan(x, z, n_t, 128, np.linspace(-0.2, 0.2, n_ang), FS, WIDTH, PITCH, C0, (1e6, 8e6), 0.0,
+                     window=fa.windows.tukey(0.5), F_number=fa.f_numbers.grating.angle_lb(60, 1.5))
+    rf = torch.randn((n_ang, 128, n_t), generator=torch.Generator(device="cuda").manual_seed(9), device="cuda")
+    ref, img = (torch.empty((192, 256), dtype=torch.complex64, device="cuda") for _ in range(2))
+    plan.execute(rf, ref)
+    torch.cuda.synchronize()
+    before, bins = plan.info(), plan.info()["n_f"]
+    assert bins * 16384 * 10 > 400e6 and 8 * 192 * 256 * bins > 512e6
+    filler = []
+    while (room := torch.cuda.mem_get_info()[0] - (256 << 20)) > (2 << 20):
+        filler.append(torch.empty(min(room, 16 << 30) // (2 << 20) * (2 << 20), dtype=torch.uint8, device="cuda"))
+    for mt, split in ((5, 2), (plan.info()["m_tiles"], bins)):
+        print(f"case no memory {mt} {split}", flush=True)
+        with pytest.raises(Exception, match="memory"):
+            plan.set_tiling(mt, split)
+        assert plan.info() == before
+        plan.execute(rf, img)
+        torch.cuda.synchronize()
+        assert torch.equal(img, ref)
+    del filler
+    torch.cuda.empty_cache()
+    plan.set_tiling(5, 2)
+    plan.execute(rf, img)
+    torch.cuda.synchronize()
+    assert rel_l2(img.cpu().numpy(), ref.cpu().numpy()) <= 1e-5
