@@ -1137,7 +1137,9 @@ int launch_lowp_planes(const fn_plan *P, const float2 *X, void *Xlp, float *xsca
     const fnk::MirrorArgs look = P->tie_later && use_mirror(P) ? mirror_args(P) : fnk::MirrorArgs{};
     if (rowscale)
         if (int st = launch_row_scales(X, rowscale, MT, P->KI, P->g.n_f, s)) return st;
-    const dim3 cg((unsigned)P->g.n_f), cb(256);
+    // a block per bin, and where the grid's mirror is looked at here, one more for each 2048 pairs of voxels
+    const long pairs = look.tie ? (long)(look.n_x / 2) * look.n_z : 0;
+    const dim3 cg((unsigned)P->g.n_f, 1 + (unsigned)std::min<long>(16, (pairs + 2047) / 2048)), cb(256);
     const double fs_over_N = P->args.f_s / P->g.N;
     switch (P->kprec) {
     case FN_PRECISION_FP32: return FN_OK;

@@ -1782,7 +1782,9 @@ static __global__ void row_scale_kernel(const float *__restrict__ peak, float *_
 // the kernels' phase words); the mirrored tiles' weights then stay alike on both sides.
 // Values that are not finite are left out of the scale and written as zeros; the bin's scale is
 // then negative and their elements are noted in bad (spread_nonfinite).  look: whether the grid
-// mirrors at this bin, for one-shot calls (null tie: known).
+// mirrors at this bin, for one-shot calls (null tie: known), by the blocks of blockIdx.y > 0, which
+// run beside the others (128 x 96 voxels: 12.7 us without the look, 18.6 with it, 32.4 in the
+// planes' own blocks).
 template <int PREC>
 __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restrict__ X, void *__restrict__ Xlp,
                                                           float *__restrict__ xscale, int MT_all, int KI,
@@ -1795,6 +1797,13 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
     auto finite = [](float2 v) { return fabsf(v.x) < INFINITY && fabsf(v.y) < INFINITY; };
     __shared__ float red[256];
     const int b = blockIdx.x;
+    if (blockIdx.y > 0) {
+        const long n = (long)(look.n_x / 2) * look.n_z, step = 256L * (gridDim.y - 1);
+        bool off = false;
+        for (long v = 256L * (blockIdx.y - 1) + threadIdx.x; v < n; v += step) off |= mirror_off(look, v, b);
+        if (off) *look.tie = 1u;
+        return;
+    }
     const int n_pairs = MT_all * KI * 64;
     const float2 *Xb = X + (size_t)b * n_pairs;
     // largest magnitude as an integer (of floats >= 0 the order is the same, and what is not finite
@@ -1841,11 +1850,6 @@ __global__ __launch_bounds__(256) void lowp_planes_kernel(const float2 *__restri
         }
     }
     if (threadIdx.x == 0) xscale[b] = any_nf ? -scale : scale;
-    if (look.tie) {
-        bool off = false;
-        for (long v = threadIdx.x; v < (long)(look.n_x / 2) * look.n_z; v += 256) off |= mirror_off(look, v, b);
-        if (off) *look.tie = 1u;
-    }
     const float inv = 1.0f / scale;
     constexpr int pl = Prec<PREC>::planes;
     const int KC = KI / 8;
